@@ -1,7 +1,7 @@
 // dynamics.hip — contact forces and the fused explicit update.
 //
-// k_pair_forces:  one lane per particle pair, the pair's contacts in order,
-//                 both sides (A with the stored normal, B with it negated).
+// k_pair_forces:  one lane per contact, both sides (A with the stored normal,
+//                 B with it negated), then the pair's sums in contact order.
 // k_particle_sum: one lane per particle, its pairs in ascending partner index
 //                 (deterministic, so the step is bit-reproducible).
 // k_integrate:    one wave per particle; every lane recomputes the particle's
@@ -37,52 +37,40 @@ __device__ __forceinline__ void load3(const double* p, int i, double v[3]) {
   v[2] = p[3 * i + 2];
 }
 
+// Orders the wave's LDS writes before its later reads of other lanes' rows.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // np_dev (may be null): the live pair count when npairs is a capacity.
 __device__ __forceinline__ bool past_pairs(int p, int npairs, const long long* np_dev) {
   return p >= npairs || (np_dev && p >= *np_dev);
 }
 
-// Pair p's contact forces on both sides into pf, and its incidence counts
-// when it carries contacts.
-__device__ __forceinline__ void pair_forces_one(const BodiesDev& b, const int* __restrict__ pairs,
-                                                int p, const dh_contact* __restrict__ cs,
-                                                const long long* __restrict__ off,
-                                                const ForceConsts& k, double* __restrict__ pf,
-                                                int* __restrict__ incidence, long long ncap) {
-  const int a = pairs[2 * p], c = pairs[2 * p + 1];
-  double posA[3], angA[3], linA[3], posB[3], angB[3], linB[3];
-  load3(b.pos, a, posA);
-  load3(b.angvel, a, angA);
-  load3(b.linvel, a, linA);
-  load3(b.pos, c, posB);
-  load3(b.angvel, c, angB);
-  load3(b.linvel, c, linB);
-  const double mA = b.mass[a], mB = b.mass[c];
-  double fA[3] = {0, 0, 0}, tA[3] = {0, 0, 0}, fB[3] = {0, 0, 0}, tB[3] = {0, 0, 0};
-  // contacts past the capacity ncap were dropped (reported by the caller)
-  const long long c0 = off[p] < ncap ? off[p] : ncap, c1 = off[p + 1] < ncap ? off[p + 1] : ncap;
-  for (long long i = c0; i < c1; ++i) {
-    const dh_contact& ct = cs[i];
-    const double n[3] = {ct.normal[0], ct.normal[1], ct.normal[2]};
-    const double nn[3] = {-1.0 * ct.normal[0], -1.0 * ct.normal[1], -1.0 * ct.normal[2]};
-    contact_force(ct.x, n, ct.depth, ct.friction != 0, posA, angA, linA, mA, posB, angB, linB, mB,
-                  k, fA, tA);
-    contact_force(ct.x, nn, ct.depth, ct.friction != 0, posB, angB, linB, mB, posA, angA, linA,
-                  mA, k, fB, tB);
-  }
-  double* o = pf + 12 * static_cast<long long>(p);
-  for (int q = 0; q < 3; ++q) {
-    o[q] = fA[q];
-    o[3 + q] = tA[q];
-    o[6 + q] = fB[q];
-    o[9 + q] = tB[q];
-  }
-  if (c1 > c0) {
-    atomicAdd(&incidence[a], 1);
-    atomicAdd(&incidence[c], 1);
-  }
-}
+// Doubles per contact row in LDS: force and torque on A, then on B, one of
+// padding (rows 13 apart put a wave's rows in different banks).
+constexpr int kForceRow = 13;
 
+// Pairs a wave of k_pair_forces takes in lists longer than kForcesFewPairs.
+constexpr int kForcesGroup = 64;
+constexpr int kForcesFewGroup = 4;
+constexpr int kForcesFewPairs = 16384;
+
+// Contact forces of both sides of every pair into pf and, with `incidence`,
+// the particles' counts of contact-carrying pairs.  A wave takes G consecutive
+// pairs, whose contacts are one contiguous range: 64 contacts at a time, a
+// lane evaluates one contact for both sides and leaves its twelve components
+// in LDS, then 64 / G lanes per pair add the pair's rows in contact order (the
+// reference's order, one component per lane and pass).  Evaluating a pair's
+// contacts in one lane, one after the other, left a funnel of 3,900 pairs and
+// 17,000 contacts at 300 us and a lattice of 484 pairs and 14,000 contacts at
+// 120 us: a serial chain of scattered loads, square roots and divisions.
+// G = 4 spreads a short list over the GPU; with more than kForcesFewPairs
+// pairs there are waves enough, and G = 64 fills the lanes of a wave where
+// most pairs carry one contact or none.
+template <int G>
 __global__ __launch_bounds__(256) void k_pair_forces(BodiesDev b, const int* __restrict__ pairs,
                                                      int npairs,
                                                      const dh_contact* __restrict__ cs,
@@ -91,13 +79,85 @@ __global__ __launch_bounds__(256) void k_pair_forces(BodiesDev b, const int* __r
                                                      int* __restrict__ incidence,
                                                      const long long* __restrict__ np_dev,
                                                      long long ncap) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (past_pairs(p, npairs, np_dev)) return;
-  pair_forces_one(b, pairs, p, cs, off, k, pf, incidence, ncap);
+  constexpr int LP = 64 / G;               // lanes per pair in the sums
+  constexpr int NC = (12 + LP - 1) / LP;   // components per lane
+  __shared__ double rows[4][64 * kForceRow];
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  double* row = rows[threadIdx.x >> 6];
+  const int live = np_dev && *np_dev < npairs ? static_cast<int>(*np_dev) : npairs;
+  const int p0 = (static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6)) * G;
+  if (p0 >= live) return;
+  // lane l < G: the first contact of pair p0 + l; contacts past the capacity
+  // ncap were dropped (reported by the caller)
+  const int np = live - p0 < G ? live - p0 : G;
+  auto first = [&](int l) {
+    const long long o = off[p0 + (l < np ? l : np)];
+    return o < ncap ? o : ncap;
+  };
+  const long long lo = first(lane);
+  const long long c0 = __shfl(lo, 0), c1 = first(np);
+  if (c1 <= c0) return;
+  const int beg = static_cast<int>(lo - c0);  // from the group's first contact
+  const int mine = lane / LP, comp = lane % LP;
+  const int pb = __shfl(beg, mine);
+  const int pe = static_cast<int>(first(mine + 1) - c0);
+  double acc[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) acc[q] = 0.0;
+  const int total = static_cast<int>(c1 - c0);
+  for (int base = 0; base < total; base += 64) {
+    const int i = base + lane;
+    // the pair of contact i: the last one that starts at or before it
+    int l = 0;
+#pragma unroll
+    for (int h = G / 2; h > 0; h >>= 1) l = __shfl(beg, l + h) <= i ? l + h : l;
+    if (i < total) {
+      const int p = p0 + l;
+      const int a = pairs[2 * p], c = pairs[2 * p + 1];
+      const dh_contact& ct = cs[c0 + i];
+      double posA[3], angA[3], linA[3], posB[3], angB[3], linB[3];
+      load3(b.pos, a, posA);
+      load3(b.angvel, a, angA);
+      load3(b.linvel, a, linA);
+      load3(b.pos, c, posB);
+      load3(b.angvel, c, angB);
+      load3(b.linvel, c, linB);
+      const double mA = b.mass[a], mB = b.mass[c];
+      const double x[3] = {ct.x[0], ct.x[1], ct.x[2]};
+      const double n[3] = {ct.normal[0], ct.normal[1], ct.normal[2]};
+      const double nn[3] = {-1.0 * n[0], -1.0 * n[1], -1.0 * n[2]};
+      double f[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+      contact_force(x, n, ct.depth, ct.friction != 0, posA, angA, linA, mA, posB, angB, linB, mB,
+                    k, f, f + 3);
+      contact_force(x, nn, ct.depth, ct.friction != 0, posB, angB, linB, mB, posA, angA, linA, mA,
+                    k, f + 6, f + 9);
+#pragma unroll
+      for (int q = 0; q < 12; ++q) row[kForceRow * lane + q] = f[q];
+    }
+    wave_lds_fence();
+    const int r0 = pb > base ? pb - base : 0, r1 = pe < base + 64 ? pe - base : 64;
+    if (NC > 1 || comp < 12) {
+#pragma unroll 4
+      for (int r = r0; r < r1; ++r)
+#pragma unroll
+        for (int q = 0; q < NC; ++q) acc[q] += row[kForceRow * r + NC * comp + q];
+    }
+    wave_lds_fence();
+  }
+  if (mine >= np || pe <= pb) return;
+  if (NC > 1 || comp < 12) {
+    double* o = pf + 12 * static_cast<long long>(p0 + mine) + NC * comp;
+#pragma unroll
+    for (int q = 0; q < NC; ++q) o[q] = acc[q];
+  }
+  if (incidence && comp == 0) {
+    atomicAdd(&incidence[pairs[2 * (p0 + mine)]], 1);
+    atomicAdd(&incidence[pairs[2 * (p0 + mine) + 1]], 1);
+  }
 }
 
 // Pair p's two incidence entries, when it carries contacts (the same test as
-// pair_forces_one's count, offsets clamped to ncap).
+// k_pair_forces' count, offsets clamped to ncap).
 __device__ __forceinline__ void fill_one(const int* __restrict__ pairs, int p,
                                          const long long* __restrict__ off,
                                          const long long* __restrict__ start,
@@ -293,26 +353,26 @@ __global__ __launch_bounds__(256) void k_particle_sum_wide(const int* __restrict
 // force stage in one workgroup.
 constexpr int kForcesSmallN = 1024;
 
-// The whole force stage of a small scene (at most kForcesSmallN particles) in
-// one workgroup, phase by phase: the pairs' forces and incidence counts, the
-// exclusive scan of the counts, the incidence entries, the narrow sums, then
+// The force stage of a small scene (at most kForcesSmallN particles) after
+// k_pair_forces, in one workgroup, phase by phase: the incidence counts, their
+// exclusive scan, the incidence entries, the narrow sums, then
 // the wide particles one after another.  Each phase is the multi-launch
 // path's own code, so the result is the same bit for bit.  The counts, fill
 // cursors and offsets live in LDS (its atomics are the workgroup's own); the
 // global rows and entries are each written once and first read after a
 // barrier.
 __global__ __launch_bounds__(1024) void k_forces_small(
-    BodiesDev b, const int* __restrict__ pairs, int npairs, const long long* __restrict__ np_dev,
-    const dh_contact* __restrict__ cs, const long long* __restrict__ off, ForceConsts k,
-    long long ncap, double* __restrict__ pf, int* __restrict__ entries,
-    double* __restrict__ force, double* __restrict__ torque, int* __restrict__ touched) {
+    int n, const int* __restrict__ pairs, int npairs, const long long* __restrict__ np_dev,
+    const long long* __restrict__ off, long long ncap, const double* __restrict__ pf,
+    int* __restrict__ entries, double* __restrict__ force, double* __restrict__ torque,
+    int* __restrict__ touched) {
   __shared__ long long key[kWideSort];  // the scan's buffer first, then the sort keys
   __shared__ double stage[256 * 6];
   __shared__ long long start[kForcesSmallN + 1];
   __shared__ int cnt[kForcesSmallN];
   __shared__ int fill[kForcesSmallN];  // fill cursors, then the wide particles
   __shared__ int nwide;
-  const int n = b.n, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const int live = np_dev && *np_dev < npairs ? static_cast<int>(*np_dev) : npairs;
   if (tid < kForcesSmallN) {
     cnt[tid] = 0;
@@ -320,7 +380,12 @@ __global__ __launch_bounds__(1024) void k_forces_small(
   }
   if (tid == 0) nwide = 0;
   __syncthreads();
-  for (int p = tid; p < live; p += 1024) pair_forces_one(b, pairs, p, cs, off, k, pf, cnt, ncap);
+  for (int p = tid; p < live; p += 1024) {
+    const long long c0 = off[p] < ncap ? off[p] : ncap, c1 = off[p + 1] < ncap ? off[p + 1] : ncap;
+    if (c1 <= c0) continue;
+    atomicAdd(&cnt[pairs[2 * p]], 1);
+    atomicAdd(&cnt[pairs[2 * p + 1]], 1);
+  }
   __syncthreads();
   // start[0..n) exclusive, start[n] the total
   const long long v = tid < n ? cnt[tid] : 0;
@@ -469,9 +534,18 @@ int contacts_forces_impl(const dh_bodies* bodies, const int* pairs_dev, int npai
   if ((rc = forces_reserve(n, npairs))) return rc;
   const BodiesDev b = to_dev(bodies);
   const ForceConsts k{fp->spring, fp->damper, fp->friction};
-  if (n <= kForcesSmallN) {  // one workgroup, one launch
-    hipLaunchKernelGGL(k_forces_small, 1, 1024, 0, st, b, pairs_dev, npairs, np_dev,
-                       contacts_dev, pair_offset_dev, k, contact_cap, g_fs.pf.as<double>(),
+  auto pair_forces = [&](int* incidence) {
+    if (npairs <= 0) return;
+    const bool few = npairs <= kForcesFewPairs;
+    const auto f = few ? k_pair_forces<kForcesFewGroup> : k_pair_forces<kForcesGroup>;
+    hipLaunchKernelGGL(f, grid_for(npairs, 4 * (few ? kForcesFewGroup : kForcesGroup)), 256, 0, st,
+                       b, pairs_dev, npairs, contacts_dev, pair_offset_dev, k,
+                       g_fs.pf.as<double>(), incidence, np_dev, contact_cap);
+  };
+  if (n <= kForcesSmallN) {  // the pairs' forces, then one workgroup for the rest
+    pair_forces(nullptr);
+    hipLaunchKernelGGL(k_forces_small, 1, 1024, 0, st, n, pairs_dev, npairs, np_dev,
+                       pair_offset_dev, contact_cap, g_fs.pf.as<double>(),
                        g_fs.entries.as<int>(), force_dev, torque_dev, touched_dev);
     DH_HIP_CHECK(hipGetLastError());
     return DH_OK;
@@ -480,12 +554,8 @@ int contacts_forces_impl(const dh_bodies* bodies, const int* pairs_dev, int npai
                           g_fs.wide.as<unsigned>(), nullptr},
                          {n + 1, n + 1, 1, 0}},
              st);
-  if (npairs > 0) {
-    hipLaunchKernelGGL(k_pair_forces, grid_for(npairs, 256), 256, 0, st, b, pairs_dev, npairs,
-                       contacts_dev, pair_offset_dev, k, g_fs.pf.as<double>(),
-                       g_fs.incid.as<int>(), np_dev, contact_cap);
-    DH_HIP_CHECK(hipGetLastError());
-  }
+  pair_forces(g_fs.incid.as<int>());
+  DH_HIP_CHECK(hipGetLastError());
   if ((rc = scan_counts(g_fs.incid.as<int>(), n, g_fs.start.as<long long>(), st))) return rc;
   if (npairs > 0) {
     hipLaunchKernelGGL(k_fill_incidence, grid_for(npairs, 256), 256, 0, st, pairs_dev, npairs,
