@@ -2,8 +2,8 @@
 //
 // k_pair_forces:  one lane per contact, both sides (A with the stored normal,
 //                 B with it negated), then the pair's sums in contact order.
-// k_particle_sum: one lane per particle, its pairs in ascending partner index
-//                 (deterministic, so the step is bit-reproducible).
+// k_particle_sum: eight lanes per particle, its pairs in ascending partner
+//                 index (deterministic, so the step is bit-reproducible).
 // k_integrate:    one wave per particle; every lane recomputes the particle's
 //                 velocity/rotation update (identical arithmetic), lane 0 stores
 //                 it, and the wave rewrites the particle's vertex replicas.
@@ -49,12 +49,34 @@ __device__ __forceinline__ bool past_pairs(int p, int npairs, const long long* n
   return p >= npairs || (np_dev && p >= *np_dev);
 }
 
+// Adds 1 to count[key] for every lane of `has` and returns the lane's own
+// place (the old count plus the lanes before it), with one atomic for each
+// run of equal keys among those lanes: the pairs of a wall follow one another
+// in the list, and an atomic each to the wall's counter serialised them
+// (about 0.1 us each across the XCDs: 32 us for the hopper's busiest wall).
+__device__ __forceinline__ int run_add(bool has, int key, int* count) {
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const unsigned long long mask = __ballot(has), below = (1ull << lane) - 1;
+  const unsigned long long before = mask & below;
+  const int prev = before ? 63 - __clzll(static_cast<long long>(before)) : lane;
+  const int prevkey = __shfl(key, prev);
+  const bool head = has && (!before || prevkey != key);
+  const unsigned long long heads = __ballot(head);
+  const unsigned long long upto = heads & (below | 1ull << lane), after = heads & ~(below | 1ull << lane);
+  const int first = upto ? 63 - __clzll(static_cast<long long>(upto)) : lane;
+  const unsigned long long run = mask & ~((1ull << first) - 1) &
+                                 (after ? (1ull << __builtin_ctzll(after)) - 1 : ~0ull);
+  int base = 0;
+  if (head) base = atomicAdd(&count[key], __popcll(run));
+  return __shfl(base, first) + __popcll(run & below);
+}
+
 // Doubles per contact row in LDS: force and torque on A, then on B, one of
 // padding (rows 13 apart put a wave's rows in different banks).
 constexpr int kForceRow = 13;
 
 // Pairs a wave of k_pair_forces takes in lists longer than kForcesFewPairs.
-constexpr int kForcesGroup = 64;
+constexpr int kForcesGroup = 16;
 constexpr int kForcesFewGroup = 4;
 constexpr int kForcesFewPairs = 16384;
 
@@ -67,9 +89,11 @@ constexpr int kForcesFewPairs = 16384;
 // contacts in one lane, one after the other, left a funnel of 3,900 pairs and
 // 17,000 contacts at 300 us and a lattice of 484 pairs and 14,000 contacts at
 // 120 us: a serial chain of scattered loads, square roots and divisions.
-// G = 4 spreads a short list over the GPU; with more than kForcesFewPairs
-// pairs there are waves enough, and G = 64 fills the lanes of a wave where
-// most pairs carry one contact or none.
+// G = 4 spreads a short list over the GPU (lattice 13.5 us, G = 16 31 us; the
+// funnel's 22 against 51 us); with more than kForcesFewPairs pairs there are
+// waves enough, and G = 16 fills more of a wave's lanes where most pairs
+// carry no contact (hopper of 1.9e5 pairs 52 us, G = 4 75 us; G = 64 71 us:
+// its waves meet up to ten rounds of 64 contacts one after the other).
 template <int G>
 __global__ __launch_bounds__(256) void k_pair_forces(BodiesDev b, const int* __restrict__ pairs,
                                                      int npairs,
@@ -136,7 +160,7 @@ __global__ __launch_bounds__(256) void k_pair_forces(BodiesDev b, const int* __r
     }
     wave_lds_fence();
     const int r0 = pb > base ? pb - base : 0, r1 = pe < base + 64 ? pe - base : 64;
-    if (NC > 1 || comp < 12) {
+    if (NC * comp < 12) {
 #pragma unroll 4
       for (int r = r0; r < r1; ++r)
 #pragma unroll
@@ -144,31 +168,40 @@ __global__ __launch_bounds__(256) void k_pair_forces(BodiesDev b, const int* __r
     }
     wave_lds_fence();
   }
-  if (mine >= np || pe <= pb) return;
-  if (NC > 1 || comp < 12) {
+  const bool any = mine < np && pe > pb;
+  if (any && NC * comp < 12) {
     double* o = pf + 12 * static_cast<long long>(p0 + mine) + NC * comp;
 #pragma unroll
     for (int q = 0; q < NC; ++q) o[q] = acc[q];
   }
-  if (incidence && comp == 0) {
-    atomicAdd(&incidence[pairs[2 * (p0 + mine)]], 1);
-    atomicAdd(&incidence[pairs[2 * (p0 + mine) + 1]], 1);
+  if (incidence) {
+    const bool has = any && comp == 0;
+    const int p = has ? p0 + mine : p0;
+    run_add(has, pairs[2 * p], incidence);
+    run_add(has, pairs[2 * p + 1], incidence);
   }
 }
 
-// Pair p's two incidence entries, when it carries contacts (the same test as
-// k_pair_forces' count, offsets clamped to ncap).
-__device__ __forceinline__ void fill_one(const int* __restrict__ pairs, int p,
-                                         const long long* __restrict__ off,
-                                         const long long* __restrict__ start,
-                                         int* __restrict__ fill, int* __restrict__ entries,
-                                         long long ncap) {
-  const long long c0 = off[p] < ncap ? off[p] : ncap, c1 = off[p + 1] < ncap ? off[p + 1] : ncap;
-  if (c1 <= c0) return;
-  const int a = pairs[2 * p], c = pairs[2 * p + 1];
-  const int ia = atomicAdd(&fill[a], 1);
-  entries[start[a] + ia] = 2 * p;  // side A
-  const int ic = atomicAdd(&fill[c], 1);
+// The two incidence entries of each lane's pair p (p < 0: none), when it
+// carries contacts (the same test as k_pair_forces' count, offsets clamped to
+// ncap).  The whole wave calls it.
+__device__ __forceinline__ void fill_entries(const int* __restrict__ pairs, int p,
+                                             const long long* __restrict__ off,
+                                             const long long* __restrict__ start,
+                                             int* __restrict__ fill, int* __restrict__ entries,
+                                             long long ncap) {
+  bool has = false;
+  int a = -1, c = -1;
+  if (p >= 0) {
+    const long long c0 = off[p] < ncap ? off[p] : ncap, c1 = off[p + 1] < ncap ? off[p + 1] : ncap;
+    has = c1 > c0;
+    a = pairs[2 * p];
+    c = pairs[2 * p + 1];
+  }
+  const int ia = run_add(has, a, fill);
+  const int ic = run_add(has, c, fill);
+  if (!has) return;
+  entries[start[a] + ia] = 2 * p;      // side A
   entries[start[c] + ic] = 2 * p + 1;  // side B
 }
 
@@ -182,12 +215,11 @@ __global__ __launch_bounds__(256) void k_fill_incidence(const int* __restrict__ 
                                                         const long long* __restrict__ np_dev,
                                                         long long ncap) {
   const int p = blockIdx.x * 256 + threadIdx.x;
-  if (past_pairs(p, npairs, np_dev)) return;
-  fill_one(pairs, p, off, start, fill, entries, ncap);
+  fill_entries(pairs, past_pairs(p, npairs, np_dev) ? -1 : p, off, start, fill, entries, ncap);
 }
 
 // Particles with more than this many contact-carrying pairs (walls, floors)
-// are summed by a workgroup each (k_particle_sum_wide); the rest by one lane.
+// are summed by a workgroup each (k_particle_sum_wide); the rest by a few lanes.
 constexpr int kNarrowSum = 64;
 constexpr int kWideSort = 4096;  // entries sorted in LDS
 
@@ -226,6 +258,61 @@ __device__ void sum_by_selection(const int* __restrict__ pairs, const int* __res
   }
 }
 
+// LDS of one narrow sum: the entries, their partners and their order.
+struct NarrowSum {
+  int entry[kNarrowSum], partner[kNarrowSum];
+  unsigned char order[kNarrowSum];
+};
+
+// Particle i's sum over its m <= kNarrowSum entries (from entries[s]) by L >= 6
+// lanes of one wave, `sub` each one's number: the entries are ranked by
+// partner in LDS, then six lanes add one component each in ascending partner
+// order (a partner that comes again is left out, as sum_by_selection does).
+// Selecting the next partner in one lane read the entries and their pairs
+// from memory m times over: 47 us for the lattice's 65 particles.
+template <int L>
+__device__ __forceinline__ void narrow_sum(int i, int m, long long s, int sub,
+                                           const int* __restrict__ pairs,
+                                           const int* __restrict__ entries,
+                                           const double* __restrict__ pf, NarrowSum& w,
+                                           double* __restrict__ force, double* __restrict__ torque,
+                                           int* __restrict__ touched) {
+  for (int e = sub; e < m; e += L) {
+    const int en = entries[s + e];
+    w.entry[e] = en;
+    w.partner[e] = entry_partner(pairs, en);
+  }
+  wave_lds_fence();
+  for (int e = sub; e < m; e += L) {
+    const int mine = w.partner[e];
+    int rank = 0;
+    for (int o = 0; o < m; ++o) {
+      const int q = w.partner[o];
+      rank += (q < mine || (q == mine && o < e)) ? 1 : 0;
+    }
+    w.order[rank] = static_cast<unsigned char>(e);
+  }
+  wave_lds_fence();
+  if (i >= 0 && sub < 6) {
+    double acc = 0.0;
+    int last = -1;
+#pragma unroll 4
+    for (int r = 0; r < m; ++r) {
+      const int e = w.order[r];
+      const double v = entry_forces(pf, w.entry[e])[sub];
+      const int q = w.partner[e];
+      acc = q > last ? acc + v : acc;
+      last = q;
+    }
+    if (sub < 3) force[3 * i + sub] = acc;
+    else torque[3 * i + sub - 3] = acc;
+    if (sub == 0 && touched) touched[i] = m > 0 ? 1 : 0;
+  }
+  wave_lds_fence();  // the next particle's entries go to the same place
+}
+
+constexpr int kSumLanes = 8;  // lanes per particle of k_particle_sum
+
 __global__ __launch_bounds__(256) void k_particle_sum(int n, const int* __restrict__ pairs,
                                                       const long long* __restrict__ start,
                                                       const int* __restrict__ count,
@@ -235,29 +322,16 @@ __global__ __launch_bounds__(256) void k_particle_sum(int n, const int* __restri
                                                       double* __restrict__ torque,
                                                       int* __restrict__ touched,
                                                       int* __restrict__ wide) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  __shared__ NarrowSum sums[256 / kSumLanes];
+  const int i = (blockIdx.x * 256 + threadIdx.x) / kSumLanes;
+  const int sub = threadIdx.x % kSumLanes;
   const int m = i < n ? count[i] : 0;
-  // listed for k_particle_sum_wide (wide[0] entries from wide[1]), each
-  // wave's in particle order
   const bool is_wide = m > kNarrowSum;
-  const unsigned long long wm = __ballot(is_wide);
-  if (wm) {
-    const int lane = static_cast<int>(threadIdx.x & 63), first = __builtin_ctzll(wm);
-    int base = 0;
-    if (lane == first) base = atomicAdd(&wide[0], __popcll(wm));
-    base = __shfl(base, first);
-    const int pre = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(wm >> 32),
-                                              __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(wm), 0));
-    if (is_wide) wide[1 + base + pre] = i;
-  }
-  if (i >= n || is_wide) return;
-  double f[3] = {0.0, 0.0, 0.0}, t[3] = {0.0, 0.0, 0.0};
-  sum_by_selection(pairs, entries, pf, start[i], m, f, t);
-  for (int q = 0; q < 3; ++q) {
-    force[3 * i + q] = f[q];
-    torque[3 * i + q] = t[q];
-  }
-  if (touched) touched[i] = m > 0 ? 1 : 0;
+  // listed for k_particle_sum_wide (wide[0] entries from wide[1])
+  if (is_wide && sub == 0) wide[1 + atomicAdd(&wide[0], 1)] = i;
+  const bool mine = i < n && !is_wide;
+  narrow_sum<kSumLanes>(mine ? i : -1, mine ? m : 0, mine ? start[i] : 0, sub, pairs, entries, pf,
+                        sums[threadIdx.x / kSumLanes], force, torque, touched);
 }
 
 // Particle i's sum over its m > kNarrowSum entries, by the NT threads of a
@@ -267,15 +341,12 @@ __global__ __launch_bounds__(256) void k_particle_sum(int n, const int* __restri
 // each, in ascending partner order: the same order and arithmetic as the
 // narrow sum.  Over kWideSort entries, one lane selects them in order.
 template <int NT>
-__device__ void wide_sum_one(int i, const int* __restrict__ pairs,
-                             const long long* __restrict__ start,
-                             const int* __restrict__ count, const int* __restrict__ entries,
+__device__ void wide_sum_one(int i, const int* __restrict__ pairs, long long s, int m,
+                             const int* __restrict__ entries,
                              const double* __restrict__ pf, double* __restrict__ force,
                              double* __restrict__ torque, int* __restrict__ touched,
                              long long* key, double* stage) {
   const int tid = threadIdx.x;
-  const int m = count[i];
-  const long long s = start[i];
   if (m > kWideSort) {
     if (tid == 0) {
       double f[3] = {0.0, 0.0, 0.0}, t[3] = {0.0, 0.0, 0.0};
@@ -344,9 +415,11 @@ __global__ __launch_bounds__(256) void k_particle_sum_wide(const int* __restrict
   __shared__ long long key[kWideSort];
   __shared__ double stage[256 * 6];
   const int nwide = wide[0];
-  for (int j = blockIdx.x; j < nwide; j += gridDim.x)
-    wide_sum_one<256>(wide[1 + j], pairs, start, count, entries, pf, force, torque, touched, key,
+  for (int j = blockIdx.x; j < nwide; j += gridDim.x) {
+    const int i = wide[1 + j];
+    wide_sum_one<256>(i, pairs, start[i], count[i], entries, pf, force, torque, touched, key,
                       stage);
+  }
 }
 
 // Particles, pairs and contact capacity for which k_forces_small does the
@@ -366,18 +439,19 @@ __global__ __launch_bounds__(1024) void k_forces_small(
     const long long* __restrict__ off, long long ncap, const double* __restrict__ pf,
     int* __restrict__ entries, double* __restrict__ force, double* __restrict__ torque,
     int* __restrict__ touched) {
-  __shared__ long long key[kWideSort];  // the scan's buffer first, then the sort keys
-  __shared__ double stage[256 * 6];
-  __shared__ long long start[kForcesSmallN + 1];
+  // the scan's buffer, then the narrow sums, then the wide sums' keys and rows
+  constexpr int kLanes = 16;  // lanes per narrow sum
+  constexpr int kSmallBytes = kWideSort * 8 + 256 * 6 * 8;
+  __shared__ __align__(16) unsigned char lds[kSmallBytes];
+  __shared__ int start[kForcesSmallN];
   __shared__ int cnt[kForcesSmallN];
   __shared__ int fill[kForcesSmallN];  // fill cursors, then the wide particles
   __shared__ int nwide;
+  static_assert(sizeof(NarrowSum) * (1024 / kLanes) <= kSmallBytes, "narrow sums fit");
   const int tid = threadIdx.x;
   const int live = np_dev && *np_dev < npairs ? static_cast<int>(*np_dev) : npairs;
-  if (tid < kForcesSmallN) {
-    cnt[tid] = 0;
-    fill[tid] = 0;
-  }
+  cnt[tid] = 0;
+  fill[tid] = 0;
   if (tid == 0) nwide = 0;
   __syncthreads();
   for (int p = tid; p < live; p += 1024) {
@@ -387,41 +461,44 @@ __global__ __launch_bounds__(1024) void k_forces_small(
     atomicAdd(&cnt[pairs[2 * p + 1]], 1);
   }
   __syncthreads();
-  // start[0..n) exclusive, start[n] the total
-  const long long v = tid < n ? cnt[tid] : 0;
-  key[tid] = v;
-  __syncthreads();
-  for (int sh = 1; sh < 1024; sh <<= 1) {
-    const long long t = tid >= sh ? key[tid - sh] : 0;
-    __syncthreads();
-    key[tid] += t;
-    __syncthreads();
+  // start[0..n), the exclusive sums of the counts: wave scans, then the waves' sums
+  int* wsum = reinterpret_cast<int*>(lds);
+  const int lane = tid & 63, v = tid < n ? cnt[tid] : 0;
+  int incl = v;
+#pragma unroll
+  for (int sh = 1; sh < 64; sh <<= 1) {
+    const int t = __shfl_up(incl, sh);
+    if (lane >= sh) incl += t;
   }
-  if (tid < n) start[tid] = key[tid] - v;
-  if (tid == 1023) start[n] = key[1023];
+  if (lane == 63) wsum[tid >> 6] = incl;
   __syncthreads();
-  for (int p = tid; p < live; p += 1024) fill_one(pairs, p, off, start, fill, entries, ncap);
+  for (int w = 0; w < (tid >> 6); ++w) incl += wsum[w];
+  if (tid < n) start[tid] = incl - v;
+  __syncthreads();
+  for (int p = tid; p < live; p += 1024) {
+    const long long c0 = off[p] < ncap ? off[p] : ncap, c1 = off[p + 1] < ncap ? off[p + 1] : ncap;
+    if (c1 <= c0) continue;
+    const int a = pairs[2 * p], c = pairs[2 * p + 1];
+    entries[start[a] + atomicAdd(&fill[a], 1)] = 2 * p;      // side A
+    entries[start[c] + atomicAdd(&fill[c], 1)] = 2 * p + 1;  // side B
+  }
   __syncthreads();
   int* wide = fill;  // the cursors are spent
-  for (int i = tid; i < n; i += 1024) {
-    const int m = cnt[i];
-    if (m > kNarrowSum) {
-      wide[atomicAdd(&nwide, 1)] = i;
-      continue;
-    }
-    double f[3] = {0.0, 0.0, 0.0}, t[3] = {0.0, 0.0, 0.0};
-    sum_by_selection(pairs, entries, pf, start[i], m, f, t);
-    for (int q = 0; q < 3; ++q) {
-      force[3 * i + q] = f[q];
-      torque[3 * i + q] = t[q];
-    }
-    if (touched) touched[i] = m > 0 ? 1 : 0;
+  NarrowSum* sums = reinterpret_cast<NarrowSum*>(lds);
+  for (int i0 = 0; i0 < n; i0 += 1024 / kLanes) {
+    const int i = i0 + tid / kLanes, sub = tid % kLanes;
+    const int m = i < n ? cnt[i] : 0;
+    if (m > kNarrowSum && sub == 0) wide[atomicAdd(&nwide, 1)] = i;
+    const bool mine = i < n && m <= kNarrowSum;
+    narrow_sum<kLanes>(mine ? i : -1, mine ? m : 0, mine ? start[i] : 0, sub, pairs, entries, pf,
+                       sums[tid / kLanes], force, torque, touched);
   }
   __syncthreads();
   const int nw = nwide;
+  long long* key = reinterpret_cast<long long*>(lds);
   for (int j = 0; j < nw; ++j)
-    wide_sum_one<1024>(wide[j], pairs, start, cnt, entries, pf, force, torque, touched, key,
-                       stage);
+    wide_sum_one<1024>(wide[j], pairs, start[wide[j]], cnt[wide[j]], entries, pf, force, torque,
+                       touched, key, reinterpret_cast<double*>(key + kWideSort));
 }
 
 struct Gravity {
@@ -564,7 +641,7 @@ int contacts_forces_impl(const dh_bodies* bodies, const int* pairs_dev, int npai
     DH_HIP_CHECK(hipGetLastError());
   }
   if (n > 0) {
-    hipLaunchKernelGGL(k_particle_sum, grid_for(n, 256), 256, 0, st, n, pairs_dev,
+    hipLaunchKernelGGL(k_particle_sum, grid_for(static_cast<int64_t>(n) * kSumLanes, 256), 256, 0, st, n, pairs_dev,
                        g_fs.start.as<long long>(), g_fs.incid.as<int>(), g_fs.entries.as<int>(),
                        g_fs.pf.as<double>(), force_dev, torque_dev, touched_dev,
                        g_fs.wide.as<int>());
