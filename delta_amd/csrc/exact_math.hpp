@@ -211,15 +211,18 @@ DH_HD void vertex_face(T& ptmin, T& ss, T& tt, int& id, const V3<T>& f0, const V
   id = better ? j : id;
 }
 
-// bfSolver: closest points P on A and Q on B.  Returns true when the
-// edge-edge result is kept (ptmin > ssmin, bf.cpp:1102).  With kZoltan the
-// output stage is that of zoltan/bf.cpp, whose switch cases 1 fall through
-// into cases 2 (zoltan/bf.cpp:527-559, 907-925): edge-edge feature 1 takes
-// its Q from B's edge 2->0 with feature 1's parameter, vertex-face feature 1
-// reports B's vertex 2.
-template <typename T, bool kZoltan = false>
-DH_HD bool bf_solver_ids(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q, int& ssid_out,
-                         int& id_out) {
+// The least edge-edge distance of a triangle pair (feature ssid, parameters
+// ssc on A's edge and ttc on B's) and the least vertex-face distance (feature
+// id, face parameters ss and tt).
+template <typename T>
+struct BfBest {
+  T ssmin, ttc, ssc, ptmin, ss, tt;
+  int ssid, id;
+};
+
+// The features of bfSolver for any input.
+template <typename T>
+DH_HD void bf_features(const Tri<T>& A, const Tri<T>& B, BfBest<T>& best) {
   T ssmin = T(1E+30), ttc = T(0), ssc = T(0);
   int ssid = 0;
   // Edge k of a triangle runs from its origin v[(k+1)%3] towards v[k].  The
@@ -268,9 +271,253 @@ DH_HD bool bf_solver_ids(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q, i
       p2 = tp;
     }
   }
+  best = {ssmin, ttc, ssc, ptmin, ss, tt, ssid, id};
+}
+
+// ---- the same features with fewer instructions, for regular pairs
+//
+// One pair per lane is bound by the instructions it issues, and the general
+// form above spends most of its own on selects, on moving the rotating
+// vertices and on the scaling that a division and a square root need for
+// extreme exponents.  bf_features_regular unrolls the features (edges, their
+// squared lengths and the faces' terms are formed once), clamps the
+// parameters instead of selecting among the clamped cases, and divides and
+// takes roots without scaling.  Every value that reaches a result is the same
+// operation on the same operands, so the results are the same bit for bit.
+// Regular means that no intermediate value leaves the range in which that
+// holds: squared edge lengths (and a face's third one, as the face's formula
+// has it) of at least 1e-30, so that a clamped parameter's numerator and
+// denominator are not taken for zero, face determinants of at least 1e-60,
+// and squared lengths and one squared distance of less than 2^180, so that
+// nothing overflows (a NaN fails that test).  MI355X, 2^24 pairs: 2,807 to about
+// 2,170 vector instructions per wave of 64 pairs, 1.467 to 1.198 ms.
+
+// a / b, correctly rounded, for 2^-400 < |a|, |b| < 2^400 (other operands: any
+// value): the reciprocal by two Newton steps, the quotient by one residual.
+DH_HD double div_regular(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(fma(-b, y, 1.0), y, y);
+  y = fma(fma(-b, y, 1.0), y, y);
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+#else
+  return a / b;
+#endif
+}
+
+// sqrt(x), correctly rounded, for x >= 2^-700 (else `ok` is cleared): by
+// Goldschmidt's iteration and two residual corrections.
+DH_HD double sqrt_regular(double x, bool& ok) {
+  ok &= x >= 0x1p-700;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  return fma(fma(-g, g, x), h, g);
+#else
+  return std::sqrt(x);
+#endif
+}
+
+// q in [0, 1] (the clamp of an instruction's result).
+DH_HD double clamp01(double q) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return fmin(fmax(q, 0.0), 1.0);
+#else
+  return q > 0.0 ? (q < 1.0 ? q : 1.0) : 0.0;
+#endif
+}
+
+// segseg and the distance for edges u (squared length a) and v (c) of a
+// regular pair, w from v's origin to u's.  The s-range's clamps are the
+// clamp of sN / D; only parallel edges that keep their t need a zero of
+// their own.
+DH_HD double edge_edge_regular(const V3<double>& u, double a, const V3<double>& v, double c,
+                               const V3<double>& w, double& sc, double& tc, bool& ok) {
+  using std::fabs;
+  const double small_num = 1E-30;
+  const double b = dot(u, v), d = dot(u, w), e = dot(v, w);
+  const double D = a * c - b * b;
+  const double sN = b * e - c * d;
+  const bool par = D < small_num;
+  const bool s_hi = !par && sN > D;
+  const bool edge = par || sN < 0.0 || s_hi;
+  const double eb = e + b, t0 = a * e - b * d, bd = b - d, nd = -d;
+  const double te = s_hi ? eb : e;
+  const double tN = edge ? te : t0;
+  const double tD = edge ? c : D;
+  const bool tlo = tN < 0.0, clamp = tlo || tN > tD;
+  const double x = tlo ? nd : bd;
+  const double num = clamp ? x : sN, den = clamp ? a : D;
+  const double qs = clamp01(div_regular(num, den));
+  const double qt = clamp01(div_regular(tN, tD));
+  sc = (fabs(num) < small_num || (par && !clamp)) ? 0.0 : qs;
+  tc = (fabs(tN) < small_num) ? 0.0 : qt;
+  const V3<double> dP = {w.x + (sc * u.x) - (tc * v.x), w.y + (sc * u.y) - (tc * v.y),
+                         w.z + (sc * u.z) - (tc * v.z)};
+  return sqrt_regular(dP.x * dP.x + dP.y * dP.y + dP.z * dP.z, ok);
+}
+
+// The terms of a face that its three points share.
+struct FaceTerms {
+  V3<double> o, e0, e1;
+  double a, b, c, det, denom;
+  DH_HD explicit FaceTerms(const Tri<double>& t)
+      : o(t.v[0]), e0(sub(t.v[1], t.v[0])), e1(sub(t.v[2], t.v[0])), a(dot(e0, e0)),
+        b(dot(e0, e1)), c(dot(e1, e1)), det(a * c - b * b), denom(a - 2.0 * b + c) {}
+};
+
+// pt_tri and the distance for a regular face: the face parameters are
+// (s0, t0) / det inside, and on the boundary one clamped quotient: along
+// t = 0, along s = 0, or along s + t = 1.  pt_tri's sums for the three
+// corners are its quadratic form at (0, 0), (1, 0) and (0, 1) term by term,
+// so only the two edges t = 0 and s = 0 have a form of their own.
+DH_HD double vertex_face_regular(const FaceTerms& f, const V3<double>& pt, double& s, double& t,
+                                 bool& ok) {
+  const V3<double> dd = sub(f.o, pt);
+  const double d = dot(f.e0, dd), e = dot(f.e1, dd), ff = dot(dd, dd);
+  const double a = f.a, b = f.b, c = f.c;
+  const double s0 = b * e - c * d, t0 = b * d - a * e;
+  const bool in = (s0 + t0) <= f.det, sneg = s0 < 0.0, tneg = t0 < 0.0, dneg = d < 0.0;
+  const double bd = b + d, be = b + e, ce = c + e, ad = a + d;
+  const bool gt2 = ce > bd, gt6 = ad > be;
+  const bool r0 = in && !sneg && !tneg;
+  const bool r1 = !in && !sneg && !tneg, r2 = !in && sneg, r6 = !in && !sneg && tneg;
+  const bool useE = (in && sneg && !(tneg && dneg)) || (r2 && !gt2);
+  const bool useD = (in && tneg && (!sneg || dneg)) || (r6 && !gt6);
+  const bool hyp6 = r6 && gt6;
+  const double h1 = ce - b - d, h2 = ce - bd, h6 = ad - be, ne = -e, nd = -d;
+  double num = r2 ? h2 : h6, den = f.denom;
+  num = r1 ? h1 : num;
+  num = useD ? nd : num;
+  den = useD ? a : den;
+  num = useE ? ne : num;
+  den = useE ? c : den;
+  num = r0 ? 1.0 : num;
+  den = r0 ? f.det : den;
+  const double q = num / den;
+  const double p = clamp01(q), p1 = 1.0 - p;
+  const double si = s0 * q, ti = t0 * q;
+  s = hyp6 ? p1 : p;
+  t = hyp6 ? p : p1;
+  t = useD ? 0.0 : t;
+  s = useE ? 0.0 : s;
+  t = useE ? p : t;
+  s = r0 ? si : s;
+  t = r0 ? ti : t;
+  const double quad = s * (a * s + b * t + 2.0 * d) + t * (b * s + c * t + 2.0 * e) + ff;
+  const double line = (useE ? e : d) * p + ff;
+  const double sqr = ((useE || useD) && num < den) ? line : quad;
+  return sqrt_regular(fmax(sqr, 0.0), ok);
+}
+
+// Forgets what the compiler has derived from a triangle's first vertex, so
+// that it forms the faces' terms again after the edges instead of keeping
+// them in registers meanwhile.
+DH_HD void forget_derived(Tri<double>& t) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(t.v[0].x), "+v"(t.v[0].y), "+v"(t.v[0].z));
+#endif
+}
+
+DH_HD void feature_fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// The features of a regular pair; false (and nothing in `best`) for others.
+DH_HD bool bf_features_regular(Tri<double> A, Tri<double> B, BfBest<double>& best) {
+  bool ok = true;
+  double least = 1E300, sum = 0.0;
+  double ssmin = 1E+30, ssc = 0.0, ttc = 0.0, ptmin = 1E+30, ss = 0.0, tt = 0.0;
+  int ssid = 0, id = 0;
+  V3<double> v[3];
+  double c[3];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    v[m] = sub(B.v[m], B.v[m == 2 ? 0 : m + 1]);
+    c[m] = dot(v[m], v[m]);
+    least = fmin(least, c[m]);
+    sum = sum + c[m];
+  }
+  // A's vertices rotate through a loop that stays rolled (three turns put
+  // them back), B's edges are unrolled
+#pragma unroll 1
+  for (int k = 0; k < 9; k += 3) {
+    const V3<double> u = sub(A.v[0], A.v[1]);
+    const double a = dot(u, u);
+    least = fmin(least, a);
+    sum = sum + a;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      feature_fence();
+      const V3<double> w = sub(A.v[1], B.v[m == 2 ? 0 : m + 1]);
+      double sc, tc;
+      const double dist = edge_edge_regular(u, a, v[m], c[m], w, sc, tc, ok);
+      const bool better = dist < ssmin;
+      ssmin = better ? dist : ssmin;
+      ssc = better ? sc : ssc;
+      ttc = better ? tc : ttc;
+      ssid = better ? k + m : ssid;
+    }
+    const V3<double> t = A.v[0];
+    A.v[0] = A.v[1];
+    A.v[1] = A.v[2];
+    A.v[2] = t;
+  }
+  forget_derived(A);
+  forget_derived(B);
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    const FaceTerms face(f ? B : A);
+    least = fmin(least, face.denom);
+    ok &= face.det >= 1E-60;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      feature_fence();
+      double s, t;
+      const double dist = vertex_face_regular(face, f ? A.v[j] : B.v[j], s, t, ok);
+      const bool better = dist < ptmin;
+      ptmin = better ? dist : ptmin;
+      ss = better ? s : ss;
+      tt = better ? t : tt;
+      id = better ? 3 * f + j : id;
+    }
+  }
+  best = {ssmin, ttc, ssc, ptmin, ss, tt, ssid, id};
+  const V3<double> ab = sub(A.v[0], B.v[0]);
+  return ok && least >= 1E-30 && sum + dot(ab, ab) < 0x1p180;
+}
+
+DH_HD void bf_features_any(const Tri<double>& A, const Tri<double>& B, BfBest<double>& best) {
+  if (!bf_features_regular(A, B, best)) bf_features(A, B, best);
+}
+
+DH_HD void bf_features_any(const Tri<float>& A, const Tri<float>& B, BfBest<float>& best) {
+  bf_features(A, B, best);
+}
+
+// bfSolver: closest points P on A and Q on B.  Returns true when the
+// edge-edge result is kept (ptmin > ssmin, bf.cpp:1102).  With kZoltan the
+// output stage is that of zoltan/bf.cpp, whose switch cases 1 fall through
+// into cases 2 (zoltan/bf.cpp:527-559, 907-925): edge-edge feature 1 takes
+// its Q from B's edge 2->0 with feature 1's parameter, vertex-face feature 1
+// reports B's vertex 2.
+template <typename T, bool kZoltan = false>
+DH_HD bool bf_solver_ids(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q, int& ssid_out,
+                         int& id_out) {
+  BfBest<T> best;
+  bf_features_any(A, B, best);
+  const int ssid = best.ssid, id = best.id;
+  const T ssc = best.ssc, ttc = best.ttc, ss = best.ss, tt = best.tt;
   ssid_out = ssid;
   id_out = id;
-  if (ptmin > ssmin) {
+  if (best.ptmin > best.ssmin) {
     const int k = ssid / 3, m = (kZoltan && ssid == 1) ? 2 : ssid - 3 * (ssid / 3);
     // register selects instead of dynamic indexing (keeps Tri out of scratch)
     const V3<T> ha = pick3(A, k), oa = pick3(A, k == 2 ? 0 : k + 1);

@@ -152,3 +152,17 @@ def test_exact_mode_flags_generated_intersections(gen_batch):
     assert hit[kind == 2].mean() > 0.99
     assert not hit[kind != 2].any()
     assert (d[hit] == 0).all()
+
+
+def test_brute_force_at_its_edges():
+    """bfSolver on the GPU against the oracle where its cases change (the sets
+    of the host test): the regular pairs' divisions, roots and clamps equal
+    the general ones bit for bit, and the other pairs take the general path."""
+    from test_hostcheck import bf_edge_sets, same_bits
+    for name, soa in bf_edge_sets(20000):
+        b = narrow.PairBatch.from_host(soa)
+        b.run("bf64")
+        P, Q, d, f = b.results()
+        Po, Qo, do, fo = oracle_pairs(0, soa)
+        assert same_bits(d, do) and same_bits(P.ravel(), Po.ravel()), name
+        assert same_bits(Q.ravel(), Qo.ravel()) and np.array_equal(f, fo), name

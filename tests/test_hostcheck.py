@@ -347,3 +347,63 @@ def test_device_sincos_is_correctly_rounded(hc):
     hc.hc_cr_sincos(ol.dptr(xs), C.c_long(n), ol.dptr(s), ol.dptr(c))
     ms = np.array([math.sin(v) for v in xs]); mc = np.array([math.cos(v) for v in xs])
     assert np.mean(s == ms) > 0.995 and np.mean(c == mc) > 0.995
+
+
+def bf_edge_sets(n, seed=5):
+    """Triangle pairs where bfSolver's cases change: small whole numbers (ties,
+    parallel and collinear edges, degenerate faces, signed zeros), coordinates
+    of any scale, slivers, shared vertices, NaN and infinities."""
+    rng = np.random.default_rng(seed)
+    ints = lambda k: rng.integers(-k, k + 1, (18, n)).astype(float)
+    uni = lambda: rng.uniform(0, 1e-3, (18, n))
+    yield "whole numbers", ints(2)
+    yield "more whole numbers", ints(9)
+    yield "signed zeros", np.where(rng.random((18, n)) < 0.3, -0.0, ints(2))
+    near = ints(3) + rng.normal(0, 1, (18, n)) * 10.0 ** rng.uniform(-18, -3, n)
+    yield "near whole numbers", near
+    for k in (160, 60, 20):
+        yield f"scaled to 1e{k}", near * 10.0 ** rng.uniform(-k, k, n)
+        yield f"coordinates to 1e{k}", rng.normal(0, 1, (18, n)) * 10.0 ** rng.uniform(-k, k, (18, n))
+    for bad in (np.nan, np.inf):
+        x = uni()
+        x[rng.random((18, n)) < 0.03] = bad
+        yield f"{bad}", x
+    x, at = uni(), rng.integers(0, 3, n)
+    for c in range(3):
+        x[9 + 3 * c] = np.where(at == 0, x[3 * c], x[9 + 3 * c])
+    yield "shared vertex", x
+    x, e, l = uni(), 10.0 ** rng.uniform(-22, -3, n), rng.uniform(-1, 2, n)
+    for c in range(3):
+        x[3 * c + 2] = x[3 * c + 1] + rng.normal(0, 1, n) * e
+    yield "slivers", x
+    x = uni()
+    for c in range(3):
+        x[3 * c + 2] = x[3 * c] + l * (x[3 * c + 1] - x[3 * c])
+    yield "collinear", x
+    x = uni()
+    for c in range(3):
+        x[9 + 3 * c + 1] = x[9 + 3 * c] + l * (x[3 * c + 1] - x[3 * c])
+    yield "parallel edges", x
+    # squared lengths about the least one of the regular pairs' path
+    yield "edges of 1e-15", ints(3) * 2.0 ** -50
+    yield "edges of 2e-15", ints(3) * 2.0 ** -49
+
+
+def same_bits(a, b):
+    return np.all((a.view(np.uint64) == b.view(np.uint64)) | (np.isnan(a) & np.isnan(b)))
+
+
+def test_brute_force_at_its_edges(hc):
+    """The host build's bfSolver, whose regular pairs take a path of their own,
+    equals the oracle bit for bit where its cases change."""
+    n = 20000
+    for name, s in bf_edge_sets(n):
+        s = np.ascontiguousarray(s)
+        outs = []
+        for lib, fn in ((ol.oracle(), "or_tri_pairs"), (hc, "hc_tri_pairs")):
+            P = np.zeros(3 * n); Q = np.zeros(3 * n); d = np.zeros(n); f = np.zeros(n, np.uint8)
+            getattr(lib, fn)(0, ol.dptr(s), C.c_long(n), C.c_double(2e-4), ol.dptr(P),
+                             ol.dptr(Q), ol.dptr(d), f.ctypes.data_as(C.c_void_p))
+            outs.append((P, Q, d, f))
+        assert all(same_bits(a, b) for a, b in zip(outs[0][:3], outs[1][:3])), name
+        assert np.array_equal(outs[0][3], outs[1][3]), name
