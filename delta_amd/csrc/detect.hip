@@ -35,10 +35,11 @@ constexpr int kChunkFlags = 1024;  // chunks of 64 rows an item tests up front
 
 enum DetectError : int { DE_NONE = 0, DE_REF_UB = 1, DE_TOO_LONG = 2 };
 
-// Per-tile counters (tile_stats) and the stats slot each one is summed into.
+// Per-tile counters (tile_stats) and the stats slot each one is summed into;
+// DH_BF keeps the first kBfStats only.
 enum TileStat : int {
-  TS_CHECKS = 0, TS_EVALUATED, TS_FALLBACK_ROWS, TS_PENALTY_FAILS, TS_BATCH_FAILS,
-  TS_BATCH_SIZE, TS_CULLED, kTileStats
+  TS_CHECKS = 0, TS_EVALUATED, TS_CULLED, kBfStats,
+  TS_FALLBACK_ROWS = kBfStats, TS_PENALTY_FAILS, TS_BATCH_FAILS, TS_BATCH_SIZE, kTileStats
 };
 
 enum StatSlot : int {
@@ -93,48 +94,67 @@ struct DetectArgs {
   // B's particle box are not loaded; a block without a near chunk is
   // skipped.
   const double* bbox;
-  // Survivor queue (null: every item solves its own survivors).  A staged
-  // single-block DH_BF item whose survivors all fit in its LDS list appends
-  // them {item, iA | iB << 16} as one contiguous range and records its start
-  // in qbase[item]; when the range does not fit in qcap entries, the item
-  // fills the part inside with {-1, 0} and solves its survivors itself.
-  int2* queue;
-  long long qcap;
-  unsigned long long* qcounter;
-  long long* qbase;
-  // Mid-phase-only launches (no solver in the kernel) append the items they
-  // cannot queue here; a second launch runs those items in full, taking its
-  // items from item_list.
+  int nstats;  // counters per tile: kBfStats (DH_BF) or kTileStats
+  // Survivor queue of a DH_BF launch (null: every item solves its own
+  // survivors).  Wave r of k_detect_wave appends its items' survivors to its
+  // own region queue[r * rcap ..] and leaves their number in rcount[r], so
+  // that no wave waits for a counter that all share.  An item of k_detect_big
+  // appends to bqueue (which follows the regions) through bcounter, as one range that it lists
+  // ({first, length, item, contacts}); a range that does not fit in bcap
+  // entries is filled with item -1 as far as it lies inside.  An item that
+  // cannot queue goes to `deferred`, for a second launch that runs those items
+  // in full, taking its items from item_list.
+  int4* queue;  // {item, triangle of A, triangle of B, iA | iB << 16}
+  int rcap, regions;
+  int* rcount;
+  int* rwant;  // [0]: most entries that a region had to hold, when more than rcap
+  int4* bqueue;
+  int bcap;
+  unsigned* bcounter;
+  int4* ranges;
+  unsigned* nranges;
+  // contacts of the queue's entries, in the entries' order, from the place of
+  // the region's or range's first entry; region r's number in
+  // rcount[regions + r], a range's in the range
+  struct QueueRecord* rec;
   int* deferred;
   unsigned* ndeferred;
-  // Items k_detect_wave takes for their rows' test but cannot stage (B has
-  // more than kWaveRows triangles) and does not cull: k_detect_big runs them.
+  // Items for k_detect_big: rows or columns that k_detect_wave does not take
   int* biglist;
   unsigned* nbig;
-  // Items k_lane_cull leaves for k_detect_wave (with wlist, k_detect_wave
-  // takes its items from this list, *nwlist long).
-  int* wlist;
+  // Items k_lane_cull leaves for k_detect_wave
+  struct WaveItem* wlist;
   unsigned* nwlist;
   const int* item_list;
   const unsigned* nitems_dev;  // with item_list: its length (else the launch's)
   int fp32_screen;             // k_queue_solve screens in binary32 first
-  int wave_items;              // small items go to k_detect_wave (mid-phase only)
   // item_skip[item] != 0: k_chunk_cull culled the item and wrote its
   // counters (a launch of DH_BF without the survivor queue skips it)
   const unsigned char* item_skip;
 };
 
-// Items of a mid-phase-only launch small enough for one wave each.
-constexpr int kWaveRows = 80;       // rows and columns staged per wave
-constexpr int kWaveSurvivors = 256; // survivors listed per wave
-__device__ __forceinline__ bool wave_item(int nrows, int nA, int nB) {
-  return nrows <= kWaveRows && nB <= kWaveRows && nA < 65536;
-}
-// Items whose rows k_detect_wave tests against B's particle box (a larger B,
-// such as a wall against a small particle, is often culled there).
-__device__ __forceinline__ bool wave_rows(int nrows, int nA, int nB) {
-  return nrows <= kWaveRows && nA < 65536 && nB < 65536;
-}
+// Items of the queue path that take one wave each: at most kWaveScan rows and
+// columns, of which at most kWaveRows each stay after the tests against the
+// other particle (their boxes are held in LDS).
+constexpr int kWaveScan = 320;
+constexpr int kWaveRows = 80;
+constexpr int kWaveSurvivors = 256;  // survivors listed per wave
+constexpr int kWavesPerGroup = 2;    // of k_detect_wave
+
+struct WaveItem {
+  int item, pa, pb;
+  int tA, tB;      // first triangles of the rows and of B
+  int r0, nrows;   // rows [r0, r0 + nrows) of A
+  int nB;
+  double epsA, epsB;
+};
+
+struct QueueRecord {
+  int item, tris;  // iA | iB << 16
+  int rank;        // among the item's contacts
+  int pad_;
+  double pq[6];
+};
 
 __device__ __forceinline__ Tri<double> load_tri(const DetectArgs& g, int t) {
   Tri<double> r;
@@ -312,11 +332,11 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
   const int k = item / g.tiles, tile = item - k * g.tiles;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * kTileStats;
+  unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * g.nstats;
   if (M == DH_BF && !QONLY && g.item_skip && g.item_skip[item]) return;  // k_chunk_cull's
   if (g.npairs_dev && k >= *g.npairs_dev) {
     if (tid == 0) g.tile_count[item] = 0;
-    if (tid < kTileStats) ts[tid] = 0;
+    if (tid < g.nstats) ts[tid] = 0;
     return;
   }
   const Pair p = load_pair(g, k);
@@ -328,13 +348,13 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
   if (M == DH_HYBRID_TRIANGLE && p.nB > p.nA) {
     if (tid == 0) atomicCAS(g.error, DE_NONE, static_cast<int>(DE_REF_UB));
     if (tid == 0) g.tile_count[item] = 0;
-    if (tid < kTileStats) ts[tid] = 0;
+    if (tid < g.nstats) ts[tid] = 0;
     return;
   }
   if ((is_hybrid || is_rowstat) && (rows > kMaxRowTriangles || p.nB > kMaxRowTriangles)) {
     if (tid == 0) atomicCAS(g.error, DE_NONE, static_cast<int>(DE_TOO_LONG));
     if (tid == 0) g.tile_count[item] = 0;
-    if (tid < kTileStats) ts[tid] = 0;
+    if (tid < g.nstats) ts[tid] = 0;
     return;
   }
   // this workgroup's rows [r0, r1)
@@ -453,14 +473,18 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
     const bool staged = p.nB <= kBoxTriangles;  // block-uniform
     const int blk = staged ? kBoxTriangles : (nrows > 0 ? nrows : 1);
     bool b_staged = false;  // B's boxes are loaded on the first block that needs them
-    long long q_first = 0;  // the item's queue range, when a block appended one
+    int q_first = 0;  // the item's queue range, when a block appended one
     int q_len = 0;
     // mid-phase-only launch: an item that cannot queue its survivors is
     // handed to the full launch (which also writes its counters)
     auto defer = [&]() {
       if (tid == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = item;
     };
-    if (QONLY && g.wave_items && wave_item(nrows, p.nA, p.nB)) return;  // k_detect_wave's
+    // an item that defers after one of its blocks has appended its range
+    auto void_range = [&]() {
+      for (int q = q_first + tid; q < q_first + q_len; q += 256)
+        g.bqueue[q] = make_int4(-1, 0, 0, 0);
+    };
     if (QONLY && !(staged && p.nA < 65536 && p.nB < 65536)) {
       defer();
       return;
@@ -632,46 +656,45 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
           __syncthreads();
         }
         if (QONLY && fpos < tested) {  // more survivors than the LDS list holds
+          void_range();
           defer();
           return;
         }
-        if (g.queue && first && fpos >= tested && staged && p.nA < 65536 && p.nB < 65536 &&
-            !(nl > 0 && q_len > 0)) {
+        if (QONLY && first && fpos >= tested && staged && !(nl > 0 && q_len > 0)) {
           // every survivor of the block is in LDS: append them, in row-major
           // order, as the item's one range of the survivor queue (solved
-          // there with every lane busy); the item solves them itself if they
-          // do not fit
-          if (tid == 0 && nl > 0)
-            chunk_base = atomicAdd(g.qcounter, static_cast<unsigned long long>(nl));
+          // there with every lane busy)
+          if (tid == 0 && nl > 0) chunk_base = atomicAdd(g.bcounter, static_cast<unsigned>(nl));
           __syncthreads();
-          const long long qb = nl > 0 ? static_cast<long long>(chunk_base) : 0;
+          const unsigned qb = nl > 0 ? static_cast<unsigned>(chunk_base) : 0u;
           __syncthreads();
-          if (qb + nl <= g.qcap) {
+          if (static_cast<long long>(qb) + nl <= g.bcap) {
             if (nl > 0) {
-              q_first = qb;
+              q_first = static_cast<int>(qb);
               q_len = nl;
+              if (tid == 0)
+                g.ranges[atomicAdd(g.nranges, 1u)] = make_int4(q_first, q_len, item, 0);
             }
-            if (tid == 0 && nl > 0) g.qbase[item] = qb;
             for (int e = tid; e < nl; e += 256) {
               int iA, iB;
               pair_of(surv[e], iA, iB);
-              g.queue[qb + e] = make_int2(
-                  item, static_cast<int>(static_cast<unsigned>(iA) | (static_cast<unsigned>(iB) << 16)));
+              g.bqueue[qb + e] = make_int4(
+                  item, p.oA + iA, p.oB + iB,
+                  static_cast<int>(static_cast<unsigned>(iA) | (static_cast<unsigned>(iB) << 16)));
             }
-            continue;  // fpos >= tested: the item is done
+            continue;  // fpos >= tested: the block is done
           }
-          for (long long q = qb + tid; q < qb + nl && q < g.qcap; q += 256)
-            g.queue[q] = make_int2(-1, 0);
-          if (QONLY) {
-            defer();
-            return;
-          }
+          for (long long q = static_cast<long long>(qb) + tid; q < static_cast<long long>(qb) + nl &&
+                                                               q < g.bcap; q += 256)
+            g.bqueue[q] = make_int4(-1, 0, 0, 0);
+          void_range();
+          defer();
+          return;
         }
-        if (QONLY && nl > 0 && q_len > 0) {
+        if (QONLY && nl > 0) {
           // a second block with survivors: the item's survivors would not
           // be one range; void the first and run the item in full
-          for (long long q = q_first + tid; q < q_first + q_len; q += 256)
-            g.queue[q] = make_int2(-1, 0);
+          void_range();
           defer();
           return;
         }
@@ -775,11 +798,13 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
         (is_hybrid ? local_stats[0] * static_cast<unsigned long long>(p.nB) : 0ull);
     ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
     ts[TS_EVALUATED] = evals;
-    ts[TS_FALLBACK_ROWS] = is_hybrid ? local_stats[0] : 0ull;
-    ts[TS_PENALTY_FAILS] = is_rowstat ? local_stats[1] : 0ull;
-    ts[TS_BATCH_FAILS] = is_rowstat ? local_stats[2] : 0ull;
-    ts[TS_BATCH_SIZE] = is_rowstat ? static_cast<unsigned long long>(nrows) * p.nB : 0ull;
     ts[TS_CULLED] = M == DH_BF ? local_stats[3] : 0ull;
+    if (M != DH_BF) {
+      ts[TS_FALLBACK_ROWS] = is_hybrid ? local_stats[0] : 0ull;
+      ts[TS_PENALTY_FAILS] = is_rowstat ? local_stats[1] : 0ull;
+      ts[TS_BATCH_FAILS] = is_rowstat ? local_stats[2] : 0ull;
+      ts[TS_BATCH_SIZE] = is_rowstat ? static_cast<unsigned long long>(nrows) * p.nB : 0ull;
+    }
   }
 }
 
@@ -801,44 +826,13 @@ __attribute__((amdgpu_waves_per_eu(M == DH_BF && !QONLY ? 3 : 1))) void k_detect
   }
 }
 
-// The workgroup mid-phase for the items k_detect_wave leaves (larger ones):
-// the first wave classifies 64 items at a time, one per lane, and the
-// workgroup runs the larger live ones, in order.
-__global__ __launch_bounds__(256) void k_detect_big(DetectArgs g, int items) {
-  __shared__ int list[64];
-  __shared__ int nlist;
-  const int tid = threadIdx.x;
-  for (int base = blockIdx.x * 64; base < items; base += gridDim.x * 64) {
-    if (tid < 64) {
-      const int item = base + tid;
-      bool big = false;
-      if (item < items) {
-        const int k = item / g.tiles, tile = item - k * g.tiles;
-        if (!(g.npairs_dev && k >= *g.npairs_dev)) {
-          const int pa = g.pairs[2 * k], pb = g.pairs[2 * k + 1];
-          const int nA = g.tri_offset[pa + 1] - g.tri_offset[pa];
-          const int nB = g.tri_offset[pb + 1] - g.tri_offset[pb];
-          const int r0 = static_cast<int>(static_cast<long long>(tile) * nA / g.tiles);
-          const int r1 = static_cast<int>(static_cast<long long>(tile + 1) * nA / g.tiles);
-          big = !wave_rows(r1 - r0, nA, nB);
-        }
-      }
-      const unsigned long long m = __ballot(big);
-      if (big) list[lane_prefix(m)] = item;
-      if (tid == 0) nlist = __popcll(m);
-    }
-    __syncthreads();
-    const int n = nlist;
-    for (int j = 0; j < n; ++j) {
-      detect_item<DH_BF, true>(g, list[j]);
-      __syncthreads();  // the next item reuses the workgroup's LDS
-    }
-  }
-  // then the items k_detect_wave (launched before) handed over
+// The workgroup mid-phase for the items that k_detect_wave does not take (listed
+// by k_lane_cull) or hands over.
+__global__ __launch_bounds__(256) void k_detect_big(DetectArgs g) {
   const int nb = static_cast<int>(*g.nbig);
   for (int j = blockIdx.x; j < nb; j += gridDim.x) {
     detect_item<DH_BF, true>(g, g.biglist[j]);
-    __syncthreads();
+    __syncthreads();  // the next item reuses the workgroup's LDS
   }
 }
 
@@ -856,13 +850,13 @@ __global__ __launch_bounds__(256) void k_chunk_cull(DetectArgs g, int items,
   for (int item = static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6);
        item < items; item += nw) {
     const int k = item / g.tiles, tile = item - k * g.tiles;
-    unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * kTileStats;
+    unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * g.nstats;
     if (g.npairs_dev && k >= *g.npairs_dev) {
       if (lane == 0) {
         g.tile_count[item] = 0;
         skip[item] = 1;
       }
-      if (lane < kTileStats) ts[lane] = 0;
+      if (lane < g.nstats) ts[lane] = 0;
       continue;
     }
     const Pair p = load_pair(g, k);
@@ -902,10 +896,6 @@ __global__ __launch_bounds__(256) void k_chunk_cull(DetectArgs g, int items,
         g.tile_count[item] = 0;
         ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
         ts[TS_EVALUATED] = total;
-        ts[TS_FALLBACK_ROWS] = 0;
-        ts[TS_PENALTY_FAILS] = 0;
-        ts[TS_BATCH_FAILS] = 0;
-        ts[TS_BATCH_SIZE] = 0;
         ts[TS_CULLED] = total;
       }
     }
@@ -915,278 +905,280 @@ __global__ __launch_bounds__(256) void k_chunk_cull(DetectArgs g, int items,
 // Rows a lane tests alone in k_lane_cull.
 constexpr int kLaneRows = 16;
 
-// One lane per item, before k_detect_wave: an item of k_detect_wave's whose
-// particles' bounding spheres are apart by more than the margin (diagonal
-// neighbours in a packing), or with at most kLaneRows rows whose rows' boxes
-// all miss B's particle box (grown by the margin: a wall of few triangles
-// against the many particles inside it), is culled here, with the counters
-// k_detect_wave would write; the other items of k_detect_wave's are listed
-// for it.
-__global__ __launch_bounds__(256) void k_lane_cull(DetectArgs g, int items) {
-  const int item = blockIdx.x * 256 + static_cast<int>(threadIdx.x);
-  bool listed = false;
+// One lane per item, before k_detect_wave: an item whose particles' bounding
+// spheres are apart by more than the margin (diagonal neighbours in a
+// packing), or with at most kLaneRows rows whose rows' boxes all miss B's
+// particle box (grown by the margin: a wall of few triangles against the many
+// particles inside it), is culled here, with the counters the mid-phase would
+// write.  The others are listed for k_detect_wave with what it needs of them
+// (its loads of triangles then wait for one load, not for three in a row), or,
+// above kWaveScan rows or columns, for k_detect_big.  One atomic per workgroup
+// and list: one per wave took most of the 43 us that the hopper's 3.8e5 items
+// spent here.
+__global__ __launch_bounds__(1024) void k_lane_cull(DetectArgs g, int items) {
+  __shared__ unsigned wave_cnt[2][16], base[2];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int item = blockIdx.x * 1024 + tid;
+  const int wave = tid >> 6;
+  int list = -1;  // 0: k_detect_wave, 1: k_detect_big
+  WaveItem it = {};
   if (item < items) {
     const int k = item / g.tiles, tile = item - k * g.tiles;
-    unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * kTileStats;
-    if (g.npairs_dev && k >= *g.npairs_dev) {
-      g.tile_count[item] = 0;
-      for (int q = 0; q < kTileStats; ++q) ts[q] = 0;
-    } else {
+    unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * g.nstats;
+    g.tile_count[item] = 0;
+    if (!(g.npairs_dev && k >= *g.npairs_dev)) {
       const Pair p = load_pair(g, k);
       const int r0 = static_cast<int>(static_cast<long long>(tile) * p.nA / g.tiles);
       const int r1 = static_cast<int>(static_cast<long long>(tile + 1) * p.nA / g.tiles);
       const int nrows = r1 - r0;
-      if (wave_rows(nrows, p.nA, p.nB)) {
-        bool near = !(g.pbox && nrows <= kLaneRows);
-        if (spheres_apart(g, p)) {
-          near = false;  // culled whole
-        } else if (!near) {
-          const double* pb = g.pbox + 6 * static_cast<long long>(p.pb);
-          for (int t = 0; t < nrows && !near; ++t) {
-            double lo[3], hi[3];
-            tri_box(load_tri(g, p.oA + r0 + t), lo, hi);
-            near = !boxes_apart(lo, hi, pb, pb + 3, p.margin);
+      const unsigned long long total = static_cast<unsigned long long>(nrows) * p.nB;
+      bool near = !(g.pbox && nrows <= kLaneRows);
+      if (spheres_apart(g, p)) {
+        near = false;  // culled whole
+      } else if (!near) {
+        const double* pb = g.pbox + 6 * static_cast<long long>(p.pb);
+        for (int t = 0; t < nrows && !near; ++t) {
+          double lo[3], hi[3];
+          tri_box(load_tri(g, p.oA + r0 + t), lo, hi);
+          near = !boxes_apart(lo, hi, pb, pb + 3, p.margin);
+        }
+      }
+      if (near && total > 0)
+        list = nrows <= kWaveScan && p.nB <= kWaveScan && p.nA < 65536 ? 0 : 1;
+      ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
+      ts[TS_EVALUATED] = total;
+      ts[TS_CULLED] = total;  // a listed item's own kernel writes its count
+      it = {item, p.pa, p.pb, p.oA + r0, p.oB, r0, nrows, p.nB, p.epsA, p.epsB};
+    }
+  }
+  const unsigned long long m0 = __ballot(list == 0), m1 = __ballot(list == 1);
+  if ((tid & 63) == 0) {
+    wave_cnt[0][wave] = static_cast<unsigned>(__popcll(m0));
+    wave_cnt[1][wave] = static_cast<unsigned>(__popcll(m1));
+  }
+  __syncthreads();
+  if (tid < 2) {
+    unsigned n = 0;
+    for (int w = 0; w < 16; ++w) {
+      const unsigned c = wave_cnt[tid][w];
+      wave_cnt[tid][w] = n;
+      n += c;
+    }
+    base[tid] = n ? atomicAdd(tid == 0 ? g.nwlist : g.nbig, n) : 0u;
+  }
+  __syncthreads();
+  if (list == 0) g.wlist[base[0] + wave_cnt[0][wave] + lane_prefix(m0)] = it;
+  if (list == 1) g.biglist[base[1] + wave_cnt[1][wave] + lane_prefix(m1)] = item;
+}
+
+// Orders a wave's LDS writes before its later reads of other lanes' values.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The largest gap between two boxes along an axis.
+__device__ __forceinline__ double box_gap(const double* loA, const double* hiA, const double* loB,
+                                          const double* hiB) {
+  double gap = -INFINITY;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) gap = fmax(gap, fmax(loB[q] - hiA[q], loA[q] - hiB[q]));
+  return gap;
+}
+
+// The mid-phase of DH_BF, one wave per listed item and no workgroup barrier:
+// the boxes of A's rows and B's columns that lie within the margin of the
+// other particle's box and bounding sphere are kept, in order, in the wave's
+// LDS; the pairs of kept rows and columns whose boxes are within the margin
+// are listed in row-major order and appended to the wave's region of the
+// survivor queue.  Items with more than kWaveRows kept rows or columns go to
+// k_detect_big, items whose survivors overflow the list or the region to the
+// full kernel.  Same survivors and counters as detect_item's box test.
+// It is bound by the latency of an item's loads, so it holds little: 16 waves
+// per CU (LDS) at the 128 registers that allow them.  Separating axes are
+// tested in k_queue_solve instead, with every lane busy (here they took 161
+// registers, 9 waves per CU, for some 10 to 40 survivors at a time), and the
+// other particle's box from the broad phase takes the place of the union of
+// its triangles' boxes (144 lane shuffles per item).  What it cost before was
+// an atomic per item on one queue counter, some 10 ns each: 610 us for the
+// hopper's 1.9e5 pairs, 87 us with a region per wave (8 workgroups per CU; 6
+// per CU: 100 us).
+__global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectArgs g) {
+  __shared__ double boxes[kWavesPerGroup][2 * kWaveRows * 6];
+  __shared__ unsigned short act[kWavesPerGroup][2 * kWaveRows];
+  __shared__ unsigned short surv[kWavesPerGroup][kWaveSurvivors];  // row << 8 | column, both kept
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  double* bx = boxes[w];
+  const int region = blockIdx.x * kWavesPerGroup + w;
+  int4* queue = g.queue + static_cast<long long>(region) * g.rcap;
+  int used = 0, want = 0;
+  const int nw = static_cast<int>(*g.nwlist);
+  for (int j = region; j < nw; j += gridDim.x * kWavesPerGroup) {
+    const WaveItem it = g.wlist[j];
+    const double margin = it.epsA + it.epsB;
+    // what the rows (side 0) and the columns (side 1) are tested against: the
+    // other particle's box, and how much of the margin lies in it already
+    double other[2][6], in[2] = {0.0, 0.0};
+    if (g.pbox) {
+      in[0] = it.epsB;
+      in[1] = it.epsA;
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        other[0][q] = g.pbox[6 * static_cast<long long>(it.pb) + q];
+        other[1][q] = g.pbox[6 * static_cast<long long>(it.pa) + q];
+      }
+    } else {  // the unions of the triangles' boxes
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        const int n = side == 0 ? it.nB : it.nrows, t0 = side == 0 ? it.tB : it.tA;
+        double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (int t = lane; t < n; t += 64) {
+          double l[3], h[3];
+          tri_box(load_tri(g, t0 + t), l, h);
+          for (int q = 0; q < 3; ++q) {
+            lo[q] = fmin(lo[q], l[q]);
+            hi[q] = fmax(hi[q], h[q]);
           }
         }
-        if (near) {
-          listed = true;
-        } else {
-          const unsigned total = static_cast<unsigned>(nrows * p.nB);
-          g.tile_count[item] = 0;
-          ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
-          ts[TS_EVALUATED] = total;
-          ts[TS_FALLBACK_ROWS] = 0;
-          ts[TS_PENALTY_FAILS] = 0;
-          ts[TS_BATCH_FAILS] = 0;
-          ts[TS_BATCH_SIZE] = 0;
-          ts[TS_CULLED] = total;
+        for (int o = 32; o > 0; o >>= 1)
+          for (int q = 0; q < 3; ++q) {
+            lo[q] = fmin(lo[q], __shfl_xor(lo[q], o));
+            hi[q] = fmax(hi[q], __shfl_xor(hi[q], o));
+          }
+        for (int q = 0; q < 3; ++q) {
+          other[side][q] = lo[q];
+          other[side][3 + q] = hi[q];
         }
       }
     }
+    // boxes apart by more than `reach` along an axis: boxes_apart's test with
+    // the largest coordinate of either particle in its rounding band
+    double mag = 0.0;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) mag = fmax(mag, fmax(fabs(other[0][q]), fabs(other[1][q])));
+    const double reach = margin * (1.0 + 0x1p-20) + mag * 0x1p-40;
+    int kept[2] = {0, 0};
+    bool handed = false;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const int n = side == 0 ? it.nrows : it.nB, t0 = side == 0 ? it.tA : it.tB;
+      const double* sph =
+          g.psph ? g.psph + 4 * static_cast<long long>(side == 0 ? it.pb : it.pa) : nullptr;
+      const double far = reach + mag * 0x1p-40 - in[side];
+      int c = 0;
+      for (int b = 0; b < n && !handed; b += 64) {
+        const int t = b + lane;
+        double lo[3], hi[3];
+        tri_box(load_tri(g, t0 + (t < n ? t : n - 1)), lo, hi);
+        const bool on = t < n && !(box_gap(lo, hi, other[side], other[side] + 3) > far) &&
+                        !(sph && box_sphere_apart(lo, hi, sph, margin));
+        const unsigned long long m = __ballot(on);
+        const int at = c + lane_prefix(m);
+        c += __popcll(m);
+        if (c > kWaveRows) {
+          handed = true;
+        } else if (on) {
+          double* d = bx + 6 * (side * kWaveRows + at);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            d[q] = lo[q];
+            d[3 + q] = hi[q];
+          }
+          act[w][side * kWaveRows + at] = static_cast<unsigned short>(t);
+        }
+      }
+      kept[side] = c;
+      if (c == 0) break;
+    }
+    if (handed) {
+      if (lane == 0) g.biglist[atomicAdd(g.nbig, 1u)] = it.item;
+      continue;
+    }
+    wave_lds_fence();
+    const int na = kept[0], nc = kept[1], tested = na * nc;
+    // survivors in row-major order over the kept rows and columns
+    int S = 0;
+    if (tested > 0) {
+      const int step_r = 64 / nc, step_c = 64 - step_r * nc;
+      int ra = lane / nc, cb = lane - ra * nc;
+      for (int f = lane; f - lane < tested; f += 64) {
+        bool keep = false;
+        if (f < tested) {
+          const double* a = bx + 6 * ra;
+          const double* b = bx + 6 * (kWaveRows + cb);
+          keep = !(box_gap(a, a + 3, b, b + 3) > reach);
+        }
+        const unsigned long long m = __ballot(keep);
+        const int at = S + lane_prefix(m);
+        if (keep && at < kWaveSurvivors) surv[w][at] = static_cast<unsigned short>(ra << 8 | cb);
+        S += __popcll(m);
+        ra += step_r;
+        cb += step_c;
+        if (cb >= nc) {
+          cb -= nc;
+          ++ra;
+        }
+      }
+    }
+    wave_lds_fence();
+    bool deferred = S > kWaveSurvivors;
+    if (!deferred) {
+      want += S;
+      deferred = used + S > g.rcap;
+    }
+    if (deferred) {
+      if (lane == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = it.item;
+    } else {
+      for (int e = lane; e < S; e += 64) {
+        const int v = surv[w][e];
+        const int r = act[w][v >> 8], c = act[w][kWaveRows + (v & 255)];
+        queue[used + e] = make_int4(it.item, it.tA + r, it.tB + c, (it.r0 + r) | c << 16);
+      }
+      used += S;
+      if (lane == 0)
+        g.tile_stats[static_cast<long long>(it.item) * g.nstats + TS_CULLED] =
+            static_cast<unsigned long long>(it.nrows) * it.nB - S;
+    }
+    wave_lds_fence();  // the next item overwrites the wave's LDS
   }
-  const unsigned long long m = __ballot(listed);
-  if (m) {
-    unsigned base = 0;
-    if ((threadIdx.x & 63) == static_cast<unsigned>(__builtin_ctzll(m)))
-      base = atomicAdd(g.nwlist, static_cast<unsigned>(__popcll(m)));
-    base = __shfl(base, __builtin_ctzll(m));
-    if (listed) g.wlist[base + lane_prefix(m)] = item;
+  if (lane == 0) {
+    g.rcount[region] = used;
+    if (want > g.rcap) atomicMax(g.rwant, want);
   }
 }
 
-// The mid-phase of DH_BF for small items, one wave per item and no
-// workgroup barrier: A's rows and B's columns (at most kWaveRows each)
-// staged as boxes in the wave's LDS, rows apart from B's particle box
-// dropped (an item with a larger B that this test does not cull goes to
-// k_detect_big), rows and columns prefiltered against the other side's union,
-// the surviving pairs listed in row-major order and appended to the
-// survivor queue as one range.  Items whose survivors overflow the list or
-// the queue are deferred to the full kernel.  Same tests, order and
-// counters as detect_item's queue path.
-__global__ __launch_bounds__(128) void k_detect_wave(DetectArgs g, int items) {
-  constexpr int kW = 2;  // waves per workgroup
-  __shared__ double boxes[kW][2 * kWaveRows * 6];
-  __shared__ unsigned char act[kW][2 * kWaveRows];
-  __shared__ int surv[kW][kWaveSurvivors];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  double* bx = boxes[w];
-  const int nw = g.wlist ? static_cast<int>(*g.nwlist) : items;
-  for (int j = blockIdx.x * kW + w; j < nw; j += gridDim.x * kW) {
-    const int item = g.wlist ? g.wlist[j] : j;
-    const int k = item / g.tiles, tile = item - k * g.tiles;
-    unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * kTileStats;
-    if (g.npairs_dev && k >= *g.npairs_dev) {
-      if (lane == 0) g.tile_count[item] = 0;
-      if (lane < kTileStats) ts[lane] = 0;
-      continue;
-    }
-    const Pair p = load_pair(g, k);
-    const int r0 = static_cast<int>(static_cast<long long>(tile) * p.nA / g.tiles);
-    const int r1 = static_cast<int>(static_cast<long long>(tile + 1) * p.nA / g.tiles);
-    const int nrows = r1 - r0;
-    if (!wave_rows(nrows, p.nA, p.nB)) continue;  // the workgroup kernel's
-    const int total = nrows * p.nB;
-    unsigned culled = 0;  // lane 0's count is the item's
-    const double* pb = g.pbox ? g.pbox + 6 * static_cast<long long>(p.pb) : nullptr;
-    // rows: boxes, and the test against B's particle box
-    bool near = false;
-    for (int t = lane; t < nrows; t += 64) {
-      double* b = bx + 6 * t;
-      tri_box(load_tri(g, p.oA + r0 + t), b, b + 3);
-      if (pb) near = near || !boxes_apart(b, b + 3, pb, pb + 3, p.margin);
-    }
-    int S = 0;
-    bool deferred = false;
-    if (pb && !__ballot(near)) {
-      culled = total;
-    } else if (p.nB > kWaveRows) {
-      if (lane == 0) g.biglist[atomicAdd(g.nbig, 1u)] = item;
-      continue;
-    } else {
-      for (int t = lane; t < p.nB; t += 64) {
-        double* b = bx + 6 * (kWaveRows + t);
-        tri_box(load_tri(g, p.oB + t), b, b + 3);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      // unions of the rows' and of B's boxes
-      double u[12];
-      for (int q = 0; q < 3; ++q) {
-        u[q] = u[6 + q] = INFINITY;
-        u[3 + q] = u[9 + q] = -INFINITY;
-      }
-      for (int t = lane; t < nrows; t += 64)
-        for (int q = 0; q < 3; ++q) {
-          u[q] = fmin(u[q], bx[6 * t + q]);
-          u[3 + q] = fmax(u[3 + q], bx[6 * t + 3 + q]);
-        }
-      for (int t = lane; t < p.nB; t += 64)
-        for (int q = 0; q < 3; ++q) {
-          u[6 + q] = fmin(u[6 + q], bx[6 * (kWaveRows + t) + q]);
-          u[9 + q] = fmax(u[9 + q], bx[6 * (kWaveRows + t) + 3 + q]);
-        }
-      for (int o = 32; o > 0; o >>= 1)
-        for (int q = 0; q < 12; ++q) {
-          const double v = __shfl_xor(u[q], o);
-          u[q] = ((q % 6) < 3) ? fmin(u[q], v) : fmax(u[q], v);
-        }
-      // ordered active rows and columns: boxes that meet the other side's
-      // union and are not apart from its particle's bounding sphere
-      int na = 0, nc = 0;
-      for (int side = 0; side < 2; ++side) {
-        const int cnt_all = side == 0 ? nrows : p.nB;
-        const double* other = u + 6 * (1 - side);
-        const double* osph =
-            g.psph ? g.psph + 4 * static_cast<long long>(side == 0 ? p.pb : p.pa) : nullptr;
-        int n_on = 0;
-        for (int t0 = 0; t0 < cnt_all; t0 += 64) {
-          const int t = t0 + lane;
-          bool on = false;
-          if (t < cnt_all) {
-            const double* b = bx + 6 * (side == 0 ? t : kWaveRows + t);
-            on = !boxes_apart(b, b + 3, other, other + 3, p.margin) &&
-                 !(osph && box_sphere_apart(b, b + 3, osph, p.margin));
-          }
-          const unsigned long long m = __ballot(on);
-          if (on) act[w][side * kWaveRows + n_on + lane_prefix(m)] = static_cast<unsigned char>(t);
-          n_on += __popcll(m);
-        }
-        if (side == 0) na = n_on; else nc = n_on;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const int tested = na * nc;
-      culled = static_cast<unsigned>(total - tested);
-      // survivors in row-major order over the active rows and columns
-      for (int f0 = 0; f0 < tested; f0 += 64) {
-        const int fe = f0 + lane;
-        bool keep = false;
-        if (fe < tested) {
-          const int ra = fe / nc, cb = fe - ra * nc;
-          const double* a = bx + 6 * act[w][ra];
-          const double* b = bx + 6 * (kWaveRows + act[w][kWaveRows + cb]);
-          keep = !boxes_apart(a, a + 3, b, b + 3, p.margin);
-        }
-        const unsigned long long m = __ballot(keep);
-        if (keep && S + lane_prefix(m) < kWaveSurvivors) surv[w][S + lane_prefix(m)] = fe;
-        S += __popcll(m);
-        culled += static_cast<unsigned>(__popcll(__ballot(fe < tested && !keep)));
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (S > 0 && S <= kWaveSurvivors) {
-        // survivors that a triangle plane or an edge-pair axis separates by
-        // more than the margin emit nothing (k_queue_solve's first test):
-        // only the rest are queued, compacted in place in row-major order
-        int S2 = 0;
-        for (int e0 = 0; e0 < S; e0 += 64) {
-          const int e = e0 + lane;
-          int fe = 0;
-          bool keep = false;
-          if (e < S) {
-            fe = surv[w][e];
-            const int ra = fe / nc, cb = fe - ra * nc;
-            keep = !axes_apart(load_tri(g, p.oA + r0 + act[w][ra]),
-                               load_tri(g, p.oB + act[w][kWaveRows + cb]), p.margin);
-          }
-          const unsigned long long m = __ballot(keep);
-          if (keep) surv[w][S2 + lane_prefix(m)] = fe;
-          S2 += __popcll(m);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        S = S2;
-      }
-      if (S > kWaveSurvivors) {
-        deferred = true;
-      } else if (S > 0) {
-        unsigned long long qb0 = 0;
-        if (lane == 0) qb0 = atomicAdd(g.qcounter, static_cast<unsigned long long>(S));
-        const long long qb = static_cast<long long>(__shfl(qb0, 0));
-        if (qb + S <= g.qcap) {
-          if (lane == 0) g.qbase[item] = qb;
-          for (int e = lane; e < S; e += 64) {
-            const int fe = surv[w][e];
-            const int ra = fe / nc, cb = fe - ra * nc;
-            const int iA = r0 + act[w][ra], iB = act[w][kWaveRows + cb];
-            g.queue[qb + e] = make_int2(
-                item, static_cast<int>(static_cast<unsigned>(iA) | (static_cast<unsigned>(iB) << 16)));
-          }
-        } else {
-          for (long long q = qb + lane; q < qb + S && q < g.qcap; q += 64)
-            g.queue[q] = make_int2(-1, 0);
-          deferred = true;
-        }
-      }
-      // the next item overwrites the wave's LDS
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    if (deferred) {
-      if (lane == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = item;
-      continue;
-    }
-    if (lane == 0) {
-      g.tile_count[item] = 0;
-      ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
-      ts[TS_EVALUATED] = static_cast<unsigned long long>(total);
-      ts[TS_FALLBACK_ROWS] = 0;
-      ts[TS_PENALTY_FAILS] = 0;
-      ts[TS_BATCH_FAILS] = 0;
-      ts[TS_BATCH_SIZE] = 0;
-      ts[TS_CULLED] = culled;
-    }
-  }
+// The stats slot of a tile counter.
+__device__ __forceinline__ int stat_slot(int q) {
+  const int slot[kTileStats] = {ST_CHECKS, ST_EVALUATED, ST_CULLED, ST_FALLBACK_ROWS,
+                                ST_PENALTY_FAILS, ST_BATCH_FAILS, ST_BATCH_SIZE};
+  return slot[q];
 }
 
 // Sums of the per-tile counters into the stats slots (one atomic per
 // workgroup and counter).
+template <int N>
 __global__ __launch_bounds__(256) void k_tile_stats(const unsigned long long* __restrict__ ts,
-                                                    long long ntiles,
+                                                    long long npairs, int tiles,
+                                                    const long long* __restrict__ npairs_dev,
                                                     unsigned long long* __restrict__ stats) {
-  __shared__ unsigned long long red[kTileStats];
-  if (threadIdx.x < kTileStats) red[threadIdx.x] = 0;
+  __shared__ unsigned long long red[N];
+  if (threadIdx.x < N) red[threadIdx.x] = 0;
   __syncthreads();
-  unsigned long long acc[kTileStats] = {};
+  const long long ntiles = (npairs_dev && *npairs_dev < npairs ? *npairs_dev : npairs) * tiles;
+  unsigned long long acc[N] = {};
   for (long long t = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; t < ntiles;
        t += static_cast<long long>(gridDim.x) * 256)
-    for (int q = 0; q < kTileStats; ++q) acc[q] += ts[t * kTileStats + q];
-  for (int q = 0; q < kTileStats; ++q) {
+    for (int q = 0; q < N; ++q) acc[q] += ts[t * N + q];
+  for (int q = 0; q < N; ++q) {
     unsigned long long v = acc[q];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     if ((threadIdx.x & 63) == 0 && v) atomicAdd(&red[q], v);
   }
   __syncthreads();
-  if (threadIdx.x < kTileStats && red[threadIdx.x]) {
-    const int slot[kTileStats] = {ST_CHECKS, ST_EVALUATED, ST_FALLBACK_ROWS, ST_PENALTY_FAILS,
-                                  ST_BATCH_FAILS, ST_BATCH_SIZE, ST_CULLED};
-    atomicAdd(&stats[slot[threadIdx.x]], red[threadIdx.x]);
-  }
+  if (threadIdx.x < N && red[threadIdx.x])
+    atomicAdd(&stats[stat_slot(threadIdx.x)], red[threadIdx.x]);
 }
 
 // The tail of a captured detection over at most kTailPairs pairs, in one
@@ -1196,19 +1188,22 @@ __global__ __launch_bounds__(256) void k_tile_stats(const unsigned long long* __
 // sums with the total at offs[npairs] (as scan_counts).
 constexpr int kTailPairs = 4096;
 
+template <int N>
 __global__ __launch_bounds__(1024) void k_detect_tail_small(
-    const unsigned long long* __restrict__ ts, long long ntiles,
+    const unsigned long long* __restrict__ ts, const long long* __restrict__ npairs_dev,
     unsigned long long* __restrict__ stats, const int* __restrict__ tile_count, int tiles,
     int npairs, int* __restrict__ counts, long long* __restrict__ offs) {
-  __shared__ unsigned long long red[kTileStats];
+  __shared__ unsigned long long red[N];
   __shared__ long long s_wave[16];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  if (t < kTileStats) red[t] = 0;
+  if (t < N) red[t] = 0;
   __syncthreads();
-  unsigned long long acc[kTileStats] = {};
+  const long long ntiles =
+      (npairs_dev && *npairs_dev < npairs ? *npairs_dev : static_cast<long long>(npairs)) * tiles;
+  unsigned long long acc[N] = {};
   for (long long k = t; k < ntiles; k += 1024)
-    for (int q = 0; q < kTileStats; ++q) acc[q] += ts[k * kTileStats + q];
-  for (int q = 0; q < kTileStats; ++q) {
+    for (int q = 0; q < N; ++q) acc[q] += ts[k * N + q];
+  for (int q = 0; q < N; ++q) {
     unsigned long long v = acc[q];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     if (lane == 0 && v) atomicAdd(&red[q], v);
@@ -1246,11 +1241,7 @@ __global__ __launch_bounds__(1024) void k_detect_tail_small(
     run += c[u];
   }
   if (t == 1023) offs[npairs] = before + incl;
-  if (t < kTileStats && red[t]) {
-    const int slot[kTileStats] = {ST_CHECKS, ST_EVALUATED, ST_FALLBACK_ROWS, ST_PENALTY_FAILS,
-                                  ST_BATCH_FAILS, ST_BATCH_SIZE, ST_CULLED};
-    atomicAdd(&stats[slot[t]], red[t]);
-  }
+  if (t < N && red[t]) atomicAdd(&stats[stat_slot(t)], red[t]);
 }
 
 // GJK over the particles' vertex replicas (gjk.cpp:25-100 with the core of
@@ -1275,10 +1266,10 @@ __global__ __launch_bounds__(256) void k_gjk(DetectArgs g) {
   const int lane = threadIdx.x & 63;
   const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (k >= g.npairs) return;
-  unsigned long long* ts = g.tile_stats + static_cast<long long>(k) * kTileStats;
+  unsigned long long* ts = g.tile_stats + static_cast<long long>(k) * g.nstats;
   if (g.npairs_dev && k >= *g.npairs_dev) {
     if (lane == 0) g.tile_count[k] = 0;
-    if (lane < kTileStats) ts[lane] = 0;
+    if (lane < g.nstats) ts[lane] = 0;
     return;
   }
   const Pair p = load_pair(g, k);
@@ -1469,132 +1460,267 @@ __global__ __launch_bounds__(256) void k_tile_sums(const int* __restrict__ tile_
 __global__ __launch_bounds__(256) void k_scatter(const dh_contact* __restrict__ temp, long long n,
                                                  const long long* __restrict__ offs,
                                                  const int* __restrict__ tile_count, int tiles,
-                                                 dh_contact* __restrict__ out,
+                                                 dh_contact* __restrict__ out, long long cap,
                                                  const unsigned long long* __restrict__ n_dev) {
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  // n is the capacity (of temp and out) when the count is read from n_dev
+  // n is the capacity of temp when the count is read from n_dev
   if (i >= n || (n_dev && static_cast<unsigned long long>(i) >= *n_dev)) return;
   dh_contact c = temp[i];
   const int pair = c.pair / tiles;
   long long dst = offs[pair] + c.pad_;
   for (int t = pair * tiles; t < c.pair; ++t) dst += tile_count[t];
-  if (dst >= n) return;  // more contacts than the capacity (reported by the caller)
+  if (dst >= cap) return;  // more contacts than the capacity (reported by the caller)
   c.pair = pair;
   c.pad_ = 0;
   out[dst] = c;
 }
 
-template <bool SCREEN>
-__device__ __forceinline__ void queue_solve_entry(const DetectArgs& g, long long e,
-                                                  int* __restrict__ flags,
-                                                  double* __restrict__ pq) {
-  const int2 en = g.queue[e];
-  if (en.x < 0) {
-    flags[e] = 0;
-    return;
-  }
+// Survivor queue, pass 2: every wave takes one region of k_detect_wave's (then
+// the ranges of k_detect_big that fall to it) through the plane test, the
+// edge-pair axes (and, when tuned on, the binary32 screen) and bfSolver.  What
+// a test leaves waits in a list in LDS until 64 entries are there, so that
+// each stage runs with every lane busy although the one before it drops most.
+// The entries stay in order, so the contacts of an item come out in row-major
+// order and their rank is a running count, and the records of a region follow
+// each other without a counter that all waves share.
+struct QueueLists {
+  int a[128], b[128];  // entries for the axes, for bfSolver
+};
+
+// Lanes' places in a wave's list of n entries; the whole wave calls it.
+__device__ __forceinline__ int list_append(int* list, int n, bool keep, int e) {
+  const unsigned long long m = __ballot(keep);
+  if (keep) list[n + lane_prefix(m)] = e;
+  wave_lds_fence();
+  return n + __popcll(m);
+}
+
+// The first 64 entries of a list of n off it: the lane's entry (-1 past the
+// end); the rest move to the front.
+__device__ __forceinline__ int list_take(int* list, int& n, int lane) {
+  const int e = lane < n ? list[lane] : -1;
+  const int rest = n > 64 ? n - 64 : 0;
+  const int r = lane < rest ? list[64 + lane] : 0;
+  wave_lds_fence();
+  if (lane < rest) list[lane] = r;
+  wave_lds_fence();
+  n = rest;
+  return e;
+}
+
+__device__ __forceinline__ double entry_margin(const DetectArgs& g, const int4& en) {
   const int k = en.x / g.tiles;
-  const int pa = g.pairs[2 * k], pb = g.pairs[2 * k + 1];
-  const int iA = static_cast<int>(static_cast<unsigned>(en.y) & 0xffffu);
-  const int iB = static_cast<int>(static_cast<unsigned>(en.y) >> 16);
-  const Tri<double> A = load_tri(g, g.tri_offset[pa] + iA);
-  const Tri<double> B = load_tri(g, g.tri_offset[pb] + iB);
-  const double margin = g.eps[pa] + g.eps[pb];
-  if (axes_apart(A, B, margin) || (SCREEN && screened_far(A, B, margin))) {
-    flags[e] = 0;
-    return;
+  return g.eps[g.pairs[2 * k]] + g.eps[g.pairs[2 * k + 1]];
+}
+
+// Ranks of the emitting lanes within their items (runs of one item, in order)
+// after `carry` contacts of item `carry_item` so far; the last lane of each
+// run writes the item's count.  The whole wave calls it.
+__device__ __forceinline__ int item_rank(const DetectArgs& g, bool emit, int item, int lane,
+                                         int& carry_item, int& carry) {
+  const unsigned long long mask = __ballot(emit), below = (1ull << lane) - 1;
+  if (!mask) return 0;
+  const unsigned long long before = mask & below;
+  const int prev = before ? 63 - __clzll(static_cast<long long>(before)) : lane;
+  const int prev_item = __shfl(item, prev);  // by every lane: prev must take part
+  const bool head = emit && (!before || prev_item != item);
+  const unsigned long long heads = __ballot(head);
+  const unsigned long long upto = heads & (below | 1ull << lane);
+  const int first = upto ? 63 - __clzll(static_cast<long long>(upto)) : lane;
+  int rank = __popcll(before & ~((1ull << first) - 1));
+  if (item == carry_item && first == __builtin_ctzll(mask)) rank += carry;
+  const int last = 63 - __clzll(static_cast<long long>(mask));
+  const unsigned long long after = mask & ~(below | 1ull << lane);
+  const bool tail = emit && (!after || (heads >> __builtin_ctzll(after) & 1));
+  if (tail) g.tile_count[item] = rank + 1;
+  carry_item = __shfl(item, last);
+  carry = __shfl(rank, last) + 1;
+  return rank;
+}
+
+// The n entries at q through the tests and bfSolver; their contacts' records
+// to rec, in order.  Returns the number of records.  With kFilter the entries
+// that the tests leave are compacted in place instead, and counted.
+template <bool SCREEN, bool kFilter>
+__device__ __forceinline__ int solve_stream(const DetectArgs& g, int4* __restrict__ q, int n,
+                                            QueueRecord* __restrict__ rec, QueueLists& L,
+                                            int lane) {
+  int na = 0, nb = 0, base = 0, out = 0, carry_item = -1, carry = 0;
+  for (;;) {
+    const bool eof = base >= n;
+    if (nb >= 64 || (eof && na == 0 && nb > 0)) {
+      const int e = list_take(L.b, nb, lane);
+      int4 en = make_int4(-1, 0, 0, 0);
+      if (e >= 0) en = q[e];
+      if (kFilter) {
+        // every entry before these has been read: the places are free
+        const unsigned long long m = __ballot(e >= 0);
+        if (e >= 0) q[out + lane_prefix(m)] = en;
+        out += __popcll(m);
+        continue;
+      }
+      bool emit = false;
+      V3<double> P = {0, 0, 0}, Q = {0, 0, 0};
+      if (e >= 0) {
+        bf_solver(load_tri(g, en.y), load_tri(g, en.z), P, Q);
+        emit = pq_dist(P, Q) <= entry_margin(g, en);
+      }
+      const int rank = item_rank(g, emit, en.x, lane, carry_item, carry);
+      const unsigned long long m = __ballot(emit);
+      if (emit) {
+        QueueRecord r;
+        r.item = en.x;
+        r.tris = en.w;
+        r.rank = rank;
+        r.pad_ = 0;
+        r.pq[0] = P.x; r.pq[1] = P.y; r.pq[2] = P.z;
+        r.pq[3] = Q.x; r.pq[4] = Q.y; r.pq[5] = Q.z;
+        rec[out + lane_prefix(m)] = r;
+      }
+      out += __popcll(m);
+    } else if (na >= 64 || (eof && na > 0)) {
+      const int e = list_take(L.a, na, lane);
+      bool keep = false;
+      if (e >= 0) {
+        const int4 en = q[e];
+        const Tri<double> A = load_tri(g, en.y), B = load_tri(g, en.z);
+        const double margin = entry_margin(g, en);
+        keep = !edge_axes_apart(A, B, axis_reach(A, B, margin)) &&
+               !(SCREEN && screened_far(A, B, margin));
+      }
+      nb = list_append(L.b, nb, keep, e);
+    } else if (!eof) {
+      const int e = base + lane;
+      bool keep = false;
+      if (e < n) {
+        const int4 en = q[e];
+        if (en.x >= 0)
+          keep = !plane_apart(load_tri(g, en.y), load_tri(g, en.z), entry_margin(g, en));
+      }
+      na = list_append(L.a, na, keep, e);
+      base += 64;
+    } else {
+      break;
+    }
   }
-  V3<double> P, Q;
-  bf_solver(A, B, P, Q);
-  const bool emit = pq_dist(P, Q) <= margin;
-  flags[e] = emit ? 1 : 0;
-  if (emit) {
-    double* o = pq + 6 * e;
-    o[0] = P.x; o[1] = P.y; o[2] = P.z;
-    o[3] = Q.x; o[4] = Q.y; o[5] = Q.z;
+  return out;
+}
+
+// A wave's streams: the regions, then the ranges.
+struct QueueStream {
+  long long at;  // first entry, from g.queue (bqueue follows the regions there)
+  int n;
+  int* contacts;  // where the number of its records goes
+};
+
+__device__ __forceinline__ QueueStream queue_stream(const DetectArgs& g, int u) {
+  if (u < g.regions)
+    return {static_cast<long long>(u) * g.rcap, g.rcount[u], g.rcount + g.regions + u};
+  int4* r = g.ranges + (u - g.regions);
+  return {static_cast<long long>(g.regions) * g.rcap + r->x, r->y, &r->w};
+}
+
+template <bool SCREEN, bool kFilter>
+__global__ __launch_bounds__(256, 3) void k_queue_solve(DetectArgs g) {
+  __shared__ QueueLists lists[4];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int nstreams = g.regions + static_cast<int>(*g.nranges);
+  for (int u = blockIdx.x * 4 + w; u < nstreams; u += gridDim.x * 4) {
+    const QueueStream s = queue_stream(g, u);
+    const int m = solve_stream<SCREEN, kFilter>(g, g.queue + s.at, s.n, g.rec + s.at, lists[w], lane);
+    if (lane == 0) {
+      if (!kFilter) *s.contacts = m;
+      else if (u < g.regions) g.rcount[u] = m;
+      else g.ranges[u - g.regions].y = m;
+    }
   }
 }
 
-
-// Survivor queue, pass 2: a lane per queued triangle pair at a time
-// (bfSolver, the contact test of bf.cpp:125); flags[e] = 1 and P, Q kept when
-// it emits.  The entries are the first n, or, with need_dev (a captured step
-// launched for the capacity n), the first min(*need_dev, n); the later passes
-// stop at the same count.
-template <bool SCREEN>
-__global__ __launch_bounds__(256) void k_queue_solve(DetectArgs g, long long n,
-                                                     const unsigned long long* __restrict__ need_dev,
-                                                     int* __restrict__ flags,
-                                                     double* __restrict__ pq) {
-  // the live entries (flags past them are not written: the scan stops there)
-  const long long live =
-      need_dev && static_cast<long long>(*need_dev) < n ? static_cast<long long>(*need_dev) : n;
-  for (long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; e < live;
-       e += static_cast<long long>(gridDim.x) * 256)
-    queue_solve_entry<SCREEN>(g, e, flags, pq);
-}
-
-// Pass 3: the queue's contacts take one range of the contact slots.
-__device__ __forceinline__ long long queue_live(long long n,
-                                                const unsigned long long* need_dev) {
-  return need_dev && static_cast<long long>(*need_dev) < n ? static_cast<long long>(*need_dev) : n;
-}
-
-__global__ void k_queue_reserve(DetectArgs g, const long long* __restrict__ pos, long long n,
-                                const unsigned long long* __restrict__ need_dev,
-                                unsigned long long* __restrict__ base) {
-  if (threadIdx.x == 0 && blockIdx.x == 0)
-    *base = atomicAdd(g.counter, static_cast<unsigned long long>(pos[queue_live(n, need_dev)]));
-}
-
-// Pass 4: contacts of the emitting entries, tagged (item, rank within the
-// item): the item's entries are contiguous and in row-major order, so the
-// rank is the number of emitting entries before it in the item's range.
-__device__ __forceinline__ void queue_emit_entry(const DetectArgs& g, long long e,
-                                                 const long long* __restrict__ pos,
-                                                 const double* __restrict__ pq,
-                                                 const unsigned long long* __restrict__ base) {
-  const int2 en = g.queue[e];
-  const int item = en.x;
-  const int k = item / g.tiles;
-  const Pair p = load_pair(g, k);
-  const int iA = static_cast<int>(static_cast<unsigned>(en.y) & 0xffffu);
-  const int iB = static_cast<int>(static_cast<unsigned>(en.y) >> 16);
-  const double* o = pq + 6 * e;
-  const V3<double> P = {o[0], o[1], o[2]}, Q = {o[3], o[4], o[5]};
-  const unsigned long long slot = *base + static_cast<unsigned long long>(pos[e]);
-  if (slot < static_cast<unsigned long long>(g.cap)) {
-    dh_contact c;
-    make_contact(p, k, iA, iB, P, Q, &c);
-    c.pair = item;
-    c.pad_ = static_cast<int>(pos[e] - pos[g.qbase[item]]);
-    g.temp[slot] = c;
+// The records of entries that another kernel has solved (flags[e], and the
+// points pq[6e..] of those that emit), in order.
+__device__ __forceinline__ int record_stream(const DetectArgs& g, const int4* __restrict__ q, int n,
+                                             const int* __restrict__ flags,
+                                             const double* __restrict__ pq,
+                                             QueueRecord* __restrict__ rec, int lane) {
+  int out = 0, carry_item = -1, carry = 0;
+  for (int base = 0; base < n; base += 64) {
+    const int e = base + lane;
+    const bool emit = e < n && flags[e] != 0;
+    int4 en = make_int4(-1, 0, 0, 0);
+    if (emit) en = q[e];
+    const int rank = item_rank(g, emit, en.x, lane, carry_item, carry);
+    const unsigned long long m = __ballot(emit);
+    if (emit) {
+      QueueRecord r;
+      r.item = en.x;
+      r.tris = en.w;
+      r.rank = rank;
+      r.pad_ = 0;
+      for (int c = 0; c < 6; ++c) r.pq[c] = pq[6 * static_cast<long long>(e) + c];
+      rec[out + lane_prefix(m)] = r;
+    }
+    out += __popcll(m);
   }
-  atomicAdd(&g.tile_count[item], 1);
+  return out;
 }
 
-__global__ __launch_bounds__(256) void k_queue_emit(DetectArgs g, long long n,
-                                                    const unsigned long long* __restrict__ need_dev,
-                                                    const int* __restrict__ flags,
-                                                    const long long* __restrict__ pos,
-                                                    const double* __restrict__ pq,
-                                                    const unsigned long long* __restrict__ base) {
-  const long long live = queue_live(n, need_dev);
-  for (long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; e < live;
-       e += static_cast<long long>(gridDim.x) * 256)
-    if (flags[e]) queue_emit_entry(g, e, pos, pq, base);
+__global__ __launch_bounds__(256) void k_queue_record(DetectArgs g, const int* __restrict__ flags,
+                                                      const double* __restrict__ pq) {
+  const int lane = threadIdx.x & 63;
+  const int nstreams = g.regions + static_cast<int>(*g.nranges);
+  for (int u = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6); u < nstreams;
+       u += gridDim.x * 4) {
+    const QueueStream s = queue_stream(g, u);
+    const int m = record_stream(g, g.queue + s.at, s.n, flags + s.at, pq + 6 * s.at, g.rec + s.at,
+                                lane);
+    if (lane == 0) *s.contacts = m;
+  }
 }
 
-int queue_learned(const int2* queue, const int* pairs, int tiles, const int* tri_offset,
+// Pass 3, after the pairs' offsets: the records' contacts, each at its place.
+// counter (may be null) receives offs[*npairs_dev], the contacts found.
+__device__ __forceinline__ void write_record(const DetectArgs& g, const QueueRecord& r,
+                                             const long long* __restrict__ offs,
+                                             dh_contact* __restrict__ out, long long cap) {
+  const int k = r.item / g.tiles;
+  long long dst = offs[k] + r.rank;
+  for (int t = k * g.tiles; t < r.item; ++t) dst += g.tile_count[t];
+  if (dst >= cap) return;  // more contacts than the capacity (reported by the caller)
+  dh_contact c;
+  const V3<double> P = {r.pq[0], r.pq[1], r.pq[2]}, Q = {r.pq[3], r.pq[4], r.pq[5]};
+  make_contact(load_pair(g, k), k, r.tris & 0xffff, static_cast<int>(static_cast<unsigned>(r.tris) >> 16),
+               P, Q, &c);
+  c.pad_ = 0;
+  out[dst] = c;
+}
+
+__global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long long* __restrict__ offs,
+                                                     dh_contact* __restrict__ out, long long cap,
+                                                     unsigned long long* __restrict__ counter) {
+  const int lane = threadIdx.x & 63;
+  const int nstreams = g.regions + static_cast<int>(*g.nranges);
+  for (int u = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6); u < nstreams;
+       u += gridDim.x * 4) {
+    const QueueStream s = queue_stream(g, u);
+    const int n = *s.contacts;
+    for (int e = lane; e < n; e += 64) write_record(g, g.rec[s.at + e], offs, out, cap);
+  }
+  if (counter && blockIdx.x == 0 && threadIdx.x == 0)
+    *counter = static_cast<unsigned long long>(
+        offs[g.npairs_dev && *g.npairs_dev < g.npairs ? *g.npairs_dev : g.npairs]);
+}
+
+int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
+                  const int* rcount, const int4* ranges, const unsigned* nranges,
                   const double* x, const double* y, const double* z, const double* eps,
-                  long long n, const unsigned long long* need_dev, int* flags, double* pq,
-                  hipStream_t st);
+                  long long n, int* flags, double* pq, hipStream_t st);
 int queue_learned_reserve(long long n);
 
 struct DetectScratch {
-  DevBuf temp, counter, stats, error, counts, offs, sums, tiles, tstats;
-  DevBuf queue, qcounter, qbase, qflags, qpos, qpq, qres, deferred, ndeferred, iskip, tmax;
-  long long qcap = 0;  // queue entries of the next eager DH_BF call
+  DevBuf temp, counter, stats, error, counts, offs, sums, tiles, tstats, iskip, tmax;
+  DevBuf queue, qrec, qcounts, rcount, ranges, deferred, wlist, qflags, qpq;
+  int rwant = 0, bwant = 0;  // what a region and bqueue had to hold in earlier eager calls
 };
 static DetectScratch g_scratch;
 
@@ -1700,43 +1826,25 @@ static unsigned detect_grid(long long items) {
 
 template <int M>
 static void launch_detect(unsigned items, size_t shm, hipStream_t st, const DetectArgs& a) {
-  if (M == DH_BF && a.queue && a.wave_items) {
-    hipLaunchKernelGGL(k_lane_cull, items > 0 ? grid_for(items, 256) : 1u, 256, 0, st, a,
-                       static_cast<int>(items));
-    // at most the workgroups one CU holds at once (3 waves per SIMD at the
-    // kernel's 161 VGPRs, 2 waves per workgroup): no partial second round
-    const long long wg = (static_cast<long long>(items) + 1) / 2;
-    const long long cap = static_cast<long long>(device_cus()) * 6;
-    hipLaunchKernelGGL(k_detect_wave, static_cast<unsigned>(wg < cap ? (wg > 0 ? wg : 1) : cap),
-                       128, 0, st, a, static_cast<int>(items));
-  }
-  if (M == DH_BF && a.queue && a.wave_items) {
-    const long long wg = (static_cast<long long>(items) + 63) / 64;
+  if (M == DH_BF && a.item_skip) {
+    const long long wg = (static_cast<long long>(items) + 3) / 4;
     const long long cap = static_cast<long long>(device_cus()) * 32;
-    hipLaunchKernelGGL(k_detect_big, static_cast<unsigned>(wg < cap ? (wg > 0 ? wg : 1) : cap),
-                       256, shm, st, a, static_cast<int>(items));
-  } else if (M == DH_BF && a.queue) {
-    hipLaunchKernelGGL((k_detect<DH_BF, true>), detect_grid(items), 256, shm, st, a,
-                       static_cast<int>(items));
-  } else {
-    if (M == DH_BF && a.item_skip) {
-      const long long wg = (static_cast<long long>(items) + 3) / 4;
-      const long long cap = static_cast<long long>(device_cus()) * 32;
-      hipLaunchKernelGGL(k_chunk_cull, static_cast<unsigned>(wg < cap ? (wg > 0 ? wg : 1) : cap),
-                         256, 0, st, a, static_cast<int>(items),
-                         const_cast<unsigned char*>(a.item_skip));
-    }
-    hipLaunchKernelGGL((k_detect<M, false>), detect_grid(items), 256, shm, st, a,
-                       static_cast<int>(items));
+    hipLaunchKernelGGL(k_chunk_cull, static_cast<unsigned>(wg < cap ? (wg > 0 ? wg : 1) : cap),
+                       256, 0, st, a, static_cast<int>(items),
+                       const_cast<unsigned char*>(a.item_skip));
   }
+  hipLaunchKernelGGL((k_detect<M, false>), detect_grid(items), 256, shm, st, a,
+                     static_cast<int>(items));
 }
 
-static void launch_tile_stats(const unsigned long long* ts, long long ntiles,
-                              unsigned long long* stats, hipStream_t st) {
+static void launch_tile_stats(const DetectArgs& a, hipStream_t st) {
+  const long long ntiles = static_cast<long long>(a.npairs) * a.tiles;
   if (ntiles <= 0) return;
   long long grid = (ntiles + 255) / 256;
   if (grid > 256) grid = 256;
-  hipLaunchKernelGGL(k_tile_stats, static_cast<unsigned>(grid), 256, 0, st, ts, ntiles, stats);
+  const auto f = a.nstats == kBfStats ? k_tile_stats<kBfStats> : k_tile_stats<kTileStats>;
+  hipLaunchKernelGGL(f, static_cast<unsigned>(grid), 256, 0, st, a.tile_stats,
+                     static_cast<long long>(a.npairs), a.tiles, a.npairs_dev, a.stats);
 }
 
 // Row ranges per particle pair: enough workgroups to fill the 256 CUs
@@ -1749,79 +1857,143 @@ static int tiles_for(long long npairs, int method) {
   return static_cast<int>(t < 1 ? 1 : (t > cap ? cap : t));
 }
 
-// Buffers of the queue passes for n entries.
-static int queue_reserve(long long n) {
-  int rc;
-  if ((rc = g_scratch.qflags.grow(sizeof(int) * (n + 1)))) return rc;
-  if ((rc = g_scratch.qpos.grow(sizeof(long long) * (n + 1)))) return rc;
-  if ((rc = g_scratch.qpq.grow(sizeof(double) * 6 * n))) return rc;
-  if ((rc = g_scratch.qres.grow(sizeof(unsigned long long)))) return rc;
-  return scan_reserve(static_cast<int>(n));
+// The survivor queue's shape for `items` items: a region per wave of
+// k_detect_wave's persistent grid (as many as the CUs hold at once), 16 entries
+// per item over the regions and 4 for bqueue, or what earlier calls needed.
+struct QueuePlan {
+  unsigned groups;
+  int regions, rcap, bcap;
+  long long entries() const { return static_cast<long long>(regions) * rcap + bcap; }
+};
+
+static QueuePlan queue_plan(long long items, int rwant, int bwant) {
+  QueuePlan q;
+  const long long wg = (items + kWavesPerGroup - 1) / kWavesPerGroup;
+  const long long most = static_cast<long long>(device_cus()) * 8;
+  q.groups = static_cast<unsigned>(wg < 1 ? 1 : (wg < most ? wg : most));
+  q.regions = static_cast<int>(q.groups) * kWavesPerGroup;
+  long long r = (16 * items + 65536) / q.regions, b = 4 * items + 65536;
+  if (r < 2 * kWaveSurvivors) r = 2 * kWaveSurvivors;
+  if (r < rwant) r = rwant;
+  if (b < bwant) b = bwant;
+  const long long rmost = (1ll << 29) / q.regions;
+  q.rcap = static_cast<int>(r < rmost ? r : rmost);
+  q.bcap = static_cast<int>(b < (1ll << 29) ? b : 1ll << 29);
+  return q;
 }
 
-// Solve, scan, reserve and emit over n queue entries (live: all of them, or
-// min(*need_dev, n) in a captured step).
-static int queue_passes(const DetectArgs& a, long long n, const unsigned long long* need_dev,
-                        bool learned, hipStream_t st) {
-  // a captured step's passes are launched for the capacity: a persistent grid
-  // strides over the live entries
-  long long g = grid_for(n, 256);
-  const long long gcap = static_cast<long long>(device_cus()) * 16;
-  if (need_dev && g > gcap) g = gcap;
-  const unsigned grid = static_cast<unsigned>(g > 0 ? g : 1);
+// Places of the queue path's counters in g_scratch.qcounts.
+enum QueueCount : int { QC_WLIST = 0, QC_BIG, QC_DEFERRED, QC_BQUEUE, QC_RANGES, QC_RWANT, kQueueCounts };
+
+// Buffers of the queue path (before a capture).
+static int queue_reserve(const QueuePlan& q, long long items, bool learned) {
   int rc;
+  if ((rc = g_scratch.queue.grow(sizeof(int4) * q.entries()))) return rc;
+  if ((rc = g_scratch.qrec.grow(sizeof(QueueRecord) * q.entries()))) return rc;
+  if ((rc = g_scratch.qcounts.grow(sizeof(unsigned) * kQueueCounts))) return rc;
+  if ((rc = g_scratch.rcount.grow(sizeof(int) * 2 * q.regions))) return rc;
+  if ((rc = g_scratch.ranges.grow(sizeof(int4) * (items + 1)))) return rc;
+  if ((rc = g_scratch.deferred.grow(sizeof(int) * 2 * (items + 1)))) return rc;
+  if ((rc = g_scratch.wlist.grow(sizeof(WaveItem) * (items + 1)))) return rc;
   if (learned) {
-    if ((rc = queue_learned(a.queue, a.pairs, a.tiles, a.tri_offset, a.x, a.y, a.z, a.eps, n,
-                            need_dev, g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>(),
-                            st)))
+    if ((rc = g_scratch.qflags.grow(sizeof(int) * q.entries()))) return rc;
+    if ((rc = g_scratch.qpq.grow(sizeof(double) * 6 * q.entries()))) return rc;
+    return queue_learned_reserve(q.entries());
+  }
+  return DH_OK;
+}
+
+static void queue_bind(DetectArgs& a, const QueuePlan& q, long long items) {
+  unsigned* c = g_scratch.qcounts.as<unsigned>();
+  const long long big = static_cast<long long>(q.regions) * q.rcap;
+  a.queue = g_scratch.queue.as<int4>();
+  a.rcap = q.rcap;
+  a.regions = q.regions;
+  a.rcount = g_scratch.rcount.as<int>();
+  a.rwant = reinterpret_cast<int*>(c + QC_RWANT);
+  a.bqueue = a.queue + big;
+  a.bcap = q.bcap;
+  a.bcounter = c + QC_BQUEUE;
+  a.ranges = g_scratch.ranges.as<int4>();
+  a.nranges = c + QC_RANGES;
+  a.rec = g_scratch.qrec.as<QueueRecord>();
+  a.deferred = g_scratch.deferred.as<int>();
+  a.ndeferred = c + QC_DEFERRED;
+  a.biglist = a.deferred + (items + 1);
+  a.nbig = c + QC_BIG;
+  a.wlist = g_scratch.wlist.as<WaveItem>();
+  a.nwlist = c + QC_WLIST;
+}
+
+// A DH_BF detection through the survivor queue: the mid-phase, the items it
+// could not queue in full (as many as *ndeferred), then the queue's solve.
+// Every launch is for the capacity and reads the live lengths, so nothing is
+// read back on the way.
+static int queue_detect(const DetectArgs& a, const QueuePlan& q, unsigned items, bool learned,
+                        hipStream_t st) {
+  const unsigned cus = static_cast<unsigned>(device_cus());
+  const unsigned few = items < 4 * cus ? items : 4 * cus;  // usually none to do
+  hipLaunchKernelGGL(k_lane_cull, items > 0 ? grid_for(items, 1024) : 1u, 1024, 0, st, a,
+                     static_cast<int>(items));
+  hipLaunchKernelGGL(k_detect_wave, q.groups, 64 * kWavesPerGroup, 0, st, a);
+  hipLaunchKernelGGL(k_detect_big, few, 256, 0, st, a);
+  DetectArgs f = a;
+  f.item_list = a.deferred;
+  f.nitems_dev = a.ndeferred;
+  hipLaunchKernelGGL((k_detect<DH_BF, false>), few, 256, 0, st, f, static_cast<int>(items));
+  const unsigned grid = grid_for(q.regions, 4);
+  if (!learned) {
+    if (a.fp32_screen)
+      hipLaunchKernelGGL((k_queue_solve<true, false>), grid, 256, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_queue_solve<false, false>), grid, 256, 0, st, a);
+  } else {
+    if (a.fp32_screen)
+      hipLaunchKernelGGL((k_queue_solve<true, true>), grid, 256, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_queue_solve<false, true>), grid, 256, 0, st, a);
+    int rc;
+    if ((rc = queue_learned(a.queue, a.pairs, a.tiles, a.regions, a.rcap, a.rcount, a.ranges,
+                            a.nranges, a.x, a.y, a.z, a.eps, q.entries(),
+                            g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>(), st)))
       return rc;
-  } else if (a.fp32_screen)
-    hipLaunchKernelGGL(k_queue_solve<true>, grid, 256, 0, st, a, n, need_dev,
-                       g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>());
-  else
-    hipLaunchKernelGGL(k_queue_solve<false>, grid, 256, 0, st, a, n, need_dev,
-                       g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>());
-  const int ni = static_cast<int>(n);
-  if (ni > 1024 && (rc = g_scratch.sums.grow(sizeof(long long) * scan_sums_len(ni)))) return rc;
-  if ((rc = scan_counts_upto(g_scratch.qflags.as<int>(), static_cast<int>(n), need_dev,
-                             g_scratch.qpos.as<long long>(), g_scratch.sums.as<long long>(), st)))
-    return rc;
-  hipLaunchKernelGGL(k_queue_reserve, 1, 64, 0, st, a, g_scratch.qpos.as<long long>(), n, need_dev,
-                     g_scratch.qres.as<unsigned long long>());
-  hipLaunchKernelGGL(k_queue_emit, grid, 256, 0, st, a, n, need_dev, g_scratch.qflags.as<int>(),
-                     g_scratch.qpos.as<long long>(), g_scratch.qpq.as<double>(),
-                     g_scratch.qres.as<unsigned long long>());
+    hipLaunchKernelGGL(k_queue_record, grid, 256, 0, st, a, g_scratch.qflags.as<int>(),
+                       g_scratch.qpq.as<double>());
+  }
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
 
-// Passes 2-4 of the survivor queue after the detection launch: the queued
-// triangle pairs solved one per lane, an exclusive scan of the emitting
-// flags, one reservation of contact slots, the contacts.  Reads the queue
-// length back (one synchronisation); the next call's queue holds this
-// call's need.
-static int solve_queue(const DetectArgs& a, bool learned, hipStream_t st) {
-  unsigned long long need = 0;
-  unsigned ndef = 0;
-  DH_HIP_CHECK(hipMemcpyAsync(&need, a.qcounter, sizeof(need), hipMemcpyDeviceToHost, st));
-  DH_HIP_CHECK(hipMemcpyAsync(&ndef, a.ndeferred, sizeof(ndef), hipMemcpyDeviceToHost, st));
-  DH_HIP_CHECK(hipStreamSynchronize(st));
-  if (ndef > 0) {
-    // the items the mid-phase launch could not queue, in full
-    DetectArgs f = a;
-    f.queue = nullptr;
-    f.item_list = a.deferred;
-    f.nitems_dev = nullptr;
-    hipLaunchKernelGGL((k_detect<DH_BF, false>), detect_grid(ndef), 256, 0, st, f,
-                       static_cast<int>(ndef));
-  }
-  if (static_cast<long long>(need) > a.qcap)
-    g_scratch.qcap = static_cast<long long>(need) + static_cast<long long>(need) / 4;
-  const long long live = static_cast<long long>(need) < a.qcap ? static_cast<long long>(need) : a.qcap;
-  if (live == 0) return DH_OK;
-  int rc;
-  if ((rc = queue_reserve(live))) return rc;
-  return queue_passes(a, live, nullptr, learned, st);
+// The DetectArgs of a call without its queue.
+static DetectArgs detect_args(const dh_geometry* geom, const int* pairs, int npairs,
+                              const long long* np_dev, long long cap, int tiles, int* tile_count,
+                              bool bf, const double* pbox, const double* bbox,
+                              const double* psph) {
+  DetectArgs a = {};
+  a.x = geom->x;
+  a.y = geom->y;
+  a.z = geom->z;
+  a.tri_offset = geom->tri_offset;
+  a.eps = geom->eps;
+  a.friction = geom->friction;
+  a.id = geom->id;
+  a.pairs = pairs;
+  a.npairs = npairs;
+  a.temp = g_scratch.temp.as<dh_contact>();
+  a.cap = cap;
+  a.counter = g_scratch.counter.as<unsigned long long>();
+  a.tiles = tiles;
+  a.tile_count = tile_count;
+  a.nstats = bf ? kBfStats : kTileStats;
+  a.tile_stats = g_scratch.tstats.as<unsigned long long>();
+  a.stats = g_scratch.stats.as<unsigned long long>();
+  a.error = g_scratch.error.as<int>();
+  a.npairs_dev = np_dev;
+  a.pbox = pbox;
+  a.psph = pbox ? psph : nullptr;
+  a.bbox = bbox;
+  a.fp32_screen = tuning().detect_fp32_screen;
+  return a;
 }
 
 int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int npairs,
@@ -1850,80 +2022,34 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
     if ((rc = g_scratch.tiles.grow(sizeof(int) * static_cast<size_t>(npairs) * tiles))) return rc;
     tile_count = g_scratch.tiles.as<int>();
   }
-  DetectArgs a;
-  a.x = geom->x;
-  a.y = geom->y;
-  a.z = geom->z;
-  a.tri_offset = geom->tri_offset;
-  a.eps = geom->eps;
-  a.friction = geom->friction;
-  a.id = geom->id;
-  a.pairs = pairs;
-  a.npairs = npairs;
-  a.temp = g_scratch.temp.as<dh_contact>();
-  a.cap = cap;
-  a.counter = g_scratch.counter.as<unsigned long long>();
-  a.tiles = tiles;
-  a.tile_count = tile_count;
-  const long long ntiles = static_cast<long long>(npairs) * tiles;
-  if ((rc = g_scratch.tstats.grow(sizeof(unsigned long long) * kTileStats * ntiles))) return rc;
-  a.tile_stats = g_scratch.tstats.as<unsigned long long>();
-  a.stats = g_scratch.stats.as<unsigned long long>();
-  a.error = g_scratch.error.as<int>();
-  a.npairs_dev = nullptr;
-  a.pbox = pbox;
-  a.psph = pbox ? psph : nullptr;
-  a.fp32_screen = tuning().detect_fp32_screen;
-  a.wave_items = 0;
-  a.item_skip = nullptr;
-  a.bbox = bbox;
-  a.queue = nullptr;
-  a.qcap = 0;
-  a.qcounter = nullptr;
-  a.qbase = nullptr;
-  a.deferred = nullptr;
-  a.ndeferred = nullptr;
-  a.biglist = nullptr;
-  a.nbig = nullptr;
-  a.wlist = nullptr;
-  a.nwlist = nullptr;
-  a.item_list = nullptr;
-  a.nitems_dev = nullptr;
   const long long nitems = static_cast<long long>(npairs) * tiles;
-  // the queue costs a read-back and four launches: for many items only
-  if (method == DH_BF && (learned || nitems >= tuning().detect_queue_min_items)) {
-    // survivor queue: sized from the last call's need, at least 16 entries
-    // per item (an overflowing item solves its own survivors)
-    long long qcap = g_scratch.qcap > 16 * nitems + 65536 ? g_scratch.qcap : 16 * nitems + 65536;
-    if (qcap > (1ll << 30)) qcap = 1ll << 30;
-    if ((rc = g_scratch.queue.grow(sizeof(int2) * qcap))) return rc;
-    if ((rc = g_scratch.qcounter.grow(sizeof(unsigned long long)))) return rc;
-    if ((rc = g_scratch.qbase.grow(sizeof(long long) * (nitems + 1)))) return rc;
-    if ((rc = g_scratch.deferred.grow(sizeof(int) * 3 * (nitems + 1)))) return rc;
-    if ((rc = g_scratch.ndeferred.grow(sizeof(unsigned) * 3))) return rc;
-    DH_HIP_CHECK(hipMemsetAsync(g_scratch.qcounter.ptr, 0, sizeof(unsigned long long), st));
-    DH_HIP_CHECK(hipMemsetAsync(g_scratch.ndeferred.ptr, 0, sizeof(unsigned) * 3, st));
-    a.deferred = g_scratch.deferred.as<int>();
-    a.ndeferred = g_scratch.ndeferred.as<unsigned>();
-    a.biglist = a.deferred + (nitems + 1);
-    a.nbig = a.ndeferred + 1;
-    a.wlist = a.deferred + 2 * (nitems + 1);
-    a.nwlist = a.ndeferred + 2;
-    a.wave_items = 1;
-    a.queue = g_scratch.queue.as<int2>();
-    a.qcap = qcap;
-    a.qcounter = g_scratch.qcounter.as<unsigned long long>();
-    a.qbase = g_scratch.qbase.as<long long>();
+  const bool bf = method == DH_BF;
+  if ((rc = g_scratch.tstats.grow(sizeof(unsigned long long) * (bf ? kBfStats : kTileStats) *
+                                  nitems)))
+    return rc;
+  DetectArgs a = detect_args(geom, pairs, npairs, nullptr, cap, tiles, tile_count, bf, pbox, bbox,
+                             psph);
+  // the queue costs launches: for many items only
+  const bool queued = bf && (learned || nitems >= tuning().detect_queue_min_items);
+  QueuePlan plan = {};
+  if (queued) {
+    plan = queue_plan(nitems, g_scratch.rwant, g_scratch.bwant);
+    if ((rc = queue_reserve(plan, nitems, learned))) return rc;
+    DH_HIP_CHECK(hipMemsetAsync(g_scratch.qcounts.ptr, 0, sizeof(unsigned) * kQueueCounts, st));
+    queue_bind(a, plan, nitems);
   }
   const size_t shm_rows = 2 * kMaxRowTriangles * sizeof(int) + 8 + kMaxRowTriangles * 8;
-  const unsigned items = static_cast<unsigned>(static_cast<long long>(npairs) * tiles);
-  if (method == DH_BF && !a.queue && pbox && bbox &&
+  const unsigned items = static_cast<unsigned>(nitems);
+  if (bf && !queued && pbox && bbox &&
       particle_max_tris(geom, st, true) > kRowBlock) {
     if ((rc = g_scratch.iskip.grow(items > 0 ? items : 1))) return rc;
     a.item_skip = g_scratch.iskip.as<unsigned char>();
   }
   switch (method) {
-    case DH_BF: launch_detect<DH_BF>(items, 0, st, a); break;
+    case DH_BF:
+      if (!queued) launch_detect<DH_BF>(items, 0, st, a);
+      else if ((rc = queue_detect(a, plan, items, learned, st))) return rc;
+      break;
     case DH_PENALTY: launch_detect<DH_PENALTY>(items, 0, st, a); break;
     case DH_PENALTY_STAT: launch_detect<DH_PENALTY_STAT>(items, 0, st, a); break;
     case DH_HYBRID_BATCH: launch_detect<DH_HYBRID_BATCH>(items, shm_rows, st, a); break;
@@ -1939,17 +2065,41 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
       return set_error(DH_ERR_UNSUPPORTED, "dh_detect_pairs: method %d", method);
   }
   DH_HIP_CHECK(hipGetLastError());
-  if (a.queue && (rc = solve_queue(a, learned, st))) return rc;
-  launch_tile_stats(a.tile_stats, ntiles, a.stats, st);
-  unsigned long long total = 0;
+  launch_tile_stats(a, st);
+  long long* offs = offs_out ? offs_out : g_scratch.offs.as<long long>();
+  auto pair_offsets = [&]() {
+    if (tiles > 1)
+      hipLaunchKernelGGL(k_tile_sums, grid_for(npairs, 256), 256, 0, st, tile_count, tiles,
+                         npairs, counts);
+    return scan_counts(counts, npairs, offs, st);
+  };
+  // the queue's contacts are counted by the pairs' offsets alone
+  if (queued && (rc = pair_offsets())) return rc;
+  unsigned long long in_temp = 0;
   int err = 0;
   unsigned long long st_host[ST_COUNT];
-  DH_HIP_CHECK(hipMemcpyAsync(&total, g_scratch.counter.ptr, sizeof(total),
+  unsigned qc[kQueueCounts] = {};
+  long long all = 0;
+  DH_HIP_CHECK(hipMemcpyAsync(&in_temp, g_scratch.counter.ptr, sizeof(in_temp),
                               hipMemcpyDeviceToHost, st));
   DH_HIP_CHECK(hipMemcpyAsync(&err, g_scratch.error.ptr, sizeof(err), hipMemcpyDeviceToHost, st));
   DH_HIP_CHECK(hipMemcpyAsync(st_host, g_scratch.stats.ptr, sizeof(st_host),
                               hipMemcpyDeviceToHost, st));
+  if (queued) {
+    DH_HIP_CHECK(hipMemcpyAsync(&all, offs + npairs, sizeof(all), hipMemcpyDeviceToHost, st));
+    DH_HIP_CHECK(hipMemcpyAsync(qc, g_scratch.qcounts.ptr, sizeof(qc), hipMemcpyDeviceToHost, st));
+  }
   DH_HIP_CHECK(hipStreamSynchronize(st));
+  if (queued) {
+    // the next call's queue holds this call's need
+    auto more = [](unsigned need, int had) {
+      const long long n = static_cast<long long>(need) + need / 4;
+      return need > static_cast<unsigned>(had) ? static_cast<int>(n < (1 << 29) ? n : 1 << 29) : 0;
+    };
+    if (const int n = more(qc[QC_RWANT], plan.rcap)) g_scratch.rwant = n;
+    if (const int n = more(qc[QC_BQUEUE], plan.bcap)) g_scratch.bwant = n;
+  }
+  const unsigned long long total = queued ? static_cast<unsigned long long>(all) : in_temp;
   if (err == DE_REF_UB)
     return set_error(DH_ERR_REF_UB,
                      "hybridWithPerTriangleFallBack reads row iA < nTriB of A: nTriB > nTriA is "
@@ -1969,17 +2119,15 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
     stats->pairs_culled += st_host[ST_CULLED];
   }
   if (static_cast<long long>(total) > cap) return DH_ERR_CAPACITY;
-  long long* offs = offs_out ? offs_out : g_scratch.offs.as<long long>();
-  if (tiles > 1)
-    hipLaunchKernelGGL(k_tile_sums, grid_for(npairs, 256), 256, 0, st, tile_count, tiles, npairs,
-                       counts);
-  if ((rc = scan_counts(counts, npairs, offs, st))) return rc;
-  if (total > 0) {
-    hipLaunchKernelGGL(k_scatter, grid_for(static_cast<int64_t>(total), 256), 256, 0, st,
-                       g_scratch.temp.as<dh_contact>(), static_cast<long long>(total), offs,
-                       tile_count, tiles, out, nullptr);
-    DH_HIP_CHECK(hipGetLastError());
-  }
+  if (!queued && (rc = pair_offsets())) return rc;
+  if (in_temp > 0)
+    hipLaunchKernelGGL(k_scatter, grid_for(static_cast<int64_t>(in_temp), 256), 256, 0, st,
+                       g_scratch.temp.as<dh_contact>(), static_cast<long long>(in_temp), offs,
+                       tile_count, tiles, out, cap, nullptr);
+  if (total > in_temp)
+    hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out, cap,
+                       nullptr);
+  DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
 
@@ -1988,13 +2136,11 @@ int detect_reserve(int pair_cap, long long contact_cap, int method);
 // Tiles of the captured step, sized for half the pair capacity live.
 static int graph_tiles(int pair_cap) { return tiles_for(pair_cap / 2 > 0 ? pair_cap / 2 : 1, DH_BF); }
 
-// Survivor-queue entries of a captured DH_BF step (0: no queue).
-static long long graph_qcap(int method, int pair_cap) {
+// Whether a captured step's detection goes through the survivor queue.
+static bool graph_queued(int method, int pair_cap) {
   const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
-  if (method == DH_BF_LEARNED) method = DH_BF;
-  else if (method != DH_BF || items < tuning().detect_queue_min_items) return 0;
-  const long long q = 16 * items + 65536;
-  return q < (1ll << 30) ? q : (1ll << 30);
+  return method == DH_BF_LEARNED ||
+         (method == DH_BF && items >= tuning().detect_queue_min_items);
 }
 
 // Detection for a captured step: launches for `pair_cap` pairs of which
@@ -2008,107 +2154,58 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
   int rc;
   if ((rc = detect_reserve(pair_cap, contact_cap, method))) return rc;
   const bool learned = method == DH_BF_LEARNED;
-  const long long qcap = graph_qcap(method, pair_cap);
+  const bool queued = graph_queued(method, pair_cap);
   if (learned) method = DH_BF;
   zero_async(ZeroRegions{{g_scratch.counter.as<unsigned>(), g_scratch.stats.as<unsigned>(),
                           g_scratch.error.as<unsigned>(),
-                          qcap > 0 ? g_scratch.qcounter.as<unsigned>() : nullptr},
-                         {2, 2 * ST_COUNT, 1, 2}},
+                          queued ? g_scratch.qcounts.as<unsigned>() : nullptr},
+                         {2, 2 * ST_COUNT, 1, kQueueCounts}},
              st);
-  DetectArgs a;
-  a.x = geom->x;
-  a.y = geom->y;
-  a.z = geom->z;
-  a.tri_offset = geom->tri_offset;
-  a.eps = geom->eps;
-  a.friction = geom->friction;
-  a.id = geom->id;
-  a.pairs = pairs;
-  a.npairs = pair_cap;
-  a.temp = g_scratch.temp.as<dh_contact>();
-  a.cap = contact_cap;
-  a.counter = g_scratch.counter.as<unsigned long long>();
   const int tiles = graph_tiles(pair_cap);
-  a.tiles = tiles;
-  a.tile_count = tiles > 1 ? g_scratch.tiles.as<int>() : counts;
-  const long long ntiles = static_cast<long long>(pair_cap) * tiles;
-  a.tile_stats = g_scratch.tstats.as<unsigned long long>();
-  a.stats = g_scratch.stats.as<unsigned long long>();
-  a.error = g_scratch.error.as<int>();
-  a.npairs_dev = np_dev;
-  a.pbox = pbox;
-  a.psph = pbox ? psph : nullptr;
-  a.fp32_screen = tuning().detect_fp32_screen;
-  a.wave_items = 0;
-  a.item_skip = nullptr;
-  a.bbox = bbox;
-  a.queue = nullptr;  // the queue needs the survivor count on the host
-  a.qcap = 0;
-  a.qcounter = nullptr;
-  a.qbase = nullptr;
-  a.deferred = nullptr;
-  a.ndeferred = nullptr;
-  a.biglist = nullptr;
-  a.nbig = nullptr;
-  a.wlist = nullptr;
-  a.nwlist = nullptr;
-  a.item_list = nullptr;
-  a.nitems_dev = nullptr;
+  const bool bf = method == DH_BF;
+  DetectArgs a = detect_args(geom, pairs, pair_cap, np_dev, contact_cap, tiles,
+                             tiles > 1 ? g_scratch.tiles.as<int>() : counts, bf, pbox, bbox, psph);
   const unsigned items = static_cast<unsigned>(static_cast<long long>(pair_cap) * tiles);
   // the chunk pre-pass on the geometries detect_prepare found walls in
-  if (method == DH_BF && qcap == 0 && pbox && bbox &&
-      particle_max_tris(geom, st, false) > kRowBlock)
+  if (bf && !queued && pbox && bbox && particle_max_tris(geom, st, false) > kRowBlock)
     a.item_skip = g_scratch.iskip.as<unsigned char>();
-  if (qcap > 0) {
-    // the survivor queue with its counts kept on the device: every pass is
-    // launched for the capacity and reads the live length
-    fill_async(g_scratch.ndeferred.as<unsigned>(), 0u, 3, st);
-    a.queue = g_scratch.queue.as<int2>();
-    a.qcap = qcap;
-    a.qcounter = g_scratch.qcounter.as<unsigned long long>();
-    a.qbase = g_scratch.qbase.as<long long>();
-    a.deferred = g_scratch.deferred.as<int>();
-    a.ndeferred = g_scratch.ndeferred.as<unsigned>();
-    a.biglist = a.deferred + (items + 1);
-    a.nbig = a.ndeferred + 1;
-    a.wlist = a.deferred + 2 * (items + 1);
-    a.nwlist = a.ndeferred + 2;
-    a.wave_items = 1;
+  QueuePlan plan = {};
+  if (queued) {
+    plan = queue_plan(items, 0, 0);
+    queue_bind(a, plan, items);
   }
   switch (method) {
-    case DH_BF: launch_detect<DH_BF>(items, 0, st, a); break;
+    case DH_BF:
+      if (!queued) launch_detect<DH_BF>(items, 0, st, a);
+      else if ((rc = queue_detect(a, plan, items, learned, st))) return rc;
+      break;
     case DH_PENALTY: launch_detect<DH_PENALTY>(items, 0, st, a); break;
     default:
       return set_error(DH_ERR_UNSUPPORTED, "captured step: method %d (use DH_BF or DH_PENALTY)",
                        method);
   }
-  if (a.queue) {
-    // the items the mid-phase launch could not queue, in full (as many as
-    // *ndeferred of the capacity), then the queue's passes
-    DetectArgs f = a;
-    f.queue = nullptr;
-    f.item_list = a.deferred;
-    f.nitems_dev = a.ndeferred;
-    // persistent over the deferred items (usually none): a grid for the
-    // capacity would cost a dispatch per item
-    const unsigned dcap = static_cast<unsigned>(device_cus()) * 4;
-    const unsigned dgrid = detect_grid(items) < dcap ? detect_grid(items) : dcap;
-    hipLaunchKernelGGL((k_detect<DH_BF, false>), dgrid, 256, 0, st, f, static_cast<int>(items));
-    if ((rc = queue_passes(a, a.qcap, a.qcounter, learned, st))) return rc;
-  }
   if (pair_cap <= kTailPairs) {
-    hipLaunchKernelGGL(k_detect_tail_small, 1, 1024, 0, st, a.tile_stats, ntiles, a.stats,
-                       a.tile_count, tiles, pair_cap, counts, offs);
+    const auto f = bf ? k_detect_tail_small<kBfStats> : k_detect_tail_small<kTileStats>;
+    hipLaunchKernelGGL(f, 1, 1024, 0, st, a.tile_stats, np_dev, a.stats, a.tile_count, tiles,
+                       pair_cap, counts, offs);
   } else {
-    launch_tile_stats(a.tile_stats, ntiles, a.stats, st);
+    launch_tile_stats(a, st);
     if (tiles > 1)
       hipLaunchKernelGGL(k_tile_sums, grid_for(pair_cap, 256), 256, 0, st, a.tile_count, tiles,
                          pair_cap, counts);
-    if ((rc = scan_counts(counts, pair_cap, offs, st))) return rc;
+    if ((rc = g_scratch.sums.grow(sizeof(long long) * scan_sums_len(pair_cap)))) return rc;
+    // the live pairs' counts (the pairs past them have none)
+    if ((rc = scan_counts_upto(counts, pair_cap,
+                               reinterpret_cast<const unsigned long long*>(np_dev), offs,
+                               g_scratch.sums.as<long long>(), st)))
+      return rc;
   }
   hipLaunchKernelGGL(k_scatter, grid_for(contact_cap, 256), 256, 0, st,
                      g_scratch.temp.as<dh_contact>(), contact_cap, offs, a.tile_count, tiles, out,
-                     g_scratch.counter.as<unsigned long long>());
+                     contact_cap, g_scratch.counter.as<unsigned long long>());
+  if (queued)
+    hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out,
+                       contact_cap, g_scratch.counter.as<unsigned long long>());
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
@@ -2117,23 +2214,15 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
 // happen inside one).
 int detect_reserve(int pair_cap, long long contact_cap, int method) {
   int rc;
-  const long long qcap = graph_qcap(method, pair_cap);
-  if (qcap > 0) {
+  if (graph_queued(method, pair_cap)) {
     const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
-    if ((rc = g_scratch.queue.grow(sizeof(int2) * qcap))) return rc;
-    if ((rc = g_scratch.qcounter.grow(sizeof(unsigned long long)))) return rc;
-    if ((rc = g_scratch.qbase.grow(sizeof(long long) * (items + 1)))) return rc;
-    if ((rc = g_scratch.deferred.grow(sizeof(int) * 3 * (items + 1)))) return rc;
-    if ((rc = g_scratch.ndeferred.grow(sizeof(unsigned) * 3))) return rc;
-    if ((rc = queue_reserve(qcap))) return rc;
-    if (method == DH_BF_LEARNED && (rc = queue_learned_reserve(qcap))) return rc;
+    if ((rc = queue_reserve(queue_plan(items, 0, 0), items, method == DH_BF_LEARNED))) return rc;
   }
   if ((rc = g_scratch.temp.grow(sizeof(dh_contact) * (contact_cap > 0 ? contact_cap : 1)))) return rc;
   if ((rc = g_scratch.counter.grow(sizeof(unsigned long long)))) return rc;
   if ((rc = g_scratch.stats.grow(sizeof(unsigned long long) * ST_COUNT))) return rc;
   if ((rc = g_scratch.error.grow(sizeof(int)))) return rc;
-  const int nb = (pair_cap + 1023) / 1024 > 0 ? (pair_cap + 1023) / 1024 : 1;
-  if ((rc = g_scratch.sums.grow(sizeof(long long) * (nb + 1)))) return rc;
+  if ((rc = g_scratch.sums.grow(sizeof(long long) * scan_sums_len(pair_cap)))) return rc;
   const int tiles = graph_tiles(pair_cap);
   if (tiles > 1 &&
       (rc = g_scratch.tiles.grow(sizeof(int) * static_cast<size_t>(pair_cap) * tiles)))

@@ -635,7 +635,8 @@ DH_HD bool edge_axes_apart(const Tri<double>& A, const Tri<double>& B, double th
   return false;
 }
 
-DH_HD bool plane_apart(const Tri<double>& A, const Tri<double>& B, double margin) {
+// The margin with its rounding band for the axes of A and B.
+DH_HD double axis_reach(const Tri<double>& A, const Tri<double>& B, double margin) {
   using std::fabs;
   double mag = 0.0;
 #pragma unroll
@@ -643,21 +644,17 @@ DH_HD bool plane_apart(const Tri<double>& A, const Tri<double>& B, double margin
     mag = fmax(mag, fmax(fmax(fabs(A.v[k].x), fabs(A.v[k].y)),
                          fmax(fmax(fabs(A.v[k].z), fabs(B.v[k].x)),
                               fmax(fabs(B.v[k].y), fabs(B.v[k].z)))));
-  const double thr = margin * (1.0 + 0x1p-20) + mag * 0x1p-40;
+  return margin * (1.0 + 0x1p-20) + mag * 0x1p-40;
+}
+
+DH_HD bool plane_apart(const Tri<double>& A, const Tri<double>& B, double margin) {
+  const double thr = axis_reach(A, B, margin);
   return plane_side_apart(A, B, thr) || plane_side_apart(B, A, thr);
 }
 
 // plane_apart, then the edge-pair axes (for the pairs the planes leave).
 DH_HD bool axes_apart(const Tri<double>& A, const Tri<double>& B, double margin) {
-  using std::fabs;
-  if (plane_apart(A, B, margin)) return true;
-  double mag = 0.0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    mag = fmax(mag, fmax(fmax(fabs(A.v[k].x), fabs(A.v[k].y)),
-                         fmax(fmax(fabs(A.v[k].z), fabs(B.v[k].x)),
-                              fmax(fabs(B.v[k].y), fabs(B.v[k].z)))));
-  return edge_axes_apart(A, B, margin * (1.0 + 0x1p-20) + mag * 0x1p-40);
+  return plane_apart(A, B, margin) || edge_axes_apart(A, B, axis_reach(A, B, margin));
 }
 
 // Screen before bfSolver in binary64: true when A and B are provably farther

@@ -777,23 +777,26 @@ k_learned(LearnedArgs a) {
 
 // ------------------------------------------------ the step's survivor queue
 // The triangle pairs that the DEM step's box mid-phase leaves (the survivor
-// queue of detect.hip, entries {item, iA | iB << 16}) through the learned
-// decision: a wave per 64 entries on a persistent grid.  A finished entry
+// queue of detect.hip, entries {item, triangle of A, triangle of B, ..} in
+// regions and ranges) through the learned decision: a wave per region or range
+// at a time, 64 entries in a round.  A finished entry
 // sets flags[e] (its pair emits a contact: d <= epsA + epsB, bf.cpp:125) and,
 // when it emits, its P, Q at pq[6e..6e+6); the rest are listed for the
 // brute force (k_queue_fallback).  Both write exactly what the brute-force
 // queue solve would.
 struct QueueLearnArgs {
-  const int2* queue;
+  const int4* queue;
   const int* pairs;
   int tiles;  // items per particle pair
-  const int* tri_offset;
+  int regions, rcap;     // region r: rcount[r] entries from r * rcap
+  const int* rcount;
+  const int4* ranges;    // then the ranges {first, length}, from regions * rcap
+  const unsigned* nranges;
   const double* x;
   const double* y;
   const double* z;
   const double* eps;
-  long long n;                         // entries of the launch
-  const unsigned long long* need_dev;  // live entries (captured step), else null
+  long long n;  // entries the queue can hold
   int* flags;
   double* pq;
   const float* W;
@@ -815,62 +818,60 @@ k_queue_learned(QueueLearnArgs a) {
   __shared__ LearnedLds L;
   stage_network<kModeFeatures>(L, a.W);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long long live =
-      a.need_dev && static_cast<long long>(*a.need_dev) < a.n ? static_cast<long long>(*a.need_dev)
-                                                              : a.n;
-  // the live entries only (the later passes stop at the same count)
-  const long long nchunks = (live + 63) / 64;
   unsigned evals = 0;
-  for (long long ch = static_cast<long long>(blockIdx.x) * kInferWaves + wave; ch < nchunks;
-       ch += static_cast<long long>(gridDim.x) * kInferWaves) {
-    const long long e = ch * 64 + lane;
-    const int2 en = e < live ? a.queue[e] : make_int2(-1, 0);
-    const bool valid = en.x >= 0;
-    Tri<double> A = {}, B = {};
-    double margin = 0.0;
-    if (valid) {
-      const int k = en.x / a.tiles;
-      const int pa = a.pairs[2 * k], pb = a.pairs[2 * k + 1];
-      const int iA = static_cast<int>(static_cast<unsigned>(en.y) & 0xffffu);
-      const int iB = static_cast<int>(static_cast<unsigned>(en.y) >> 16);
-      A = load_tri_xyz(a.x, a.y, a.z, a.tri_offset[pa] + iA);
-      B = load_tri_xyz(a.x, a.y, a.z, a.tri_offset[pb] + iB);
-      margin = a.eps[pa] + a.eps[pb];
-    }
-    V3<double> P, Q;
-    bool done;
-    learned_pair<kModeFeatures>(L, A, B, valid, P, Q, done, evals);
-    if (e < live && !(valid && !done)) {
-      const bool emit = valid && pq_dist(P, Q) <= margin;
-      a.flags[e] = emit ? 1 : 0;
-      if (emit) {
-        double* o = a.pq + 6 * e;
-        o[0] = P.x; o[1] = P.y; o[2] = P.z;
-        o[3] = Q.x; o[4] = Q.y; o[5] = Q.z;
+  const int nr = static_cast<int>(*a.nranges);
+  const long long big = static_cast<long long>(a.regions) * a.rcap;
+  for (int u = blockIdx.x * kInferWaves + wave; u < a.regions + nr;
+       u += gridDim.x * kInferWaves) {
+    const bool is_range = u >= a.regions;
+    const int4 range = is_range ? a.ranges[u - a.regions] : make_int4(0, 0, 0, 0);
+    const long long at = is_range ? big + range.x : static_cast<long long>(u) * a.rcap;
+    const int live = is_range ? range.y : a.rcount[u];
+    for (int base = 0; base < live; base += 64) {
+      const long long e = at + base + lane;
+      const int4 en = base + lane < live ? a.queue[e] : make_int4(-1, 0, 0, 0);
+      const bool valid = en.x >= 0;
+      Tri<double> A = {}, B = {};
+      double margin = 0.0;
+      if (valid) {
+        const int k = en.x / a.tiles;
+        A = load_tri_xyz(a.x, a.y, a.z, en.y);
+        B = load_tri_xyz(a.x, a.y, a.z, en.z);
+        margin = a.eps[a.pairs[2 * k]] + a.eps[a.pairs[2 * k + 1]];
       }
-    }
-    // the rest to the brute force: one append per wave
-    const bool need = valid && !done;
-    const unsigned long long mask = __ballot(need);
-    if (mask) {
-      unsigned base = 0;
-      if (lane == 0) base = atomicAdd(a.fb_count, static_cast<unsigned>(__popcll(mask)));
-      base = __shfl(base, 0);
-      const int pre = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
-                                                __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0));
-      if (need) a.fb_list[base + pre] = static_cast<int>(e);
+      V3<double> P, Q;
+      bool done;
+      learned_pair<kModeFeatures>(L, A, B, valid, P, Q, done, evals);
+      if (base + lane < live && !(valid && !done)) {
+        const bool emit = valid && pq_dist(P, Q) <= margin;
+        a.flags[e] = emit ? 1 : 0;
+        if (emit) {
+          double* o = a.pq + 6 * e;
+          o[0] = P.x; o[1] = P.y; o[2] = P.z;
+          o[3] = Q.x; o[4] = Q.y; o[5] = Q.z;
+        }
+      }
+      // the rest to the brute force: one append per wave
+      const bool need = valid && !done;
+      const unsigned long long mask = __ballot(need);
+      if (mask) {
+        unsigned slot = 0;
+        if (lane == 0) slot = atomicAdd(a.fb_count, static_cast<unsigned>(__popcll(mask)));
+        slot = __shfl(slot, 0);
+        const int pre = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0));
+        if (need) a.fb_list[slot + pre] = static_cast<int>(e);
+      }
     }
   }
 }
 
 __device__ __forceinline__ void queue_fallback_entry(const QueueLearnArgs& a, long long e) {
-  const int2 en = a.queue[e];
+  const int4 en = a.queue[e];
   const int k = en.x / a.tiles;
   const int pa = a.pairs[2 * k], pb = a.pairs[2 * k + 1];
-  const int iA = static_cast<int>(static_cast<unsigned>(en.y) & 0xffffu);
-  const int iB = static_cast<int>(static_cast<unsigned>(en.y) >> 16);
-  const Tri<double> A = load_tri_xyz(a.x, a.y, a.z, a.tri_offset[pa] + iA);
-  const Tri<double> B = load_tri_xyz(a.x, a.y, a.z, a.tri_offset[pb] + iB);
+  const Tri<double> A = load_tri_xyz(a.x, a.y, a.z, en.y);
+  const Tri<double> B = load_tri_xyz(a.x, a.y, a.z, en.z);
   V3<double> P, Q;
   bf_solver(A, B, P, Q);
   const bool emit = pq_dist(P, Q) <= a.eps[pa] + a.eps[pb];
@@ -911,31 +912,27 @@ int queue_learned_reserve(long long n) {
   return g_qlearn.fb_count.grow(sizeof(unsigned));
 }
 
-// The survivor queue's n entries (live: *need_dev when set) through the
-// learned decision, then the brute force for the rest; fills instead of
-// memsets (captured steps).
-int queue_learned(const int2* queue, const int* pairs, int tiles, const int* tri_offset,
+// The survivor queue's entries through the learned decision, then the brute
+// force for the rest; a fill instead of a memset (captured steps).
+int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
+                  const int* rcount, const int4* ranges, const unsigned* nranges,
                   const double* x, const double* y, const double* z, const double* eps,
-                  long long n, const unsigned long long* need_dev, int* flags, double* pq,
-                  hipStream_t st) {
+                  long long n, int* flags, double* pq, hipStream_t st) {
   if (!g_learned.model)
     return set_error(DH_ERR_ARG, "DH_BF_LEARNED: no network set (dh_learned_set_model)");
   int rc;
   if ((rc = queue_learned_reserve(n))) return rc;
-  QueueLearnArgs a{queue, pairs, tiles, tri_offset, x, y, z, eps, n, need_dev, flags, pq,
-                   g_learned.model, g_qlearn.fb_list.as<int>(), g_qlearn.fb_count.as<unsigned>()};
+  QueueLearnArgs a{queue, pairs, tiles, regions, rcap, rcount, ranges, nranges, x, y, z, eps, n,
+                   flags, pq, g_learned.model, g_qlearn.fb_list.as<int>(),
+                   g_qlearn.fb_count.as<unsigned>()};
   fill_async(g_qlearn.fb_count.as<unsigned>(), 0u, 1, st);
-  if (n > 0) {
-    const long long chunks = (n + 63) / 64;
-    long long grid = (chunks + kInferWaves - 1) / kInferWaves;
-    const long long max_grid = static_cast<long long>(device_cus()) * 4;
-    if (grid > max_grid) grid = max_grid;
-    hipLaunchKernelGGL(k_queue_learned, static_cast<unsigned>(grid), 64 * kInferWaves, 0, st, a);
-    long long fgrid = grid_for(n, 256);
-    const long long fcap = static_cast<long long>(device_cus()) * 16;
-    if (need_dev && fgrid > fcap) fgrid = fcap;
-    hipLaunchKernelGGL(k_queue_fallback, static_cast<unsigned>(fgrid), 256, 0, st, a);
-  }
+  const long long cus = device_cus();
+  long long grid = (regions + kInferWaves - 1) / kInferWaves;
+  if (grid > 4 * cus) grid = 4 * cus;
+  hipLaunchKernelGGL(k_queue_learned, static_cast<unsigned>(grid), 64 * kInferWaves, 0, st, a);
+  long long fgrid = grid_for(n, 256);
+  if (fgrid > 16 * cus) fgrid = 16 * cus;
+  hipLaunchKernelGGL(k_queue_fallback, static_cast<unsigned>(fgrid), 256, 0, st, a);
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
