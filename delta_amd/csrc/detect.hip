@@ -98,30 +98,18 @@ struct DetectArgs {
   // Survivor queue of a DH_BF launch (null: every item solves its own
   // survivors).  Wave r of k_detect_wave appends its items' survivors to its
   // own region queue[r * rcap ..] and leaves their number in rcount[r], so
-  // that no wave waits for a counter that all share.  An item of k_detect_big
-  // appends to bqueue (which follows the regions) through bcounter, as one range that it lists
-  // ({first, length, item, contacts}); a range that does not fit in bcap
-  // entries is filled with item -1 as far as it lies inside.  An item that
-  // cannot queue goes to `deferred`, for a second launch that runs those items
-  // in full, taking its items from item_list.
+  // that no wave waits for a counter that all share.  An item that cannot
+  // queue goes to `deferred`, for a launch that runs those items in full,
+  // taking its items from item_list.
   int4* queue;  // {item, triangle of A, triangle of B, iA | iB << 16}
   int rcap, regions;
   int* rcount;
-  int* rwant;  // [0]: most entries that a region had to hold, when more than rcap
-  int4* bqueue;
-  int bcap;
-  unsigned* bcounter;
-  int4* ranges;
-  unsigned* nranges;
+  int* rwant;  // most entries that a region had to hold, when more than rcap
   // contacts of the queue's entries, in the entries' order, from the place of
-  // the region's or range's first entry; region r's number in
-  // rcount[regions + r], a range's in the range
+  // the region's first entry; region r's number in rcount[regions + r]
   struct QueueRecord* rec;
   int* deferred;
   unsigned* ndeferred;
-  // Items for k_detect_big: rows or columns that k_detect_wave does not take
-  int* biglist;
-  unsigned* nbig;
   // Items k_lane_cull leaves for k_detect_wave
   struct WaveItem* wlist;
   unsigned* nwlist;
@@ -133,19 +121,16 @@ struct DetectArgs {
   const unsigned char* item_skip;
 };
 
-// Items of the queue path that take one wave each: at most kWaveScan rows and
-// columns, of which at most kWaveRows each stay after the tests against the
-// other particle (their boxes are held in LDS).
-constexpr int kWaveScan = 320;
-constexpr int kWaveRows = 80;
-constexpr int kWaveSurvivors = 256;  // survivors listed per wave
+// Triangles of A's rows and B's columns, together, whose boxes a wave of
+// k_detect_wave holds in LDS after the tests against the other particle.
+constexpr int kWaveBoxes = 160;
 constexpr int kWavesPerGroup = 2;    // of k_detect_wave
 
 struct WaveItem {
   int item, pa, pb;
-  int tA, tB;      // first triangles of the rows and of B
+  int oA, oB;      // first triangles of A and of B
   int r0, nrows;   // rows [r0, r0 + nrows) of A
-  int nB;
+  int nB, chunked; // chunked: A's 64-row chunks have boxes in bbox
   double epsA, epsB;
 };
 
@@ -322,7 +307,7 @@ __device__ __forceinline__ void make_contact(const Pair& p, int k, int iA, int i
 // One (particle pair, row range) item of the detection: `item` = pair *
 // tiles + tile.  Returns when the item is done; the caller synchronises the
 // workgroup before its next item.
-template <int M, bool QONLY>
+template <int M>
 __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item) {
   extern __shared__ unsigned char smem[];
   __shared__ int wave_cnt[4];
@@ -333,7 +318,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   unsigned long long* ts = g.tile_stats + static_cast<long long>(item) * g.nstats;
-  if (M == DH_BF && !QONLY && g.item_skip && g.item_skip[item]) return;  // k_chunk_cull's
+  if (M == DH_BF && g.item_skip && g.item_skip[item]) return;  // k_chunk_cull's
   if (g.npairs_dev && k >= *g.npairs_dev) {
     if (tid == 0) g.tile_count[item] = 0;
     if (tid < g.nstats) ts[tid] = 0;
@@ -473,22 +458,6 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
     const bool staged = p.nB <= kBoxTriangles;  // block-uniform
     const int blk = staged ? kBoxTriangles : (nrows > 0 ? nrows : 1);
     bool b_staged = false;  // B's boxes are loaded on the first block that needs them
-    int q_first = 0;  // the item's queue range, when a block appended one
-    int q_len = 0;
-    // mid-phase-only launch: an item that cannot queue its survivors is
-    // handed to the full launch (which also writes its counters)
-    auto defer = [&]() {
-      if (tid == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = item;
-    };
-    // an item that defers after one of its blocks has appended its range
-    auto void_range = [&]() {
-      for (int q = q_first + tid; q < q_first + q_len; q += 256)
-        g.bqueue[q] = make_int4(-1, 0, 0, 0);
-    };
-    if (QONLY && !(staged && p.nA < 65536 && p.nB < 65536)) {
-      defer();
-      return;
-    }
     // the whole pair beyond the margin by its bounding spheres
     const bool far_pair = spheres_apart(g, p);
     if (far_pair) culled += tid == 0 ? static_cast<unsigned>(nrows * p.nB) : 0u;
@@ -626,7 +595,6 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
       culled += tid == 0 ? static_cast<unsigned>(nrb * p.nB - tested) : 0u;
       for (int fpos = 0; fpos < tested;) {
         int nl = 0;
-        const bool first = fpos == 0;
         while (fpos < tested && nl <= kSurvivors - 256) {
           const int fe = fpos + tid;
           bool keep = false;
@@ -655,84 +623,39 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
           fpos += 256;
           __syncthreads();
         }
-        if (QONLY && fpos < tested) {  // more survivors than the LDS list holds
-          void_range();
-          defer();
-          return;
-        }
-        if (QONLY && first && fpos >= tested && staged && !(nl > 0 && q_len > 0)) {
-          // every survivor of the block is in LDS: append them, in row-major
-          // order, as the item's one range of the survivor queue (solved
-          // there with every lane busy)
-          if (tid == 0 && nl > 0) chunk_base = atomicAdd(g.bcounter, static_cast<unsigned>(nl));
-          __syncthreads();
-          const unsigned qb = nl > 0 ? static_cast<unsigned>(chunk_base) : 0u;
-          __syncthreads();
-          if (static_cast<long long>(qb) + nl <= g.bcap) {
-            if (nl > 0) {
-              q_first = static_cast<int>(qb);
-              q_len = nl;
-              if (tid == 0)
-                g.ranges[atomicAdd(g.nranges, 1u)] = make_int4(q_first, q_len, item, 0);
-            }
-            for (int e = tid; e < nl; e += 256) {
-              int iA, iB;
-              pair_of(surv[e], iA, iB);
-              g.bqueue[qb + e] = make_int4(
-                  item, p.oA + iA, p.oB + iB,
-                  static_cast<int>(static_cast<unsigned>(iA) | (static_cast<unsigned>(iB) << 16)));
-            }
-            continue;  // fpos >= tested: the block is done
+        // the survivors that a triangle plane separates by more than the
+        // margin (and, with the binary32 screen, those it proves far) drop
+        // out; the rest are compacted in place (order kept) for the
+        // binary64 solve.  (The edge-pair axes of the queue paths do not
+        // pay here: an item keeps one wave's bfSolver round as long as a
+        // survivor is left, whatever their number.)
+        int n2 = 0;
+        for (int b = 0; b < nl; b += 256) {
+          const int e = b + tid;
+          int v = 0;
+          bool keep2 = false;
+          if (e < nl) {
+            v = surv[e];
+            int iA, iB;
+            pair_of(v, iA, iB);
+            const Tri<double> A = load_tri(g, p.oA + iA), B = load_tri(g, p.oB + iB);
+            keep2 = !plane_apart(A, B, p.margin) &&
+                    !(g.fp32_screen && screened_far(A, B, p.margin));
           }
-          for (long long q = static_cast<long long>(qb) + tid; q < static_cast<long long>(qb) + nl &&
-                                                               q < g.bcap; q += 256)
-            g.bqueue[q] = make_int4(-1, 0, 0, 0);
-          void_range();
-          defer();
-          return;
-        }
-        if (QONLY && nl > 0) {
-          // a second block with survivors: the item's survivors would not
-          // be one range; void the first and run the item in full
-          void_range();
-          defer();
-          return;
-        }
-        if (!QONLY) {
-          // the survivors that a triangle plane separates by more than the
-          // margin (and, with the binary32 screen, those it proves far) drop
-          // out; the rest are compacted in place (order kept) for the
-          // binary64 solve.  (The edge-pair axes of the queue paths do not
-          // pay here: an item keeps one wave's bfSolver round as long as a
-          // survivor is left, whatever their number.)
-          int n2 = 0;
-          for (int b = 0; b < nl; b += 256) {
-            const int e = b + tid;
-            int v = 0;
-            bool keep2 = false;
-            if (e < nl) {
-              v = surv[e];
-              int iA, iB;
-              pair_of(v, iA, iB);
-              const Tri<double> A = load_tri(g, p.oA + iA), B = load_tri(g, p.oB + iB);
-              keep2 = !plane_apart(A, B, p.margin) &&
-                      !(g.fp32_screen && screened_far(A, B, p.margin));
-            }
-            const unsigned long long m = __ballot(keep2);
-            if (lane == 0) wave_cnt[wave] = __popcll(m);
-            __syncthreads();
-            int off = 0, cnt = 0;
-            for (int w = 0; w < 4; ++w) {
-              off += (w < wave) ? wave_cnt[w] : 0;
-              cnt += wave_cnt[w];
-            }
-            if (keep2) surv[n2 + off + lane_prefix(m)] = v;
-            n2 += cnt;
-            __syncthreads();
+          const unsigned long long m = __ballot(keep2);
+          if (lane == 0) wave_cnt[wave] = __popcll(m);
+          __syncthreads();
+          int off = 0, cnt = 0;
+          for (int w = 0; w < 4; ++w) {
+            off += (w < wave) ? wave_cnt[w] : 0;
+            cnt += wave_cnt[w];
           }
-          nl = n2;
+          if (keep2) surv[n2 + off + lane_prefix(m)] = v;
+          n2 += cnt;
+          __syncthreads();
         }
-        for (int b = 0; b < (QONLY ? 0 : nl); b += 256) {
+        nl = n2;
+        for (int b = 0; b < nl; b += 256) {
           const int e = b + tid;
           bool emit = false;
           V3<double> P = {0, 0, 0}, Q = {0, 0, 0};
@@ -814,24 +737,13 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
 // workgroups of one launch.  The brute force is held to 168 registers
 // (three waves per SIMD; a few spill), which its latency-bound item loop
 // needs more than the registers.
-template <int M, bool QONLY = false>
+template <int M>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(M == DH_BF && !QONLY ? 3 : 1))) void k_detect(DetectArgs g,
-                                                                                 int items) {
+__attribute__((amdgpu_waves_per_eu(M == DH_BF ? 3 : 1))) void k_detect(DetectArgs g, int items) {
   if (g.item_list && g.nitems_dev && static_cast<int>(*g.nitems_dev) < items)
     items = static_cast<int>(*g.nitems_dev);
   for (int t = blockIdx.x; t < items; t += gridDim.x) {
-    detect_item<M, QONLY>(g, g.item_list ? g.item_list[t] : t);
-    __syncthreads();  // the next item reuses the workgroup's LDS
-  }
-}
-
-// The workgroup mid-phase for the items that k_detect_wave does not take (listed
-// by k_lane_cull) or hands over.
-__global__ __launch_bounds__(256) void k_detect_big(DetectArgs g) {
-  const int nb = static_cast<int>(*g.nbig);
-  for (int j = blockIdx.x; j < nb; j += gridDim.x) {
-    detect_item<DH_BF, true>(g, g.biglist[j]);
+    detect_item<M>(g, g.item_list ? g.item_list[t] : t);
     __syncthreads();  // the next item reuses the workgroup's LDS
   }
 }
@@ -911,16 +823,16 @@ constexpr int kLaneRows = 16;
 // particle box (grown by the margin: a wall of few triangles against the many
 // particles inside it), is culled here, with the counters the mid-phase would
 // write.  The others are listed for k_detect_wave with what it needs of them
-// (its loads of triangles then wait for one load, not for three in a row), or,
-// above kWaveScan rows or columns, for k_detect_big.  One atomic per workgroup
-// and list: one per wave took most of the 43 us that the hopper's 3.8e5 items
-// spent here.
+// (its loads of triangles then wait for one load, not for three in a row).
+// Items whose triangle numbers do not fit a queue entry are deferred.  One
+// atomic per workgroup and list: one per wave took most of the 43 us that the
+// hopper's 3.8e5 items spent here (11 us now).
 __global__ __launch_bounds__(1024) void k_lane_cull(DetectArgs g, int items) {
-  __shared__ unsigned wave_cnt[2][16], base[2];
+  __shared__ unsigned wave_cnt[16], base;
   const int tid = static_cast<int>(threadIdx.x);
   const int item = blockIdx.x * 1024 + tid;
   const int wave = tid >> 6;
-  int list = -1;  // 0: k_detect_wave, 1: k_detect_big
+  bool listed = false;
   WaveItem it = {};
   if (item < items) {
     const int k = item / g.tiles, tile = item - k * g.tiles;
@@ -943,32 +855,31 @@ __global__ __launch_bounds__(1024) void k_lane_cull(DetectArgs g, int items) {
           near = !boxes_apart(lo, hi, pb, pb + 3, p.margin);
         }
       }
-      if (near && total > 0)
-        list = nrows <= kWaveScan && p.nB <= kWaveScan && p.nA < 65536 ? 0 : 1;
       ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
       ts[TS_EVALUATED] = total;
       ts[TS_CULLED] = total;  // a listed item's own kernel writes its count
-      it = {item, p.pa, p.pb, p.oA + r0, p.oB, r0, nrows, p.nB, p.epsA, p.epsB};
+      if (near && total > 0) {
+        listed = p.nA < 65536 && p.nB < 65536;
+        if (!listed) g.deferred[atomicAdd(g.ndeferred, 1u)] = item;
+      }
+      it = {item, p.pa, p.pb, p.oA, p.oB, r0, nrows, p.nB,
+            g.pbox && g.bbox && p.nA > kRowBlock ? 1 : 0, p.epsA, p.epsB};
     }
   }
-  const unsigned long long m0 = __ballot(list == 0), m1 = __ballot(list == 1);
-  if ((tid & 63) == 0) {
-    wave_cnt[0][wave] = static_cast<unsigned>(__popcll(m0));
-    wave_cnt[1][wave] = static_cast<unsigned>(__popcll(m1));
-  }
+  const unsigned long long m = __ballot(listed);
+  if ((tid & 63) == 0) wave_cnt[wave] = static_cast<unsigned>(__popcll(m));
   __syncthreads();
-  if (tid < 2) {
+  if (tid == 0) {
     unsigned n = 0;
     for (int w = 0; w < 16; ++w) {
-      const unsigned c = wave_cnt[tid][w];
-      wave_cnt[tid][w] = n;
+      const unsigned c = wave_cnt[w];
+      wave_cnt[w] = n;
       n += c;
     }
-    base[tid] = n ? atomicAdd(tid == 0 ? g.nwlist : g.nbig, n) : 0u;
+    base = n ? atomicAdd(g.nwlist, n) : 0u;
   }
   __syncthreads();
-  if (list == 0) g.wlist[base[0] + wave_cnt[0][wave] + lane_prefix(m0)] = it;
-  if (list == 1) g.biglist[base[1] + wave_cnt[1][wave] + lane_prefix(m1)] = item;
+  if (listed) g.wlist[base + wave_cnt[wave] + lane_prefix(m)] = it;
 }
 
 // Orders a wave's LDS writes before its later reads of other lanes' values.
@@ -990,24 +901,23 @@ __device__ __forceinline__ double box_gap(const double* loA, const double* hiA, 
 // The mid-phase of DH_BF, one wave per listed item and no workgroup barrier:
 // the boxes of A's rows and B's columns that lie within the margin of the
 // other particle's box and bounding sphere are kept, in order, in the wave's
-// LDS; the pairs of kept rows and columns whose boxes are within the margin
-// are listed in row-major order and appended to the wave's region of the
-// survivor queue.  Items with more than kWaveRows kept rows or columns go to
-// k_detect_big, items whose survivors overflow the list or the region to the
-// full kernel.  Same survivors and counters as detect_item's box test.
+// LDS (the rows of a large A chunk by chunk, those of far chunks unread); the
+// pairs of kept rows and columns whose boxes are within the margin are
+// appended, in row-major order, to the wave's region of the survivor queue.
+// Items with more than kWaveBoxes kept rows and columns, or more survivors
+// than the region has room for, are deferred to the full kernel.  Same
+// survivors and counters as detect_item's box test.
 // It is bound by the latency of an item's loads, so it holds little: 16 waves
-// per CU (LDS) at the 128 registers that allow them.  Separating axes are
-// tested in k_queue_solve instead, with every lane busy (here they took 161
-// registers, 9 waves per CU, for some 10 to 40 survivors at a time), and the
-// other particle's box from the broad phase takes the place of the union of
-// its triangles' boxes (144 lane shuffles per item).  What it cost before was
-// an atomic per item on one queue counter, some 10 ns each: 610 us for the
-// hopper's 1.9e5 pairs, 87 us with a region per wave (8 workgroups per CU; 6
-// per CU: 100 us).
+// per CU.  Separating axes are tested in k_queue_solve instead, with every
+// lane busy (here they took 161 registers, 9 waves per CU, for some 10 to 40
+// survivors at a time), and the other particle's box from the broad phase
+// takes the place of the union of its triangles' boxes (144 lane shuffles per
+// item).  What it cost before was an atomic per item on one queue counter,
+// some 10 ns each: 610 us for the hopper's 1.9e5 pairs, 87 us with a region
+// per wave (8 workgroups per CU; 6 per CU: 100 us).
 __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectArgs g) {
-  __shared__ double boxes[kWavesPerGroup][2 * kWaveRows * 6];
-  __shared__ unsigned short act[kWavesPerGroup][2 * kWaveRows];
-  __shared__ unsigned short surv[kWavesPerGroup][kWaveSurvivors];  // row << 8 | column, both kept
+  __shared__ double boxes[kWavesPerGroup][kWaveBoxes * 6];
+  __shared__ unsigned short act[kWavesPerGroup][kWaveBoxes];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   double* bx = boxes[w];
@@ -1032,7 +942,8 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
     } else {  // the unions of the triangles' boxes
 #pragma unroll
       for (int side = 0; side < 2; ++side) {
-        const int n = side == 0 ? it.nB : it.nrows, t0 = side == 0 ? it.tB : it.tA;
+        const int n = side == 0 ? it.nB : it.nrows;
+        const int t0 = side == 0 ? it.oB : it.oA + it.r0;
         double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
         for (int t = lane; t < n; t += 64) {
           double l[3], h[3];
@@ -1059,60 +970,77 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
 #pragma unroll
     for (int q = 0; q < 6; ++q) mag = fmax(mag, fmax(fabs(other[0][q]), fabs(other[1][q])));
     const double reach = margin * (1.0 + 0x1p-20) + mag * 0x1p-40;
-    int kept[2] = {0, 0};
-    bool handed = false;
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int n = side == 0 ? it.nrows : it.nB, t0 = side == 0 ? it.tA : it.tB;
+    // keeps the triangles of [t, t + 64) and below `end` that are on side's
+    // own; false when the LDS is full
+    int kept = 0;
+    auto scan = [&](int side, int t0, int t, int end) {
       const double* sph =
           g.psph ? g.psph + 4 * static_cast<long long>(side == 0 ? it.pb : it.pa) : nullptr;
       const double far = reach + mag * 0x1p-40 - in[side];
-      int c = 0;
-      for (int b = 0; b < n && !handed; b += 64) {
-        const int t = b + lane;
-        double lo[3], hi[3];
-        tri_box(load_tri(g, t0 + (t < n ? t : n - 1)), lo, hi);
-        const bool on = t < n && !(box_gap(lo, hi, other[side], other[side] + 3) > far) &&
-                        !(sph && box_sphere_apart(lo, hi, sph, margin));
-        const unsigned long long m = __ballot(on);
-        const int at = c + lane_prefix(m);
-        c += __popcll(m);
-        if (c > kWaveRows) {
-          handed = true;
-        } else if (on) {
-          double* d = bx + 6 * (side * kWaveRows + at);
+      const int i = t + lane;
+      double lo[3], hi[3];
+      tri_box(load_tri(g, t0 + (i < end ? i : end - 1)), lo, hi);
+      const bool on = i < end && !(box_gap(lo, hi, other[side], other[side] + 3) > far) &&
+                      !(sph && box_sphere_apart(lo, hi, sph, margin));
+      const unsigned long long m = __ballot(on);
+      const int at = kept + lane_prefix(m);
+      kept += __popcll(m);
+      if (kept > kWaveBoxes) return false;
+      if (on) {
+        double* d = bx + 6 * at;
 #pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            d[q] = lo[q];
-            d[3 + q] = hi[q];
-          }
-          act[w][side * kWaveRows + at] = static_cast<unsigned short>(t);
+        for (int q = 0; q < 3; ++q) {
+          d[q] = lo[q];
+          d[3 + q] = hi[q];
+        }
+        act[w][at] = static_cast<unsigned short>(i);
+      }
+      return true;
+    };
+    bool fits = true;
+    const int r1 = it.r0 + it.nrows;
+    if (it.chunked) {
+      for (int c0 = it.r0 / 64; c0 <= (r1 - 1) / 64 && fits; c0 += 64) {
+        const int c = c0 + lane;
+        bool cn = false;
+        if (c <= (r1 - 1) / 64) {
+          const double* cb = g.bbox + 6 * (static_cast<long long>(it.oA / 64) + it.pa + c);
+          cn = !boxes_apart(cb, cb + 3, other[0], other[0] + 3, margin);
+        }
+        for (unsigned long long m = __ballot(cn); m && fits; m &= m - 1) {
+          const int r = 64 * (c0 + __builtin_ctzll(m));
+          // rows of the chunk before r0 belong to the tile before
+          const int lo = r < it.r0 ? it.r0 : r, hi = r + 64 < r1 ? r + 64 : r1;
+          fits = scan(0, it.oA, lo, hi);
         }
       }
-      kept[side] = c;
-      if (c == 0) break;
+    } else {
+      for (int r = it.r0; r < r1 && fits; r += 64) fits = scan(0, it.oA, r, r1);
     }
-    if (handed) {
-      if (lane == 0) g.biglist[atomicAdd(g.nbig, 1u)] = it.item;
-      continue;
-    }
+    const int na = kept;
+    for (int t = 0; t < it.nB && fits && na > 0; t += 64) fits = scan(1, it.oB, t, it.nB);
+    const int nc = kept - na, tested = na * nc;
     wave_lds_fence();
-    const int na = kept[0], nc = kept[1], tested = na * nc;
     // survivors in row-major order over the kept rows and columns
     int S = 0;
-    if (tested > 0) {
+    if (fits && tested > 0) {
       const int step_r = 64 / nc, step_c = 64 - step_r * nc;
       int ra = lane / nc, cb = lane - ra * nc;
       for (int f = lane; f - lane < tested; f += 64) {
         bool keep = false;
         if (f < tested) {
           const double* a = bx + 6 * ra;
-          const double* b = bx + 6 * (kWaveRows + cb);
+          const double* b = bx + 6 * (na + cb);
           keep = !(box_gap(a, a + 3, b, b + 3) > reach);
         }
         const unsigned long long m = __ballot(keep);
-        const int at = S + lane_prefix(m);
-        if (keep && at < kWaveSurvivors) surv[w][at] = static_cast<unsigned short>(ra << 8 | cb);
+        const int at = used + S + lane_prefix(m);
+        if (keep && at < g.rcap) {
+          const int r = act[w][ra], c = act[w][na + cb];
+          queue[at] = make_int4(it.item, it.oA + r, it.oB + c,
+                                static_cast<int>(static_cast<unsigned>(r) |
+                                                 (static_cast<unsigned>(c) << 16)));
+        }
         S += __popcll(m);
         ra += step_r;
         cb += step_c;
@@ -1122,20 +1050,10 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
         }
       }
     }
-    wave_lds_fence();
-    bool deferred = S > kWaveSurvivors;
-    if (!deferred) {
-      want += S;
-      deferred = used + S > g.rcap;
-    }
-    if (deferred) {
+    want += S;
+    if (!fits || used + S > g.rcap) {
       if (lane == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = it.item;
     } else {
-      for (int e = lane; e < S; e += 64) {
-        const int v = surv[w][e];
-        const int r = act[w][v >> 8], c = act[w][kWaveRows + (v & 255)];
-        queue[used + e] = make_int4(it.item, it.tA + r, it.tB + c, (it.r0 + r) | c << 16);
-      }
       used += S;
       if (lane == 0)
         g.tile_stats[static_cast<long long>(it.item) * g.nstats + TS_CULLED] =
@@ -1460,29 +1378,31 @@ __global__ __launch_bounds__(256) void k_tile_sums(const int* __restrict__ tile_
 __global__ __launch_bounds__(256) void k_scatter(const dh_contact* __restrict__ temp, long long n,
                                                  const long long* __restrict__ offs,
                                                  const int* __restrict__ tile_count, int tiles,
-                                                 dh_contact* __restrict__ out, long long cap,
+                                                 dh_contact* __restrict__ out,
                                                  const unsigned long long* __restrict__ n_dev) {
   const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  // n is the capacity of temp when the count is read from n_dev
+  // n is the capacity (of temp and out) when the count is read from n_dev
   if (i >= n || (n_dev && static_cast<unsigned long long>(i) >= *n_dev)) return;
   dh_contact c = temp[i];
   const int pair = c.pair / tiles;
   long long dst = offs[pair] + c.pad_;
   for (int t = pair * tiles; t < c.pair; ++t) dst += tile_count[t];
-  if (dst >= cap) return;  // more contacts than the capacity (reported by the caller)
+  if (dst >= n) return;  // more contacts than the capacity (reported by the caller)
   c.pair = pair;
   c.pad_ = 0;
   out[dst] = c;
 }
 
-// Survivor queue, pass 2: every wave takes one region of k_detect_wave's (then
-// the ranges of k_detect_big that fall to it) through the plane test, the
-// edge-pair axes (and, when tuned on, the binary32 screen) and bfSolver.  What
-// a test leaves waits in a list in LDS until 64 entries are there, so that
-// each stage runs with every lane busy although the one before it drops most.
-// The entries stay in order, so the contacts of an item come out in row-major
-// order and their rank is a running count, and the records of a region follow
-// each other without a counter that all waves share.
+// Survivor queue, pass 2: every wave takes one region of k_detect_wave's through
+// the plane test, the edge-pair axes (and, when tuned on, the binary32 screen)
+// and bfSolver.  What a test leaves waits in a list in LDS until 64 entries
+// are there, so that each stage runs with every lane busy although the one
+// before it drops most.  The entries stay in order, so the contacts of an item
+// come out in row-major order and their rank is a running count, and the
+// records of a region follow each other without a counter that all waves
+// share.  Bound by vector issue: 152 us for the hopper's 1.78e6 entries and
+// 644,000 contacts (a lane per entry, with its scan, reservation and unordered
+// contacts: 250 us); four waves per SIMD would spill (166 us).
 struct QueueLists {
   int a[128], b[128];  // entries for the axes, for bfSolver
 };
@@ -1594,8 +1514,7 @@ __device__ __forceinline__ int solve_stream(const DetectArgs& g, int4* __restric
       bool keep = false;
       if (e < n) {
         const int4 en = q[e];
-        if (en.x >= 0)
-          keep = !plane_apart(load_tri(g, en.y), load_tri(g, en.z), entry_margin(g, en));
+        keep = !plane_apart(load_tri(g, en.y), load_tri(g, en.z), entry_margin(g, en));
       }
       na = list_append(L.a, na, keep, e);
       base += 64;
@@ -1606,121 +1525,104 @@ __device__ __forceinline__ int solve_stream(const DetectArgs& g, int4* __restric
   return out;
 }
 
-// A wave's streams: the regions, then the ranges.
-struct QueueStream {
-  long long at;  // first entry, from g.queue (bqueue follows the regions there)
-  int n;
-  int* contacts;  // where the number of its records goes
-};
-
-__device__ __forceinline__ QueueStream queue_stream(const DetectArgs& g, int u) {
-  if (u < g.regions)
-    return {static_cast<long long>(u) * g.rcap, g.rcount[u], g.rcount + g.regions + u};
-  int4* r = g.ranges + (u - g.regions);
-  return {static_cast<long long>(g.regions) * g.rcap + r->x, r->y, &r->w};
-}
-
 template <bool SCREEN, bool kFilter>
 __global__ __launch_bounds__(256, 3) void k_queue_solve(DetectArgs g) {
   __shared__ QueueLists lists[4];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const int nstreams = g.regions + static_cast<int>(*g.nranges);
-  for (int u = blockIdx.x * 4 + w; u < nstreams; u += gridDim.x * 4) {
-    const QueueStream s = queue_stream(g, u);
-    const int m = solve_stream<SCREEN, kFilter>(g, g.queue + s.at, s.n, g.rec + s.at, lists[w], lane);
-    if (lane == 0) {
-      if (!kFilter) *s.contacts = m;
-      else if (u < g.regions) g.rcount[u] = m;
-      else g.ranges[u - g.regions].y = m;
-    }
-  }
+  const int r = blockIdx.x * 4 + w;
+  if (r >= g.regions) return;
+  const long long at = static_cast<long long>(r) * g.rcap;
+  const int m = solve_stream<SCREEN, kFilter>(g, g.queue + at, g.rcount[r], g.rec + at, lists[w],
+                                              lane);
+  if (lane == 0) g.rcount[(kFilter ? 0 : g.regions) + r] = m;
 }
 
 // The records of entries that another kernel has solved (flags[e], and the
 // points pq[6e..] of those that emit), in order.
-__device__ __forceinline__ int record_stream(const DetectArgs& g, const int4* __restrict__ q, int n,
-                                             const int* __restrict__ flags,
-                                             const double* __restrict__ pq,
-                                             QueueRecord* __restrict__ rec, int lane) {
-  int out = 0, carry_item = -1, carry = 0;
-  for (int base = 0; base < n; base += 64) {
-    const int e = base + lane;
-    const bool emit = e < n && flags[e] != 0;
-    int4 en = make_int4(-1, 0, 0, 0);
-    if (emit) en = q[e];
-    const int rank = item_rank(g, emit, en.x, lane, carry_item, carry);
-    const unsigned long long m = __ballot(emit);
-    if (emit) {
-      QueueRecord r;
-      r.item = en.x;
-      r.tris = en.w;
-      r.rank = rank;
-      r.pad_ = 0;
-      for (int c = 0; c < 6; ++c) r.pq[c] = pq[6 * static_cast<long long>(e) + c];
-      rec[out + lane_prefix(m)] = r;
-    }
-    out += __popcll(m);
-  }
-  return out;
-}
-
 __global__ __launch_bounds__(256) void k_queue_record(DetectArgs g, const int* __restrict__ flags,
                                                       const double* __restrict__ pq) {
   const int lane = threadIdx.x & 63;
-  const int nstreams = g.regions + static_cast<int>(*g.nranges);
-  for (int u = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6); u < nstreams;
-       u += gridDim.x * 4) {
-    const QueueStream s = queue_stream(g, u);
-    const int m = record_stream(g, g.queue + s.at, s.n, flags + s.at, pq + 6 * s.at, g.rec + s.at,
-                                lane);
-    if (lane == 0) *s.contacts = m;
+  const int r = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
+  if (r >= g.regions) return;
+  const long long at = static_cast<long long>(r) * g.rcap;
+  const int n = g.rcount[r];
+  int out = 0, carry_item = -1, carry = 0;
+  for (int base = 0; base < n; base += 64) {
+    const long long e = at + base + lane;
+    const bool emit = base + lane < n && flags[e] != 0;
+    int4 en = make_int4(-1, 0, 0, 0);
+    if (emit) en = g.queue[e];
+    const int rank = item_rank(g, emit, en.x, lane, carry_item, carry);
+    const unsigned long long m = __ballot(emit);
+    if (emit) {
+      QueueRecord q;
+      q.item = en.x;
+      q.tris = en.w;
+      q.rank = rank;
+      q.pad_ = 0;
+      for (int c = 0; c < 6; ++c) q.pq[c] = pq[6 * e + c];
+      g.rec[at + out + lane_prefix(m)] = q;
+    }
+    out += __popcll(m);
   }
+  if (lane == 0) g.rcount[g.regions + r] = out;
 }
 
-// Pass 3, after the pairs' offsets: the records' contacts, each at its place.
-// counter (may be null) receives offs[*npairs_dev], the contacts found.
-__device__ __forceinline__ void write_record(const DetectArgs& g, const QueueRecord& r,
-                                             const long long* __restrict__ offs,
-                                             dh_contact* __restrict__ out, long long cap) {
-  const int k = r.item / g.tiles;
-  long long dst = offs[k] + r.rank;
-  for (int t = k * g.tiles; t < r.item; ++t) dst += g.tile_count[t];
-  if (dst >= cap) return;  // more contacts than the capacity (reported by the caller)
-  dh_contact c;
-  const V3<double> P = {r.pq[0], r.pq[1], r.pq[2]}, Q = {r.pq[3], r.pq[4], r.pq[5]};
-  make_contact(load_pair(g, k), k, r.tris & 0xffff, static_cast<int>(static_cast<unsigned>(r.tris) >> 16),
-               P, Q, &c);
-  c.pad_ = 0;
-  out[dst] = c;
+// Pass 3, after the pairs' offsets: the records' contacts, each at its place,
+// and those that the full kernel left in `temp` (*in_temp of them).
+__device__ __forceinline__ long long contact_place(const DetectArgs& g, int item, int rank,
+                                                   const long long* __restrict__ offs) {
+  const int k = item / g.tiles;
+  long long dst = offs[k] + rank;
+  for (int t = k * g.tiles; t < item; ++t) dst += g.tile_count[t];
+  return dst;
 }
 
 __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long long* __restrict__ offs,
                                                      dh_contact* __restrict__ out, long long cap,
-                                                     unsigned long long* __restrict__ counter) {
+                                                     const unsigned long long* __restrict__ in_temp,
+                                                     unsigned long long* __restrict__ found) {
   const int lane = threadIdx.x & 63;
-  const int nstreams = g.regions + static_cast<int>(*g.nranges);
-  for (int u = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6); u < nstreams;
-       u += gridDim.x * 4) {
-    const QueueStream s = queue_stream(g, u);
-    const int n = *s.contacts;
-    for (int e = lane; e < n; e += 64) write_record(g, g.rec[s.at + e], offs, out, cap);
+  const int r = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
+  // contacts past the capacity are dropped (reported by the caller)
+  const int n = r < g.regions ? g.rcount[g.regions + r] : 0;
+  for (int e = lane; e < n; e += 64) {
+    const QueueRecord q = g.rec[static_cast<long long>(r) * g.rcap + e];
+    const long long dst = contact_place(g, q.item, q.rank, offs);
+    if (dst >= cap) continue;
+    const int k = q.item / g.tiles;
+    const unsigned tris = static_cast<unsigned>(q.tris);
+    dh_contact c;
+    make_contact(load_pair(g, k), k, static_cast<int>(tris & 0xffffu), static_cast<int>(tris >> 16),
+                 V3<double>{q.pq[0], q.pq[1], q.pq[2]}, V3<double>{q.pq[3], q.pq[4], q.pq[5]}, &c);
+    c.pad_ = 0;
+    out[dst] = c;
   }
-  if (counter && blockIdx.x == 0 && threadIdx.x == 0)
-    *counter = static_cast<unsigned long long>(
+  const unsigned long long nt = *in_temp < static_cast<unsigned long long>(g.cap)
+                                    ? *in_temp : static_cast<unsigned long long>(g.cap);
+  for (unsigned long long i = blockIdx.x * 256ull + threadIdx.x; i < nt; i += gridDim.x * 256ull) {
+    dh_contact c = g.temp[i];
+    const long long dst = contact_place(g, c.pair, c.pad_, offs);
+    if (dst >= cap) continue;
+    c.pair /= g.tiles;
+    c.pad_ = 0;
+    out[dst] = c;
+  }
+  if (found && blockIdx.x == 0 && threadIdx.x == 0)
+    *found = static_cast<unsigned long long>(
         offs[g.npairs_dev && *g.npairs_dev < g.npairs ? *g.npairs_dev : g.npairs]);
 }
 
 int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
-                  const int* rcount, const int4* ranges, const unsigned* nranges,
-                  const double* x, const double* y, const double* z, const double* eps,
-                  long long n, int* flags, double* pq, hipStream_t st);
+                  const int* rcount, const double* x, const double* y, const double* z,
+                  const double* eps, int* flags, double* pq, hipStream_t st);
 int queue_learned_reserve(long long n);
 
 struct DetectScratch {
   DevBuf temp, counter, stats, error, counts, offs, sums, tiles, tstats, iskip, tmax;
-  DevBuf queue, qrec, qcounts, rcount, ranges, deferred, wlist, qflags, qpq;
-  int rwant = 0, bwant = 0;  // what a region and bqueue had to hold in earlier eager calls
+  DevBuf queue, qrec, qcounts, rcount, deferred, wlist, found, qflags, qpq;
+  int rwant = 0;  // what a region had to hold in earlier eager calls
 };
 static DetectScratch g_scratch;
 
@@ -1833,7 +1735,7 @@ static void launch_detect(unsigned items, size_t shm, hipStream_t st, const Dete
                        256, 0, st, a, static_cast<int>(items),
                        const_cast<unsigned char*>(a.item_skip));
   }
-  hipLaunchKernelGGL((k_detect<M, false>), detect_grid(items), 256, shm, st, a,
+  hipLaunchKernelGGL(k_detect<M>, detect_grid(items), 256, shm, st, a,
                      static_cast<int>(items));
 }
 
@@ -1859,31 +1761,30 @@ static int tiles_for(long long npairs, int method) {
 
 // The survivor queue's shape for `items` items: a region per wave of
 // k_detect_wave's persistent grid (as many as the CUs hold at once), 16 entries
-// per item over the regions and 4 for bqueue, or what earlier calls needed.
+// per item over the regions and at least 1,024 in each, or what earlier calls
+// needed.
 struct QueuePlan {
   unsigned groups;
-  int regions, rcap, bcap;
-  long long entries() const { return static_cast<long long>(regions) * rcap + bcap; }
+  int regions, rcap;
+  long long entries() const { return static_cast<long long>(regions) * rcap; }
 };
 
-static QueuePlan queue_plan(long long items, int rwant, int bwant) {
+static QueuePlan queue_plan(long long items, int rwant) {
   QueuePlan q;
   const long long wg = (items + kWavesPerGroup - 1) / kWavesPerGroup;
   const long long most = static_cast<long long>(device_cus()) * 8;
   q.groups = static_cast<unsigned>(wg < 1 ? 1 : (wg < most ? wg : most));
   q.regions = static_cast<int>(q.groups) * kWavesPerGroup;
-  long long r = (16 * items + 65536) / q.regions, b = 4 * items + 65536;
-  if (r < 2 * kWaveSurvivors) r = 2 * kWaveSurvivors;
+  long long r = (16 * items + 65536) / q.regions;
+  if (r < 1024) r = 1024;
   if (r < rwant) r = rwant;
-  if (b < bwant) b = bwant;
-  const long long rmost = (1ll << 29) / q.regions;
+  const long long rmost = (1ll << 30) / q.regions;
   q.rcap = static_cast<int>(r < rmost ? r : rmost);
-  q.bcap = static_cast<int>(b < (1ll << 29) ? b : 1ll << 29);
   return q;
 }
 
 // Places of the queue path's counters in g_scratch.qcounts.
-enum QueueCount : int { QC_WLIST = 0, QC_BIG, QC_DEFERRED, QC_BQUEUE, QC_RANGES, QC_RWANT, kQueueCounts };
+enum QueueCount : int { QC_WLIST = 0, QC_DEFERRED, QC_RWANT, kQueueCounts };
 
 // Buffers of the queue path (before a capture).
 static int queue_reserve(const QueuePlan& q, long long items, bool learned) {
@@ -1892,9 +1793,9 @@ static int queue_reserve(const QueuePlan& q, long long items, bool learned) {
   if ((rc = g_scratch.qrec.grow(sizeof(QueueRecord) * q.entries()))) return rc;
   if ((rc = g_scratch.qcounts.grow(sizeof(unsigned) * kQueueCounts))) return rc;
   if ((rc = g_scratch.rcount.grow(sizeof(int) * 2 * q.regions))) return rc;
-  if ((rc = g_scratch.ranges.grow(sizeof(int4) * (items + 1)))) return rc;
-  if ((rc = g_scratch.deferred.grow(sizeof(int) * 2 * (items + 1)))) return rc;
+  if ((rc = g_scratch.deferred.grow(sizeof(int) * (items + 1)))) return rc;
   if ((rc = g_scratch.wlist.grow(sizeof(WaveItem) * (items + 1)))) return rc;
+  if ((rc = g_scratch.found.grow(sizeof(unsigned long long)))) return rc;
   if (learned) {
     if ((rc = g_scratch.qflags.grow(sizeof(int) * q.entries()))) return rc;
     if ((rc = g_scratch.qpq.grow(sizeof(double) * 6 * q.entries()))) return rc;
@@ -1903,24 +1804,16 @@ static int queue_reserve(const QueuePlan& q, long long items, bool learned) {
   return DH_OK;
 }
 
-static void queue_bind(DetectArgs& a, const QueuePlan& q, long long items) {
+static void queue_bind(DetectArgs& a, const QueuePlan& q) {
   unsigned* c = g_scratch.qcounts.as<unsigned>();
-  const long long big = static_cast<long long>(q.regions) * q.rcap;
   a.queue = g_scratch.queue.as<int4>();
   a.rcap = q.rcap;
   a.regions = q.regions;
   a.rcount = g_scratch.rcount.as<int>();
   a.rwant = reinterpret_cast<int*>(c + QC_RWANT);
-  a.bqueue = a.queue + big;
-  a.bcap = q.bcap;
-  a.bcounter = c + QC_BQUEUE;
-  a.ranges = g_scratch.ranges.as<int4>();
-  a.nranges = c + QC_RANGES;
   a.rec = g_scratch.qrec.as<QueueRecord>();
   a.deferred = g_scratch.deferred.as<int>();
   a.ndeferred = c + QC_DEFERRED;
-  a.biglist = a.deferred + (items + 1);
-  a.nbig = c + QC_BIG;
   a.wlist = g_scratch.wlist.as<WaveItem>();
   a.nwlist = c + QC_WLIST;
 }
@@ -1932,30 +1825,23 @@ static void queue_bind(DetectArgs& a, const QueuePlan& q, long long items) {
 static int queue_detect(const DetectArgs& a, const QueuePlan& q, unsigned items, bool learned,
                         hipStream_t st) {
   const unsigned cus = static_cast<unsigned>(device_cus());
-  const unsigned few = items < 4 * cus ? items : 4 * cus;  // usually none to do
   hipLaunchKernelGGL(k_lane_cull, items > 0 ? grid_for(items, 1024) : 1u, 1024, 0, st, a,
                      static_cast<int>(items));
   hipLaunchKernelGGL(k_detect_wave, q.groups, 64 * kWavesPerGroup, 0, st, a);
-  hipLaunchKernelGGL(k_detect_big, few, 256, 0, st, a);
   DetectArgs f = a;
   f.item_list = a.deferred;
   f.nitems_dev = a.ndeferred;
-  hipLaunchKernelGGL((k_detect<DH_BF, false>), few, 256, 0, st, f, static_cast<int>(items));
+  // usually none to do: a grid for the capacity would cost a dispatch per item
+  hipLaunchKernelGGL(k_detect<DH_BF>, items < 4 * cus ? items : 4 * cus, 256, 0, st, f,
+                     static_cast<int>(items));
   const unsigned grid = grid_for(q.regions, 4);
-  if (!learned) {
-    if (a.fp32_screen)
-      hipLaunchKernelGGL((k_queue_solve<true, false>), grid, 256, 0, st, a);
-    else
-      hipLaunchKernelGGL((k_queue_solve<false, false>), grid, 256, 0, st, a);
-  } else {
-    if (a.fp32_screen)
-      hipLaunchKernelGGL((k_queue_solve<true, true>), grid, 256, 0, st, a);
-    else
-      hipLaunchKernelGGL((k_queue_solve<false, true>), grid, 256, 0, st, a);
+  const auto solve = learned ? (a.fp32_screen ? k_queue_solve<true, true> : k_queue_solve<false, true>)
+                             : (a.fp32_screen ? k_queue_solve<true, false> : k_queue_solve<false, false>);
+  hipLaunchKernelGGL(solve, grid, 256, 0, st, a);
+  if (learned) {
     int rc;
-    if ((rc = queue_learned(a.queue, a.pairs, a.tiles, a.regions, a.rcap, a.rcount, a.ranges,
-                            a.nranges, a.x, a.y, a.z, a.eps, q.entries(),
-                            g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>(), st)))
+    if ((rc = queue_learned(a.queue, a.pairs, a.tiles, a.regions, a.rcap, a.rcount, a.x, a.y, a.z,
+                            a.eps, g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>(), st)))
       return rc;
     hipLaunchKernelGGL(k_queue_record, grid, 256, 0, st, a, g_scratch.qflags.as<int>(),
                        g_scratch.qpq.as<double>());
@@ -2033,10 +1919,10 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
   const bool queued = bf && (learned || nitems >= tuning().detect_queue_min_items);
   QueuePlan plan = {};
   if (queued) {
-    plan = queue_plan(nitems, g_scratch.rwant, g_scratch.bwant);
+    plan = queue_plan(nitems, g_scratch.rwant);
     if ((rc = queue_reserve(plan, nitems, learned))) return rc;
     DH_HIP_CHECK(hipMemsetAsync(g_scratch.qcounts.ptr, 0, sizeof(unsigned) * kQueueCounts, st));
-    queue_bind(a, plan, nitems);
+    queue_bind(a, plan);
   }
   const size_t shm_rows = 2 * kMaxRowTriangles * sizeof(int) + 8 + kMaxRowTriangles * 8;
   const unsigned items = static_cast<unsigned>(nitems);
@@ -2091,13 +1977,10 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
   }
   DH_HIP_CHECK(hipStreamSynchronize(st));
   if (queued) {
-    // the next call's queue holds this call's need
-    auto more = [](unsigned need, int had) {
-      const long long n = static_cast<long long>(need) + need / 4;
-      return need > static_cast<unsigned>(had) ? static_cast<int>(n < (1 << 29) ? n : 1 << 29) : 0;
-    };
-    if (const int n = more(qc[QC_RWANT], plan.rcap)) g_scratch.rwant = n;
-    if (const int n = more(qc[QC_BQUEUE], plan.bcap)) g_scratch.bwant = n;
+    // the next call's regions hold this call's need
+    const long long want = qc[QC_RWANT];
+    if (want > plan.rcap)
+      g_scratch.rwant = static_cast<int>(want + want / 4 < (1 << 29) ? want + want / 4 : 1 << 29);
   }
   const unsigned long long total = queued ? static_cast<unsigned long long>(all) : in_temp;
   if (err == DE_REF_UB)
@@ -2120,13 +2003,15 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
   }
   if (static_cast<long long>(total) > cap) return DH_ERR_CAPACITY;
   if (!queued && (rc = pair_offsets())) return rc;
-  if (in_temp > 0)
-    hipLaunchKernelGGL(k_scatter, grid_for(static_cast<int64_t>(in_temp), 256), 256, 0, st,
-                       g_scratch.temp.as<dh_contact>(), static_cast<long long>(in_temp), offs,
-                       tile_count, tiles, out, cap, nullptr);
-  if (total > in_temp)
-    hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out, cap,
-                       nullptr);
+  if (queued) {
+    if (total > 0)
+      hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out, cap,
+                         a.counter, nullptr);
+  } else if (total > 0) {
+    hipLaunchKernelGGL(k_scatter, grid_for(static_cast<int64_t>(total), 256), 256, 0, st,
+                       g_scratch.temp.as<dh_contact>(), static_cast<long long>(total), offs,
+                       tile_count, tiles, out, nullptr);
+  }
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
@@ -2171,8 +2056,8 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
     a.item_skip = g_scratch.iskip.as<unsigned char>();
   QueuePlan plan = {};
   if (queued) {
-    plan = queue_plan(items, 0, 0);
-    queue_bind(a, plan, items);
+    plan = queue_plan(items, 0);
+    queue_bind(a, plan);
   }
   switch (method) {
     case DH_BF:
@@ -2200,12 +2085,13 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
                                g_scratch.sums.as<long long>(), st)))
       return rc;
   }
-  hipLaunchKernelGGL(k_scatter, grid_for(contact_cap, 256), 256, 0, st,
-                     g_scratch.temp.as<dh_contact>(), contact_cap, offs, a.tile_count, tiles, out,
-                     contact_cap, g_scratch.counter.as<unsigned long long>());
   if (queued)
     hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out,
-                       contact_cap, g_scratch.counter.as<unsigned long long>());
+                       contact_cap, a.counter, g_scratch.found.as<unsigned long long>());
+  else
+    hipLaunchKernelGGL(k_scatter, grid_for(contact_cap, 256), 256, 0, st,
+                       g_scratch.temp.as<dh_contact>(), contact_cap, offs, a.tile_count, tiles, out,
+                       g_scratch.counter.as<unsigned long long>());
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
@@ -2216,7 +2102,7 @@ int detect_reserve(int pair_cap, long long contact_cap, int method) {
   int rc;
   if (graph_queued(method, pair_cap)) {
     const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
-    if ((rc = queue_reserve(queue_plan(items, 0, 0), items, method == DH_BF_LEARNED))) return rc;
+    if ((rc = queue_reserve(queue_plan(items, 0), items, method == DH_BF_LEARNED))) return rc;
   }
   if ((rc = g_scratch.temp.grow(sizeof(dh_contact) * (contact_cap > 0 ? contact_cap : 1)))) return rc;
   if ((rc = g_scratch.counter.grow(sizeof(unsigned long long)))) return rc;
@@ -2236,9 +2122,12 @@ int detect_reserve(int pair_cap, long long contact_cap, int method) {
   return DH_OK;
 }
 
-// Device addresses of the detection counters: [0] contacts found, and the
-// error flag.
-const unsigned long long* detect_counter_dev() { return g_scratch.counter.as<unsigned long long>(); }
+// Device addresses of the detection counters of a captured step: the contacts
+// found, the error flag and the statistics.
+const unsigned long long* detect_counter_dev(int method, int pair_cap) {
+  return graph_queued(method, pair_cap) ? g_scratch.found.as<unsigned long long>()
+                                        : g_scratch.counter.as<unsigned long long>();
+}
 const int* detect_error_dev() { return g_scratch.error.as<int>(); }
 const unsigned long long* detect_stats_dev() { return g_scratch.stats.as<unsigned long long>(); }
 

@@ -25,7 +25,7 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
                        const double* bbox, const double* psph);
 int detect_reserve(int pair_cap, long long contact_cap, int method);
 int detect_prepare(const dh_geometry* geom, hipStream_t st);
-const unsigned long long* detect_counter_dev();
+const unsigned long long* detect_counter_dev(int method, int pair_cap);
 const int* detect_error_dev();
 const unsigned long long* detect_stats_dev();
 int forces_reserve(int n, int npairs);
@@ -199,7 +199,9 @@ static int record_step(dh_step_graph* g, hipStream_t st) {
     return rc;
   if (ad && (rc = adaptive_finish(s->bodies.linvel, s->bodies.obstacle, s->bodies.n, ad, st)))
     return rc;
-  hipLaunchKernelGGL(k_step_status, 1, 64, 0, st, np_dev, detect_counter_dev(), detect_error_dev(),
+  hipLaunchKernelGGL(k_step_status, 1, 64, 0, st, np_dev,
+                     detect_counter_dev(g->params.method, static_cast<int>(g->pair_cap)),
+                     detect_error_dev(),
                      detect_stats_dev(), g->pair_cap, g->contact_cap, g->status.as<long long>());
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;

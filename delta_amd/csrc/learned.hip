@@ -778,8 +778,8 @@ k_learned(LearnedArgs a) {
 // ------------------------------------------------ the step's survivor queue
 // The triangle pairs that the DEM step's box mid-phase leaves (the survivor
 // queue of detect.hip, entries {item, triangle of A, triangle of B, ..} in
-// regions and ranges) through the learned decision: a wave per region or range
-// at a time, 64 entries in a round.  A finished entry
+// regions) through the learned decision: a wave per region at a time, 64
+// entries in a round.  A finished entry
 // sets flags[e] (its pair emits a contact: d <= epsA + epsB, bf.cpp:125) and,
 // when it emits, its P, Q at pq[6e..6e+6); the rest are listed for the
 // brute force (k_queue_fallback).  Both write exactly what the brute-force
@@ -790,13 +790,10 @@ struct QueueLearnArgs {
   int tiles;  // items per particle pair
   int regions, rcap;     // region r: rcount[r] entries from r * rcap
   const int* rcount;
-  const int4* ranges;    // then the ranges {first, length}, from regions * rcap
-  const unsigned* nranges;
   const double* x;
   const double* y;
   const double* z;
   const double* eps;
-  long long n;  // entries the queue can hold
   int* flags;
   double* pq;
   const float* W;
@@ -819,14 +816,9 @@ k_queue_learned(QueueLearnArgs a) {
   stage_network<kModeFeatures>(L, a.W);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   unsigned evals = 0;
-  const int nr = static_cast<int>(*a.nranges);
-  const long long big = static_cast<long long>(a.regions) * a.rcap;
-  for (int u = blockIdx.x * kInferWaves + wave; u < a.regions + nr;
-       u += gridDim.x * kInferWaves) {
-    const bool is_range = u >= a.regions;
-    const int4 range = is_range ? a.ranges[u - a.regions] : make_int4(0, 0, 0, 0);
-    const long long at = is_range ? big + range.x : static_cast<long long>(u) * a.rcap;
-    const int live = is_range ? range.y : a.rcount[u];
+  for (int r = blockIdx.x * kInferWaves + wave; r < a.regions; r += gridDim.x * kInferWaves) {
+    const long long at = static_cast<long long>(r) * a.rcap;
+    const int live = a.rcount[r];
     for (int base = 0; base < live; base += 64) {
       const long long e = at + base + lane;
       const int4 en = base + lane < live ? a.queue[e] : make_int4(-1, 0, 0, 0);
@@ -886,8 +878,7 @@ __device__ __forceinline__ void queue_fallback_entry(const QueueLearnArgs& a, lo
 // The listed entries by the brute force, a lane each at a time (a captured
 // step launches a persistent grid and strides over the list's length).
 __global__ __launch_bounds__(256) void k_queue_fallback(QueueLearnArgs a) {
-  const long long nfb = static_cast<long long>(*a.fb_count) < a.n
-                            ? static_cast<long long>(*a.fb_count) : a.n;
+  const long long nfb = *a.fb_count;
   for (long long j = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; j < nfb;
        j += static_cast<long long>(gridDim.x) * 256)
     queue_fallback_entry(a, a.fb_list[j]);
@@ -915,14 +906,14 @@ int queue_learned_reserve(long long n) {
 // The survivor queue's entries through the learned decision, then the brute
 // force for the rest; a fill instead of a memset (captured steps).
 int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
-                  const int* rcount, const int4* ranges, const unsigned* nranges,
-                  const double* x, const double* y, const double* z, const double* eps,
-                  long long n, int* flags, double* pq, hipStream_t st) {
+                  const int* rcount, const double* x, const double* y, const double* z,
+                  const double* eps, int* flags, double* pq, hipStream_t st) {
+  const long long n = static_cast<long long>(regions) * rcap;
   if (!g_learned.model)
     return set_error(DH_ERR_ARG, "DH_BF_LEARNED: no network set (dh_learned_set_model)");
   int rc;
   if ((rc = queue_learned_reserve(n))) return rc;
-  QueueLearnArgs a{queue, pairs, tiles, regions, rcap, rcount, ranges, nranges, x, y, z, eps, n,
+  QueueLearnArgs a{queue, pairs, tiles, regions, rcap, rcount, x, y, z, eps,
                    flags, pq, g_learned.model, g_qlearn.fb_list.as<int>(),
                    g_qlearn.fb_count.as<unsigned>()};
   fill_async(g_qlearn.fb_count.as<unsigned>(), 0u, 1, st);
