@@ -108,6 +108,8 @@ struct DetectArgs {
   // contacts of the queue's entries, in the entries' order, from the place of
   // the region's first entry; region r's number in rcount[regions + r]
   struct QueueRecord* rec;
+  int heavy;    // regions with more entries are solved in four parts
+  int* rparts;  // a heavy region's: each part's contacts and rank base
   int* deferred;
   unsigned* ndeferred;
   // Items k_lane_cull leaves for k_detect_wave
@@ -1018,6 +1020,30 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
       for (int r = it.r0; r < r1 && fits; r += 64) fits = scan(0, it.oA, r, r1);
     }
     const int na = kept;
+    if (na > 0 && fits && (it.chunked || na + it.nB > kWaveBoxes)) {
+      // the columns might not fit: they are tested against the union of the
+      // kept rows' boxes instead of A's (a funnel's box holds every particle)
+      wave_lds_fence();
+      double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+      for (int t = lane; t < na; t += 64)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          lo[q] = fmin(lo[q], bx[6 * t + q]);
+          hi[q] = fmax(hi[q], bx[6 * t + 3 + q]);
+        }
+      for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          lo[q] = fmin(lo[q], __shfl_xor(lo[q], o));
+          hi[q] = fmax(hi[q], __shfl_xor(hi[q], o));
+        }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        other[1][q] = lo[q];
+        other[1][3 + q] = hi[q];
+      }
+      in[1] = 0.0;
+    }
     for (int t = 0; t < it.nB && fits && na > 0; t += 64) fits = scan(1, it.oB, t, it.nB);
     const int nc = kept - na, tested = na * nc;
     wave_lds_fence();
@@ -1459,13 +1485,19 @@ __device__ __forceinline__ int item_rank(const DetectArgs& g, bool emit, int ite
 }
 
 // The n entries at q through the tests and bfSolver; their contacts' records
-// to rec, in order.  Returns the number of records.  With kFilter the entries
-// that the tests leave are compacted in place instead, and counted.
+// to rec, in order.  Returns the number of records, and the first and the last
+// item that has one with their counts.  With kFilter the entries that the tests
+// leave are compacted in place instead, and counted.
+struct StreamEnds {
+  int n, first, nfirst, last, nlast;
+};
+
 template <bool SCREEN, bool kFilter>
-__device__ __forceinline__ int solve_stream(const DetectArgs& g, int4* __restrict__ q, int n,
-                                            QueueRecord* __restrict__ rec, QueueLists& L,
-                                            int lane) {
+__device__ __forceinline__ StreamEnds solve_stream(const DetectArgs& g, int4* __restrict__ q, int n,
+                                                   QueueRecord* __restrict__ rec, QueueLists& L,
+                                                   int lane) {
   int na = 0, nb = 0, base = 0, out = 0, carry_item = -1, carry = 0;
+  int first = -1, nfirst = 0;
   for (;;) {
     const bool eof = base >= n;
     if (nb >= 64 || (eof && na == 0 && nb > 0)) {
@@ -1497,6 +1529,8 @@ __device__ __forceinline__ int solve_stream(const DetectArgs& g, int4* __restric
         r.pq[3] = Q.x; r.pq[4] = Q.y; r.pq[5] = Q.z;
         rec[out + lane_prefix(m)] = r;
       }
+      if (m && out == 0) first = __shfl(en.x, __builtin_ctzll(m));
+      nfirst += __popcll(__ballot(emit && en.x == first));
       out += __popcll(m);
     } else if (na >= 64 || (eof && na > 0)) {
       const int e = list_take(L.a, na, lane);
@@ -1522,20 +1556,62 @@ __device__ __forceinline__ int solve_stream(const DetectArgs& g, int4* __restric
       break;
     }
   }
-  return out;
+  return {out, first, nfirst, carry_item, carry};
 }
 
+// The part of a heavy region's n entries that each of a workgroup's waves
+// takes, in whole rounds of 64.
+__device__ __forceinline__ int region_part(int n) { return (n + 255) / 256 * 64; }
+
+// A wave per region; then the workgroup's four waves share each of its regions
+// with more than g.heavy entries, so that one pair of particles in deep
+// contact does not keep a single wave at work (the funnel's heaviest pairs
+// have 400 contacts: 100 us without, 69 us with).  An item that goes on from
+// one part of a region to the next has the later part's ranks raised by the
+// contacts before (applied in k_queue_write).
 template <bool SCREEN, bool kFilter>
 __global__ __launch_bounds__(256, 3) void k_queue_solve(DetectArgs g) {
   __shared__ QueueLists lists[4];
+  __shared__ StreamEnds ends[4];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const int r = blockIdx.x * 4 + w;
-  if (r >= g.regions) return;
-  const long long at = static_cast<long long>(r) * g.rcap;
-  const int m = solve_stream<SCREEN, kFilter>(g, g.queue + at, g.rcount[r], g.rec + at, lists[w],
-                                              lane);
-  if (lane == 0) g.rcount[(kFilter ? 0 : g.regions) + r] = m;
+  for (int p = -1; p < 4; ++p) {
+    // a workgroup's regions lie far apart: neighbours hold neighbouring pairs,
+    // which are heavy together
+    const int r = (p < 0 ? w : p) * gridDim.x + blockIdx.x;
+    const int total = r < g.regions ? g.rcount[r] : 0;
+    if (p >= 0 && total <= g.heavy) continue;  // the same for the whole workgroup
+    int begin = 0, n = total <= g.heavy ? total : 0;
+    if (p >= 0) {
+      const int part = region_part(total);
+      begin = w * part < total ? w * part : total;
+      n = total - begin < part ? total - begin : part;
+    }
+    const long long at = static_cast<long long>(r) * g.rcap + begin;
+    const StreamEnds e = solve_stream<SCREEN, kFilter>(g, g.queue + at, n, g.rec + at, lists[w], lane);
+    if (p < 0) {
+      if (lane == 0 && r < g.regions && total <= g.heavy)
+        g.rcount[(kFilter ? 0 : g.regions) + r] = e.n;
+      continue;
+    }
+    if (lane == 0) ends[w] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int item = -1, count = 0;
+      for (int q = 0; q < 4; ++q) {
+        const StreamEnds s = ends[q];
+        const int base = s.n > 0 && s.first == item ? count : 0;
+        int* c = g.rparts + 8 * static_cast<long long>(r) + 2 * q;
+        c[0] = s.n;
+        c[1] = base;
+        if (s.n == 0) continue;
+        if (base > 0) g.tile_count[s.first] = base + s.nfirst;
+        count = s.first == s.last ? base + s.nfirst : s.nlast;
+        item = s.last;
+      }
+    }
+    __syncthreads();
+  }
 }
 
 // The records of entries that another kernel has solved (flags[e], and the
@@ -1585,19 +1661,28 @@ __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long lo
                                                      unsigned long long* __restrict__ found) {
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
-  // contacts past the capacity are dropped (reported by the caller)
-  const int n = r < g.regions ? g.rcount[g.regions + r] : 0;
-  for (int e = lane; e < n; e += 64) {
-    const QueueRecord q = g.rec[static_cast<long long>(r) * g.rcap + e];
-    const long long dst = contact_place(g, q.item, q.rank, offs);
-    if (dst >= cap) continue;
-    const int k = q.item / g.tiles;
-    const unsigned tris = static_cast<unsigned>(q.tris);
-    dh_contact c;
-    make_contact(load_pair(g, k), k, static_cast<int>(tris & 0xffffu), static_cast<int>(tris >> 16),
-                 V3<double>{q.pq[0], q.pq[1], q.pq[2]}, V3<double>{q.pq[3], q.pq[4], q.pq[5]}, &c);
-    c.pad_ = 0;
-    out[dst] = c;
+  const int total = r < g.regions ? g.rcount[r] : 0;
+  const bool heavy = total > g.heavy;
+  for (int p = 0; p < (heavy ? 4 : total > 0 ? 1 : 0); ++p) {
+    const int* c = g.rparts + 8 * static_cast<long long>(r) + 2 * p;
+    const int n = heavy ? c[0] : g.rcount[g.regions + r];
+    if (n == 0) continue;
+    const QueueRecord* rec =
+        g.rec + static_cast<long long>(r) * g.rcap + (heavy ? p * region_part(total) : 0);
+    const int base = heavy ? c[1] : 0, first = rec[0].item;
+    for (int e = lane; e < n; e += 64) {
+      const QueueRecord q = rec[e];
+      const long long dst = contact_place(g, q.item, q.rank + (q.item == first ? base : 0), offs);
+      if (dst >= cap) continue;  // past the capacity: dropped (reported by the caller)
+      const int k = q.item / g.tiles;
+      const unsigned tris = static_cast<unsigned>(q.tris);
+      dh_contact ct;
+      make_contact(load_pair(g, k), k, static_cast<int>(tris & 0xffffu),
+                   static_cast<int>(tris >> 16), V3<double>{q.pq[0], q.pq[1], q.pq[2]},
+                   V3<double>{q.pq[3], q.pq[4], q.pq[5]}, &ct);
+      ct.pad_ = 0;
+      out[dst] = ct;
+    }
   }
   const unsigned long long nt = *in_temp < static_cast<unsigned long long>(g.cap)
                                     ? *in_temp : static_cast<unsigned long long>(g.cap);
@@ -1621,7 +1706,7 @@ int queue_learned_reserve(long long n);
 
 struct DetectScratch {
   DevBuf temp, counter, stats, error, counts, offs, sums, tiles, tstats, iskip, tmax;
-  DevBuf queue, qrec, qcounts, rcount, deferred, wlist, found, qflags, qpq;
+  DevBuf queue, qrec, qcounts, rcount, rparts, deferred, wlist, found, qflags, qpq;
   int rwant = 0;  // what a region had to hold in earlier eager calls
 };
 static DetectScratch g_scratch;
@@ -1763,9 +1848,11 @@ static int tiles_for(long long npairs, int method) {
 // k_detect_wave's persistent grid (as many as the CUs hold at once), 16 entries
 // per item over the regions and at least 1,024 in each, or what earlier calls
 // needed.
+// With fewer than 16 items per region, those with more than 256 entries are
+// shared by four waves in k_queue_solve; with more, the regions are alike.
 struct QueuePlan {
   unsigned groups;
-  int regions, rcap;
+  int regions, rcap, heavy;
   long long entries() const { return static_cast<long long>(regions) * rcap; }
 };
 
@@ -1780,6 +1867,7 @@ static QueuePlan queue_plan(long long items, int rwant) {
   if (r < rwant) r = rwant;
   const long long rmost = (1ll << 30) / q.regions;
   q.rcap = static_cast<int>(r < rmost ? r : rmost);
+  q.heavy = items < 16ll * q.regions ? 256 : 0x7fffffff;
   return q;
 }
 
@@ -1793,6 +1881,7 @@ static int queue_reserve(const QueuePlan& q, long long items, bool learned) {
   if ((rc = g_scratch.qrec.grow(sizeof(QueueRecord) * q.entries()))) return rc;
   if ((rc = g_scratch.qcounts.grow(sizeof(unsigned) * kQueueCounts))) return rc;
   if ((rc = g_scratch.rcount.grow(sizeof(int) * 2 * q.regions))) return rc;
+  if ((rc = g_scratch.rparts.grow(sizeof(int) * 8 * q.regions))) return rc;
   if ((rc = g_scratch.deferred.grow(sizeof(int) * (items + 1)))) return rc;
   if ((rc = g_scratch.wlist.grow(sizeof(WaveItem) * (items + 1)))) return rc;
   if ((rc = g_scratch.found.grow(sizeof(unsigned long long)))) return rc;
@@ -1810,6 +1899,8 @@ static void queue_bind(DetectArgs& a, const QueuePlan& q) {
   a.rcap = q.rcap;
   a.regions = q.regions;
   a.rcount = g_scratch.rcount.as<int>();
+  a.rparts = g_scratch.rparts.as<int>();
+  a.heavy = q.heavy;
   a.rwant = reinterpret_cast<int*>(c + QC_RWANT);
   a.rec = g_scratch.qrec.as<QueueRecord>();
   a.deferred = g_scratch.deferred.as<int>();
@@ -1882,6 +1973,18 @@ static DetectArgs detect_args(const dh_geometry* geom, const int* pairs, int npa
   return a;
 }
 
+// Items as detect_queue_min_items counts them: one for every 16 triangles of
+// the mean particle.  The queue's launches and their chain of dependent loads
+// cost some 40 us; without it each item is a workgroup's, which the larger
+// particles make the costlier (captured steps with and without the queue: 36
+// pairs of 80 triangles 92 and 83 us, 484 pairs 113 and 124, 2,500 pairs 134
+// and 169, 33,000 pairs 235 and 612).
+static long long queue_items(long long items, const dh_geometry* geom) {
+  const long long per = geom->nparticles > 0
+                            ? static_cast<long long>(geom->ntri_total) / geom->nparticles / 16 : 0;
+  return per > 1 ? items * per : items;
+}
+
 int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int npairs,
                       dh_contact* out, long long cap, long long* n_total, int* pair_count_user,
                       long long* offs_out, dh_stats* stats, hipStream_t st,
@@ -1916,10 +2019,12 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
   DetectArgs a = detect_args(geom, pairs, npairs, nullptr, cap, tiles, tile_count, bf, pbox, bbox,
                              psph);
   // the queue costs launches: for many items only
-  const bool queued = bf && (learned || nitems >= tuning().detect_queue_min_items);
+  const bool queued =
+      bf && (learned || queue_items(nitems, geom) >= tuning().detect_queue_min_items);
   QueuePlan plan = {};
   if (queued) {
     plan = queue_plan(nitems, g_scratch.rwant);
+    if (learned) plan.heavy = 0x7fffffff;
     if ((rc = queue_reserve(plan, nitems, learned))) return rc;
     DH_HIP_CHECK(hipMemsetAsync(g_scratch.qcounts.ptr, 0, sizeof(unsigned) * kQueueCounts, st));
     queue_bind(a, plan);
@@ -2016,16 +2121,16 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
   return DH_OK;
 }
 
-int detect_reserve(int pair_cap, long long contact_cap, int method);
+int detect_reserve(const dh_geometry* geom, int pair_cap, long long contact_cap, int method);
 
 // Tiles of the captured step, sized for half the pair capacity live.
 static int graph_tiles(int pair_cap) { return tiles_for(pair_cap / 2 > 0 ? pair_cap / 2 : 1, DH_BF); }
 
 // Whether a captured step's detection goes through the survivor queue.
-static bool graph_queued(int method, int pair_cap) {
+static bool graph_queued(int method, const dh_geometry* geom, int pair_cap) {
   const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
   return method == DH_BF_LEARNED ||
-         (method == DH_BF && items >= tuning().detect_queue_min_items);
+         (method == DH_BF && queue_items(items, geom) >= tuning().detect_queue_min_items);
 }
 
 // Detection for a captured step: launches for `pair_cap` pairs of which
@@ -2037,9 +2142,9 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
                        int* counts, long long* offs, hipStream_t st, const double* pbox,
                        const double* bbox, const double* psph) {
   int rc;
-  if ((rc = detect_reserve(pair_cap, contact_cap, method))) return rc;
+  if ((rc = detect_reserve(geom, pair_cap, contact_cap, method))) return rc;
   const bool learned = method == DH_BF_LEARNED;
-  const bool queued = graph_queued(method, pair_cap);
+  const bool queued = graph_queued(method, geom, pair_cap);
   if (learned) method = DH_BF;
   zero_async(ZeroRegions{{g_scratch.counter.as<unsigned>(), g_scratch.stats.as<unsigned>(),
                           g_scratch.error.as<unsigned>(),
@@ -2057,6 +2162,7 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
   QueuePlan plan = {};
   if (queued) {
     plan = queue_plan(items, 0);
+    if (learned) plan.heavy = 0x7fffffff;
     queue_bind(a, plan);
   }
   switch (method) {
@@ -2098,9 +2204,9 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
 
 // Buffers of detect_pairs_graph (call before a capture: no allocation may
 // happen inside one).
-int detect_reserve(int pair_cap, long long contact_cap, int method) {
+int detect_reserve(const dh_geometry* geom, int pair_cap, long long contact_cap, int method) {
   int rc;
-  if (graph_queued(method, pair_cap)) {
+  if (graph_queued(method, geom, pair_cap)) {
     const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
     if ((rc = queue_reserve(queue_plan(items, 0), items, method == DH_BF_LEARNED))) return rc;
   }
@@ -2124,8 +2230,9 @@ int detect_reserve(int pair_cap, long long contact_cap, int method) {
 
 // Device addresses of the detection counters of a captured step: the contacts
 // found, the error flag and the statistics.
-const unsigned long long* detect_counter_dev(int method, int pair_cap) {
-  return graph_queued(method, pair_cap) ? g_scratch.found.as<unsigned long long>()
+const unsigned long long* detect_counter_dev(int method, const dh_geometry* geom,
+                                             int pair_cap) {
+  return graph_queued(method, geom, pair_cap) ? g_scratch.found.as<unsigned long long>()
                                         : g_scratch.counter.as<unsigned long long>();
 }
 const int* detect_error_dev() { return g_scratch.error.as<int>(); }

@@ -78,7 +78,7 @@ constexpr int kForceRow = 13;
 // Pairs a wave of k_pair_forces takes in lists longer than kForcesFewPairs.
 constexpr int kForcesGroup = 16;
 constexpr int kForcesFewGroup = 4;
-constexpr int kForcesFewPairs = 16384;
+constexpr int kForcesFewPairs = 131072;
 
 // Contact forces of both sides of every pair into pf and, with `incidence`,
 // the particles' counts of contact-carrying pairs.  A wave takes G consecutive
@@ -90,8 +90,8 @@ constexpr int kForcesFewPairs = 16384;
 // 17,000 contacts at 300 us and a lattice of 484 pairs and 14,000 contacts at
 // 120 us: a serial chain of scattered loads, square roots and divisions.
 // G = 4 spreads a short list over the GPU (lattice 13.5 us, G = 16 31 us; the
-// funnel's 22 against 51 us); with more than kForcesFewPairs pairs there are
-// waves enough, and G = 16 fills more of a wave's lanes where most pairs
+// funnel's 15,700 pairs 22 against 51 us); with more than kForcesFewPairs pairs
+// there are waves enough, and G = 16 fills more of a wave's lanes where most pairs
 // carry no contact (hopper of 1.9e5 pairs 52 us, G = 4 75 us; G = 64 71 us:
 // its waves meet up to ten rounds of 64 contacts one after the other).
 template <int G>

@@ -23,9 +23,9 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
                        const long long* np_dev, dh_contact* out, long long contact_cap,
                        int* counts, long long* offs, hipStream_t st, const double* pbox,
                        const double* bbox, const double* psph);
-int detect_reserve(int pair_cap, long long contact_cap, int method);
+int detect_reserve(const dh_geometry* geom, int pair_cap, long long contact_cap, int method);
 int detect_prepare(const dh_geometry* geom, hipStream_t st);
-const unsigned long long* detect_counter_dev(int method, int pair_cap);
+const unsigned long long* detect_counter_dev(int method, const dh_geometry* geom, int pair_cap);
 const int* detect_error_dev();
 const unsigned long long* detect_stats_dev();
 int forces_reserve(int n, int npairs);
@@ -200,7 +200,7 @@ static int record_step(dh_step_graph* g, hipStream_t st) {
   if (ad && (rc = adaptive_finish(s->bodies.linvel, s->bodies.obstacle, s->bodies.n, ad, st)))
     return rc;
   hipLaunchKernelGGL(k_step_status, 1, 64, 0, st, np_dev,
-                     detect_counter_dev(g->params.method, static_cast<int>(g->pair_cap)),
+                     detect_counter_dev(g->params.method, &s->geom, static_cast<int>(g->pair_cap)),
                      detect_error_dev(),
                      detect_stats_dev(), g->pair_cap, g->contact_cap, g->status.as<long long>());
   DH_HIP_CHECK(hipGetLastError());
@@ -248,9 +248,10 @@ int dh_step_graph_create(const dh_scene* scene, const dh_step_params* params, in
       (rc = g->torque.grow(sizeof(double) * 3 * (n + 1))) ||
       (rc = g->touched.grow(sizeof(int) * (n + 1))) ||
       (rc = g->status.grow(sizeof(long long) * 6)) || (rc = broadphase_reserve(n, scene->geom.ntri_total)) ||
-      (rc = detect_reserve(static_cast<int>(pair_cap > n ? pair_cap : n), contact_cap,
+      (rc = detect_reserve(&scene->geom, static_cast<int>(pair_cap > n ? pair_cap : n), contact_cap,
                            params->method)) ||
-      (rc = detect_reserve(static_cast<int>(pair_cap), contact_cap, params->method)) ||
+      (rc = detect_reserve(&scene->geom, static_cast<int>(pair_cap), contact_cap,
+                           params->method)) ||
       (rc = forces_reserve(n, static_cast<int>(pair_cap)))) {
     destroy_graph(g);
     return rc;

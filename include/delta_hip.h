@@ -348,9 +348,10 @@ typedef struct dh_tuning {
                                  per (pair, rows) item; else a persistent grid
                                  of this many workgroups per CU (1..64)      */
   int32_t detect_queue_min_items; /* DH_BF detection of at least this many
-                                 items (pairs x tiles) solves the survivors of
-                                 the box test from one queue, one per lane
-                                 (0..2^30)                                   */
+                                 items (pairs x tiles, each counted once per 16
+                                 triangles of the mean particle) solves the
+                                 survivors of the box test from a queue, one
+                                 per lane (0..2^30)                          */
   int32_t detect_fp32_screen; /* 1: queued survivors are first solved in
                                  binary32 (coordinates relative to A's first
                                  vertex); those at twice the margin or more
