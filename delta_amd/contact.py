@@ -61,13 +61,20 @@ def _sig(f):
     return f
 
 
+_bound = False
+
+
 def _bind():
+    global _bound
+    if _bound:
+        return
     L = _lib.lib()
     L.dh_detect_pair.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int,
                                  C.c_double, C.c_int, C.c_int, C.c_void_p, C.c_void_p,
                                  C.c_void_p, C.c_int, C.c_double, C.c_int, C.c_int, C.c_void_p,
                                  C.c_int, C.POINTER(C.c_int), C.POINTER(_lib.DhStats)]
     L.dh_detect_pair.restype = C.c_int
+    _bound = True
 
 
 def bf(xA, yA, zA, numberOfTrianglesOfGeometryA, epsilonA, frictionA, particleA,

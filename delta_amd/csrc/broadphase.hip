@@ -786,11 +786,19 @@ static void grid_fill(const GridArgs& g, const BpBuffers& b, long long cap, int*
                      64 * kBpWaves, 0, st, g, b.start, cap, pairs);
 }
 
-// The eager broad phase on the buffers b: the total is read back, and the
-// pairs are written only if it fits cap.
+// The eager broad phase on the buffers b: the total is read back (through the
+// library's pinned mailbox, or by a copy where nothing may be allocated), and
+// the pairs are written only if it fits cap.
 static int broadphase_run(const dh_geometry* geom, const int* obstacle_dev, double cell,
-                          const BpBuffers& b, int* pairs, long long cap, long long* npairs,
-                          hipStream_t st) {
+                          const BpBuffers& b, bool mailbox, int* pairs, long long cap,
+                          long long* npairs, hipStream_t st) {
+  auto read_total = [&](long long* total) -> int {
+    if (mailbox) return read_back(b.start + geom->nparticles, 2, total, st);
+    DH_HIP_CHECK(hipMemcpyAsync(total, b.start + geom->nparticles, sizeof(long long),
+                                hipMemcpyDeviceToHost, st));
+    DH_HIP_CHECK(hipStreamSynchronize(st));
+    return DH_OK;
+  };
   const int n = geom->nparticles;
   if (n <= kSmallScene) {
     // one workgroup tests every pair; nothing is written past cap, so the
@@ -803,10 +811,8 @@ static int broadphase_run(const dh_geometry* geom, const int* obstacle_dev, doub
       DH_HIP_CHECK(hipGetLastError());
     }
     long long total = 0;
-    if (n > 0)
-      DH_HIP_CHECK(hipMemcpyAsync(&total, b.start + n, sizeof(long long), hipMemcpyDeviceToHost,
-                                  st));
-    DH_HIP_CHECK(hipStreamSynchronize(st));
+    int rc;
+    if (n > 0 && (rc = read_total(&total))) return rc;
     *npairs = total;
     return total > cap ? DH_ERR_CAPACITY : DH_OK;
   }
@@ -815,8 +821,7 @@ static int broadphase_run(const dh_geometry* geom, const int* obstacle_dev, doub
   int rc;
   if ((rc = grid_build(geom, obstacle_dev, cell, b, g, st))) return rc;
   long long total = 0;
-  DH_HIP_CHECK(hipMemcpyAsync(&total, b.start + n, sizeof(long long), hipMemcpyDeviceToHost, st));
-  DH_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = read_total(&total))) return rc;
   *npairs = total;
   if (*npairs > cap) return DH_ERR_CAPACITY;
   grid_fill(g, b, cap, pairs, st);
@@ -828,7 +833,7 @@ int broadphase_impl(const dh_geometry* geom, const int* obstacle_dev, double cel
                     long long cap, long long* npairs, hipStream_t st) {
   int rc;
   if ((rc = broadphase_reserve(geom->nparticles, geom->ntri_total))) return rc;
-  return broadphase_run(geom, obstacle_dev, cell, library_buffers(), pairs, cap, npairs, st);
+  return broadphase_run(geom, obstacle_dev, cell, library_buffers(), true, pairs, cap, npairs, st);
 }
 
 // The broad phase for a captured step: the same kernels with no host
@@ -965,7 +970,7 @@ extern "C" int dh_broadphase_noalloc(const dh_geometry* geom, const int* obstacl
   if (noalloc_layout(base, geom->nparticles, geom->ntri_total, &b) > kNaScratchBytes)
     return set_error(DH_ERR_CAPACITY, "dh_broadphase_noalloc: scratch layout too large");
   long long np = 0;
-  rc = broadphase_run(geom, obstacle_dev, cell, b, pairs_dev, cap, &np, as_stream(stream));
+  rc = broadphase_run(geom, obstacle_dev, cell, b, false, pairs_dev, cap, &np, as_stream(stream));
   *npairs = static_cast<int>(np);
   return rc;
 }

@@ -1405,18 +1405,22 @@ __global__ __launch_bounds__(256) void k_scatter(const dh_contact* __restrict__ 
                                                  const long long* __restrict__ offs,
                                                  const int* __restrict__ tile_count, int tiles,
                                                  dh_contact* __restrict__ out,
-                                                 const unsigned long long* __restrict__ n_dev) {
-  const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-  // n is the capacity (of temp and out) when the count is read from n_dev
-  if (i >= n || (n_dev && static_cast<unsigned long long>(i) >= *n_dev)) return;
-  dh_contact c = temp[i];
-  const int pair = c.pair / tiles;
-  long long dst = offs[pair] + c.pad_;
-  for (int t = pair * tiles; t < c.pair; ++t) dst += tile_count[t];
-  if (dst >= n) return;  // more contacts than the capacity (reported by the caller)
-  c.pair = pair;
-  c.pad_ = 0;
-  out[dst] = c;
+                                                 const unsigned long long* __restrict__ n_dev,
+                                                 Report report) {
+  // n is the capacity (of temp and out), the count is read from n_dev
+  const long long live = static_cast<long long>(*n_dev) < n ? static_cast<long long>(*n_dev) : n;
+  for (long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; i < live;
+       i += static_cast<long long>(gridDim.x) * 256) {
+    dh_contact c = temp[i];
+    const int pair = c.pair / tiles;
+    long long dst = offs[pair] + c.pad_;
+    for (int t = pair * tiles; t < c.pair; ++t) dst += tile_count[t];
+    if (dst >= n) continue;  // more contacts than the capacity (reported by the caller)
+    c.pair = pair;
+    c.pad_ = 0;
+    out[dst] = c;
+  }
+  if (blockIdx.x == 0) report_write(report, threadIdx.x, 256);
 }
 
 // Survivor queue, pass 2: every wave takes one region of k_detect_wave's through
@@ -1658,7 +1662,8 @@ __device__ __forceinline__ long long contact_place(const DetectArgs& g, int item
 __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long long* __restrict__ offs,
                                                      dh_contact* __restrict__ out, long long cap,
                                                      const unsigned long long* __restrict__ in_temp,
-                                                     unsigned long long* __restrict__ found) {
+                                                     unsigned long long* __restrict__ found,
+                                                     Report report) {
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
   const int total = r < g.regions ? g.rcount[r] : 0;
@@ -1697,6 +1702,7 @@ __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long lo
   if (found && blockIdx.x == 0 && threadIdx.x == 0)
     *found = static_cast<unsigned long long>(
         offs[g.npairs_dev && *g.npairs_dev < g.npairs ? *g.npairs_dev : g.npairs]);
+  if (blockIdx.x == 0) report_write(report, threadIdx.x, 256);
 }
 
 int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
@@ -1973,6 +1979,28 @@ static DetectArgs detect_args(const dh_geometry* geom, const int* pairs, int npa
   return a;
 }
 
+// After the detection: the tile counters summed, the pairs' contact counts and
+// their offsets (of the live pairs).
+static int pair_offsets(const DetectArgs& a, int* counts, long long* offs, hipStream_t st) {
+  if (a.npairs <= kTailPairs) {
+    const auto f = a.nstats == kBfStats ? k_detect_tail_small<kBfStats>
+                                        : k_detect_tail_small<kTileStats>;
+    hipLaunchKernelGGL(f, 1, 1024, 0, st, a.tile_stats, a.npairs_dev, a.stats, a.tile_count,
+                       a.tiles, a.npairs, counts, offs);
+    DH_HIP_CHECK(hipGetLastError());
+    return DH_OK;
+  }
+  launch_tile_stats(a, st);
+  if (a.tiles > 1)
+    hipLaunchKernelGGL(k_tile_sums, grid_for(a.npairs, 256), 256, 0, st, a.tile_count, a.tiles,
+                       a.npairs, counts);
+  int rc = g_scratch.sums.grow(sizeof(long long) * scan_sums_len(a.npairs));
+  if (rc) return rc;
+  return scan_counts_upto(counts, a.npairs,
+                          reinterpret_cast<const unsigned long long*>(a.npairs_dev), offs,
+                          g_scratch.sums.as<long long>(), st);
+}
+
 // Items as detect_queue_min_items counts them: one for every 16 triangles of
 // the mean particle.  The queue's launches and their chain of dependent loads
 // cost some 40 us; without it each item is a workgroup's, which the larger
@@ -2001,9 +2029,6 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
   if ((rc = g_scratch.error.grow(sizeof(int)))) return rc;
   if ((rc = g_scratch.counts.grow(sizeof(int) * (npairs + 1)))) return rc;
   if ((rc = g_scratch.offs.grow(sizeof(long long) * (npairs + 1)))) return rc;
-  DH_HIP_CHECK(hipMemsetAsync(g_scratch.counter.ptr, 0, sizeof(unsigned long long), st));
-  DH_HIP_CHECK(hipMemsetAsync(g_scratch.stats.ptr, 0, sizeof(unsigned long long) * ST_COUNT, st));
-  DH_HIP_CHECK(hipMemsetAsync(g_scratch.error.ptr, 0, sizeof(int), st));
   int* counts = pair_count_user ? pair_count_user : g_scratch.counts.as<int>();
   const int tiles = tiles_for(npairs, method);
   int* tile_count = counts;
@@ -2026,9 +2051,13 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
     plan = queue_plan(nitems, g_scratch.rwant);
     if (learned) plan.heavy = 0x7fffffff;
     if ((rc = queue_reserve(plan, nitems, learned))) return rc;
-    DH_HIP_CHECK(hipMemsetAsync(g_scratch.qcounts.ptr, 0, sizeof(unsigned) * kQueueCounts, st));
     queue_bind(a, plan);
   }
+  zero_async(ZeroRegions{{g_scratch.counter.as<unsigned>(), g_scratch.stats.as<unsigned>(),
+                          g_scratch.error.as<unsigned>(),
+                          queued ? g_scratch.qcounts.as<unsigned>() : nullptr},
+                         {2, 2 * ST_COUNT, 1, kQueueCounts}},
+             st);
   const size_t shm_rows = 2 * kMaxRowTriangles * sizeof(int) + 8 + kMaxRowTriangles * 8;
   const unsigned items = static_cast<unsigned>(nitems);
   if (bf && !queued && pbox && bbox &&
@@ -2056,38 +2085,36 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
       return set_error(DH_ERR_UNSUPPORTED, "dh_detect_pairs: method %d", method);
   }
   DH_HIP_CHECK(hipGetLastError());
-  launch_tile_stats(a, st);
   long long* offs = offs_out ? offs_out : g_scratch.offs.as<long long>();
-  auto pair_offsets = [&]() {
-    if (tiles > 1)
-      hipLaunchKernelGGL(k_tile_sums, grid_for(npairs, 256), 256, 0, st, tile_count, tiles,
-                         npairs, counts);
-    return scan_counts(counts, npairs, offs, st);
-  };
-  // the queue's contacts are counted by the pairs' offsets alone
-  if (queued && (rc = pair_offsets())) return rc;
-  unsigned long long in_temp = 0;
-  int err = 0;
-  unsigned long long st_host[ST_COUNT];
-  unsigned qc[kQueueCounts] = {};
-  long long all = 0;
-  DH_HIP_CHECK(hipMemcpyAsync(&in_temp, g_scratch.counter.ptr, sizeof(in_temp),
-                              hipMemcpyDeviceToHost, st));
-  DH_HIP_CHECK(hipMemcpyAsync(&err, g_scratch.error.ptr, sizeof(err), hipMemcpyDeviceToHost, st));
-  DH_HIP_CHECK(hipMemcpyAsync(st_host, g_scratch.stats.ptr, sizeof(st_host),
-                              hipMemcpyDeviceToHost, st));
+  if ((rc = pair_offsets(a, counts, offs, st))) return rc;
+  // the contacts to their places, with the counts reported: one wait for all
+  Report report;
+  if ((rc = report_open(report))) return rc;
+  report_add(report, offs + npairs, 2);
+  report_add(report, g_scratch.error.ptr, 1);
+  report_add(report, g_scratch.stats.ptr, 2 * ST_COUNT);
   if (queued) {
-    DH_HIP_CHECK(hipMemcpyAsync(&all, offs + npairs, sizeof(all), hipMemcpyDeviceToHost, st));
-    DH_HIP_CHECK(hipMemcpyAsync(qc, g_scratch.qcounts.ptr, sizeof(qc), hipMemcpyDeviceToHost, st));
+    report_add(report, g_scratch.qcounts.ptr, kQueueCounts);
+    hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out, cap,
+                       a.counter, nullptr, report);
+  } else {
+    const long long wg = (cap + 255) / 256;
+    hipLaunchKernelGGL(k_scatter, static_cast<unsigned>(wg < 1 ? 1 : (wg < 2048 ? wg : 2048)), 256,
+                       0, st, a.temp, cap, offs, tile_count, tiles, out, a.counter, report);
   }
-  DH_HIP_CHECK(hipStreamSynchronize(st));
+  if ((rc = report_wait(st))) return rc;
+  unsigned long long total;
+  int err;
+  unsigned long long st_host[ST_COUNT];
+  std::memcpy(&total, report.mail, sizeof(total));
+  std::memcpy(&err, report.mail + 2, sizeof(err));
+  std::memcpy(st_host, report.mail + 3, sizeof(st_host));
   if (queued) {
     // the next call's regions hold this call's need
-    const long long want = qc[QC_RWANT];
+    const long long want = report.mail[3 + 2 * ST_COUNT + QC_RWANT];
     if (want > plan.rcap)
       g_scratch.rwant = static_cast<int>(want + want / 4 < (1 << 29) ? want + want / 4 : 1 << 29);
   }
-  const unsigned long long total = queued ? static_cast<unsigned long long>(all) : in_temp;
   if (err == DE_REF_UB)
     return set_error(DH_ERR_REF_UB,
                      "hybridWithPerTriangleFallBack reads row iA < nTriB of A: nTriB > nTriA is "
@@ -2107,17 +2134,6 @@ int detect_pairs_impl(int method, const dh_geometry* geom, const int* pairs, int
     stats->pairs_culled += st_host[ST_CULLED];
   }
   if (static_cast<long long>(total) > cap) return DH_ERR_CAPACITY;
-  if (!queued && (rc = pair_offsets())) return rc;
-  if (queued) {
-    if (total > 0)
-      hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out, cap,
-                         a.counter, nullptr);
-  } else if (total > 0) {
-    hipLaunchKernelGGL(k_scatter, grid_for(static_cast<int64_t>(total), 256), 256, 0, st,
-                       g_scratch.temp.as<dh_contact>(), static_cast<long long>(total), offs,
-                       tile_count, tiles, out, nullptr);
-  }
-  DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
 
@@ -2175,29 +2191,15 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
       return set_error(DH_ERR_UNSUPPORTED, "captured step: method %d (use DH_BF or DH_PENALTY)",
                        method);
   }
-  if (pair_cap <= kTailPairs) {
-    const auto f = bf ? k_detect_tail_small<kBfStats> : k_detect_tail_small<kTileStats>;
-    hipLaunchKernelGGL(f, 1, 1024, 0, st, a.tile_stats, np_dev, a.stats, a.tile_count, tiles,
-                       pair_cap, counts, offs);
-  } else {
-    launch_tile_stats(a, st);
-    if (tiles > 1)
-      hipLaunchKernelGGL(k_tile_sums, grid_for(pair_cap, 256), 256, 0, st, a.tile_count, tiles,
-                         pair_cap, counts);
-    if ((rc = g_scratch.sums.grow(sizeof(long long) * scan_sums_len(pair_cap)))) return rc;
-    // the live pairs' counts (the pairs past them have none)
-    if ((rc = scan_counts_upto(counts, pair_cap,
-                               reinterpret_cast<const unsigned long long*>(np_dev), offs,
-                               g_scratch.sums.as<long long>(), st)))
-      return rc;
-  }
-  if (queued)
+  if ((rc = pair_offsets(a, counts, offs, st))) return rc;
+  if (queued) {
     hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out,
-                       contact_cap, a.counter, g_scratch.found.as<unsigned long long>());
-  else
-    hipLaunchKernelGGL(k_scatter, grid_for(contact_cap, 256), 256, 0, st,
-                       g_scratch.temp.as<dh_contact>(), contact_cap, offs, a.tile_count, tiles, out,
-                       g_scratch.counter.as<unsigned long long>());
+                       contact_cap, a.counter, g_scratch.found.as<unsigned long long>(), Report{});
+  } else {
+    const long long wg = (contact_cap + 255) / 256;
+    hipLaunchKernelGGL(k_scatter, static_cast<unsigned>(wg < 2048 ? wg : 2048), 256, 0, st, a.temp,
+                       contact_cap, offs, a.tile_count, tiles, out, a.counter, Report{});
+  }
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }
@@ -2237,6 +2239,17 @@ const unsigned long long* detect_counter_dev(int method, const dh_geometry* geom
 }
 const int* detect_error_dev() { return g_scratch.error.as<int>(); }
 const unsigned long long* detect_stats_dev() { return g_scratch.stats.as<unsigned long long>(); }
+
+// Contacts of a host call that come back through pinned memory (65,536 of them
+// take 9.4 MB); more are copied.
+constexpr size_t kPinnedContactBytes = 16u << 20;
+
+__global__ __launch_bounds__(256) void k_fetch(const double* __restrict__ src,
+                                               double* __restrict__ dst, long long n) {
+  for (long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; i < n;
+       i += static_cast<long long>(gridDim.x) * 256)
+    dst[i] = src[i];
+}
 
 // _batchError of the *Stat drivers: maxErr added once per row, in row order
 // and pair order (hybrid.cpp:240,530).
@@ -2308,45 +2321,43 @@ int dh_detect_pair(int method, const double* xA, const double* yA, const double*
                      "hybridWithPerTriangleFallBack reads row iA < nTriB of A: nTriB > nTriA is "
                      "out of bounds in the reference (hybrid.cpp:130)");
   if (nTriA == 0 || nTriB == 0) return DH_OK;
-  static DevBuf geo, meta, pairs_buf, outbuf;
-  const size_t nv = 3 * static_cast<size_t>(nTriA + nTriB);
-  if ((rc = geo.grow(3 * nv * sizeof(double)))) return rc;
-  if ((rc = meta.grow(64 + 2 * sizeof(double) + 9 * sizeof(int)))) return rc;
-  if ((rc = pairs_buf.grow(2 * sizeof(int)))) return rc;
-  double* gx = geo.as<double>();
-  double* gy = gx + nv;
-  double* gz = gy + nv;
-  const size_t na = 3 * static_cast<size_t>(nTriA), nb = 3 * static_cast<size_t>(nTriB);
-  DH_HIP_CHECK(hipMemcpy(gx, xA, na * 8, hipMemcpyHostToDevice));
-  DH_HIP_CHECK(hipMemcpy(gx + na, xB, nb * 8, hipMemcpyHostToDevice));
-  DH_HIP_CHECK(hipMemcpy(gy, yA, na * 8, hipMemcpyHostToDevice));
-  DH_HIP_CHECK(hipMemcpy(gy + na, yB, nb * 8, hipMemcpyHostToDevice));
-  DH_HIP_CHECK(hipMemcpy(gz, zA, na * 8, hipMemcpyHostToDevice));
-  DH_HIP_CHECK(hipMemcpy(gz + na, zB, nb * 8, hipMemcpyHostToDevice));
+  // The two particles go to the device in one block, staged in pinned memory
+  // and fetched from there by a kernel, and the contacts come back into pinned
+  // memory, written by the kernel that orders them: one wait per call (seven
+  // copies in and one out cost 170 of the 205 us of a 20 x 20 call).
   struct Meta {
     double eps[2];
     int off[3];
     int fric[2];
     int id[2];
     int pairs[2];
-  } m;
-  m.eps[0] = epsA;
-  m.eps[1] = epsB;
-  m.off[0] = 0;
-  m.off[1] = nTriA;
-  m.off[2] = nTriA + nTriB;
-  m.fric[0] = frictionA ? 1 : 0;
-  m.fric[1] = frictionB ? 1 : 0;
-  m.id[0] = idA;
-  m.id[1] = idB;
-  m.pairs[0] = 0;
-  m.pairs[1] = 1;
-  DH_HIP_CHECK(hipMemcpy(meta.ptr, &m, sizeof(m), hipMemcpyHostToDevice));
-  const Meta* dm = meta.as<Meta>();
+    int pad_[3];
+  };
+  static_assert(sizeof(Meta) % 16 == 0, "the vertices follow on a 16-byte boundary");
+  static DevBuf geo, outbuf;
+  static PinnedBuf stage, pinned_out;
+  const size_t na = 3 * static_cast<size_t>(nTriA), nb = 3 * static_cast<size_t>(nTriB);
+  const size_t nv = na + nb, block = sizeof(Meta) + 3 * nv * sizeof(double);
+  if ((rc = geo.grow(block))) return rc;
+  if ((rc = stage.grow(block))) return rc;
+  const Meta m = {{epsA, epsB},   {0, nTriA, nTriA + nTriB}, {frictionA ? 1 : 0, frictionB ? 1 : 0},
+                  {idA, idB},     {0, 1},                    {0, 0, 0}};
+  std::memcpy(stage.ptr, &m, sizeof(m));
+  double* v = reinterpret_cast<double*>(static_cast<char*>(stage.ptr) + sizeof(Meta));
+  const double* axes[3][2] = {{xA, xB}, {yA, yB}, {zA, zB}};
+  for (int q = 0; q < 3; ++q) {
+    std::memcpy(v + q * nv, axes[q][0], na * sizeof(double));
+    std::memcpy(v + q * nv + na, axes[q][1], nb * sizeof(double));
+  }
+  const long long words = static_cast<long long>(block / 8);
+  hipLaunchKernelGGL(k_fetch, grid_for(words, 256) < 256 ? grid_for(words, 256) : 256, 256, 0,
+                     nullptr, static_cast<const double*>(stage.ptr), geo.as<double>(), words);
+  DH_HIP_CHECK(hipGetLastError());
+  const Meta* dm = geo.as<Meta>();
   dh_geometry g;
-  g.x = gx;
-  g.y = gy;
-  g.z = gz;
+  g.x = reinterpret_cast<double*>(geo.as<char>() + sizeof(Meta));
+  g.y = g.x + nv;
+  g.z = g.y + nv;
   g.tri_offset = dm->off;
   g.eps = dm->eps;
   g.friction = dm->fric;
@@ -2354,16 +2365,21 @@ int dh_detect_pair(int method, const double* xA, const double* yA, const double*
   g.nparticles = 2;
   g.ntri_total = nTriA + nTriB;
   const long long dcap = cap > 0 ? cap : 1;
-  if ((rc = outbuf.grow(sizeof(dh_contact) * dcap))) return rc;
+  const size_t out_bytes = sizeof(dh_contact) * dcap;
+  const bool direct = out_bytes <= kPinnedContactBytes;
+  if ((rc = direct ? pinned_out.grow(out_bytes) : outbuf.grow(out_bytes))) return rc;
+  dh_contact* dev_out = direct ? static_cast<dh_contact*>(pinned_out.ptr) : outbuf.as<dh_contact>();
   long long total = 0;
-  rc = detect_pairs_impl(method, &g, dm->pairs, 1, outbuf.as<dh_contact>(), cap, &total, nullptr,
+  rc = detect_pairs_impl(method, &g, dm->pairs, 1, dev_out, cap, &total, nullptr,
                          nullptr, stats, nullptr, nullptr, nullptr, nullptr);
   *n_out = static_cast<int>(total);
   if (rc != DH_OK) return rc;
   if (stats && (method == DH_HYBRID_BATCH_STAT || method == DH_HYBRID_TRIANGLE_STAT))
     stats->batch_error = batch_error_sum(stats->batch_error, (epsA + epsB) / 16, nTriA);
-  if (total > 0)
-    DH_HIP_CHECK(hipMemcpy(out, outbuf.ptr, sizeof(dh_contact) * total, hipMemcpyDeviceToHost));
+  if (total > 0 && direct)
+    std::memcpy(out, dev_out, sizeof(dh_contact) * total);
+  else if (total > 0)
+    DH_HIP_CHECK(hipMemcpy(out, dev_out, sizeof(dh_contact) * total, hipMemcpyDeviceToHost));
   return DH_OK;
 }
 

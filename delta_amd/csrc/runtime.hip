@@ -69,6 +69,46 @@ int DevBuf::grow(size_t need) {
   return DH_OK;
 }
 
+int PinnedBuf::grow(size_t need) {
+  if (need <= bytes && ptr) return DH_OK;
+  if (ptr) DH_HIP_CHECK(hipHostFree(ptr));
+  ptr = nullptr;
+  bytes = 0;
+  const size_t n = need < 4096 ? 4096 : need;
+  DH_HIP_CHECK(hipHostMalloc(&ptr, n, hipHostMallocMapped | hipHostMallocCoherent));
+  bytes = n;
+  return DH_OK;
+}
+
+static PinnedBuf g_mail;
+
+__global__ __launch_bounds__(64) void k_report(Report r) { report_write(r, threadIdx.x, 64); }
+
+int report_open(Report& r) {
+  r = {};
+  int rc = g_mail.grow(sizeof(unsigned) * Report::kWords);
+  if (rc) return rc;
+  r.mail = static_cast<unsigned*>(g_mail.ptr);
+  return DH_OK;
+}
+
+int report_wait(hipStream_t st) {
+  DH_HIP_CHECK(hipGetLastError());
+  DH_HIP_CHECK(hipStreamSynchronize(st));
+  return DH_OK;
+}
+
+int read_back(const void* src, int words, void* dst, hipStream_t st) {
+  Report r;
+  int rc = report_open(r);
+  if (rc) return rc;
+  report_add(r, src, words);
+  hipLaunchKernelGGL(k_report, 1, 64, 0, st, r);
+  if ((rc = report_wait(st))) return rc;
+  std::memcpy(dst, r.mail, sizeof(unsigned) * words);
+  return DH_OK;
+}
+
 }  // namespace dh
 
 using namespace dh;

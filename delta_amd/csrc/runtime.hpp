@@ -93,4 +93,51 @@ inline void zero_async(ZeroRegions z, hipStream_t st) {
   if (m > 0) hipLaunchKernelGGL(k_zero_regions, dim3(grid_for(m, 256), 4), 256, 0, st, z);
 }
 
+// Small results of device work for the host without a copy: a kernel writes
+// them to pinned host memory that the device sees, and the stream is waited
+// for once.  (Each hipMemcpyAsync to ordinary host memory and its wait cost
+// some 25 us, and a call read back three to five.)  One report is under way
+// at a time, like the library's scratch.
+struct Report {
+  enum { kParts = 6, kWords = 128 };
+  const unsigned* src[kParts];
+  int words[kParts];
+  unsigned* mail;  // kWords words of pinned host memory
+};
+
+// Adds `words` 32-bit words at src (device) to the report.
+inline void report_add(Report& r, const void* src, int words) {
+  for (int p = 0; p < Report::kParts; ++p)
+    if (!r.src[p]) {
+      r.src[p] = static_cast<const unsigned*>(src);
+      r.words[p] = words;
+      return;
+    }
+}
+
+// An empty report with the library's mailbox.
+int report_open(Report& r);
+// Waits for the stream; the words are then in r.mail, parts one after another.
+int report_wait(hipStream_t st);
+// The same for one part: writes, waits and copies it to dst.
+int read_back(const void* src, int words, void* dst, hipStream_t st);
+
+// Writes the report; by one workgroup of at least a wave.
+__device__ __forceinline__ void report_write(const Report& r, int tid, int nthreads) {
+  int at = 0;
+  for (int p = 0; p < Report::kParts; ++p) {
+    if (!r.src[p]) break;
+    for (int w = tid; w < r.words[p]; w += nthreads) r.mail[at + w] = r.src[p][w];
+    at += r.words[p];
+  }
+  __threadfence_system();
+}
+
+// A pinned host buffer that the device sees, growing like DevBuf.
+struct PinnedBuf {
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  int grow(size_t need);
+};
+
 }  // namespace dh
