@@ -250,7 +250,7 @@ def step(dscene, params, stream=None):
 class StepGraph:
     """dh_step_graph: the whole explicit step (broad phase, detection,
     forces, integration) captured once into a HIP graph with fixed pair and
-    contact capacities; each launch() replays it on the graph's own stream
+    contact capacities; each launch() replays it on the library's stream
     without host synchronisation.  status() reads the last replay's counts
     and the overflow bits of every replay since the previous status() (1
     pairs, 2 contacts, 4 detection error): a replay that overflowed dropped

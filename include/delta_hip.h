@@ -584,7 +584,7 @@ int dh_step(dh_scene* scene, const dh_step_params* params, dh_step_info* info, v
  * capacities.
  * A graph keeps the scene pointers it was created with, and shares the
  * library's scratch with the other entry points.  dh_step_graph_launch
- * replays on `stream`, or on the graph's own blocking stream when NULL; a
+ * replays on `stream`, or on the library's own blocking stream when NULL; a
  * non-blocking stream is rejected (DH_ERR_ARG), since it would not wait for
  * eager work on the null stream.  Each launch waits for the previous launch
  * of any graph, so replays of different graphs never overlap; eager entry
