@@ -23,141 +23,242 @@ struct Aabb {
   double lo[3], hi[3];
 };
 
-// Vertex replicas per lane that the box pass loads at once and keeps for the
-// sphere pass (a particle of up to 64 * kAabbHeld replicas is read once).
-constexpr int kAabbHeld = 8;
+// Pairs of vertex replicas per lane that the box pass loads at once and keeps
+// for the sphere pass (a particle of up to 128 * kAabbHeld replicas is read
+// once).
+constexpr int kAabbHeld = 4;
+constexpr int kAabbWaves = 8;  // particles per workgroup
 
-__global__ __launch_bounds__(64) void k_particle_aabb(const double* __restrict__ x,
-                                                      const double* __restrict__ y,
-                                                      const double* __restrict__ z,
-                                                      const int* __restrict__ tri_offset,
-                                                      const double* __restrict__ eps,
-                                                      Aabb* __restrict__ box,
-                                                      Aabb* __restrict__ cbox,
-                                                      double* __restrict__ sph) {
-  const int i = blockIdx.x;
-  const int lane = static_cast<int>(threadIdx.x);
-  const int t0 = tri_offset[i], t1 = tri_offset[i + 1];
-  // a particle with more triangles than one row block keeps the box of each
-  // chunk of 64 of its triangles, chunk c at cbox[t0 / 64 + i + c] (an index
-  // that grows with i and c, so no two chunks share it)
-  const bool chunked = cbox && t1 - t0 > kRowBlock;
-  const int v0 = 3 * t0, nv = t1 > t0 ? 3 * (t1 - t0) : 0;
-  double plo[3] = {INFINITY, INFINITY, INFINITY}, phi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  // the held replicas (NaN past the end: min, max and the sphere skip NaN)
-  double hx[kAabbHeld], hy[kAabbHeld], hz[kAabbHeld];
-  auto load_block = [&](int b) {
+// Two consecutive doubles, loaded as 16 bytes from any 8-byte boundary (a
+// particle's replicas start at one).
+struct alignas(8) Two {
+  double a, b;
+};
+
+// The vertices [0, nv) from v0 in blocks of 128 * kAabbHeld, a lane's two at a
+// time; NaN past the end (min, max and the sphere skip NaN).
+struct HeldVertices {
+  Two x[kAabbHeld], y[kAabbHeld], z[kAabbHeld];
+
+  __device__ __forceinline__ void load(const double* __restrict__ px,
+                                       const double* __restrict__ py,
+                                       const double* __restrict__ pz, int v0, int b, int nv,
+                                       int lane) {
 #pragma unroll
     for (int k = 0; k < kAabbHeld; ++k) {
-      const int v = b + 64 * k + lane;
-      const bool in = v < nv;
-      hx[k] = in ? x[v0 + v] : NAN;
-      hy[k] = in ? y[v0 + v] : NAN;
-      hz[k] = in ? z[v0 + v] : NAN;
-    }
-  };
-  if (!chunked) {
-    for (int b = 0; b < nv; b += 64 * kAabbHeld) {
-      load_block(b);
-#pragma unroll
-      for (int k = 0; k < kAabbHeld; ++k) {
-        plo[0] = fmin(plo[0], hx[k]);
-        plo[1] = fmin(plo[1], hy[k]);
-        plo[2] = fmin(plo[2], hz[k]);
-        phi[0] = fmax(phi[0], hx[k]);
-        phi[1] = fmax(phi[1], hy[k]);
-        phi[2] = fmax(phi[2], hz[k]);
-      }
-    }
-    for (int o = 32; o > 0; o >>= 1)
-      for (int q = 0; q < 3; ++q) {
-        plo[q] = fmin(plo[q], __shfl_xor(plo[q], o));
-        phi[q] = fmax(phi[q], __shfl_xor(phi[q], o));
-      }
-  } else {
-    // kChunkGroup chunks at a time, their loads issued together
-    constexpr int kChunkGroup = 4;
-    for (int g0 = t0; g0 < t1; g0 += 64 * kChunkGroup) {
-      double lo[kChunkGroup][3], hi[kChunkGroup][3];
-#pragma unroll
-      for (int c = 0; c < kChunkGroup; ++c) {
-        const int b0 = g0 + 64 * c, b1 = b0 + 64 < t1 ? b0 + 64 : t1;
-        double cx[3], cy[3], cz[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const int v = 3 * b0 + 64 * k + lane;
-          const bool in = v < 3 * b1;
-          cx[k] = in ? x[v] : NAN;
-          cy[k] = in ? y[v] : NAN;
-          cz[k] = in ? z[v] : NAN;
-        }
-        // from +-inf, as the box of no (or only NaN) coordinates
-        lo[c][0] = fmin(fmin(fmin(INFINITY, cx[0]), cx[1]), cx[2]);
-        lo[c][1] = fmin(fmin(fmin(INFINITY, cy[0]), cy[1]), cy[2]);
-        lo[c][2] = fmin(fmin(fmin(INFINITY, cz[0]), cz[1]), cz[2]);
-        hi[c][0] = fmax(fmax(fmax(-INFINITY, cx[0]), cx[1]), cx[2]);
-        hi[c][1] = fmax(fmax(fmax(-INFINITY, cy[0]), cy[1]), cy[2]);
-        hi[c][2] = fmax(fmax(fmax(-INFINITY, cz[0]), cz[1]), cz[2]);
-      }
-      for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int c = 0; c < kChunkGroup; ++c)
-          for (int q = 0; q < 3; ++q) {
-            lo[c][q] = fmin(lo[c][q], __shfl_xor(lo[c][q], o));
-            hi[c][q] = fmax(hi[c][q], __shfl_xor(hi[c][q], o));
-          }
-#pragma unroll
-      for (int c = 0; c < kChunkGroup; ++c) {
-        const int b0 = g0 + 64 * c;
-        if (b0 >= t1) break;
-        if (lane == 0) {
-          Aabb bx;
-          for (int q = 0; q < 3; ++q) {
-            bx.lo[q] = lo[c][q];
-            bx.hi[q] = hi[c][q];
-          }
-          cbox[t0 / 64 + i + (b0 - t0) / 64] = bx;
-        }
-        for (int q = 0; q < 3; ++q) {
-          plo[q] = fmin(plo[q], lo[c][q]);
-          phi[q] = fmax(phi[q], hi[c][q]);
-        }
+      const int v = b + 128 * k + 2 * lane;
+      x[k] = y[k] = z[k] = Two{NAN, NAN};
+      if (v + 1 < nv) {
+        x[k] = *reinterpret_cast<const Two*>(px + v0 + v);
+        y[k] = *reinterpret_cast<const Two*>(py + v0 + v);
+        z[k] = *reinterpret_cast<const Two*>(pz + v0 + v);
+      } else if (v < nv) {
+        x[k].a = px[v0 + v];
+        y[k].a = py[v0 + v];
+        z[k].a = pz[v0 + v];
       }
     }
   }
-  if (lane == 0) {
-    const double m = eps[i] + 0.5e-9;
-    Aabb bx;
-    for (int q = 0; q < 3; ++q) {
-      bx.lo[q] = plo[q] - m;
-      bx.hi[q] = phi[q] + m;
-    }
-    box[i] = bx;
-  }
-  if (sph) {
-    // a bounding sphere: the vertex box's centre and the largest vertex
-    // distance from it (NaN coordinates drop out, as from the box); the
-    // replicas come from registers when one block held them all
-    const double c[3] = {0.5 * (plo[0] + phi[0]), 0.5 * (plo[1] + phi[1]),
-                         0.5 * (plo[2] + phi[2])};
+  __device__ __forceinline__ double far2(const double c[3]) const {
     double r2 = 0.0;
-    const bool held = !chunked && nv <= 64 * kAabbHeld;
-    for (int b = 0; b < nv; b += 64 * kAabbHeld) {
-      if (!held) load_block(b);
 #pragma unroll
-      for (int k = 0; k < kAabbHeld; ++k) {
-        const double dx = hx[k] - c[0], dy = hy[k] - c[1], dz = hz[k] - c[2];
-        r2 = fmax(r2, dx * dx + dy * dy + dz * dz);
+    for (int k = 0; k < kAabbHeld; ++k) {
+      double dx = x[k].a - c[0], dy = y[k].a - c[1], dz = z[k].a - c[2];
+      r2 = fmax(r2, dx * dx + dy * dy + dz * dz);
+      dx = x[k].b - c[0], dy = y[k].b - c[1], dz = z[k].b - c[2];
+      r2 = fmax(r2, dx * dx + dy * dy + dz * dz);
+    }
+    return r2;
+  }
+};
+
+// v of the lane that `ctrl` (a DPP control) names, which is in the same row of 16.
+template <int ctrl>
+__device__ __forceinline__ double row_move(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// The smallest over each row of 16 lanes, in all of them, without LDS: lanes
+// xor 1, xor 2, then the row's halves and the row mirrored.
+__device__ __forceinline__ double row_min(double v) {
+  v = fmin(v, row_move<0xb1>(v));
+  v = fmin(v, row_move<0x4e>(v));
+  v = fmin(v, row_move<0x141>(v));
+  return fmin(v, row_move<0x140>(v));
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+__device__ __forceinline__ double wave_min(double v) {
+  v = row_min(v);
+  return fmin(fmin(lane_value(v, 0), lane_value(v, 16)),
+              fmin(lane_value(v, 32), lane_value(v, 48)));
+}
+
+// The box of the wave's lanes' boxes, in all lanes.  A first exchange leaves
+// lo in the lower and -hi in the upper 32 lanes, so that one reduction does
+// for both.
+__device__ __forceinline__ void wave_box(double lo[3], double hi[3]) {
+  const bool upper = __lane_id() >= 32;
+  for (int q = 0; q < 3; ++q) {
+    const double up = -hi[q];
+    const double other = __shfl_xor(upper ? lo[q] : up, 32);
+    const double v = row_min(fmin(upper ? up : lo[q], other));
+    lo[q] = fmin(lane_value(v, 0), lane_value(v, 16));
+    hi[q] = -fmin(lane_value(v, 32), lane_value(v, 48));
+  }
+}
+
+__device__ __forceinline__ void store_box(Aabb* __restrict__ box, const double* __restrict__ eps,
+                                          int i, const double lo[3], const double hi[3]) {
+  const double m = eps[i] + 0.5e-9;
+  Aabb bx;
+  for (int q = 0; q < 3; ++q) {
+    bx.lo[q] = lo[q] - m;
+    bx.hi[q] = hi[q] + m;
+  }
+  box[i] = bx;
+}
+
+__device__ __forceinline__ void store_sphere(double* __restrict__ sph, int i, const double c[3],
+                                             double r2) {
+  sph[4 * i] = c[0];
+  sph[4 * i + 1] = c[1];
+  sph[4 * i + 2] = c[2];
+  sph[4 * i + 3] = sqrt(r2);
+}
+
+// A particle's box (inflated by its margin), its chunks' boxes when it has
+// more triangles than one row block (chunk c of 64 triangles at
+// cbox[t0 / 64 + i + c], an index that grows with i and c, so no two chunks
+// share it) and, with sph, a bounding sphere: the vertex box's centre and the
+// largest vertex distance from it (NaN coordinates drop out, as from the box).
+// A wave per particle, its replicas read once; the workgroup's waves share a
+// particle with chunks (one wave took 51 us for a 2,048-triangle funnel, the
+// longest chain of the scene's pass: 23 us now).  HBM bound: the 1.5 GB of the
+// 2e5-particle box take 287 us (5.2 TB/s; 304 us with reductions through LDS
+// shuffles and 8-byte loads, 348 us where all workgroups wait for the one
+// particle that they share).
+__global__ __launch_bounds__(64 * kAabbWaves) void k_particle_aabb(
+    int n, const double* __restrict__ x, const double* __restrict__ y,
+    const double* __restrict__ z, const int* __restrict__ tri_offset,
+    const double* __restrict__ eps, Aabb* __restrict__ box, Aabb* __restrict__ cbox,
+    double* __restrict__ sph) {
+  __shared__ double red[kAabbWaves][7];
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  {
+    const int i = blockIdx.x * kAabbWaves + w;
+    const int t0 = i < n ? tri_offset[i] : 0, t1 = i < n ? tri_offset[i + 1] : 0;
+    const bool chunked = cbox && t1 - t0 > kRowBlock;
+    const int v0 = 3 * t0, nv = t1 > t0 ? 3 * (t1 - t0) : 0;
+    if (i < n && !chunked) {
+      double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+      HeldVertices h;
+      for (int b = 0; b < nv; b += 128 * kAabbHeld) {
+        h.load(x, y, z, v0, b, nv, lane);
+#pragma unroll
+        for (int k = 0; k < kAabbHeld; ++k) {
+          lo[0] = fmin(fmin(lo[0], h.x[k].a), h.x[k].b);
+          lo[1] = fmin(fmin(lo[1], h.y[k].a), h.y[k].b);
+          lo[2] = fmin(fmin(lo[2], h.z[k].a), h.z[k].b);
+          hi[0] = fmax(fmax(hi[0], h.x[k].a), h.x[k].b);
+          hi[1] = fmax(fmax(hi[1], h.y[k].a), h.y[k].b);
+          hi[2] = fmax(fmax(hi[2], h.z[k].a), h.z[k].b);
+        }
+      }
+      wave_box(lo, hi);
+      if (lane == 0) store_box(box, eps, i, lo, hi);
+      if (sph) {
+        const double c[3] = {0.5 * (lo[0] + hi[0]), 0.5 * (lo[1] + hi[1]), 0.5 * (lo[2] + hi[2])};
+        double r2 = 0.0;
+        // the replicas come from registers when one block held them all
+        for (int b = 0; b < nv; b += 128 * kAabbHeld) {
+          if (nv > 128 * kAabbHeld) h.load(x, y, z, v0, b, nv, lane);
+          r2 = fmax(r2, h.far2(c));
+        }
+        r2 = -wave_min(-r2);
+        if (lane == 0) store_sphere(sph, i, c, r2);
       }
     }
-    for (int o = 32; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o));
-    if (lane == 0) {
-      sph[4 * i] = c[0];
-      sph[4 * i + 1] = c[1];
-      sph[4 * i + 2] = c[2];
-      sph[4 * i + 3] = sqrt(r2);
-    }
   }
+  if (!cbox) return;
+  for (int p = 0; p < kAabbWaves; ++p) {
+    const int i = blockIdx.x * kAabbWaves + p;
+    if (i >= n) break;
+    const int t0 = tri_offset[i], t1 = tri_offset[i + 1];
+    if (t1 - t0 <= kRowBlock) continue;  // the same for the whole workgroup
+    const int v0 = 3 * t0, nv = 3 * (t1 - t0);
+    double plo[3] = {INFINITY, INFINITY, INFINITY}, phi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int c = w; 64 * c < t1 - t0; c += kAabbWaves) {
+      const int b0 = 64 * c, b1 = b0 + 64 < t1 - t0 ? b0 + 64 : t1 - t0;
+      double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int v = 3 * b0 + 64 * k + lane;
+        const bool in = v < 3 * b1;
+        const double cx = in ? x[v0 + v] : NAN, cy = in ? y[v0 + v] : NAN,
+                     cz = in ? z[v0 + v] : NAN;
+        lo[0] = fmin(lo[0], cx);
+        lo[1] = fmin(lo[1], cy);
+        lo[2] = fmin(lo[2], cz);
+        hi[0] = fmax(hi[0], cx);
+        hi[1] = fmax(hi[1], cy);
+        hi[2] = fmax(hi[2], cz);
+      }
+      wave_box(lo, hi);
+      if (lane == 0) {
+        Aabb bx;
+        for (int q = 0; q < 3; ++q) {
+          bx.lo[q] = lo[q];
+          bx.hi[q] = hi[q];
+        }
+        cbox[t0 / 64 + i + c] = bx;
+      }
+      for (int q = 0; q < 3; ++q) {
+        plo[q] = fmin(plo[q], lo[q]);
+        phi[q] = fmax(phi[q], hi[q]);
+      }
+    }
+    if (lane == 0)
+      for (int q = 0; q < 3; ++q) {
+        red[w][q] = plo[q];
+        red[w][3 + q] = phi[q];
+      }
+    __syncthreads();
+    for (int o = 0; o < kAabbWaves; ++o)
+      for (int q = 0; q < 3; ++q) {
+        plo[q] = fmin(plo[q], red[o][q]);
+        phi[q] = fmax(phi[q], red[o][3 + q]);
+      }
+    if (threadIdx.x == 0) store_box(box, eps, i, plo, phi);
+    if (sph) {
+      const double c[3] = {0.5 * (plo[0] + phi[0]), 0.5 * (plo[1] + phi[1]),
+                           0.5 * (plo[2] + phi[2])};
+      double r2 = 0.0;
+      for (int b = 128 * kAabbHeld * w; b < nv; b += 128 * kAabbHeld * kAabbWaves) {
+        HeldVertices h;
+        h.load(x, y, z, v0, b, nv, lane);
+        r2 = fmax(r2, h.far2(c));
+      }
+      r2 = -wave_min(-r2);
+      if (lane == 0) red[w][6] = r2;
+      __syncthreads();
+      for (int o = 0; o < kAabbWaves; ++o) r2 = fmax(r2, red[o][6]);
+      if (threadIdx.x == 0) store_sphere(sph, i, c, r2);
+    }
+    __syncthreads();  // the next particle reuses the reductions
+  }
+}
+
+static void launch_aabb(const dh_geometry* g, Aabb* box, Aabb* cbox, double* sph, hipStream_t st) {
+  hipLaunchKernelGGL(k_particle_aabb, grid_for(g->nparticles, kAabbWaves), 64 * kAabbWaves, 0, st,
+                     g->nparticles, g->x, g->y, g->z, g->tri_offset, g->eps, box, cbox, sph);
 }
 
 __device__ __forceinline__ bool overlap(const Aabb& a, const Aabb& b) {
@@ -180,9 +281,21 @@ __device__ __forceinline__ unsigned hash_cell(long long cx, long long cy, long l
 }
 
 // The grid is a cell list sorted by hash bucket: bucket b holds the
-// particles sorted[cstart[b] .. cstart[b+1]) (a counting sort: counts,
+// particles entry[cstart[b] .. cstart[b+1]) (a counting sort: counts,
 // exclusive scan, scatter), so a bucket is one contiguous range and its
 // members load without pointer chasing.
+//
+// A member is found with its box and cell beside its number, so that a search
+// waits for one load per round (with the number first and the box after it,
+// and 64-bit cells formed again for every candidate, the 2e5-particle box took
+// 198 us; 123 us now).  Cells are compared in their low 32 bits: two that agree there and
+// differ are 2^32 cells apart and their boxes do not overlap.
+struct alignas(64) GridEntry {
+  Aabb box;
+  int cell[3];
+  int id;
+};
+
 struct GridArgs {
   const Aabb* box;
   const int* obstacle;  // may be null
@@ -192,7 +305,7 @@ struct GridArgs {
   int* ccount;               // particles per bucket
   int* cfill;                // scatter cursor per bucket
   const long long* cstart;   // bucket starts (mask + 2 entries)
-  int* sorted;               // particle ids by bucket
+  GridEntry* entry;          // particles by bucket
   unsigned* cellh;           // bucket of each particle (large: unused)
   int* large;                // indices of large particles (any order)
   int* nlarge;
@@ -232,16 +345,17 @@ __global__ __launch_bounds__(256) void k_grid_bin(GridArgs g) {
 __global__ __launch_bounds__(256) void k_grid_scatter(GridArgs g) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= g.n) return;
-  if (is_large(g, i, g.box[i])) return;
+  GridEntry e;
+  e.box = g.box[i];
+  if (is_large(g, i, e.box)) return;
   const unsigned hsh = g.cellh[i];
-  g.sorted[g.cstart[hsh] + atomicAdd(&g.cfill[hsh], 1)] = i;
+  long long c[3];
+  cell_of(e.box, g.inv_h, c);
+  for (int q = 0; q < 3; ++q) e.cell[q] = static_cast<int>(c[q]);
+  e.id = i;
+  g.entry[g.cstart[hsh] + atomicAdd(&g.cfill[hsh], 1)] = e;
 }
 
-// One wave searches the partners j > i of one particle i: the 27 neighbour
-// buckets are walked by 27 lanes at once, one member per lane per round, and
-// the large-particle list is strided over the wave.  A large particle's scan
-// over all j is split into chunks, one wave each.  Finds are compacted with ballots, so every lane sees the
-// running count.
 constexpr int kBpWaves = 4;    // particles per workgroup
 constexpr int kBpList = 512;   // partners sorted in LDS per particle (else a serial sort)
 constexpr int kBpKeep = 64;    // partners kept by the count pass per particle (one per lane)
@@ -251,52 +365,73 @@ __device__ __forceinline__ int bp_lane_prefix(unsigned long long mask) {
                                    __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0));
 }
 
-// Calls put(position, j) on the finding lane for every partner of a
-// particle i that is not large, positions 0.. in discovery order; returns
-// the number of partners (wave-uniform).
-template <typename F>
-__device__ int grid_partners(const GridArgs& g, int i, const Aabb& bi, int lane, F put) {
+// The partners j > i of a particle i that is not large, by L = 32 or 64 lanes
+// of a wave (`active`: they have one): calls put(position, j) on the finding
+// lane for every partner, positions 0.. in discovery order; returns their
+// number.  27 lanes look up the neighbour cells' buckets; the buckets' members
+// then form one list that all L lanes go through.  A member counts for the
+// lane whose cell is its own, so that two cells that share a bucket do not find
+// it twice.  The large particles are strided over the lanes.  Finds are
+// compacted with ballots, so every lane sees the running count.
+template <int L, typename F>
+__device__ __forceinline__ int grid_partners(const GridArgs& g, int i, const Aabb& bi, bool active,
+                                             int lane, F put) {
+  const int sl = lane & (L - 1), first = lane - sl;
+  auto part = [&](unsigned long long m) { return L == 64 ? m : (m >> first) & 0xffffffffull; };
+  const unsigned long long below = (1ull << sl) - 1;
   long long c[3];
   cell_of(bi, g.inv_h, c);
-  const int dx = lane / 9 - 1, dy = (lane / 3) % 3 - 1, dz = lane % 3 - 1;
-  const unsigned hsh = lane < 27 ? hash_cell(c[0] + dx, c[1] + dy, c[2] + dz, g.mask) : 0u;
-  // distinct neighbour cells may share a bucket: its lowest lane walks it
-  bool walk = lane < 27;
-  for (int l = 0; l < 26; ++l) {
-    const unsigned o = __shfl(hsh, l);
-    if (l < lane && o == hsh) walk = false;
+  const bool walk = active && sl < 27;
+  c[0] += sl / 9 - 1;
+  c[1] += (sl / 3) % 3 - 1;
+  c[2] += sl % 3 - 1;
+  const unsigned hsh = hash_cell(c[0], c[1], c[2], g.mask);
+  const int s0 = walk ? static_cast<int>(g.cstart[hsh]) : 0;
+  const int len = walk ? static_cast<int>(g.cstart[hsh + 1]) - s0 : 0;
+  int incl = len;
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) {
+    const int t = __shfl_up(incl, o, 32);
+    if (sl >= o) incl += t;
   }
-  long long pos = walk ? g.cstart[hsh] : 0, end = walk ? g.cstart[hsh + 1] : 0;
+  const int excl = incl - len;  // lanes 27.. hold the total
+  const int total = __shfl(incl, first + 31);
   int found = 0;
-  while (__ballot(pos < end)) {
+  for (int f0 = 0; __ballot(f0 < total); f0 += L) {
+    const int f = f0 + sl;
+    // the bucket of member f: the last of the 27 that starts at or before it
+    int b = 0;
+#pragma unroll
+    for (int h = 16; h > 0; h >>= 1) {
+      const int at = __shfl(excl, first + b + h);
+      if (b + h < 27 && at <= f) b += h;
+    }
+    const int bs = __shfl(s0, first + b), be = __shfl(excl, first + b);
+    const int cx = __shfl(static_cast<int>(c[0]), first + b);
+    const int cy = __shfl(static_cast<int>(c[1]), first + b);
+    const int cz = __shfl(static_cast<int>(c[2]), first + b);
     bool e = false;
     int cand = -1;
-    if (pos < end) {
-      cand = g.sorted[pos];
-      if (cand > i) {
-        const Aabb bj = g.box[cand];
-        long long cj[3];
-        cell_of(bj, g.inv_h, cj);
-        e = cj[0] - c[0] >= -1 && cj[0] - c[0] <= 1 && cj[1] - c[1] >= -1 && cj[1] - c[1] <= 1 &&
-            cj[2] - c[2] >= -1 && cj[2] - c[2] <= 1 && overlap(bi, bj);
-      }
-      ++pos;
+    if (f < total) {
+      const GridEntry m = g.entry[bs + (f - be)];
+      cand = m.id;
+      e = cand > i && m.cell[0] == cx && m.cell[1] == cy && m.cell[2] == cz && overlap(bi, m.box);
     }
-    const unsigned long long mask = __ballot(e);
-    if (e) put(found + bp_lane_prefix(mask), cand);
+    const unsigned long long mask = part(__ballot(e));
+    if (e) put(found + __popcll(mask & below), cand);
     found += __popcll(mask);
   }
   const int nl = *g.nlarge;
-  for (int o0 = 0; o0 < nl; o0 += 64) {
-    const int o = o0 + lane;
+  for (int o0 = 0; o0 < nl; o0 += L) {
+    const int o = o0 + sl;
     bool e = false;
     int cand = -1;
-    if (o < nl) {
+    if (active && o < nl) {
       cand = g.large[o];
       e = cand > i && overlap(bi, g.box[cand]);
     }
-    const unsigned long long mask = __ballot(e);
-    if (e) put(found + bp_lane_prefix(mask), cand);
+    const unsigned long long mask = part(__ballot(e));
+    if (e) put(found + __popcll(mask & below), cand);
     found += __popcll(mask);
   }
   return found;
@@ -384,59 +519,6 @@ __global__ __launch_bounds__(64 * kBpWaves) void k_large_fill(GridArgs g,
   }
 }
 
-// grid_partners for two particles per wave: half h = lane / 32 searches
-// particle i (each half's i, bi and `found` are its own); the same partner
-// set as grid_partners, in another discovery order.
-template <typename F>
-__device__ int grid_partners_half(const GridArgs& g, int i, const Aabb& bi, bool active, int lane,
-                                  F put) {
-  const int h = lane >> 5, sl = lane & 31;
-  long long c[3];
-  cell_of(bi, g.inv_h, c);
-  const int dx = sl / 9 - 1, dy = (sl / 3) % 3 - 1, dz = sl % 3 - 1;
-  const unsigned hsh = (active && sl < 27) ? hash_cell(c[0] + dx, c[1] + dy, c[2] + dz, g.mask) : 0u;
-  bool walk = active && sl < 27;
-  for (int l = 0; l < 26; ++l) {
-    const unsigned o = __shfl(hsh, (h << 5) + l);
-    if (l < sl && o == hsh) walk = false;
-  }
-  long long pos = walk ? g.cstart[hsh] : 0, end = walk ? g.cstart[hsh + 1] : 0;
-  const unsigned below = (1u << sl) - 1u;
-  int found = 0;
-  while (__ballot(pos < end)) {
-    bool e = false;
-    int cand = -1;
-    if (pos < end) {
-      cand = g.sorted[pos];
-      if (cand > i) {
-        const Aabb bj = g.box[cand];
-        long long cj[3];
-        cell_of(bj, g.inv_h, cj);
-        e = cj[0] - c[0] >= -1 && cj[0] - c[0] <= 1 && cj[1] - c[1] >= -1 && cj[1] - c[1] <= 1 &&
-            cj[2] - c[2] >= -1 && cj[2] - c[2] <= 1 && overlap(bi, bj);
-      }
-      ++pos;
-    }
-    const unsigned hm = static_cast<unsigned>(__ballot(e) >> (32 * h));
-    if (e) put(found + __popc(hm & below), cand);
-    found += __popc(hm);
-  }
-  const int nl = *g.nlarge;
-  for (int o0 = 0; o0 < nl; o0 += 32) {
-    const int o = o0 + sl;
-    bool e = false;
-    int cand = -1;
-    if (active && o < nl) {
-      cand = g.large[o];
-      e = cand > i && overlap(bi, g.box[cand]);
-    }
-    const unsigned hm = static_cast<unsigned>(__ballot(e) >> (32 * h));
-    if (e) put(found + __popc(hm & below), cand);
-    found += __popc(hm);
-  }
-  return found;
-}
-
 // Partner counts, two particles per wave (the walk is latency bound: two
 // searches share each round of dependent loads).
 __global__ __launch_bounds__(64 * kBpWaves) void k_grid_count2(GridArgs g,
@@ -450,24 +532,9 @@ __global__ __launch_bounds__(64 * kBpWaves) void k_grid_count2(GridArgs g,
   auto keep = [&](int pos, int j) {
     if (pos < kBpKeep) kept[pos] = j;
   };
-  const int m = grid_partners_half(g, i, bi, active, lane, keep);
+  const int m = grid_partners<32>(g, i, bi, active, lane, keep);
   // large particles: k_large_count / k_large_sum, launched after this
   if (valid && (lane & 31) == 0) count[i] = active ? m : 0;
-}
-
-__global__ __launch_bounds__(64 * kBpWaves) void k_grid_count(GridArgs g,
-                                                               int* __restrict__ count) {
-  const int lane = threadIdx.x & 63;
-  const int i = blockIdx.x * kBpWaves + (threadIdx.x >> 6);
-  if (i >= g.n) return;  // wave-uniform
-  const Aabb bi = g.box[i];
-  int* kept = g.keep + static_cast<long long>(i) * kBpKeep;
-  auto keep = [&](int pos, int j) {
-    if (pos < kBpKeep) kept[pos] = j;
-  };
-  // large particles: k_large_count / k_large_sum, launched after this
-  const int m = is_large(g, i, bi) ? 0 : grid_partners(g, i, bi, lane, keep);
-  if (lane == 0) count[i] = m;
 }
 
 // Writes the partners of i at start[i].. in ascending order (pairs beyond
@@ -505,7 +572,7 @@ __global__ __launch_bounds__(64 * kBpWaves) void k_grid_fill(GridArgs g,
   }
   if (m > kBpList) {
     // more partners than the LDS list holds: unsorted, then a serial sort
-    grid_partners(g, i, bi, lane, direct);
+    grid_partners<64>(g, i, bi, true, lane, direct);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
     if (lane == 0) {
       const long long e = s + m < cap ? s + m : cap;
@@ -522,7 +589,7 @@ __global__ __launch_bounds__(64 * kBpWaves) void k_grid_fill(GridArgs g,
     return;
   }
   int* lst = list[w];
-  const int found = grid_partners(g, i, bi, lane, [&](int pos, int j) {
+  const int found = grid_partners<64>(g, i, bi, true, lane, [&](int pos, int j) {
     if (pos < kBpList) lst[pos] = j;
   });
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -537,23 +604,25 @@ __global__ __launch_bounds__(64 * kBpWaves) void k_grid_fill(GridArgs g,
   }
 }
 
-// Scenes of at most kSmallScene particles: every pair (i < j) tested in one
-// workgroup of 16 waves, in place of the grid's dozen launches.  The same
+// Scenes of at most kSmallScene particles: every pair (i < j) tested, in place
+// of the grid's dozen launches.  Up to kOneGroupScene of them by this one
+// workgroup of 16 waves (65 particles: 8 us; 1,001 particles took it 400 us).  The same
 // candidate set (boxes overlap, not both obstacles) in the same order (i
 // ascending, then j ascending), with the same outputs: start[0..n] (start[n]
 // the total, which may exceed cap) and the pairs that fit cap.  A wave per
 // particle i sweeps j > i in strips of 64: counts, their prefix sums, then
 // the same sweep writes each partner at start[i] + its rank.
 constexpr int kSmallScene = 1024;
+constexpr int kOneGroupScene = 128;
 
 __global__ __launch_bounds__(1024) void k_small_pairs(const Aabb* __restrict__ box,
                                                       const int* __restrict__ obstacle, int n,
                                                       long long* __restrict__ start,
                                                       long long cap, int* __restrict__ pairs) {
   // the boxes and obstacle flags staged once: both sweeps read LDS only
-  __shared__ Aabb s_box[kSmallScene];
-  __shared__ unsigned char s_obst[kSmallScene];
-  __shared__ long long s_start[kSmallScene + 1];
+  __shared__ Aabb s_box[kOneGroupScene];
+  __shared__ unsigned char s_obst[kOneGroupScene];
+  __shared__ long long s_start[kOneGroupScene + 1];
   __shared__ long long s_wave[16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int t = threadIdx.x;
@@ -614,6 +683,38 @@ __global__ __launch_bounds__(1024) void k_small_pairs(const Aabb* __restrict__ b
   }
 }
 
+// The same set for more particles (to kSmallScene): a wave per particle i
+// sweeps j > i, once for the counts and, after their scan, once more for the
+// pairs: start[0..n] and the pairs that fit cap.  1,001 particles: 11 + 5 +
+// 11 us, 129: 14 us in all (15.5 us by the one workgroup, 8 us at 65: the line
+// lies where the two more launches are paid back).
+template <bool kFill>
+__global__ __launch_bounds__(256) void k_all_pairs(const Aabb* __restrict__ box,
+                                                   const int* __restrict__ obstacle, int n,
+                                                   int* __restrict__ count,
+                                                   const long long* __restrict__ start,
+                                                   long long cap, int* __restrict__ pairs) {
+  const int lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
+  if (i >= n) return;  // wave-uniform
+  const Aabb bi = box[i];
+  const bool oi = obstacle && obstacle[i];
+  const long long s0 = kFill ? start[i] : 0;
+  int found = 0;
+  for (int j0 = i + 1; j0 < n; j0 += 64) {
+    const int j = j0 + lane;
+    const bool e = j < n && !(oi && obstacle[j]) && overlap(bi, box[j]);
+    const unsigned long long mask = __ballot(e);
+    const long long q = s0 + found + bp_lane_prefix(mask);
+    if (kFill && e && q < cap) {
+      pairs[2 * q] = i;
+      pairs[2 * q + 1] = j;
+    }
+    found += __popcll(mask);
+  }
+  if (!kFill && lane == 0) count[i] = found;
+}
+
 int scan_counts(const int* counts, int n, long long* offs, hipStream_t st);
 int scan_counts_with(const int* counts, int n, long long* offs, long long* sums,
                      hipStream_t st);
@@ -621,7 +722,7 @@ int scan_sums_len(int n);
 int scan_reserve(int n);
 
 struct BpScratch {
-  DevBuf box, ccount, cfill, cstart, sorted, cellh, count, start, err, obst, lcount, keep, cbox,
+  DevBuf box, ccount, cfill, cstart, entry, cellh, count, start, err, obst, lcount, keep, cbox,
       sph;
 };
 static BpScratch g_bp;
@@ -659,7 +760,7 @@ struct BpBuffers {
   int* ccount;         // tbl + 1
   int* cfill;          // tbl
   long long* cstart;   // tbl + 1
-  int* sorted;         // n + 1
+  GridEntry* entry;    // n + 1
   unsigned* cellh;     // n + 1
   int* count;          // n + 1
   long long* start;    // n + 1
@@ -673,7 +774,7 @@ struct BpBuffers {
 
 static BpBuffers library_buffers() {
   return BpBuffers{g_bp.box.as<Aabb>(),     g_bp.cbox.as<Aabb>(),    g_bp.ccount.as<int>(),
-                   g_bp.cfill.as<int>(),    g_bp.cstart.as<long long>(), g_bp.sorted.as<int>(),
+                   g_bp.cfill.as<int>(),    g_bp.cstart.as<long long>(), g_bp.entry.as<GridEntry>(),
                    g_bp.cellh.as<unsigned>(), g_bp.count.as<int>(),  g_bp.start.as<long long>(),
                    g_bp.err.as<int>(),      g_bp.obst.as<int>(),     g_bp.lcount.as<int>(),
                    g_bp.keep.as<int>(),     nullptr,                 g_bp.sph.as<double>()};
@@ -701,9 +802,7 @@ int particle_boxes(const dh_geometry* geom, const double** out, hipStream_t st) 
   if ((rc = g_bp.cbox.grow(sizeof(Aabb) * ((geom->ntri_total + 63) / 64 + n + 1)))) return rc;
   if ((rc = g_bp.sph.grow(sizeof(double) * 4 * (n + 1)))) return rc;
   if (n > 0)
-    hipLaunchKernelGGL(k_particle_aabb, n, 64, 0, st, geom->x, geom->y, geom->z,
-                       geom->tri_offset, geom->eps, g_bp.box.as<Aabb>(), g_bp.cbox.as<Aabb>(),
-                       g_bp.sph.as<double>());
+    launch_aabb(geom, g_bp.box.as<Aabb>(), g_bp.cbox.as<Aabb>(), g_bp.sph.as<double>(), st);
   DH_HIP_CHECK(hipGetLastError());
   *out = g_bp.box.as<double>();
   return DH_OK;
@@ -719,7 +818,7 @@ int broadphase_reserve(int n, int ntri) {
   if ((rc = g_bp.ccount.grow(sizeof(int) * (tbl + 1)))) return rc;
   if ((rc = g_bp.cfill.grow(sizeof(int) * tbl))) return rc;
   if ((rc = g_bp.cstart.grow(sizeof(long long) * (tbl + 1)))) return rc;
-  if ((rc = g_bp.sorted.grow(sizeof(int) * (n + 1)))) return rc;
+  if ((rc = g_bp.entry.grow(sizeof(GridEntry) * (n + 1)))) return rc;
   if ((rc = g_bp.cellh.grow(sizeof(unsigned) * (n + 1)))) return rc;
   if ((rc = g_bp.count.grow(sizeof(int) * (n + 1)))) return rc;
   if ((rc = g_bp.start.grow(sizeof(long long) * (n + 1)))) return rc;
@@ -747,8 +846,7 @@ static int grid_build(const dh_geometry* geom, const int* obstacle_dev, double c
                       const BpBuffers& b, GridArgs& g, hipStream_t st) {
   const int n = geom->nparticles;
   const unsigned tbl = table_size(n);
-  hipLaunchKernelGGL(k_particle_aabb, n, 64, 0, st, geom->x, geom->y, geom->z,
-                     geom->tri_offset, geom->eps, b.box, b.cbox, b.sph);
+  launch_aabb(geom, b.box, b.cbox, b.sph, st);
   g.box = b.box;
   g.obstacle = obstacle_dev;
   g.n = n;
@@ -758,7 +856,7 @@ static int grid_build(const dh_geometry* geom, const int* obstacle_dev, double c
   g.ccount = b.ccount;
   g.cfill = b.cfill;
   g.cstart = b.cstart;
-  g.sorted = b.sorted;
+  g.entry = b.entry;
   g.cellh = b.cellh;
   g.large = b.large;
   g.nlarge = b.nlarge;
@@ -786,6 +884,27 @@ static void grid_fill(const GridArgs& g, const BpBuffers& b, long long cap, int*
                      64 * kBpWaves, 0, st, g, b.start, cap, pairs);
 }
 
+// The broad phase of at most kSmallScene particles: nothing is written past
+// cap, so the pairs come with the count.
+static int small_pairs(const dh_geometry* geom, const int* obstacle_dev, const BpBuffers& b,
+                       int* pairs, long long cap, hipStream_t st) {
+  const int n = geom->nparticles;
+  if (n > 0) launch_aabb(geom, b.box, b.cbox, b.sph, st);
+  if (n <= kOneGroupScene) {
+    hipLaunchKernelGGL(k_small_pairs, 1, 1024, 0, st, b.box, obstacle_dev, n, b.start, cap, pairs);
+  } else {
+    const unsigned grid = grid_for(n, 4);
+    hipLaunchKernelGGL(k_all_pairs<false>, grid, 256, 0, st, b.box, obstacle_dev, n, b.count,
+                       b.start, cap, pairs);
+    int rc;
+    if ((rc = scan_into(b, b.count, n, b.start, st))) return rc;
+    hipLaunchKernelGGL(k_all_pairs<true>, grid, 256, 0, st, b.box, obstacle_dev, n, b.count,
+                       b.start, cap, pairs);
+  }
+  DH_HIP_CHECK(hipGetLastError());
+  return DH_OK;
+}
+
 // The eager broad phase on the buffers b: the total is read back (through the
 // library's pinned mailbox, or by a copy where nothing may be allocated), and
 // the pairs are written only if it fits cap.
@@ -801,17 +920,9 @@ static int broadphase_run(const dh_geometry* geom, const int* obstacle_dev, doub
   };
   const int n = geom->nparticles;
   if (n <= kSmallScene) {
-    // one workgroup tests every pair; nothing is written past cap, so the
-    // pairs come with the count
-    if (n > 0) {
-      hipLaunchKernelGGL(k_particle_aabb, n, 64, 0, st, geom->x, geom->y, geom->z,
-                         geom->tri_offset, geom->eps, b.box, b.cbox, b.sph);
-      hipLaunchKernelGGL(k_small_pairs, 1, 1024, 0, st, b.box, obstacle_dev, n, b.start, cap,
-                         pairs);
-      DH_HIP_CHECK(hipGetLastError());
-    }
-    long long total = 0;
     int rc;
+    if (n > 0 && (rc = small_pairs(geom, obstacle_dev, b, pairs, cap, st))) return rc;
+    long long total = 0;
     if (n > 0 && (rc = read_total(&total))) return rc;
     *npairs = total;
     return total > cap ? DH_ERR_CAPACITY : DH_OK;
@@ -846,15 +957,7 @@ int broadphase_graph(const dh_geometry* geom, const int* obstacle_dev, double ce
   if ((rc = broadphase_reserve(n, geom->ntri_total))) return rc;
   const BpBuffers b = library_buffers();
   *np_dev = b.start + n;
-  if (n <= kSmallScene) {
-    if (n > 0)
-      hipLaunchKernelGGL(k_particle_aabb, n, 64, 0, st, geom->x, geom->y, geom->z,
-                         geom->tri_offset, geom->eps, b.box, b.cbox, b.sph);
-    hipLaunchKernelGGL(k_small_pairs, 1, 1024, 0, st, b.box, obstacle_dev, n, b.start, cap,
-                       pairs);
-    DH_HIP_CHECK(hipGetLastError());
-    return DH_OK;
-  }
+  if (n <= kSmallScene) return small_pairs(geom, obstacle_dev, b, pairs, cap, st);
   grid_clear(b, table_size(n), st);
   GridArgs g;
   if ((rc = grid_build(geom, obstacle_dev, cell, b, g, st))) return rc;
@@ -886,11 +989,15 @@ static size_t noalloc_layout(char* base, int n, int ntri, BpBuffers* b) {
   };
   BpBuffers t;
   t.box = reinterpret_cast<Aabb*>(take(sizeof(Aabb) * np1));
-  t.cbox = reinterpret_cast<Aabb*>(take(sizeof(Aabb) * ((ntri + 63) / 64 + np1)));
+  // the chunk boxes, which only the detection reads, are not kept here: their
+  // place holds the grid's entries
+  t.cbox = nullptr;
+  const size_t chunks = sizeof(Aabb) * ((ntri + 63) / 64 + np1), entries = sizeof(GridEntry) * np1;
+  t.entry = reinterpret_cast<GridEntry*>(take(chunks > entries ? chunks : entries));
   t.ccount = reinterpret_cast<int*>(take(sizeof(int) * (tbl + 1)));
   t.cfill = reinterpret_cast<int*>(take(sizeof(int) * tbl));
   t.cstart = reinterpret_cast<long long*>(take(sizeof(long long) * (tbl + 1)));
-  t.sorted = reinterpret_cast<int*>(take(sizeof(int) * np1));
+  take(sizeof(int) * np1);  // unused: the array's published size is kept
   t.cellh = reinterpret_cast<unsigned*>(take(sizeof(unsigned) * np1));
   t.count = reinterpret_cast<int*>(take(sizeof(int) * np1));
   t.start = reinterpret_cast<long long*>(take(sizeof(long long) * np1));

@@ -82,6 +82,37 @@ def test_broadphase_equals_all_pairs(scene):
     assert got2 == got
 
 
+@pytest.mark.parametrize("n", [2, 64, 127, 128, 129, 255, 1023, 1024, 1025, 1301])
+def test_broadphase_across_scene_sizes(n):
+    """Sizes on both sides of the one-workgroup, all-pairs and grid searches;
+    particles of one vertex block, several, and with chunk boxes (321 and 700
+    triangles), obstacles among them; every third grid box is crowded."""
+    rng = np.random.default_rng(n)
+    sizes = [1, 20, 42, 43, 85, 86, 170, 171, 320, 321, 700, 3]
+    tris = np.array([sizes[(7 * i + i // 12) % 12] for i in range(n)])
+    off = np.concatenate([[0], np.cumsum(tris)]).astype(np.int32)
+    centre = rng.uniform(-1.0, 1.0, (n, 3))
+    centre[::3] *= 0.3
+    r = 0.6 / max(n, 8) ** (1.0 / 3.0)
+    v = np.repeat(centre, 3 * tris, axis=0) + rng.uniform(-r, r, (3 * off[-1], 3))
+    eps = rng.uniform(0.0, 1e-2, n)
+    hs = type("Scene", (), {})()
+    hs.n, hs.tri_offset, hs.eps = n, off, eps
+    hs.x, hs.y, hs.z = (np.ascontiguousarray(v[:, q]) for q in range(3))
+    hs.obstacle = (rng.random(n) < 0.1).astype(np.int32)
+    ds = type("Device", (), {})()
+    ds.buf = {k: DeviceArray.from_host(np.ascontiguousarray(getattr(hs, k)))
+              for k in ("x", "y", "z", "tri_offset", "eps", "obstacle")}
+    ds.scene = type("Scene", (), {})()
+    ds.scene.geom = _lib.DhGeometry(ds.buf["x"].ptr, ds.buf["y"].ptr, ds.buf["z"].ptr,
+                                    ds.buf["tri_offset"].ptr, ds.buf["eps"].ptr, None, None,
+                                    n, int(off[-1]))
+    want = host_candidates(hs)
+    for cell in (2.0 * r + 0.03, r):  # all particles in the grid; the big ones outside it
+        got, _ = gpu_pairs(ds, hs, cell)
+        assert got == want, (len(got), len(want))
+
+
 def test_forces_and_update_match_oracle():
     hs = spinning_scene()
     ds = engine.DeviceScene(hs)
