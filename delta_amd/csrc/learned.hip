@@ -182,17 +182,58 @@ struct TrainArgs {
   float* loss;      // [1], accumulated
 };
 
-constexpr int kTrainPairs = 64;  // pairs per wave iteration (4 MFMA tiles)
+// A workgroup of kTrainWaves waves takes chunks of 16 pairs per wave: each
+// wave runs its pairs forward and backward, then the waves share the tiles of
+// the chunk's weight gradients, whose sums stay in registers until the end.
+// What bounds a small batch is one chunk's chain and the sums over workgroups,
+// float atomics that the eight XCDs resolve in memory: so few workgroups, of
+// many waves, which start on different tiles.  8,192 pairs: ... us (46 us by
+// 128 one-wave workgroups that summed through LDS atomics).
+constexpr int kTrainWaves = 8;
+constexpr int kTrainPairs = 16 * kTrainWaves;
+constexpr int kTrainGroups = 256;  // workgroups of a large batch: one per CU
 
-__global__ __launch_bounds__(64) void k_mlp_train(TrainArgs a) {
-  __shared__ uint16_t x_s[kTrainPairs][kIn];
-  __shared__ uint16_t a1_s[kHid][kTrainPairs];
-  __shared__ uint16_t a2_s[kHid][kTrainPairs];
-  __shared__ uint16_t d1_s[kHid][kTrainPairs];
-  __shared__ uint16_t d2_s[kHid][kTrainPairs];
-  __shared__ uint16_t d3_s[kOut][kTrainPairs];
-  __shared__ float g_s[kNumParams];
-  const int lane = threadIdx.x;
+// Rows of the chunk's LDS array, [unit][pair]: inputs, activations, dL/dz.
+// The padding keeps the 16 rows that a wave reads together apart in the banks.
+constexpr int kRowX = 0, kRowA1 = kRowX + kIn, kRowA2 = kRowA1 + kHid, kRowD1 = kRowA2 + kHid,
+              kRowD2 = kRowD1 + kHid, kRowD3 = kRowD2 + kHid, kTrainRows = kRowD3 + kOut;
+constexpr int kTrainRow = kTrainPairs + 8;
+
+// The 16 x 16 tiles of the gradients: per layer its weights, then its biases
+// (an input of ones).
+struct GradTile {
+  int act, dz;   // first rows of the operands
+  int out, row;  // gradient of (0, 0) and the distance between two inputs'
+  bool bias;
+};
+
+constexpr int kGradTiles1 = (kIn / 16 + 1) * (kHid / 16),
+              kGradTiles2 = (kHid / 16 + 1) * (kHid / 16),
+              kGradTiles3 = (kHid / 16 + 1) * (kOut / 16),
+              kGradTiles = kGradTiles1 + kGradTiles2 + kGradTiles3;
+constexpr int kTilesPerWave = (kGradTiles + kTrainWaves - 1) / kTrainWaves;
+
+__device__ __forceinline__ GradTile grad_tile(int t) {
+  int act = kRowX, dz = kRowD1, k = kIn, n = kHid, w = kW1, b = kB1;
+  if (t >= kGradTiles1) {
+    t -= kGradTiles1;
+    act = kRowA1, dz = kRowD2, k = kHid, w = kW2, b = kB2;
+    if (t >= kGradTiles2) {
+      t -= kGradTiles2;
+      act = kRowA2, dz = kRowD3, n = kOut, w = kW3, b = kB3;
+    }
+  }
+  const int tk = t / (n / 16), tn = t % (n / 16);
+  const bool bias = 16 * tk == k;
+  return {act + (bias ? 0 : 16 * tk), dz + 16 * tn, bias ? b + 16 * tn : w + 16 * tk * n + 16 * tn,
+          n, bias};
+}
+
+__global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train(TrainArgs a) {
+  __shared__ __align__(16) uint16_t rows[kTrainRows][kTrainRow];
+  __shared__ float loss_s[kTrainWaves];
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int g = lane >> 4, c = lane & 15;
   const float* W = a.W;
   FwdWeights fw;
@@ -206,26 +247,27 @@ __global__ __launch_bounds__(64) void k_mlp_train(TrainArgs a) {
   for (int tk = 0; tk < 4; ++tk)
 #pragma unroll
     for (int tn = 0; tn < 4; ++tn) w2b[tk][tn] = load_w(W + kW2, kHid, tk, tn, lane);
-  for (int i = lane; i < kNumParams; i += 64) g_s[i] = 0.f;
+  v4f sum[kTilesPerWave];
+#pragma unroll
+  for (int q = 0; q < kTilesPerWave; ++q) sum[q] = v4f{0.f, 0.f, 0.f, 0.f};
+  const int first = wave + 5 * static_cast<int>(blockIdx.x % kGradTiles);
   float loss_acc = 0.f;
   const float inv_b = 1.0f / static_cast<float>(a.batch);
-  const int nchunks = (a.batch + kTrainPairs - 1) / kTrainPairs;
-  __syncthreads();
+  const int nchunks = (a.batch - 1) / kTrainPairs + 1;
   for (int ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-    const int base = ch * kTrainPairs;
-    {  // stage the chunk's inputs (one pair per lane)
-      const int p = base + lane;
-      const bool v = p < a.batch;
-      const uint16_t* src = a.X + (a.offset + p) * kIn;
-      for (int k = 0; k < kIn; ++k) x_s[lane][k] = v ? src[k] : 0;
-    }
-    __syncthreads();
-#pragma unroll 1
-    for (int s = 0; s < 4; ++s) {
-      const int pl = s * 16 + c;  // pair within the chunk
-      const int p = base + pl;
+    {
+      const int pl = wave * 16 + c;  // pair within the chunk
+      const int64_t p = static_cast<int64_t>(ch) * kTrainPairs + pl;
       const bool valid = p < a.batch;
-      v4s xb[2] = {x_operand(&x_s[pl][0], 0, lane), x_operand(&x_s[pl][0], 1, lane)};
+      v4s xb[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+      if (valid) {
+        const uint16_t* xrow = a.X + (a.offset + p) * kIn;
+        xb[0] = x_operand(xrow, 0, lane);
+        xb[1] = x_operand(xrow, 1, lane);
+      }
+      for (int tk = 0; tk < 2; ++tk)
+        for (int j = 0; j < 4; ++j)
+          rows[kRowX + 16 * tk + 4 * g + j][pl] = static_cast<uint16_t>(xb[tk][j]);
       v4f z1[4], z2[4], z3[2];
       forward16(fw, W, xb, lane, z1, z2, z3);
       // activations for the weight gradients, [unit][pair]
@@ -233,8 +275,8 @@ __global__ __launch_bounds__(64) void k_mlp_train(TrainArgs a) {
       for (int to = 0; to < 4; ++to)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          a1_s[to * 16 + 4 * g + j][pl] = bf16_bits(relu(z1[to][j]));
-          a2_s[to * 16 + 4 * g + j][pl] = bf16_bits(relu(z2[to][j]));
+          rows[kRowA1 + to * 16 + 4 * g + j][pl] = bf16_bits(relu(z1[to][j]));
+          rows[kRowA2 + to * 16 + 4 * g + j][pl] = bf16_bits(relu(z2[to][j]));
         }
       // loss and dL/dz3 (tile 0: logits 0..14 and the flag 15; tile 1: 16..19)
       const int64_t gp = a.offset + (valid ? p : 0);
@@ -285,7 +327,7 @@ __global__ __launch_bounds__(64) void k_mlp_train(TrainArgs a) {
       for (int tn = 0; tn < 2; ++tn) {
         dz3b[tn] = pack4(dz3[tn][0], dz3[tn][1], dz3[tn][2], dz3[tn][3]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) d3_s[tn * 16 + 4 * g + j][pl] = bf16_bits(dz3[tn][j]);
+        for (int j = 0; j < 4; ++j) rows[kRowD3 + tn * 16 + 4 * g + j][pl] = bf16_bits(dz3[tn][j]);
       }
       v4s dz2b[4];
 #pragma unroll
@@ -297,7 +339,7 @@ __global__ __launch_bounds__(64) void k_mlp_train(TrainArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           d[j] = acc[j] * relu_grad(z2[tu][j]);
-          d2_s[tu * 16 + 4 * g + j][pl] = bf16_bits(d[j]);
+          rows[kRowD2 + tu * 16 + 4 * g + j][pl] = bf16_bits(d[j]);
         }
         dz2b[tu] = pack4(d[0], d[1], d[2], d[3]);
       }
@@ -308,46 +350,45 @@ __global__ __launch_bounds__(64) void k_mlp_train(TrainArgs a) {
         for (int tn = 0; tn < 4; ++tn) acc = mfma16(w2b[tu][tn], dz2b[tn], acc);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          d1_s[tu * 16 + 4 * g + j][pl] = bf16_bits(acc[j] * relu_grad(z1[tu][j]));
+          rows[kRowD1 + tu * 16 + 4 * g + j][pl] = bf16_bits(acc[j] * relu_grad(z1[tu][j]));
       }
     }
     __syncthreads();
     // weight gradients of the chunk: dW[k][n] = sum_p act[k][p] dz[n][p]
-    auto wgrad = [&](const uint16_t* act, int act_stride, bool act_is_x, const uint16_t* dz,
-                     int K, int N, int woff, int boff) {
-      for (int tk = 0; tk < K / 16; ++tk)
-        for (int tn = 0; tn < N / 16; ++tn) {
-          v4f acc = {0.f, 0.f, 0.f, 0.f};
-          for (int ps = 0; ps < 4; ++ps) {
-            const int p0 = ps * 16 + 4 * g;
-            v4s A, Bm;
-            for (int j = 0; j < 4; ++j) {
-              const int k = tk * 16 + c;
-              A[j] = static_cast<short>(act_is_x ? x_s[p0 + j][k] : act[k * act_stride + p0 + j]);
-              Bm[j] = static_cast<short>(dz[(tn * 16 + c) * kTrainPairs + p0 + j]);
-            }
-            acc = mfma16(A, Bm, acc);
-          }
-          for (int j = 0; j < 4; ++j)
-            atomicAdd(&g_s[woff + (tk * 16 + 4 * g + j) * N + tn * 16 + c], acc[j]);
-        }
-      // bias gradient: sum over the chunk's pairs
-      for (int nn = lane; nn < N; nn += 64) {
-        float sacc = 0.f;
-        for (int p = 0; p < kTrainPairs; ++p) sacc += from_bf16(dz[nn * kTrainPairs + p]);
-        atomicAdd(&g_s[boff + nn], sacc);
+#pragma unroll
+    for (int q = 0; q < kTilesPerWave; ++q) {
+      const int slot = (first + kTrainWaves * q) % (kTilesPerWave * kTrainWaves);
+      if (slot >= kGradTiles) continue;
+      const GradTile t = grad_tile(slot);
+#pragma unroll
+      for (int ps = 0; ps < kTrainPairs; ps += 32) {
+        const short one = 0x3f80;
+        const v8s ones = {one, one, one, one, one, one, one, one};
+        const v8s act = t.bias ? ones : *reinterpret_cast<const v8s*>(&rows[t.act + c][ps + 8 * g]);
+        const v8s dz = *reinterpret_cast<const v8s*>(&rows[t.dz + c][ps + 8 * g]);
+        sum[q] = mfma32(act, dz, sum[q]);
       }
-    };
-    wgrad(nullptr, 0, true, &d1_s[0][0], kIn, kHid, kW1, kB1);
-    wgrad(&a1_s[0][0], kTrainPairs, false, &d2_s[0][0], kHid, kHid, kW2, kB2);
-    wgrad(&a2_s[0][0], kTrainPairs, false, &d3_s[0][0], kHid, kOut, kW3, kB3);
+    }
     __syncthreads();
   }
-  __syncthreads();
-  for (int i = lane; i < kNumParams; i += 64)
-    if (g_s[i] != 0.f) atomicAdd(&a.grad[i], g_s[i]);
   for (int o = 32; o > 0; o >>= 1) loss_acc += __shfl_xor(loss_acc, o);
-  if (lane == 0) atomicAdd(a.loss, loss_acc * inv_b);
+  if (lane == 0) loss_s[wave] = loss_acc;
+#pragma unroll
+  for (int q = 0; q < kTilesPerWave; ++q) {
+    const int slot = (first + kTrainWaves * q) % (kTilesPerWave * kTrainWaves);
+    if (slot >= kGradTiles) continue;
+    const GradTile t = grad_tile(slot);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if ((!t.bias || 4 * g + j == 0) && sum[q][j] != 0.f)
+        atomicAdd(&a.grad[t.out + (4 * g + j) * t.row + c], sum[q][j]);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float l = 0.f;
+    for (int w = 0; w < kTrainWaves; ++w) l += loss_s[w];
+    atomicAdd(a.loss, l * inv_b);
+  }
 }
 
 // Adam on the FP32 parameters; padded input rows of W1 and unused outputs
@@ -1021,12 +1062,14 @@ int dh_mlp_grad(const float* params_dev, const uint16_t* X_dev, const uint8_t* f
       !loss_dev)
     return set_error(DH_ERR_ARG, "dh_mlp_grad: bad arguments");
   const hipStream_t st = as_stream(stream);
-  DH_HIP_CHECK(hipMemsetAsync(grad_dev, 0, sizeof(float) * kNumParams, st));
-  DH_HIP_CHECK(hipMemsetAsync(loss_dev, 0, sizeof(float), st));
+  zero_async(ZeroRegions{{reinterpret_cast<unsigned*>(grad_dev),
+                          reinterpret_cast<unsigned*>(loss_dev), nullptr, nullptr},
+                         {kNumParams, 1, 0, 0}},
+             st);
   TrainArgs a{params_dev, X_dev, feat_dev, bary_dev, flag_dev, offset, batch, grad_dev, loss_dev};
-  int grid = (batch + kTrainPairs - 1) / kTrainPairs;
-  if (grid > 1024) grid = 1024;
-  hipLaunchKernelGGL(k_mlp_train, grid, 64, 0, st, a);
+  int grid = (batch - 1) / kTrainPairs + 1;
+  if (grid > kTrainGroups) grid = kTrainGroups;
+  hipLaunchKernelGGL(k_mlp_train, grid, 64 * kTrainWaves, 0, st, a);
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
 }

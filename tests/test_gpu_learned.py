@@ -49,6 +49,24 @@ def test_gradient_matches_numpy(train_set):
         assert seg < 3e-2, (lo, seg)
 
 
+@pytest.mark.parametrize("batch", [1, 15, 16, 17, 127, 128, 129, 1000, 256 * 128 + 77])
+def test_gradient_across_batch_sizes(batch, train_set):
+    """Partial 16-pair tiles and 128-pair chunks, several workgroups, and more
+    chunks than workgroups, from an odd first pair.  bf16 operands (2^-8 each,
+    rounded at other sums) bound the relative difference as above."""
+    _, ds = train_set
+    tr = learn.Trainer(seed=5)
+    first = 61
+    assert ds.n >= first + batch
+    g, loss = tr.grad_at(ds, first, batch)
+    rows = slice(first, first + batch)
+    lref, gref = mlp_ref.loss_and_grad(learn.init_params(5), ds.X.download()[rows],
+                                       ds.feat.download()[rows].astype(np.int64),
+                                       ds.bary.download()[rows], ds.flag.download()[rows])
+    assert loss == pytest.approx(lref, rel=1e-3)
+    assert np.linalg.norm(g - gref) < 1e-2 * np.linalg.norm(gref)
+
+
 def run_learned(batch, method="learned"):
     batch.run(method)
     L = _lib.lib()
