@@ -306,6 +306,38 @@ DH_HD double div_regular(double a, double b) {
 #endif
 }
 
+// div_regular in two parts, for several quotients by one b.
+DH_HD double recip_regular(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(fma(-b, y, 1.0), y, y);
+  return fma(fma(-b, y, 1.0), y, y);
+#else
+  return 1.0 / b;
+#endif
+}
+
+DH_HD double quotient_regular(double a, double b, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+#else
+  (void)y;
+  return a / b;
+#endif
+}
+
+// The smaller of e and a's binary exponent (0 for a = 0).
+DH_HD int least_exponent(int e, double a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int x = __builtin_amdgcn_frexp_exp(a);
+#else
+  int x = 0;
+  std::frexp(a, &x);
+#endif
+  return x < e ? x : e;
+}
+
 // sqrt(x), correctly rounded, for x >= 2^-700 (else `ok` is cleared): by
 // Goldschmidt's iteration and two residual corrections.
 DH_HD double sqrt_regular(double x, bool& ok) {
@@ -784,6 +816,78 @@ struct Penalty {
     dx[0] = (b[0] - (a[4] * dx[1] + h[8] * dx[2] + h[12] * dx[3])) / a[0];
   }
 
+  // Whether step_regular may be tried: edges of some 2^-20 to 2^20 (the sum of
+  // their squares), a first vertex within 2^30.
+  DH_HD bool regular() const {
+    const double trace = h[0] + h[5] + h[10] + h[15];
+    return trace >= 0x1p-40 && trace <= 0x1p40 && fabs(A0.x) <= 0x1p30 && fabs(A0.y) <= 0x1p30 &&
+           fabs(A0.z) <= 0x1p30 && fabs(B0.x) <= 0x1p30 && fabs(B0.y) <= 0x1p30 &&
+           fabs(B0.z) <= 0x1p30;
+  }
+
+  // step() on a regular pair: the same sums, with the penalty terms selected
+  // instead of multiplied by 0, 1 or -1, and one reciprocal per pivot for its
+  // quotients (238 vector instructions a step for 333, the divisions' half of
+  // them; the penalty over 363 pairs of 80 x 80 triangles 153 -> 130 us, with
+  // its vector units busy 9 cycles in 10).  The quotients are correctly rounded, as
+  // division is, where no pivot is below 2^-10 of the trace, every non-zero
+  // numerator is at least 2^-600 (`low` is the least binary exponent seen) and
+  // the new x stays within 2^20, which with regular() keeps everything finite;
+  // else the caller takes the general path.  The fused
+  // doublings round once, as the sums after an exact product do.  (The sign of a zero quotient may
+  // differ from division's; no sum here ends in a zero whose sign shows.)
+  DH_HD bool step_regular(const double x[4], double reg, double dx[4], int& low) const {
+    const bool c0 = x[0] >= 0.0, c1 = x[1] >= 0.0, c3 = x[2] >= 0.0, c4 = x[3] >= 0.0;
+    const double over0 = x[0] + x[1] - 1.0, over1 = x[2] + x[3] - 1.0;
+    const bool c2 = over0 <= 0.0, c5 = over1 <= 0.0;
+    const double r0 = c0 ? 0.0 : r, r1 = c1 ? 0.0 : r, r2 = c2 ? 0.0 : r;
+    const double r3 = c3 ? 0.0 : r, r4 = c4 ? 0.0 : r, r5 = c5 ? 0.0 : r;
+    const double m2 = c2 ? 0.0 : over0, m5 = c5 ? 0.0 : over1;
+    const V3<double> sxy = {
+        (A0.x + (BA.x * x[0]) + (CA.x * x[1])) - (B0.x + (ED.x * x[2]) + (FD.x * x[3])),
+        (A0.y + (BA.y * x[0]) + (CA.y * x[1])) - (B0.y + (ED.y * x[2]) + (FD.y * x[3])),
+        (A0.z + (BA.z * x[0]) + (CA.z * x[1])) - (B0.z + (ED.z * x[2]) + (FD.z * x[3]))};
+    const double least = (h[0] + h[5] + h[10] + h[15]) * 0x1p-10;
+    const double p0 = h[0] + (r0 + r2) + reg;
+    const double y0 = recip_regular(p0);
+    const double a4 = h[4] + r2;
+    const double tmp1 = quotient_regular(a4, p0, y0);
+    const double tmp2 = quotient_regular(h[2], p0, y0);
+    const double tmp3 = quotient_regular(h[3], p0, y0);
+    const double b0 = fma(2.0, dot(sxy, BA), r * ((c0 ? 0.0 : x[0]) + m2));
+    const double b1 = fma(2.0, dot(sxy, CA), r * ((c1 ? 0.0 : x[1]) + m2)) - b0 * tmp1;
+    const double a13 = h[13] - h[12] * tmp1;
+    const double a9 = h[9] - h[8] * tmp1;
+    const double p1 = (h[5] + (r1 + r2) + reg) - a4 * tmp1;
+    const double y1 = recip_regular(p1);
+    const double n4 = h[6] - a4 * tmp2, n5 = h[7] - a4 * tmp3;
+    const double tmp4 = quotient_regular(n4, p1, y1);
+    const double tmp5 = quotient_regular(n5, p1, y1);
+    const double a14 = ((h[14] + r5) - h[12] * tmp2) - a13 * tmp4;
+    const double p2 = ((h[10] + (r3 + r5) + reg) - h[8] * tmp2) - a9 * tmp4;
+    const double y2 = recip_regular(p2);
+    const double b2 =
+        (fma(-2.0, dot(sxy, ED), r * ((c3 ? 0.0 : x[2]) + m5)) - b0 * tmp2) - b1 * tmp4;
+    const double n6 = ((h[11] + r5) - h[8] * tmp3) - a9 * tmp5;
+    const double tmp6 = quotient_regular(n6, p2, y2);
+    const double d3 = ((fma(-2.0, dot(sxy, FD), r * ((c4 ? 0.0 : x[3]) + m5)) - b2 * tmp6) -
+                       b0 * tmp3) - b1 * tmp5;
+    const double p3 =
+        (((h[15] + (r4 + r5) + reg) - h[12] * tmp3) - a13 * tmp5) - a14 * tmp6;
+    dx[3] = quotient_regular(d3, p3, recip_regular(p3));
+    const double d2 = b2 - (a14 * dx[3]);
+    dx[2] = quotient_regular(d2, p2, y2);
+    const double d1 = b1 - (a9 * dx[2] + a13 * dx[3]);
+    dx[1] = quotient_regular(d1, p1, y1);
+    const double d0 = b0 - (a4 * dx[1] + h[8] * dx[2] + h[12] * dx[3]);
+    dx[0] = quotient_regular(d0, p0, y0);
+    low = least_exponent(least_exponent(low, a4), n4);
+    low = least_exponent(least_exponent(low, n5), n6);
+    low = least_exponent(least_exponent(low, d0), d1);
+    low = least_exponent(least_exponent(low, d2), d3);
+    return p0 >= least && p1 >= least && p2 >= least && p3 >= least;
+  }
+
   DH_HD void points(const T x[4], V3<T>& P, V3<T>& Q) const {
     P = {A0.x + (BA.x * x[0]) + (CA.x * x[1]), A0.y + (BA.y * x[0]) + (CA.y * x[1]),
          A0.z + (BA.z * x[0]) + (CA.z * x[1])};
@@ -804,18 +908,36 @@ DH_HD bool penalty_fixed(const Tri<T>& A, const Tri<T>& B, const T x0[4], int it
                          V3<T>& P, V3<T>& Q, T xo[4]) {
   Penalty<T> pen;
   pen.setup(A, B);
-  T x[4] = {x0[0], x0[1], x0[2], x0[3]};
+  T x[4] = {x0[0], x0[1], x0[2], x0[3]}, dx[4];
   T reg = pen.reg0;
-  bool failed = false;
-  for (int i = 0; i < iters; ++i) {
-    T dx[4];
-    pen.step(x, reg, dx);
-    reg = T(1E4) * reg;
+  bool failed = false, done = false;
+  if constexpr (sizeof(T) == 8) {
+    bool ok = pen.regular() && iters > 0;
+    int low = least_exponent(least_exponent(0, pen.h[2]), pen.h[3]);
+#pragma unroll 1
+    for (int i = 0; i < iters; ++i) {
+      if (i > 0)
+        for (int q = 0; q < 4; ++q) x[q] -= dx[q];
+      ok = pen.step_regular(x, reg, dx, low) && ok;
+      reg = T(1E4) * reg;
+      for (int q = 0; q < 4; ++q) ok = fabs(x[q] - dx[q]) <= 0x1p20 && ok;
+    }
+    done = ok && low >= -600;
+  }
+  if (!done) {
+    for (int q = 0; q < 4; ++q) x[q] = x0[q];
+    reg = pen.reg0;
+#pragma unroll 1
+    for (int i = 0; i < iters; ++i) {
+      if (i > 0)
+        for (int q = 0; q < 4; ++q) x[q] -= dx[q];
+      pen.step(x, reg, dx);
+      reg = T(1E4) * reg;
+    }
+  }
+  if (iters > 0) {
     failed = (dot4(dx, dx) / dot4(x, x) > max_err * max_err);
-    x[0] -= dx[0];
-    x[1] -= dx[1];
-    x[2] -= dx[2];
-    x[3] -= dx[3];
+    for (int q = 0; q < 4; ++q) x[q] -= dx[q];
   }
   pen.points(x, P, Q);
   if (xo) {

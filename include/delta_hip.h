@@ -343,7 +343,8 @@ typedef struct dh_tuning {
                                  dh_tri_pairs: 64, 128, 192 or 256           */
   int32_t detect_tile_target; /* particle-pair detection: workgroups per pair
                                  = clamp(ceil(target / npairs), 1, max)      */
-  int32_t detect_max_tiles;   /* that max (1..64)                            */
+  int32_t detect_max_tiles;   /* that max (1..64); dh_detect_pair, which knows
+                                 its particles' sizes, takes up to 64        */
   int32_t detect_wg_per_cu;   /* particle-pair detection: 0 = one workgroup
                                  per (pair, rows) item; else a persistent grid
                                  of this many workgroups per CU (1..64)      */

@@ -59,6 +59,38 @@ def test_pair_driver_matches_oracle(method, case):
     assert st.batch_error == ost.batch_error
 
 
+def soup(n, seed, shift=0.0):
+    """n triangles of 0.3 across in a unit cube: crossing, close and apart."""
+    rng = np.random.default_rng(seed)
+    t = rng.uniform(0.0, 1.0, (n, 1, 3)) + rng.uniform(-0.15, 0.15, (n, 3, 3))
+    t[:, :, 0] += shift
+    return t
+
+
+@pytest.mark.parametrize("method", ["bf", "penalty", "hybrid_batch", "hybrid_triangle",
+                                    "hybrid_batch_stat"])
+@pytest.mark.parametrize("na,nb,eps", [(1, 1, 0.2), (16, 16, 0.1), (17, 15, 0.1),
+                                       (321, 79, 1e-3), (321, 79, 1e-5),
+                                       (1100, 1000, 1e-3), (1100, 1000, 1e-5)])
+def test_tiles_of_one_pair_match_oracle(method, na, nb, eps):
+    """Partial tiles, rows over several workgroups, and (1,100 x 1,000) tiles
+    of more pairs than a hybrid tile notes; at 1e-5 most rows fall back, at
+    the larger margins none."""
+    if na * nb > 1 << 20 and method not in ("hybrid_batch", "hybrid_triangle"):
+        pytest.skip("the notes are the hybrids'")
+    A, B = soup(na, 3), soup(nb, 4, 0.4)
+    fn, code = METHODS[method]
+    contact.reset_all_statistics()
+    got = fn(*shapes.to_soa(A), na, eps, True, 7, *shapes.to_soa(B), nb, eps, True, 9)
+    st = contact._stats
+    rc, want, ost = ol.or_detect(code, A, B, eps, eps, 1, 1, 7, 9)
+    assert rc == 0
+    same_contacts(got, want)
+    for f in ("penalty_fails", "batch_fails", "batch_size", "triangle_checks",
+              "pairs_evaluated", "fallback_rows"):
+        assert getattr(st, f) == getattr(ost, f), f
+
+
 def test_hybrid_triangle_rejects_reference_out_of_bounds():
     A = scenes.particle(0, 0.5e-3, 1, [0, 0, 0])
     B = scenes.particle(1, 0.5e-3, 2, [1e-3, 0, 0])

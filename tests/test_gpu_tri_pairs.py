@@ -166,3 +166,16 @@ def test_brute_force_at_its_edges():
         Po, Qo, do, fo = oracle_pairs(0, soa)
         assert same_bits(d, do) and same_bits(P.ravel(), Po.ravel()), name
         assert same_bits(Q.ravel(), Qo.ravel()) and np.array_equal(f, fo), name
+
+
+@pytest.mark.parametrize("method,code", [("penalty64", 1), ("hybrid64", 2)])
+def test_penalty_at_its_edges(method, code):
+    """The penalty's shared reciprocals and its bounds on the GPU, as above."""
+    from test_hostcheck import penalty_edge_sets, same_bits
+    for name, soa in penalty_edge_sets(20000):
+        b = narrow.PairBatch.from_host(soa)
+        b.run(method)
+        P, Q, d, f = b.results()
+        Po, Qo, do, fo = oracle_pairs(code, soa)
+        assert same_bits(d, do) and same_bits(P.ravel(), Po.ravel()), name
+        assert same_bits(Q.ravel(), Qo.ravel()) and np.array_equal(f, fo), name

@@ -407,3 +407,37 @@ def test_brute_force_at_its_edges(hc):
             outs.append((P, Q, d, f))
         assert all(same_bits(a, b) for a, b in zip(outs[0][:3], outs[1][:3])), name
         assert np.array_equal(outs[0][3], outs[1][3]), name
+
+
+def penalty_edge_sets(n, seed=6):
+    """bf_edge_sets, and pairs about the bounds of the penalty's regular path:
+    edges of 2^-20 and 2^20, first vertices at 2^30, constraints met exactly
+    (a start on a face's border), and 1e-320 numerators."""
+    yield from bf_edge_sets(n, seed)
+    rng = np.random.default_rng(seed)
+    x = rng.normal(0, 1, (18, n))
+    for k in (-22, -21, -20, -19, 19, 20, 21):
+        yield f"edges of 2^{k}", x * 2.0 ** k
+    yield "far from the origin", x + 2.0 ** 30 * rng.uniform(0.5, 2.0, n)
+    flat = x.copy()
+    flat[6:9] = 0.0
+    flat[15:18] *= 10.0 ** rng.uniform(-320, -280, n)
+    yield "nearly coplanar", flat
+
+
+def test_penalty_at_its_edges(hc):
+    """The same of the penalty and the hybrid, whose regular pairs have steps of
+    their own."""
+    n = 20000
+    for name, s in penalty_edge_sets(n):
+        s = np.ascontiguousarray(s)
+        for method in (1, 2):
+            outs = []
+            for lib, fn in ((ol.oracle(), "or_tri_pairs"), (hc, "hc_tri_pairs")):
+                P = np.zeros(3 * n); Q = np.zeros(3 * n); d = np.zeros(n)
+                f = np.zeros(n, np.uint8)
+                getattr(lib, fn)(method, ol.dptr(s), C.c_long(n), C.c_double(2e-4), ol.dptr(P),
+                                 ol.dptr(Q), ol.dptr(d), f.ctypes.data_as(C.c_void_p))
+                outs.append((P, Q, d, f))
+            assert all(same_bits(a, b) for a, b in zip(outs[0][:3], outs[1][:3])), (name, method)
+            assert np.array_equal(outs[0][3], outs[1][3]), (name, method)
