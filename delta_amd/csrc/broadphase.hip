@@ -311,7 +311,7 @@ struct GridArgs {
   int* nlarge;
   // partners of a large particle are searched in chunks of `chunk`
   // candidates j (nchunks per particle, chunk c covers [c*chunk, (c+1)*chunk)),
-  // one wave per (large particle, chunk); lcount[slot * nchunks + c] holds
+  // one workgroup per (large particle, chunk); lcount[slot * nchunks + c] holds
   // each chunk's partner count
   int chunk, nchunks;
   int* lcount;
@@ -437,46 +437,58 @@ __device__ __forceinline__ int grid_partners(const GridArgs& g, int i, const Aab
   return found;
 }
 
-// Partners j of a large particle i in chunk c: every j > i of the chunk
-// (not both obstacles), in ascending order; put(position, j) as above.
+// Partners j of a large particle i in chunk c: every j > i of the chunk (not
+// both obstacles), ascending, 1,024 a round over the workgroup's four waves;
+// put(position, j) on the finding lane.  Returns their number.
 template <typename F>
-__device__ int large_chunk(const GridArgs& g, int i, const Aabb& bi, int c, int lane, F put) {
+__device__ __forceinline__ int large_chunk(const GridArgs& g, int i, int c, int* wave_count,
+                                           F put) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const Aabb bi = g.box[i];
   const bool obst_i = g.obstacle && g.obstacle[i];
   const int lo = c * g.chunk > i + 1 ? c * g.chunk : i + 1;
   const int hi = (c + 1) * g.chunk < g.n ? (c + 1) * g.chunk : g.n;
   int found = 0;
-  // four strips of 64 per round: their loads are issued together
-  for (int j0 = lo; j0 < hi; j0 += 256) {
+  for (int j0 = lo; j0 < hi; j0 += 256 * kBpWaves) {
+    // four strips of 64 per wave: their loads are issued together
     bool e[4];
+    int m = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int j = j0 + 64 * q + lane;
+      const int j = j0 + 256 * w + 64 * q + lane;
       e[q] = j < hi && !(obst_i && g.obstacle && g.obstacle[j]) && overlap(bi, g.box[j]);
+      m += __popcll(__ballot(e[q]));
+    }
+    if (lane == 0) wave_count[w] = m;
+    __syncthreads();
+    int at = found;
+    for (int o = 0; o < kBpWaves; ++o) {
+      at += o < w ? wave_count[o] : 0;
+      found += wave_count[o];
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const unsigned long long mask = __ballot(e[q]);
-      if (e[q]) put(found + bp_lane_prefix(mask), j0 + 64 * q + lane);
-      found += __popcll(mask);
+      if (e[q]) put(at + bp_lane_prefix(mask), j0 + 256 * w + 64 * q + lane);
+      at += __popcll(mask);
     }
+    __syncthreads();  // the next round overwrites the counts
   }
   return found;
 }
 
-// Large particles, one wave per (slot, chunk) item, strided over a
+// Large particles, one workgroup per (slot, chunk) item, strided over a
 // persistent grid (the number of large particles is known on the device
-// only): chunk partner counts.
+// only): chunk partner counts.  Few items: the latency of a chunk's loads is
+// what they cost (a wave per item, four rounds: 16 us in a hopper of 15,651
+// particles, 7 us now; the fill 14 and 6).
 __global__ __launch_bounds__(64 * kBpWaves) void k_large_count(GridArgs g) {
-  const int lane = threadIdx.x & 63;
-  const long long nw = static_cast<long long>(gridDim.x) * kBpWaves;
+  __shared__ int wave_count[kBpWaves];
   const long long items = static_cast<long long>(*g.nlarge) * g.nchunks;
-  auto none = [](int, int) {};
-  for (long long t = static_cast<long long>(blockIdx.x) * kBpWaves + (threadIdx.x >> 6);
-       t < items; t += nw) {
+  for (long long t = blockIdx.x; t < items; t += gridDim.x) {
     const int o = static_cast<int>(t / g.nchunks), c = static_cast<int>(t - o * static_cast<long long>(g.nchunks));
-    const int i = g.large[o];
-    const int m = large_chunk(g, i, g.box[i], c, lane, none);
-    if (lane == 0) g.lcount[t] = m;
+    const int m = large_chunk(g, g.large[o], c, wave_count, [](int, int) {});
+    if (threadIdx.x == 0) g.lcount[t] = m;
   }
 }
 
@@ -498,18 +510,17 @@ __global__ __launch_bounds__(64 * kBpWaves) void k_large_fill(GridArgs g,
                                                                const long long* __restrict__ start,
                                                                long long cap,
                                                                int* __restrict__ pairs) {
+  __shared__ int wave_count[kBpWaves];
   const int lane = threadIdx.x & 63;
-  const long long nw = static_cast<long long>(gridDim.x) * kBpWaves;
   const long long items = static_cast<long long>(*g.nlarge) * g.nchunks;
-  for (long long t = static_cast<long long>(blockIdx.x) * kBpWaves + (threadIdx.x >> 6);
-       t < items; t += nw) {
+  for (long long t = blockIdx.x; t < items; t += gridDim.x) {
     const int o = static_cast<int>(t / g.nchunks), c = static_cast<int>(t - o * static_cast<long long>(g.nchunks));
     const int i = g.large[o];
     long long before = 0;
     for (int q = lane; q < c; q += 64) before += g.lcount[t - c + q];
     for (int k = 32; k > 0; k >>= 1) before += __shfl_xor(before, k);
     const long long s = start[i] + before;
-    large_chunk(g, i, g.box[i], c, lane, [&](int pos, int j) {
+    large_chunk(g, i, c, wave_count, [&](int pos, int j) {
       const long long q = s + pos;
       if (q < cap) {
         pairs[2 * q] = i;
@@ -727,8 +738,7 @@ struct BpScratch {
 };
 static BpScratch g_bp;
 
-// Candidates per large-particle chunk: 1024 (four rounds of 256 loads per
-// wave), more for very large n so that a particle has at most 256 chunks.
+// Candidates per large-particle chunk: 1024 (one round of a workgroup), more for very large n so that a particle has at most 256 chunks.
 static int large_chunk_len(int n) {
   int c = 1024;
   while (static_cast<long long>(c) * 256 < n) c *= 2;
@@ -742,8 +752,7 @@ static int large_chunks(int n) {
 
 // Persistent grid of the large-particle kernels.
 static unsigned large_grid(long long items) {
-  const long long g = (items + kBpWaves - 1) / kBpWaves;
-  return static_cast<unsigned>(g < 1 ? 1 : (g > 2048 ? 2048 : g));
+  return static_cast<unsigned>(items < 1 ? 1 : (items > 2048 ? 2048 : items));
 }
 
 static unsigned table_size(int n) {
@@ -871,7 +880,7 @@ static int grid_build(const dh_geometry* geom, const int* obstacle_dev, double c
   hipLaunchKernelGGL(k_grid_count2, grid_for(n, 2 * kBpWaves), 64 * kBpWaves, 0, st, g, b.count);
   const long long items = static_cast<long long>(n) * g.nchunks;  // bound on the device count
   hipLaunchKernelGGL(k_large_count, large_grid(items), 64 * kBpWaves, 0, st, g);
-  hipLaunchKernelGGL(k_large_sum, large_grid(n), 64 * kBpWaves, 0, st, g, b.count);
+  hipLaunchKernelGGL(k_large_sum, large_grid((n + kBpWaves - 1) / kBpWaves), 64 * kBpWaves, 0, st, g, b.count);
   DH_HIP_CHECK(hipGetLastError());
   return scan_into(b, b.count, n, b.start, st);
 }

@@ -1684,7 +1684,10 @@ __global__ __launch_bounds__(256) void k_queue_record(DetectArgs g, const int* _
 }
 
 // Pass 3, after the pairs' offsets: the records' contacts, each at its place,
-// and those that the full kernel left in `temp` (*in_temp of them).
+// and those that the full kernel left in `temp` (*in_temp of them).  A
+// workgroup per region: a record waits for a chain of loads, which a wave per
+// region went through once per 64 records (hopper of 15,651 spheres 51 us,
+// 46 us now, near the copy rate).
 __device__ __forceinline__ long long contact_place(const DetectArgs& g, int item, int rank,
                                                    const long long* __restrict__ offs) {
   const int k = item / g.tiles;
@@ -1698,9 +1701,8 @@ __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long lo
                                                      const unsigned long long* __restrict__ in_temp,
                                                      unsigned long long* __restrict__ found,
                                                      Report report) {
-  const int lane = threadIdx.x & 63;
-  const int r = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
-  const int total = r < g.regions ? g.rcount[r] : 0;
+  const int r = blockIdx.x;
+  const int total = g.rcount[r];
   const bool heavy = total > g.heavy;
   for (int p = 0; p < (heavy ? 4 : total > 0 ? 1 : 0); ++p) {
     const int* c = g.rparts + 8 * static_cast<long long>(r) + 2 * p;
@@ -1709,7 +1711,7 @@ __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long lo
     const QueueRecord* rec =
         g.rec + static_cast<long long>(r) * g.rcap + (heavy ? p * region_part(total) : 0);
     const int base = heavy ? c[1] : 0, first = rec[0].item;
-    for (int e = lane; e < n; e += 64) {
+    for (int e = threadIdx.x; e < n; e += 256) {
       const QueueRecord q = rec[e];
       const long long dst = contact_place(g, q.item, q.rank + (q.item == first ? base : 0), offs);
       if (dst >= cap) continue;  // past the capacity: dropped (reported by the caller)
@@ -2133,7 +2135,7 @@ static int detect_pairs_tiled(int method, const dh_geometry* geom, const int* pa
   report_add(report, g_scratch.stats.ptr, 2 * ST_COUNT);
   if (queued) {
     report_add(report, g_scratch.qcounts.ptr, kQueueCounts);
-    hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out, cap,
+    hipLaunchKernelGGL(k_queue_write, static_cast<unsigned>(plan.regions), 256, 0, st, a, offs, out, cap,
                        a.counter, nullptr, report);
   } else {
     const long long wg = (cap + 255) / 256;
@@ -2239,7 +2241,7 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
   }
   if ((rc = pair_offsets(a, counts, offs, st))) return rc;
   if (queued) {
-    hipLaunchKernelGGL(k_queue_write, grid_for(plan.regions, 4), 256, 0, st, a, offs, out,
+    hipLaunchKernelGGL(k_queue_write, static_cast<unsigned>(plan.regions), 256, 0, st, a, offs, out,
                        contact_cap, a.counter, g_scratch.found.as<unsigned long long>(), Report{});
   } else {
     const long long wg = (contact_cap + 255) / 256;
