@@ -121,17 +121,37 @@ def test_batched_bf_through_the_survivor_queue(max_tiles, screen):
         tuning.set(**tuning.default())
 
 
-def _batched_pairs(method):
-    parts = [scenes.particle(1 + (i % 2), 0.5e-3, 50 + i, [0.98e-3 * i, 0.05e-3 * (i % 3), 0])
-             for i in range(6)]
-    parts.append(scenes.floor(-0.45e-3))
-    pairs = [(i, i + 1) for i in range(5)] + [(i, 6) for i in range(6)] + [(0, 2)]
+@pytest.mark.parametrize("max_tiles", [1, 7])
+@pytest.mark.parametrize("eps", [1e-3, 5e-3, 2e-2, 1e-1])
+def test_survivor_queue_at_its_limits(eps, max_tiles):
+    """Regions below and above the 256 entries that one wave takes and the
+    1,024 they hold, items of more than 160 kept boxes, uneven ones, empty ones
+    and one triangle: with and without deferral the contacts, their order and
+    the counters are the oracle's."""
+    from delta_amd import tuning
+    parts = [soup(80, 1), soup(80, 2, 0.1), soup(320, 3, 0.5), soup(100, 4, 0.7), soup(8, 5, 0.2),
+             soup(1, 6), soup(700, 7, 5.0), soup(64, 8, 4.2)]
+    pairs = [(0, 1), (0, 2), (0, 4), (1, 2), (1, 3), (2, 3), (2, 4), (4, 2), (5, 0), (0, 6), (6, 7)]
+    tuning.set(detect_queue_min_items=0, detect_max_tiles=max_tiles)
+    try:
+        for _ in range(2):  # an eager call sizes the next one's regions
+            _batched_pairs("bf", parts, pairs, eps)
+    finally:
+        tuning.set(**tuning.default())
+
+
+def _batched_pairs(method, parts=None, pairs=None, eps=EPS):
+    if parts is None:
+        parts = [scenes.particle(1 + (i % 2), 0.5e-3, 50 + i, [0.98e-3 * i, 0.05e-3 * (i % 3), 0])
+                 for i in range(6)]
+        parts.append(scenes.floor(-0.45e-3))
+        pairs = [(i, i + 1) for i in range(5)] + [(i, 6) for i in range(6)] + [(0, 2)]
     offs = np.cumsum([0] + [len(p) for p in parts]).astype(np.int32)
     allm = np.concatenate(parts)
     x, y, z = (DeviceArray.from_host(v) for v in shapes.to_soa(allm))
     d_off = DeviceArray.from_host(offs)
     n = len(parts)
-    d_eps = DeviceArray.from_host(np.full(n, EPS))
+    d_eps = DeviceArray.from_host(np.full(n, eps))
     d_fr = DeviceArray.from_host(np.ones(n, np.int32))
     d_id = DeviceArray.from_host(np.arange(n, dtype=np.int32) * 10)
     d_pairs = DeviceArray.from_host(np.array(pairs, np.int32).reshape(-1))
@@ -154,7 +174,7 @@ def _batched_pairs(method):
     want = []
     ost_total = ol.DhStats()
     for k, (a, b) in enumerate(pairs):
-        rc, w, ost = ol.or_detect(code, parts[a], parts[b], EPS, EPS, 1, 1, 10 * a, 10 * b)
+        rc, w, ost = ol.or_detect(code, parts[a], parts[b], eps, eps, 1, 1, 10 * a, 10 * b)
         assert rc == 0
         assert counts[k] == len(w)
         w = w.copy()
