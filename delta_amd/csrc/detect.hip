@@ -693,7 +693,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
           int iA = 0, iB = 0;
           if (e < nl) {
             pair_of(surv[e], iA, iB);
-            bf_solver(load_tri(g, p.oA + iA), load_tri(g, p.oB + iB), P, Q);
+            bf_solver_general(load_tri(g, p.oA + iA), load_tri(g, p.oB + iB), P, Q);
             emit = pq_dist(P, Q) <= p.margin;
           }
           emit_chunk(emit, iA, iB, P, Q);

@@ -526,10 +526,13 @@ DH_HD bool bf_features_regular(Tri<double> A, Tri<double> B, BfBest<double>& bes
   return ok && least >= 1E-30 && sum + dot(ab, ab) < 0x1p180;
 }
 
+// kGeneral: no regular path (see bf_solver_general).
+template <bool kGeneral>
 DH_HD void bf_features_any(const Tri<double>& A, const Tri<double>& B, BfBest<double>& best) {
-  if (!bf_features_regular(A, B, best)) bf_features(A, B, best);
+  if (kGeneral || !bf_features_regular(A, B, best)) bf_features(A, B, best);
 }
 
+template <bool kGeneral>
 DH_HD void bf_features_any(const Tri<float>& A, const Tri<float>& B, BfBest<float>& best) {
   bf_features(A, B, best);
 }
@@ -540,11 +543,11 @@ DH_HD void bf_features_any(const Tri<float>& A, const Tri<float>& B, BfBest<floa
 // into cases 2 (zoltan/bf.cpp:527-559, 907-925): edge-edge feature 1 takes
 // its Q from B's edge 2->0 with feature 1's parameter, vertex-face feature 1
 // reports B's vertex 2.
-template <typename T, bool kZoltan = false>
+template <typename T, bool kZoltan = false, bool kGeneral = false>
 DH_HD bool bf_solver_ids(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q, int& ssid_out,
                          int& id_out) {
   BfBest<T> best;
-  bf_features_any(A, B, best);
+  bf_features_any<kGeneral>(A, B, best);
   const int ssid = best.ssid, id = best.id;
   const T ssc = best.ssc, ttc = best.ttc, ss = best.ss, tt = best.tt;
   ssid_out = ssid;
@@ -576,6 +579,18 @@ template <typename T>
 DH_HD bool bf_solver(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q) {
   int ssid, id;
   return bf_solver_ids(A, B, P, Q, ssid, id);
+}
+
+// The same by the general path alone, for the detection without the survivor
+// queue: its few survivors per item wait for loads and barriers rather than
+// for instructions, while the particles of a run that has left all bounds
+// (NaN, or so far out that their triangles round to lines) pair with every
+// other and would take both paths (the lattice's 2,000 steps: 0.178 ms a step,
+// 0.23 with both).
+DH_HD bool bf_solver_general(const Tri<double>& A, const Tri<double>& B, V3<double>& P,
+                             V3<double>& Q) {
+  int ssid, id;
+  return bf_solver_ids<double, false, true>(A, B, P, Q, ssid, id);
 }
 
 // |Q-P| in the caller's order (bf.cpp:117, contactpoint.cpp:157-159).
@@ -915,7 +930,7 @@ DH_HD bool penalty_fixed(const Tri<T>& A, const Tri<T>& B, const T x0[4], int it
     bool ok = pen.regular() && iters > 0;
     int low = least_exponent(least_exponent(0, pen.h[2]), pen.h[3]);
 #pragma unroll 1
-    for (int i = 0; i < iters; ++i) {
+    for (int i = 0; ok && i < iters; ++i) {
       if (i > 0)
         for (int q = 0; q < 4; ++q) x[q] -= dx[q];
       ok = pen.step_regular(x, reg, dx, low) && ok;
