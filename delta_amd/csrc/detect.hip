@@ -19,6 +19,7 @@
 
 #include "exact_math.hpp"
 #include "gjk.hpp"
+#include "pair_range.hpp"
 #include "runtime.hpp"
 
 namespace dh {
@@ -365,22 +366,17 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
   // chunks of 256, which leave no wave of the last round idle (rows of 80 did
   // for the penalty's 12 tiles of 6,400 pairs: 137 us, 133 us so)
   constexpr bool kFlat = M == DH_PENALTY || M == DH_PENALTY_STAT;
-  int total = nrows * p.nB, f0 = r0 * p.nB;
-  if (kFlat) {
-    // at most 64 tiles and 2^23 chunks: products of 32 bits
-    const unsigned all = static_cast<unsigned>(rows * p.nB), chunks = (all + 255) / 256;
-    const unsigned n = static_cast<unsigned>(g.tiles), t = static_cast<unsigned>(tile);
-    const unsigned a = 256 * (t * chunks / n), b = 256 * ((t + 1) * chunks / n);
-    f0 = static_cast<int>(a);
-    total = static_cast<int>((b < all ? b : all) - a);
-  }
+  const PairRange range = kFlat ? pair_range(rows, p.nB, g.tiles, tile)
+                                : PairRange{static_cast<long long>(nrows) * p.nB, r0, 0};
   // the pairs of a hybrid tile whose penalty points are within the margin, so
   // that a row which does not fall back is not solved again for the others
   // (a tile of more pairs solves all of them twice)
   constexpr bool kNoted = M == DH_HYBRID_BATCH || M == DH_HYBRID_TRIANGLE;
   constexpr int kNotedPairs = 16384;
   __shared__ unsigned long long close_bits[kNoted ? kNotedPairs / 64 : 1];
-  const bool noted = kNoted && total <= kNotedPairs;
+  const bool noted = kNoted && range.count <= kNotedPairs;
+  // the hybrids' pairs, of at most kMaxRowTriangles rows and columns
+  const int f0 = is_hybrid ? r0 * p.nB : 0, total = is_hybrid ? nrows * p.nB : 0;
 
   if (is_hybrid) {
     for (int r = tid; r < nrows; r += 256) {
@@ -442,7 +438,8 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
   // chunks): block prefix over the emitting lanes, one global atomic for the
   // chunk's slots, rank within the tile in pad_.
   unsigned long long running = 0;
-  unsigned culled = 0;
+  bool far_pair = false;
+  unsigned culled = 0;  // of a lane; a whole pair's are counted at the end
   auto emit_chunk = [&](bool emit, int iA, int iB, const V3<double>& P, const V3<double>& Q) {
     const unsigned long long mask = __ballot(emit);
     const int pre = lane_prefix(mask);
@@ -487,11 +484,12 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
     __shared__ unsigned char row_far[kBoxTriangles];  // row in a chunk apart from B
     __shared__ unsigned char chunk_near[kChunkFlags];  // the item's chunks against B's box
     const bool staged = p.nB <= kBoxTriangles;  // block-uniform
-    const int blk = staged ? kBoxTriangles : (nrows > 0 ? nrows : 1);
+    // an unstaged block's pairs are numbered in 32 bits
+    const int most = p.nB > 0 ? (1 << 30) / p.nB : 1 << 30;
+    const int blk = staged ? kBoxTriangles : (nrows < most ? (nrows > 0 ? nrows : 1) : (most > 0 ? most : 1));
     bool b_staged = false;  // B's boxes are loaded on the first block that needs them
     // the whole pair beyond the margin by its bounding spheres
-    const bool far_pair = spheres_apart(g, p);
-    if (far_pair) culled += tid == 0 ? static_cast<unsigned>(nrows * p.nB) : 0u;
+    far_pair = spheres_apart(g, p);
     // A in chunks of 64 rows with their boxes (a wall or a funnel): every
     // chunk of the item tested against B's particle box once, up front
     const bool chunked = staged && g.bbox && g.pbox && p.nA > kRowBlock;
@@ -521,7 +519,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
         for (int c = rs / 64; c <= (rs + nrb - 1) / 64; ++c)
           any_near = any_near || chunk_near[c - c_first] != 0;
         if (!any_near) {  // every chunk of the block is apart
-          culled += tid == 0 ? static_cast<unsigned>(nrb * p.nB) : 0u;
+          culled += tid == 0 ? nrb * p.nB : 0;
           continue;
         }
       } else if (chunked) {
@@ -529,7 +527,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
         for (int c = rs / 64 + tid; c <= (rs + nrb - 1) / 64; c += 256)
           any_near = any_near || !chunk_far(64 * c);
         if (!__syncthreads_or(any_near)) {  // every chunk of the block is apart
-          culled += tid == 0 ? static_cast<unsigned>(nrb * p.nB) : 0u;
+          culled += tid == 0 ? nrb * p.nB : 0;
           continue;
         }
       }
@@ -545,7 +543,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
         }
         if (g.pbox && !__syncthreads_or(near)) {
           // every row of the block misses B's particle box
-          culled += tid == 0 ? static_cast<unsigned>(nrb * p.nB) : 0u;
+          culled += tid == 0 ? nrb * p.nB : 0;
           continue;
         }
         if (!b_staged) {
@@ -623,7 +621,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
         iB = staged ? act[kBoxTriangles + cb] : cb;
       };
       const int tested = nra * nca;
-      culled += tid == 0 ? static_cast<unsigned>(nrb * p.nB - tested) : 0u;
+      culled += tid == 0 ? nrb * p.nB - tested : 0;
       for (int fpos = 0; fpos < tested;) {
         int nl = 0;
         while (fpos < tested && nl <= kSurvivors - 256) {
@@ -639,7 +637,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
             } else {
               keep = !boxes_apart(load_tri(g, p.oA + iA), load_tri(g, p.oB + iB), p.margin);
             }
-            culled += keep ? 0u : 1u;
+            culled += keep ? 0 : 1;
           }
           const unsigned long long m = __ballot(keep);
           if (lane == 0) wave_cnt[wave] = __popcll(m);
@@ -703,14 +701,13 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
       __syncthreads();
     }
   } else {
-    for (int base = 0; base < total; base += 256) {
-      const int f = base + tid;
+    PairWalk at(range, p.nB, tid);
+    for (long long left = range.count; left > 0; left -= kPairChunk) {
+      const int f = static_cast<int>(range.count - left) + tid;  // read where the tile is noted
       bool emit = false;
       V3<double> P = {0, 0, 0}, Q = {0, 0, 0};
-      int iA = 0, iB = 0;
-      if (f < total) {
-        iA = (f0 + f) / p.nB;
-        iB = (f0 + f) - iA * p.nB;
+      const int iA = at.iA, iB = at.iB;
+      if (tid < left) {
         if (M == DH_PENALTY_STAT) {
           const Tri<double> A = load_tri(g, p.oA + iA);
           const Tri<double> B = load_tri(g, p.oB + iB);
@@ -740,12 +737,14 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
         }
       }
       emit_chunk(emit, iA, iB, P, Q);
+      at.next(p.nB);
     }
   }
   if (M == DH_BF) {
     // slot 3 of local_stats (zeroed at the start, unused by BF otherwise)
-    for (int o = 32; o > 0; o >>= 1) culled += __shfl_xor(culled, o);
-    if (lane == 0) atomicAdd(&local_stats[3], static_cast<unsigned long long>(culled));
+    unsigned long long sum = far_pair && tid == 0 ? range.count : culled;
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if (lane == 0) atomicAdd(&local_stats[3], sum);
     __syncthreads();
   }
   if (tid == 0) {
@@ -753,7 +752,7 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
     // evaluations the reference performs: every pair once, plus bfSolver
     // again over each fallback row (sums over the tiles)
     const unsigned long long evals =
-        static_cast<unsigned long long>(total) +
+        static_cast<unsigned long long>(range.count) +
         (is_hybrid ? local_stats[0] * static_cast<unsigned long long>(p.nB) : 0ull);
     ts[TS_CHECKS] = tile == 0 ? static_cast<unsigned long long>(p.nA) * p.nB : 0ull;
     ts[TS_EVALUATED] = evals;

@@ -353,3 +353,27 @@ extern "C" void hc_cr_sincos(const double* x, long n, double* s, double* c) {
     c[i] = dh::cr_sincos(x[i], true);
   }
 }
+
+#include <initializer_list>
+
+#include "pair_range.hpp"
+
+// The pairs that the tiles of a rows x cols list take, walked chunk by chunk as
+// the kernel does: 0 when they are all of them, each once and in order, else the
+// number of the first tile (from 1) that is wrong.
+extern "C" int hc_pair_ranges(int rows, int cols, int tiles) {
+  long long at = 0;
+  for (int tile = 0; tile < tiles; ++tile) {
+    const dh::PairRange r = dh::pair_range(rows, cols, tiles, tile);
+    int row = r.row, col = r.col;
+    for (int t : {0, 1, dh::kPairChunk - 1}) {  // lanes of the workgroup
+      dh::PairWalk w(r, cols, t);
+      for (long long f = t; f < r.count; f += dh::kPairChunk, w.next(cols))
+        if (w.iA < 0 || w.iA >= rows || w.iB < 0 || w.iB >= cols ||
+            static_cast<long long>(w.iA) * cols + w.iB != at + f)
+          return tile + 1;
+    }
+    at += r.count;
+  }
+  return at == static_cast<long long>(rows) * cols ? 0 : tiles + 1;
+}

@@ -224,3 +224,33 @@ def test_bf_large_particle_matches_oracle(max_tiles, swap, queue):
     rc, want, _ = ol.or_detect(_lib.DH_BF, A, B, EPS, EPS, 1, 1, 7, 9)
     assert rc == 0 and len(want) > 0
     same_contacts(got, want)
+
+
+def _facing_lines(n):
+    """n triangles on a line, 1 cm apart, and n beside them: every 4,001st within
+    the margin, the others 1 m away."""
+    rng = np.random.default_rng(9)
+    tri = rng.uniform(-1e-3, 1e-3, (3, 3))
+    at = 1e-2 * np.arange(n)[:, None, None] * np.array([1.0, 0.0, 0.0])
+    A, B = tri + at, tri + at + np.array([0.0, 1.0, 0.0])
+    B[::4001, :, 1] -= 1.0 - 5e-5
+    return A, B
+
+
+@pytest.mark.parametrize("n", [46341, 65537])
+def test_penalty_over_more_pairs_than_32_bits_number(n):
+    """n x n triangles are more than 2^31 (2^32) pairs: the contacts are those
+    of A called part by part, in order, and come from every tile."""
+    A, B = _facing_lines(n)
+    contact.reset_all_statistics()
+    got = contact.penalty(*shapes.to_soa(A), n, EPS, True, 7, *shapes.to_soa(B), n, EPS, True, 9)
+    assert contact._stats.pairs_evaluated == n * n
+    want = []
+    for lo in range(0, n, 16384):
+        a = A[lo:lo + 16384]
+        w = contact.penalty(*shapes.to_soa(a), len(a), EPS, True, 7, *shapes.to_soa(B), n, EPS,
+                            True, 9).copy()
+        w["triA"] += lo
+        want.append(w)
+    same_contacts(got, np.concatenate(want))
+    assert set(range(0, n, 4001)) <= set(got["triB"].tolist())

@@ -441,3 +441,16 @@ def test_penalty_at_its_edges(hc):
                 outs.append((P, Q, d, f))
             assert all(same_bits(a, b) for a, b in zip(outs[0][:3], outs[1][:3])), (name, method)
             assert np.array_equal(outs[0][3], outs[1][3]), (name, method)
+
+
+@pytest.mark.parametrize("rows,cols,tiles", [
+    (1, 1, 1), (1, 1, 64), (7, 36, 3), (16, 16, 1), (16, 16, 2), (17, 15, 5), (80, 80, 12),
+    (1, 100000, 7), (100000, 1, 7), (300, 255, 3), (300, 256, 3), (300, 257, 3), (0, 5, 4), (5, 0, 4),
+    (46340, 46341, 1), (46341, 46341, 1), (46341, 46341, 64),  # either side of 2^31
+    (65535, 65537, 64), (65536, 65535, 64),  # the last of 32 bits
+    (65536, 65536, 1), (65536, 65536, 64), (65537, 65536, 7),  # 2^32 and above
+    (3, 2147483391, 2), (2147483391, 3, 2)])
+def test_pair_ranges_of_the_tiles(hc, rows, cols, tiles):
+    """The flat tiles take every triangle pair once and in order, on both
+    sides of the products that pass 31 and 32 bits."""
+    assert hc.hc_pair_ranges(C.c_int(rows), C.c_int(cols), C.c_int(tiles)) == 0
