@@ -250,7 +250,7 @@ __device__ __forceinline__ bool box_sphere_apart(const double* lo, const double*
 __device__ __forceinline__ bool penalty_pair(const Tri<double>& A, const Tri<double>& B,
                                              double max_err, V3<double>& P, V3<double>& Q) {
   const double x0[4] = {0.33, 0.33, 0.33, 0.33};
-  return penalty_fixed(A, B, x0, 4, max_err, P, Q, (double*)nullptr);
+  return penalty_fixed(A, B, x0, 4, max_err, P, Q);
 }
 
 // False for triangles that DH_BF's box or plane test proves to be further

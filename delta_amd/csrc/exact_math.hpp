@@ -287,10 +287,16 @@ DH_HD void bf_features(const Tri<T>& A, const Tri<T>& B, BfBest<T>& best) {
 // Regular means that no intermediate value leaves the range in which that
 // holds: squared edge lengths (and a face's third one, as the face's formula
 // has it) of at least 1e-30, so that a clamped parameter's numerator and
-// denominator are not taken for zero, face determinants of at least 1e-60,
-// and squared lengths and one squared distance of less than 2^180, so that
-// nothing overflows (a NaN fails that test).  MI355X, 2^24 pairs: 2,807 to about
-// 2,170 vector instructions per wave of 64 pairs, 1.467 to 1.198 ms.
+// denominator are not taken for zero, and of less than 2^180, so that nothing
+// overflows (a feature further away than the 1e30 that the minima start from
+// is not taken, whatever its value), no point over the inside of a face
+// whose determinant is in (0, 1e-60), and no feature's distance in (0, 2^-350).
+// Coordinates that are NaN are regular: as in the general form, the distance
+// of each feature that they are part of is NaN, which is never the least.
+// MI355X, 2^24 pairs: 2,807 to about 2,170 vector instructions per wave of 64
+// pairs, 1.467 to 1.198 ms.  A wave leaves as soon as one of its lanes has too
+// short or too long an edge: with two such pairs in 100, 2^20 pairs took 148
+// us where the others went on, 102 by the general form alone.
 
 // a / b, correctly rounded, for 2^-400 < |a|, |b| < 2^400 (other operands: any
 // value): the reciprocal by two Newton steps, the quotient by one residual.
@@ -338,12 +344,16 @@ DH_HD int least_exponent(int e, double a) {
   return x < e ? x : e;
 }
 
-// sqrt(x), correctly rounded, for x >= 2^-700 (else `ok` is cleared): by
-// Goldschmidt's iteration and two residual corrections.
-DH_HD double sqrt_regular(double x, bool& ok) {
-  ok &= x >= 0x1p-700;
+// The square root at which a squared distance is too small for sqrt_regular.
+constexpr double kSqrtLeast = 0x1p-349;
+
+// sqrt(x), correctly rounded, for x >= 2^-700 and x = 0, by Goldschmidt's
+// iteration and two residual corrections.  Between them the value is positive
+// and below kSqrtLeast: the estimate y of 1 / sqrt(2^-700) gives g = x * y in
+// (0, 2^-350), and every correction adds a factor of 1 to 1.5.
+DH_HD double sqrt_regular(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const double y = __builtin_amdgcn_rsq(x);
+  const double y = __builtin_amdgcn_rsq(fmax(x, 0x1p-700));
   double g = x * y, h = 0.5 * y;
   const double r = fma(-h, g, 0.5);
   g = fma(g, r, g);
@@ -369,7 +379,7 @@ DH_HD double clamp01(double q) {
 // clamp of sN / D; only parallel edges that keep their t need a zero of
 // their own.
 DH_HD double edge_edge_regular(const V3<double>& u, double a, const V3<double>& v, double c,
-                               const V3<double>& w, double& sc, double& tc, bool& ok) {
+                               const V3<double>& w, double& sc, double& tc) {
   using std::fabs;
   const double small_num = 1E-30;
   const double b = dot(u, v), d = dot(u, w), e = dot(v, w);
@@ -391,23 +401,26 @@ DH_HD double edge_edge_regular(const V3<double>& u, double a, const V3<double>& 
   tc = (fabs(tN) < small_num) ? 0.0 : qt;
   const V3<double> dP = {w.x + (sc * u.x) - (tc * v.x), w.y + (sc * u.y) - (tc * v.y),
                          w.z + (sc * u.z) - (tc * v.z)};
-  return sqrt_regular(dP.x * dP.x + dP.y * dP.y + dP.z * dP.z, ok);
+  return sqrt_regular(dP.x * dP.x + dP.y * dP.y + dP.z * dP.z);
 }
 
 // The terms of a face that its three points share.
 struct FaceTerms {
   V3<double> o, e0, e1;
   double a, b, c, det, denom;
+  bool inside;  // 1 / det does not overflow, or is the infinity that leaves NaN
   DH_HD explicit FaceTerms(const Tri<double>& t)
       : o(t.v[0]), e0(sub(t.v[1], t.v[0])), e1(sub(t.v[2], t.v[0])), a(dot(e0, e0)),
-        b(dot(e0, e1)), c(dot(e1, e1)), det(a * c - b * b), denom(a - 2.0 * b + c) {}
+        b(dot(e0, e1)), c(dot(e1, e1)), det(a * c - b * b), denom(a - 2.0 * b + c),
+        inside(det >= 1E-60 || det == 0.0) {}
 };
 
 // pt_tri and the distance for a regular face: the face parameters are
 // (s0, t0) / det inside, and on the boundary one clamped quotient: along
 // t = 0, along s = 0, or along s + t = 1.  pt_tri's sums for the three
 // corners are its quadratic form at (0, 0), (1, 0) and (0, 1) term by term,
-// so only the two edges t = 0 and s = 0 have a form of their own.
+// so only the two edges t = 0 and s = 0 have a form of their own.  `ok` is
+// cleared over the inside of a face that is nearly, but not quite, a line.
 DH_HD double vertex_face_regular(const FaceTerms& f, const V3<double>& pt, double& s, double& t,
                                  bool& ok) {
   const V3<double> dd = sub(f.o, pt);
@@ -444,7 +457,8 @@ DH_HD double vertex_face_regular(const FaceTerms& f, const V3<double>& pt, doubl
   const double quad = s * (a * s + b * t + 2.0 * d) + t * (b * s + c * t + 2.0 * e) + ff;
   const double line = (useE ? e : d) * p + ff;
   const double sqr = ((useE || useD) && num < den) ? line : quad;
-  return sqrt_regular(fmax(sqr, 0.0), ok);
+  ok &= !r0 || f.inside;
+  return fma(sqr, 0.0, sqrt_regular(fmax(sqr, 0.0)));  // NaN stays, which fmax drops
 }
 
 // Forgets what the compiler has derived from a triangle's first vertex, so
@@ -462,10 +476,19 @@ DH_HD void feature_fence() {
 #endif
 }
 
-// The features of a regular pair; false (and nothing in `best`) for others.
+// Whether `ok` holds for every lane of the wave (on the host: for this pair).
+DH_HD bool whole_wave(bool ok) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __all(ok);
+#else
+  return ok;
+#endif
+}
+
+// The features of a regular pair; false (and `best` to be ignored) for others.
 DH_HD bool bf_features_regular(Tri<double> A, Tri<double> B, BfBest<double>& best) {
   bool ok = true;
-  double least = 1E300, sum = 0.0;
+  double least = 1E300, most = 0.0;  // fmin and fmax skip NaN
   double ssmin = 1E+30, ssc = 0.0, ttc = 0.0, ptmin = 1E+30, ss = 0.0, tt = 0.0;
   int ssid = 0, id = 0;
   V3<double> v[3];
@@ -474,23 +497,24 @@ DH_HD bool bf_features_regular(Tri<double> A, Tri<double> B, BfBest<double>& bes
   for (int m = 0; m < 3; ++m) {
     v[m] = sub(B.v[m], B.v[m == 2 ? 0 : m + 1]);
     c[m] = dot(v[m], v[m]);
-    least = fmin(least, c[m]);
-    sum = sum + c[m];
+    const V3<double> u = sub(A.v[m], A.v[m == 2 ? 0 : m + 1]);
+    const double a = fma(u.x, u.x, fma(u.y, u.y, u.z * u.z));  // dot(u, u) but for rounding
+    least = fmin(least, fmin(a, c[m]));
+    most = fmax(most, fmax(a, c[m]));
   }
+  if (!whole_wave(least >= 1.0001E-30 && most < 0x1p179)) return false;
   // A's vertices rotate through a loop that stays rolled (three turns put
   // them back), B's edges are unrolled
 #pragma unroll 1
   for (int k = 0; k < 9; k += 3) {
     const V3<double> u = sub(A.v[0], A.v[1]);
     const double a = dot(u, u);
-    least = fmin(least, a);
-    sum = sum + a;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
       feature_fence();
       const V3<double> w = sub(A.v[1], B.v[m == 2 ? 0 : m + 1]);
       double sc, tc;
-      const double dist = edge_edge_regular(u, a, v[m], c[m], w, sc, tc, ok);
+      const double dist = edge_edge_regular(u, a, v[m], c[m], w, sc, tc);
       const bool better = dist < ssmin;
       ssmin = better ? dist : ssmin;
       ssc = better ? sc : ssc;
@@ -508,7 +532,6 @@ DH_HD bool bf_features_regular(Tri<double> A, Tri<double> B, BfBest<double>& bes
   for (int f = 0; f < 2; ++f) {
     const FaceTerms face(f ? B : A);
     least = fmin(least, face.denom);
-    ok &= face.det >= 1E-60;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       feature_fence();
@@ -522,36 +545,21 @@ DH_HD bool bf_features_regular(Tri<double> A, Tri<double> B, BfBest<double>& bes
     }
   }
   best = {ssmin, ttc, ssc, ptmin, ss, tt, ssid, id};
-  const V3<double> ab = sub(A.v[0], B.v[0]);
-  return ok && least >= 1E-30 && sum + dot(ab, ab) < 0x1p180;
+  // a distance that sqrt_regular did not round is the least of its kind
+  ok &= (ssmin >= kSqrtLeast || ssmin == 0.0) && (ptmin >= kSqrtLeast || ptmin == 0.0);
+  return ok && least >= 1E-30;
 }
 
-// kGeneral: no regular path (see bf_solver_general).
-template <bool kGeneral>
-DH_HD void bf_features_any(const Tri<double>& A, const Tri<double>& B, BfBest<double>& best) {
-  if (kGeneral || !bf_features_regular(A, B, best)) bf_features(A, B, best);
-}
-
-template <bool kGeneral>
-DH_HD void bf_features_any(const Tri<float>& A, const Tri<float>& B, BfBest<float>& best) {
-  bf_features(A, B, best);
-}
-
-// bfSolver: closest points P on A and Q on B.  Returns true when the
-// edge-edge result is kept (ptmin > ssmin, bf.cpp:1102).  With kZoltan the
-// output stage is that of zoltan/bf.cpp, whose switch cases 1 fall through
-// into cases 2 (zoltan/bf.cpp:527-559, 907-925): edge-edge feature 1 takes
-// its Q from B's edge 2->0 with feature 1's parameter, vertex-face feature 1
-// reports B's vertex 2.
-template <typename T, bool kZoltan = false, bool kGeneral = false>
-DH_HD bool bf_solver_ids(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q, int& ssid_out,
-                         int& id_out) {
-  BfBest<T> best;
-  bf_features_any<kGeneral>(A, B, best);
+// The closest points of the better feature; true when it is the edge-edge one
+// (ptmin > ssmin, bf.cpp:1102).  With kZoltan the output stage is that of
+// zoltan/bf.cpp, whose switch cases 1 fall through into cases 2
+// (zoltan/bf.cpp:527-559, 907-925): edge-edge feature 1 takes its Q from B's
+// edge 2->0 with feature 1's parameter, vertex-face feature 1 reports B's
+// vertex 2.
+template <typename T, bool kZoltan = false>
+DH_HD bool bf_points(const Tri<T>& A, const Tri<T>& B, const BfBest<T>& best, V3<T>& P, V3<T>& Q) {
   const int ssid = best.ssid, id = best.id;
   const T ssc = best.ssc, ttc = best.ttc, ss = best.ss, tt = best.tt;
-  ssid_out = ssid;
-  id_out = id;
   if (best.ptmin > best.ssmin) {
     const int k = ssid / 3, m = (kZoltan && ssid == 1) ? 2 : ssid - 3 * (ssid / 3);
     // register selects instead of dynamic indexing (keeps Tri out of scratch)
@@ -575,6 +583,27 @@ DH_HD bool bf_solver_ids(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q, i
   return false;
 }
 
+// bfSolver: closest points P on A and Q on B, and the least features of both
+// kinds.  Returns true when the edge-edge result is kept.
+template <bool kZoltan = false>
+DH_HD bool bf_solver_ids(const Tri<double>& A, const Tri<double>& B, V3<double>& P, V3<double>& Q,
+                         int& ssid_out, int& id_out) {
+  BfBest<double> best;
+  if (!bf_features_regular(A, B, best)) bf_features(A, B, best);
+  ssid_out = best.ssid;
+  id_out = best.id;
+  return bf_points<double, kZoltan>(A, B, best, P, Q);
+}
+
+DH_HD bool bf_solver_ids(const Tri<float>& A, const Tri<float>& B, V3<float>& P, V3<float>& Q,
+                         int& ssid_out, int& id_out) {
+  BfBest<float> best;
+  bf_features(A, B, best);
+  ssid_out = best.ssid;
+  id_out = best.id;
+  return bf_points(A, B, best, P, Q);
+}
+
 template <typename T>
 DH_HD bool bf_solver(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q) {
   int ssid, id;
@@ -583,14 +612,14 @@ DH_HD bool bf_solver(const Tri<T>& A, const Tri<T>& B, V3<T>& P, V3<T>& Q) {
 
 // The same by the general path alone, for the detection without the survivor
 // queue: its few survivors per item wait for loads and barriers rather than
-// for instructions, while the particles of a run that has left all bounds
-// (NaN, or so far out that their triangles round to lines) pair with every
-// other and would take both paths (the lattice's 2,000 steps: 0.178 ms a step,
-// 0.23 with both).
+// for instructions, while the particles of a run that has left all bounds (so
+// far out that their triangles round to lines and points) pair with every
+// other.
 DH_HD bool bf_solver_general(const Tri<double>& A, const Tri<double>& B, V3<double>& P,
                              V3<double>& Q) {
-  int ssid, id;
-  return bf_solver_ids<double, false, true>(A, B, P, Q, ssid, id);
+  BfBest<double> best;
+  bf_features(A, B, best);
+  return bf_points(A, B, best, P, Q);
 }
 
 // |Q-P| in the caller's order (bf.cpp:117, contactpoint.cpp:157-159).
@@ -916,30 +945,32 @@ DH_HD T dot4(const T a[4], const T b[4]) {
   return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
 }
 
-// penaltySolver(..., bool& failed): `iters` fixed steps (4 in the reference),
-// regularisation x1e4 after every step, `failed` from the last step.
+// penaltySolver(..., bool& failed): `iters` >= 1 fixed steps (4 in the
+// reference), regularisation x1e4 after every step, `failed` from the last
+// step.  By step_regular where it takes the pair.  A pair that regular() refuses
+// (NaN, extreme sizes) sends its whole wave to step(), so that no wave pays for
+// both (2 in 100 pairs with a NaN, 2^20 pairs: 78 us with both, 60 by step()
+// alone); `regular` (may be null) says which way a pair went.
 template <typename T>
 DH_HD bool penalty_fixed(const Tri<T>& A, const Tri<T>& B, const T x0[4], int iters, T max_err,
-                         V3<T>& P, V3<T>& Q, T xo[4]) {
+                         V3<T>& P, V3<T>& Q, bool* regular = nullptr) {
   Penalty<T> pen;
   pen.setup(A, B);
   T x[4] = {x0[0], x0[1], x0[2], x0[3]}, dx[4];
   T reg = pen.reg0;
-  bool failed = false, done = false;
-  if constexpr (sizeof(T) == 8) {
-    bool ok = pen.regular() && iters > 0;
-    int low = least_exponent(least_exponent(0, pen.h[2]), pen.h[3]);
+  bool ok = whole_wave(pen.regular());
+  int low = least_exponent(least_exponent(0, pen.h[2]), pen.h[3]);
 #pragma unroll 1
-    for (int i = 0; ok && i < iters; ++i) {
-      if (i > 0)
-        for (int q = 0; q < 4; ++q) x[q] -= dx[q];
-      ok = pen.step_regular(x, reg, dx, low) && ok;
-      reg = T(1E4) * reg;
-      for (int q = 0; q < 4; ++q) ok = fabs(x[q] - dx[q]) <= 0x1p20 && ok;
-    }
-    done = ok && low >= -600;
+  for (int i = 0; ok && i < iters; ++i) {
+    if (i > 0)
+      for (int q = 0; q < 4; ++q) x[q] -= dx[q];
+    ok = pen.step_regular(x, reg, dx, low) && ok;
+    reg = T(1E4) * reg;
+    for (int q = 0; q < 4; ++q) ok = fabs(x[q] - dx[q]) <= 0x1p20 && ok;
   }
-  if (!done) {
+  ok = ok && low >= -600;
+  if (regular) *regular = ok;
+  if (!ok) {
     for (int q = 0; q < 4; ++q) x[q] = x0[q];
     reg = pen.reg0;
 #pragma unroll 1
@@ -950,17 +981,9 @@ DH_HD bool penalty_fixed(const Tri<T>& A, const Tri<T>& B, const T x0[4], int it
       reg = T(1E4) * reg;
     }
   }
-  if (iters > 0) {
-    failed = (dot4(dx, dx) / dot4(x, x) > max_err * max_err);
-    for (int q = 0; q < 4; ++q) x[q] -= dx[q];
-  }
+  const bool failed = dot4(dx, dx) / dot4(x, x) > max_err * max_err;
+  for (int q = 0; q < 4; ++q) x[q] -= dx[q];
   pen.points(x, P, Q);
-  if (xo) {
-    xo[0] = x[0];
-    xo[1] = x[1];
-    xo[2] = x[2];
-    xo[3] = x[3];
-  }
   return failed;
 }
 

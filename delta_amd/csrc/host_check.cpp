@@ -27,7 +27,7 @@ extern "C" void hc_tri_pairs(int method, const double* soa, long n, double eps_t
     if (method == 0) {
       if (dh::bf_solver(A, B, p, q)) fl |= 4;
     } else if (method == 1 || method == 2) {
-      bool f = dh::penalty_fixed(A, B, x0, 4, max_err, p, q, (double*)nullptr);
+      bool f = dh::penalty_fixed(A, B, x0, 4, max_err, p, q);
       if (f) fl |= 1;
       if (method == 2 && f) {
         fl |= 2;
@@ -40,6 +40,19 @@ extern "C" void hc_tri_pairs(int method, const double* soa, long n, double eps_t
     Q[i] = q.x; Q[n + i] = q.y; Q[2 * n + i] = q.z;
     d[i] = dh::pq_dist(p, q);
     if (flags) flags[i] = fl;
+  }
+}
+
+// Which pairs take the regular paths: bit 0 the brute force, bit 1 the penalty.
+extern "C" void hc_regular(const double* soa, long n, double eps_total, unsigned char* out) {
+  const double x0[4] = {0.33, 0.33, 0.33, 0.33};
+  for (long i = 0; i < n; ++i) {
+    const Tri<double> A = load(soa, n, i, 0), B = load(soa, n, i, 9);
+    V3<double> p, q;
+    dh::BfBest<double> best;
+    bool pen = false;
+    dh::penalty_fixed(A, B, x0, 4, eps_total / 16.0, p, q, &pen);
+    out[i] = (dh::bf_features_regular(A, B, best) ? 1 : 0) | (pen ? 2 : 0);
   }
 }
 

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void k_tri_pairs_exact(const double* __restric
     if (bf_solver(A, B, p, q)) fl |= DH_FLAG_EDGE;
   } else if (METHOD == DH_PAIR_PENALTY64 || METHOD == DH_PAIR_HYBRID64) {
     const double x0[4] = {0.33, 0.33, 0.33, 0.33};
-    const bool failed = penalty_fixed(A, B, x0, 4, max_err, p, q, (double*)nullptr);
+    const bool failed = penalty_fixed(A, B, x0, 4, max_err, p, q);
     if (failed) fl |= DH_FLAG_FAILED;
     if (METHOD == DH_PAIR_HYBRID64 && failed) {
       fl |= DH_FLAG_RECHECK;

@@ -43,7 +43,7 @@ DH_HD int zoltan_bf(const Tri<double>& A, const Tri<double>& B, V3<double>& P, V
     if (n0 == 0 && m1 == 0 && m2 == 0) return -1;
   }
   int ssid, id;
-  return bf_solver_ids<double, true>(A, B, P, Q, ssid, id) ? 1 : 0;
+  return bf_solver_ids<true>(A, B, P, Q, ssid, id) ? 1 : 0;
 }
 
 // Hessian, regularisation seed and the square root of its trace scale.

@@ -179,3 +179,42 @@ def test_penalty_at_its_edges(method, code):
         Po, Qo, do, fo = oracle_pairs(code, soa)
         assert same_bits(d, do) and same_bits(P.ravel(), Po.ravel()), name
         assert same_bits(Q.ravel(), Qo.ravel()) and np.array_equal(f, fo), name
+
+
+def test_touching_pairs():
+    """Distance zero, and gaps on both sides of the least squared distance that
+    the regular path's root takes: the oracle's bits."""
+    from test_hostcheck import same_bits, touching_sets
+    for name, soa, _ in touching_sets(20000):
+        b = narrow.PairBatch.from_host(soa)
+        for method in ("bf64", "hybrid64", "bf64_exact"):
+            b.run(method)
+            P, Q, d, f = b.results()
+            Po, Qo, do, fo = oracle_pairs(narrow.METHODS[method], soa)
+            assert same_bits(d, do) and same_bits(P.ravel(), Po.ravel()), (name, method)
+            assert same_bits(Q.ravel(), Qo.ravel()) and np.array_equal(f, fo), (name, method)
+
+
+@pytest.mark.parametrize("share", [0.02, 1.0])
+@pytest.mark.parametrize("n", [1, 63, 65, 100001])
+def test_irregular_pairs_among_others(n, share):
+    """Edges of no length, in all pairs and in few of a wave's: the pairs next
+    to them leave the regular path with them."""
+    from test_hostcheck import same_bits
+    soa = narrow.PairBatch(n, seed=29).soa.download()
+    at = np.random.default_rng(n).random(n) < share
+    at[-1] = True
+    for c in range(3):
+        soa[3 * c + 2, at] = soa[3 * c + 1, at]
+    b = narrow.PairBatch.from_host(soa)
+    b.make_f32()
+    for method in ("bf64", "penalty64", "hybrid64", "bf64_exact", "mixed", "penalty_cert"):
+        b.run(method, eps_total=2e-2)
+        P, Q, d, f = b.results()
+        queued = method in ("mixed", "penalty_cert")  # rechecked: the brute force's
+        Po, Qo, do, fo = oracle_pairs(0 if queued else narrow.METHODS[method], soa, 2e-2)
+        at = (f & 2) != 0 if queued else np.ones(n, bool)
+        assert same_bits(d[at], do[at]), method
+        assert same_bits(P[:, at].ravel(), Po[:, at].ravel()), method
+        assert same_bits(Q[:, at].ravel(), Qo[:, at].ravel()), method
+        assert np.array_equal(f[at] & ~np.uint8(2) if queued else f, fo[at]), method

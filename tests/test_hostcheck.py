@@ -443,6 +443,62 @@ def test_penalty_at_its_edges(hc):
             assert np.array_equal(outs[0][3], outs[1][3]), (name, method)
 
 
+def touching_sets(n, seed=8):
+    """Pairs at distance zero, with lines for faces and with a NaN, which are
+    regular, edges of no length, and gaps of 2^-k about the least root of the
+    regular path (2^-350); whether they are regular (None: some)."""
+    rng = np.random.default_rng(seed)
+    A = rng.integers(-64, 65, (n, 3, 3)) / 8.0 + rng.integers(-64, 65, (n, 3, 3)) / 1024.0
+    B = rng.uniform(-8, 8, (n, 3, 3))
+    V = B.copy(); V[:, 0] = A[:, 1]
+    yield "shared vertex", soa_of(A, V), True
+    V = B.copy(); V[:, :2] = A[:, 1:]
+    yield "shared edge", soa_of(A, V), True
+    yield "the same triangle", soa_of(A, A[:, [2, 0, 1]]), True
+    V = B.copy(); V[:, 2] = 0.5 * A[:, 0] + 0.5 * A[:, 2]
+    yield "vertex on an edge", soa_of(A, V), True
+    V = B.copy(); V[:, 1] = 0.25 * A[:, 0] + 0.25 * A[:, 1] + 0.5 * A[:, 2]
+    yield "vertex on a face", soa_of(A, V), True
+    F = A.copy(); F[:, 2] = F[:, 0] + rng.uniform(-1, 2, (n, 1)) * (F[:, 1] - F[:, 0])
+    yield "a face that is a line", soa_of(F, B), True
+    F = A.copy(); F.reshape(n, 9)[np.arange(n), rng.integers(0, 9, n)] = np.nan
+    yield "a NaN", soa_of(F, B), True
+    yield "far apart", soa_of(A, B + 10.0 ** rng.uniform(10, 300, (n, 1, 1)) * [1, 0, 0]), None
+    F = A.copy(); F[:, 2] = F[:, 1]
+    yield "a vertex twice", soa_of(F, B), False
+    F, V = A.copy(), B.copy()
+    F[:, :, 2] = 0.0
+    V[:, 0, :2] = F[:, 0, :2]
+    V[:, :, 2] = 2.0 ** -rng.integers(300, 349, n)[:, None]
+    yield "gaps of 2^-300 to 2^-348", soa_of(F, V), True
+    V = V.copy()
+    V[:, :, 2] = 2.0 ** -rng.integers(352, 400, n)[:, None].astype(float)
+    yield "gaps of 2^-352 to 2^-399", soa_of(F, V), False
+    V = V.copy()
+    V[:, :, 2] = 2.0 ** -rng.integers(345, 1074, n)[:, None].astype(float)
+    yield "gaps of 2^-345 to 2^-1073", soa_of(F, V), None
+
+
+def test_touching_pairs(hc):
+    """Distance zero and next to it: the oracle's bits, by the regular path
+    unless a squared distance is below its least."""
+    n = 20000
+    for name, s, regular in touching_sets(n):
+        outs = []
+        for lib, fn in ((ol.oracle(), "or_tri_pairs"), (hc, "hc_tri_pairs")):
+            P = np.zeros(3 * n); Q = np.zeros(3 * n); d = np.zeros(n); f = np.zeros(n, np.uint8)
+            getattr(lib, fn)(0, ol.dptr(s), C.c_long(n), C.c_double(2e-4), ol.dptr(P),
+                             ol.dptr(Q), ol.dptr(d), f.ctypes.data_as(C.c_void_p))
+            outs.append((P, Q, d, f))
+        assert all(same_bits(a, b) for a, b in zip(outs[0][:3], outs[1][:3])), name
+        assert np.array_equal(outs[0][3], outs[1][3]), name
+        took = np.zeros(n, np.uint8)
+        hc.hc_regular(ol.dptr(s), C.c_long(n), C.c_double(2e-4), took.ctypes.data_as(C.c_void_p))
+        share = (took & 1).mean()  # whole numbers make an edge of no length now and then
+        if regular is not None:
+            assert share > 0.99 if regular else share < 0.01, (name, share)
+
+
 @pytest.mark.parametrize("rows,cols,tiles", [
     (1, 1, 1), (1, 1, 64), (7, 36, 3), (16, 16, 1), (16, 16, 2), (17, 15, 5), (80, 80, 12),
     (1, 100000, 7), (100000, 1, 7), (300, 255, 3), (300, 256, 3), (300, 257, 3), (0, 5, 4), (5, 0, 4),
