@@ -20,6 +20,7 @@
 #include "exact_math.hpp"
 #include "gjk.hpp"
 #include "pair_range.hpp"
+#include "queue_shape.hpp"
 #include "runtime.hpp"
 
 namespace dh {
@@ -97,20 +98,24 @@ struct DetectArgs {
   const double* bbox;
   int nstats;  // counters per tile: kBfStats (DH_BF) or kTileStats
   // Survivor queue of a DH_BF launch (null: every item solves its own
-  // survivors).  Wave r of k_detect_wave appends its items' survivors to its
-  // own region queue[r * rcap ..] and leaves their number in rcount[r], so
-  // that no wave waits for a counter that all share.  An item that cannot
-  // queue goes to `deferred`, for a launch that runs those items in full,
-  // taking its items from item_list.
+  // survivors), in segments: one of rcap entries for every wave of
+  // k_detect_wave, so that no wave waits for a counter that all share, and
+  // behind those the blocks of the pool.  An item that does not fit what is
+  // left of its wave's segment takes as many blocks in a row as it needs, which
+  // are the wave's segment from then on.  rcount[r] is segment r's number of
+  // entries (one of several blocks goes by the first block's number; the
+  // others' stays 0).  An item that cannot queue goes to `deferred`, for a
+  // launch that runs those items in full, taking its items from item_list.
   int4* queue;  // {item, triangle of A, triangle of B, iA | iB << 16}
-  int rcap, regions;
+  QueueShape shape;
+  int most;        // entries of an item that may queue
+  unsigned* pool;  // blocks taken of each part, kPoolStride apart
   int* rcount;
-  int* rwant;  // most entries that a region had to hold, when more than rcap
   // contacts of the queue's entries, in the entries' order, from the place of
-  // the region's first entry; region r's number in rcount[regions + r]
+  // the segment's first entry; segment r's number in rcount[segments + r]
   struct QueueRecord* rec;
-  int heavy;    // regions with more entries are solved in four parts
-  int* rparts;  // a heavy region's: each part's contacts and rank base
+  int heavy;    // segments with more entries are solved in four parts
+  int* rparts;  // a heavy segment's: each part's contacts and rank base
   int* deferred;
   unsigned* ndeferred;
   // Items k_lane_cull leaves for k_detect_wave
@@ -118,6 +123,7 @@ struct DetectArgs {
   unsigned* nwlist;
   const int* item_list;
   const unsigned* nitems_dev;  // with item_list: its length (else the launch's)
+  unsigned* item_next;         // counts the items taken after each workgroup's first
   int fp32_screen;             // k_queue_solve screens in binary32 first
   // item_skip[item] != 0: k_chunk_cull culled the item and wrote its
   // counters (a launch of DH_BF without the survivor queue skips it)
@@ -767,7 +773,8 @@ __device__ __forceinline__ void detect_item(const DetectArgs& g, const int item)
 }
 
 // Persistent over the items: workgroup b takes items b, b + gridDim.x, ...
-// (with as many workgroups as items, one each).  Pairs of very uneven cost
+// (with as many workgroups as items, one each), or with item_next the next one
+// that no workgroup has yet.  Pairs of very uneven cost
 // (a 2,048-triangle funnel against 20-triangle particles) share the
 // workgroups of one launch.  The brute force is held to 168 registers
 // (three waves per SIMD; a few spill), which its latency-bound item loop
@@ -777,9 +784,17 @@ __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(M == DH_BF ? 3 : 1))) void k_detect(DetectArgs g, int items) {
   if (g.item_list && g.nitems_dev && static_cast<int>(*g.nitems_dev) < items)
     items = static_cast<int>(*g.nitems_dev);
-  for (int t = blockIdx.x; t < items; t += gridDim.x) {
+  __shared__ int next;
+  for (int t = blockIdx.x; t < items;) {
     detect_item<M>(g, g.item_list ? g.item_list[t] : t);
     __syncthreads();  // the next item reuses the workgroup's LDS
+    if (g.item_next) {
+      if (threadIdx.x == 0) next = static_cast<int>(gridDim.x + atomicAdd(g.item_next, 1u));
+      __syncthreads();
+      t = next;
+    } else {
+      t += gridDim.x;
+    }
   }
 }
 
@@ -943,17 +958,19 @@ __device__ __forceinline__ double box_gap(const double* loA, const double* hiA, 
 // other particle's box and bounding sphere are kept, in order, in the wave's
 // LDS (the rows of a large A chunk by chunk, those of far chunks unread); the
 // pairs of kept rows and columns whose boxes are within the margin are
-// appended, in row-major order, to the wave's region of the survivor queue.
+// appended, in row-major order, to the wave's segment of the survivor queue.
 // Items with more than kWaveBoxes kept rows and columns, or more survivors
-// than the region has room for, are deferred to the full kernel.  Same
-// survivors and counters as detect_item's box test.
+// than an item may queue or the pool has left, are deferred to the full
+// kernel.  The survivors are fewer than detect_item's box test leaves (that one
+// does not know the bounding spheres), so pairs_culled depends on the path an
+// item took; the contacts do not.
 // It is bound by the latency of an item's loads, so it holds little: 16 waves
 // per CU.  Separating axes are tested in k_queue_solve instead, with every
 // lane busy (here they took 161 registers, 9 waves per CU, for some 10 to 40
 // survivors at a time), and the other particle's box from the broad phase
 // takes the place of the union of its triangles' boxes (144 lane shuffles per
 // item).  What it cost before was an atomic per item on one queue counter,
-// some 10 ns each: 610 us for the hopper's 1.9e5 pairs, 87 us with a region
+// some 10 ns each: 610 us for the hopper's 1.9e5 pairs, 87 us with a segment
 // per wave (8 workgroups per CU; 6 per CU: 100 us).
 __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectArgs g) {
   __shared__ double boxes[kWavesPerGroup][kWaveBoxes * 6];
@@ -962,8 +979,9 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   double* bx = boxes[w];
   const int region = blockIdx.x * kWavesPerGroup + w;
-  int4* queue = g.queue + static_cast<long long>(region) * g.rcap;
-  int used = 0, want = 0;
+  int segment = region, cap = g.shape.rcap, used = 0;
+  int4* queue = g.queue + static_cast<long long>(region) * g.shape.rcap;
+  bool dry = false;  // the pool has nothing left
   const int nw = static_cast<int>(*g.nwlist);
   for (int j = region; j < nw; j += gridDim.x * kWavesPerGroup) {
     const WaveItem it = g.wlist[j];
@@ -1010,6 +1028,14 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
 #pragma unroll
     for (int q = 0; q < 6; ++q) mag = fmax(mag, fmax(fabs(other[0][q]), fabs(other[1][q])));
     const double reach = margin * (1.0 + 0x1p-20) + mag * 0x1p-40;
+    if (margin > 0.0 && mag * 0x1p-26 > margin) {
+      // coordinates of more than 13 km at a margin of 0.2 mm: particles that have
+      // grown past all bounds, as an unstable run's do, keep a fifth of their
+      // pairs and more through all tests, and k_detect takes those with full
+      // lanes (lattice after 1,000 such steps: 143 us, 310 through the queue)
+      if (lane == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = it.item;
+      continue;
+    }
     // keeps the triangles of [t, t + 64) and below `end` that are on side's
     // own; false when the LDS is full
     int kept = 0;
@@ -1085,12 +1111,31 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
     for (int t = 0; t < it.nB && fits && na > 0; t += 64) fits = scan(1, it.oB, t, it.nB);
     const int nc = kept - na, tested = na * nc;
     wave_lds_fence();
-    // survivors in row-major order over the kept rows and columns
+    // Survivors in row-major order over the kept rows and columns, 64 pairs a
+    // round (at most 100): put() writes a round's.  Lane l keeps the survivors
+    // of rounds l and 64 + l for an item that turns out not to fit and is
+    // written again, to blocks of the pool that hold it.
+    unsigned long long rounds[2] = {0, 0};
+    const int step_r = nc > 0 ? 64 / nc : 0, step_c = 64 - step_r * nc;
+    int ra = nc > 0 ? lane / nc : 0, cb = lane - ra * nc;
+    auto put = [&](unsigned long long m, int at) {
+      at += lane_prefix(m);
+      if ((m >> lane & 1) && at < cap) {
+        const int r = act[w][ra], c = act[w][na + cb];
+        queue[at] = make_int4(it.item, it.oA + r, it.oB + c,
+                              static_cast<int>(static_cast<unsigned>(r) |
+                                               (static_cast<unsigned>(c) << 16)));
+      }
+      ra += step_r;
+      cb += step_c;
+      if (cb >= nc) {
+        cb -= nc;
+        ++ra;
+      }
+    };
     int S = 0;
-    if (fits && tested > 0) {
-      const int step_r = 64 / nc, step_c = 64 - step_r * nc;
-      int ra = lane / nc, cb = lane - ra * nc;
-      for (int f = lane; f - lane < tested; f += 64) {
+    if (fits)
+      for (int f = lane, k = 0; f - lane < tested; f += 64, ++k) {
         bool keep = false;
         if (f < tested) {
           const double* a = bx + 6 * ra;
@@ -1098,24 +1143,45 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
           keep = !(box_gap(a, a + 3, b, b + 3) > reach);
         }
         const unsigned long long m = __ballot(keep);
-        const int at = used + S + lane_prefix(m);
-        if (keep && at < g.rcap) {
-          const int r = act[w][ra], c = act[w][na + cb];
-          queue[at] = make_int4(it.item, it.oA + r, it.oB + c,
-                                static_cast<int>(static_cast<unsigned>(r) |
-                                                 (static_cast<unsigned>(c) << 16)));
-        }
+        if (lane == (k & 63)) rounds[k >> 6] = m;
+        put(m, used + S);
         S += __popcll(m);
-        ra += step_r;
-        cb += step_c;
-        if (cb >= nc) {
-          cb -= nc;
-          ++ra;
+      }
+    if (used + S > cap && S <= g.most && !dry) {
+      const int n = (S + g.shape.block - 1) / g.shape.block;
+      int first = -1, part = 0;
+      while (first < 0) {
+        // the parts with room, from the workgroup's own on
+        const int q = (static_cast<int>(blockIdx.x) + lane) % kPoolParts;
+        const bool room = lane < kPoolParts &&
+                          static_cast<int>(__hip_atomic_load(&g.pool[kPoolStride * q], __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT)) + n <= g.shape.blocks;
+        const unsigned long long m = __ballot(room);
+        if (!m) break;
+        part = __shfl(q, __builtin_ctzll(m));
+        if (lane == 0) first = static_cast<int>(atomicAdd(&g.pool[kPoolStride * part], static_cast<unsigned>(n)));
+        first = __shfl(first, 0);
+        // another wave took them: the count only grows, so the loop ends
+        if (first + n > g.shape.blocks) first = -1;
+      }
+      dry = first < 0;
+      if (!dry) {
+        if (lane == 0) g.rcount[segment] = used;
+        segment = g.shape.pool_segment(part, first);
+        queue = g.queue + g.shape.place(segment);
+        cap = n * g.shape.block;
+        used = 0;
+        ra = lane / nc;
+        cb = lane - ra * nc;
+        for (int k = 0, at = 0; 64 * k < tested; ++k) {
+          const unsigned long long mine = k < 64 ? rounds[0] : rounds[1];
+          const unsigned long long m = __shfl(mine, k & 63);
+          put(m, at);
+          at += __popcll(m);
         }
       }
     }
-    want += S;
-    if (!fits || used + S > g.rcap) {
+    if (!fits || used + S > cap) {
       if (lane == 0) g.deferred[atomicAdd(g.ndeferred, 1u)] = it.item;
     } else {
       used += S;
@@ -1125,10 +1191,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
     }
     wave_lds_fence();  // the next item overwrites the wave's LDS
   }
-  if (lane == 0) {
-    g.rcount[region] = used;
-    if (want > g.rcap) atomicMax(g.rwant, want);
-  }
+  if (lane == 0) g.rcount[segment] = used;
 }
 
 // The stats slot of a tile counter.
@@ -1461,13 +1524,13 @@ __global__ __launch_bounds__(256) void k_scatter(const dh_contact* __restrict__ 
   if (blockIdx.x == 0) report_write(report, threadIdx.x, 256);
 }
 
-// Survivor queue, pass 2: every wave takes one region of k_detect_wave's through
+// Survivor queue, pass 2: every wave takes one segment of k_detect_wave's through
 // the plane test, the edge-pair axes (and, when tuned on, the binary32 screen)
 // and bfSolver.  What a test leaves waits in a list in LDS until 64 entries
 // are there, so that each stage runs with every lane busy although the one
 // before it drops most.  The entries stay in order, so the contacts of an item
 // come out in row-major order and their rank is a running count, and the
-// records of a region follow each other without a counter that all waves
+// records of a segment follow each other without a counter that all waves
 // share.  Bound by vector issue: 152 us for the hopper's 1.78e6 entries and
 // 644,000 contacts (a lane per entry, with its scan, reservation and unordered
 // contacts: 250 us); four waves per SIMD would spill (166 us).
@@ -1601,15 +1664,15 @@ __device__ __forceinline__ StreamEnds solve_stream(const DetectArgs& g, int4* __
   return {out, first, nfirst, carry_item, carry};
 }
 
-// The part of a heavy region's n entries that each of a workgroup's waves
+// The part of a heavy segment's n entries that each of a workgroup's waves
 // takes, in whole rounds of 64.
-__device__ __forceinline__ int region_part(int n) { return (n + 255) / 256 * 64; }
+__device__ __forceinline__ int segment_part(int n) { return (n + 255) / 256 * 64; }
 
-// A wave per region; then the workgroup's four waves share each of its regions
+// A wave per segment; then the workgroup's four waves share each of its segments
 // with more than g.heavy entries, so that one pair of particles in deep
 // contact does not keep a single wave at work (the funnel's heaviest pairs
 // have 400 contacts: 100 us without, 69 us with).  An item that goes on from
-// one part of a region to the next has the later part's ranks raised by the
+// one part of a segment to the next has the later part's ranks raised by the
 // contacts before (applied in k_queue_write).
 template <bool SCREEN, bool kFilter>
 __global__ __launch_bounds__(256, 3) void k_queue_solve(DetectArgs g) {
@@ -1617,80 +1680,102 @@ __global__ __launch_bounds__(256, 3) void k_queue_solve(DetectArgs g) {
   __shared__ StreamEnds ends[4];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  for (int p = -1; p < 4; ++p) {
-    // a workgroup's regions lie far apart: neighbours hold neighbouring pairs,
-    // which are heavy together
-    const int r = (p < 0 ? w : p) * gridDim.x + blockIdx.x;
-    const int total = r < g.regions ? g.rcount[r] : 0;
-    if (p >= 0 && total <= g.heavy) continue;  // the same for the whole workgroup
-    int begin = 0, n = total <= g.heavy ? total : 0;
-    if (p >= 0) {
-      const int part = region_part(total);
-      begin = w * part < total ? w * part : total;
-      n = total - begin < part ? total - begin : part;
+  // the workgroup's segments: four of the waves' own, then of the pool's.  They
+  // lie far apart: neighbours hold neighbouring pairs, which are heavy together
+  const int grid = static_cast<int>(gridDim.x), b = static_cast<int>(blockIdx.x);
+  const int most = 4 + (g.shape.segments() - g.shape.regions + grid - 1) / grid;
+  auto number = [&](int i) { return i < 4 ? i * grid + b : g.shape.regions + (i - 4) * grid + b; };
+  auto count = [&](int i) {
+    const int r = number(i);
+    return i < most && r < (i < 4 ? g.shape.regions : g.shape.segments()) ? g.rcount[r] : 0;
+  };
+  for (int i0 = 0; i0 < most; i0 += 64) {  // 64 of them at a time
+    unsigned long long light, heavy;       // the wave's; the same in all waves
+    {
+      const int entries = count(i0 + lane);
+      light = __ballot(entries > 0 && entries <= g.heavy && (lane & 3) == w);
+      heavy = __ballot(entries > g.heavy);
     }
-    const long long at = static_cast<long long>(r) * g.rcap + begin;
-    const StreamEnds e = solve_stream<SCREEN, kFilter>(g, g.queue + at, n, g.rec + at, lists[w], lane);
-    if (p < 0) {
-      if (lane == 0 && r < g.regions && total <= g.heavy)
-        g.rcount[(kFilter ? 0 : g.regions) + r] = e.n;
-      continue;
-    }
-    if (lane == 0) ends[w] = e;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int item = -1, count = 0;
-      for (int q = 0; q < 4; ++q) {
-        const StreamEnds s = ends[q];
-        const int base = s.n > 0 && s.first == item ? count : 0;
-        int* c = g.rparts + 8 * static_cast<long long>(r) + 2 * q;
-        c[0] = s.n;
-        c[1] = base;
-        if (s.n == 0) continue;
-        if (base > 0) g.tile_count[s.first] = base + s.nfirst;
-        count = s.first == s.last ? base + s.nfirst : s.nlast;
-        item = s.last;
+    while (light | heavy) {
+      const bool shared = light == 0;
+      const int l = __builtin_ctzll(shared ? heavy : light);
+      if (shared) heavy &= heavy - 1;
+      else light &= light - 1;
+      const int r = number(i0 + l), total = g.rcount[r];
+      int begin = 0, n = total;
+      if (shared) {
+        const int part = segment_part(total);
+        begin = w * part < total ? w * part : total;
+        n = total - begin < part ? total - begin : part;
       }
+      const long long at = g.shape.place(r) + begin;
+      const StreamEnds e = solve_stream<SCREEN, kFilter>(g, g.queue + at, n, g.rec + at, lists[w], lane);
+      if (!shared) {
+        if (lane == 0) g.rcount[(kFilter ? 0 : g.shape.segments()) + r] = e.n;
+        continue;
+      }
+      if (lane == 0) ends[w] = e;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        int item = -1, count = 0;
+        for (int q = 0; q < 4; ++q) {
+          const StreamEnds s = ends[q];
+          const int base = s.n > 0 && s.first == item ? count : 0;
+          int* c = g.rparts + 8 * static_cast<long long>(r) + 2 * q;
+          c[0] = s.n;
+          c[1] = base;
+          if (s.n == 0) continue;
+          if (base > 0) g.tile_count[s.first] = base + s.nfirst;
+          count = s.first == s.last ? base + s.nfirst : s.nlast;
+          item = s.last;
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
   }
 }
 
-// The records of entries that another kernel has solved (flags[e], and the
-// points pq[6e..] of those that emit), in order.
-__global__ __launch_bounds__(256) void k_queue_record(DetectArgs g, const int* __restrict__ flags,
-                                                      const double* __restrict__ pq) {
+// The records of entries that another kernel has solved and left in the
+// records' places by entry (`rank` of those that emit is not 0), moved to the
+// front in order.
+__global__ __launch_bounds__(256) void k_queue_record(DetectArgs g) {
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.x * 4 + static_cast<int>(threadIdx.x >> 6);
-  if (r >= g.regions) return;
-  const long long at = static_cast<long long>(r) * g.rcap;
+  if (r >= g.shape.segments()) return;
+  const long long at = g.shape.place(r);
   const int n = g.rcount[r];
   int out = 0, carry_item = -1, carry = 0;
   for (int base = 0; base < n; base += 64) {
     const long long e = at + base + lane;
-    const bool emit = base + lane < n && flags[e] != 0;
+    const bool emit = base + lane < n && g.rec[e].rank != 0;
     int4 en = make_int4(-1, 0, 0, 0);
-    if (emit) en = g.queue[e];
+    double pq[6] = {};
+    if (emit) {
+      en = g.queue[e];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) pq[c] = g.rec[e].pq[c];
+    }
     const int rank = item_rank(g, emit, en.x, lane, carry_item, carry);
     const unsigned long long m = __ballot(emit);
-    if (emit) {
+    if (emit) {  // every record up to here has been read: the places are free
       QueueRecord q;
       q.item = en.x;
       q.tris = en.w;
       q.rank = rank;
       q.pad_ = 0;
-      for (int c = 0; c < 6; ++c) q.pq[c] = pq[6 * e + c];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) q.pq[c] = pq[c];
       g.rec[at + out + lane_prefix(m)] = q;
     }
     out += __popcll(m);
   }
-  if (lane == 0) g.rcount[g.regions + r] = out;
+  if (lane == 0) g.rcount[g.shape.segments() + r] = out;
 }
 
 // Pass 3, after the pairs' offsets: the records' contacts, each at its place,
 // and those that the full kernel left in `temp` (*in_temp of them).  A
-// workgroup per region: a record waits for a chain of loads, which a wave per
-// region went through once per 64 records (hopper of 15,651 spheres 51 us,
+// workgroup per segment: a record waits for a chain of loads, which a wave per
+// segment went through once per 64 records (hopper of 15,651 spheres 51 us,
 // 46 us now, near the copy rate).
 __device__ __forceinline__ long long contact_place(const DetectArgs& g, int item, int rank,
                                                    const long long* __restrict__ offs) {
@@ -1710,10 +1795,10 @@ __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long lo
   const bool heavy = total > g.heavy;
   for (int p = 0; p < (heavy ? 4 : total > 0 ? 1 : 0); ++p) {
     const int* c = g.rparts + 8 * static_cast<long long>(r) + 2 * p;
-    const int n = heavy ? c[0] : g.rcount[g.regions + r];
+    const int n = heavy ? c[0] : g.rcount[g.shape.segments() + r];
     if (n == 0) continue;
     const QueueRecord* rec =
-        g.rec + static_cast<long long>(r) * g.rcap + (heavy ? p * region_part(total) : 0);
+        g.rec + g.shape.place(r) + (heavy ? p * segment_part(total) : 0);
     const int base = heavy ? c[1] : 0, first = rec[0].item;
     for (int e = threadIdx.x; e < n; e += 256) {
       const QueueRecord q = rec[e];
@@ -1745,15 +1830,15 @@ __global__ __launch_bounds__(256) void k_queue_write(DetectArgs g, const long lo
   if (blockIdx.x == 0) report_write(report, threadIdx.x, 256);
 }
 
-int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
+int queue_learned(const int4* queue, const int* pairs, int tiles, const QueueShape& shape,
                   const int* rcount, const double* x, const double* y, const double* z,
-                  const double* eps, int* flags, double* pq, hipStream_t st);
+                  const double* eps, int* flags, int flag_stride, double* pq, int pq_stride,
+                  hipStream_t st);
 int queue_learned_reserve(long long n);
 
 struct DetectScratch {
   DevBuf temp, counter, stats, error, counts, offs, sums, tiles, tstats, iskip, tmax;
-  DevBuf queue, qrec, qcounts, rcount, rparts, deferred, wlist, found, qflags, qpq;
-  int rwant = 0;  // what a region had to hold in earlier eager calls
+  DevBuf queue, qrec, qcounts, rparts, deferred, wlist, found;
 };
 static DetectScratch g_scratch;
 
@@ -1890,64 +1975,78 @@ static int tiles_for(long long npairs, int method) {
   return static_cast<int>(t < 1 ? 1 : (t > cap ? cap : t));
 }
 
-// The survivor queue's shape for `items` items: a region per wave of
-// k_detect_wave's persistent grid (as many as the CUs hold at once), 16 entries
-// per item over the regions and at least 1,024 in each, or what earlier calls
-// needed.
-// With fewer than 16 items per region, those with more than 256 entries are
-// shared by four waves in k_queue_solve; with more, the regions are alike.
+// Entries of the survivor queue for `items` items and `cap` contacts: 16 per item
+// and 65,536, or 2.5 per contact where that is more (packings leave 2.1 to 2.9
+// survivors per contact), the latter up to 2^24.  What does not fit is deferred.
+static long long queue_total(long long items, long long cap) {
+  const long long by_items = 16 * items + 65536, contacts = cap < 1ll << 24 ? cap : 1ll << 24;
+  const long long by_contacts = 5 * contacts / 2 < 1ll << 24 ? 5 * contacts / 2 : 1ll << 24;
+  const long long n = by_items > by_contacts ? by_items : by_contacts;
+  return n < 1ll << 28 ? n : 1ll << 28;
+}
+
+// The queue's shape: half of the entries, and at least 1,024 each, are the
+// waves' own segments (as many waves as the CUs hold at once; 335 MB), the
+// other half the pool.  (Own segments of 512 or 256 entries with the pool for
+// the rest: funnel fill's step 2 and 3 % slower, as a wave whose items go on in
+// the pool waits for it.)  With fewer than 16 items per wave, segments with more
+// than 256 entries are shared by four waves in k_queue_solve; with more, the
+// segments are alike.  An item may queue up to 2,048 entries, 1,024 where one
+// wave alone takes a segment through the learned decision.
 struct QueuePlan {
   unsigned groups;
-  int regions, rcap, heavy;
-  long long entries() const { return static_cast<long long>(regions) * rcap; }
+  QueueShape shape;
+  int heavy, most;
 };
 
-static QueuePlan queue_plan(long long items, int rwant) {
+static QueuePlan queue_plan(long long items, long long total, bool learned) {
   QueuePlan q;
   const long long wg = (items + kWavesPerGroup - 1) / kWavesPerGroup;
-  const long long most = static_cast<long long>(device_cus()) * 8;
-  q.groups = static_cast<unsigned>(wg < 1 ? 1 : (wg < most ? wg : most));
-  q.regions = static_cast<int>(q.groups) * kWavesPerGroup;
-  long long r = (16 * items + 65536) / q.regions;
-  if (r < 1024) r = 1024;
-  if (r < rwant) r = rwant;
-  const long long rmost = (1ll << 30) / q.regions;
-  q.rcap = static_cast<int>(r < rmost ? r : rmost);
-  q.heavy = items < 16ll * q.regions ? 256 : 0x7fffffff;
+  const long long waves = static_cast<long long>(device_cus()) * 8;
+  q.groups = static_cast<unsigned>(wg < 1 ? 1 : (wg < waves ? wg : waves));
+  q.shape.regions = static_cast<int>(q.groups) * kWavesPerGroup;
+  const long long half = total / 2, own = half / q.shape.regions / 64 * 64;
+  q.shape.rcap = static_cast<int>(own < 1024 ? 1024 : own);
+  const long long block = (half / 8192 + 63) / 64 * 64;
+  q.shape.block = static_cast<int>(block < 1024 ? 1024 : block);
+  const long long blocks = half / q.shape.block / kPoolParts;
+  q.shape.blocks = static_cast<int>(blocks < 1 ? 1 : blocks);
+  q.heavy = !learned && items < 16ll * q.shape.regions ? 256 : 0x7fffffff;
+  q.most = learned ? 1024 : 2048;
   return q;
 }
 
-// Places of the queue path's counters in g_scratch.qcounts.
-enum QueueCount : int { QC_WLIST = 0, QC_DEFERRED, QC_RWANT, kQueueCounts };
+// Places of the queue path's counters in g_scratch.qcounts: the lists' lengths,
+// the pool's parts, then the segments' entries and contacts.
+enum QueueCount : int {
+  QC_WLIST = 0, QC_DEFERRED, QC_NEXT, QC_POOL,
+  QC_SEGMENTS = QC_POOL + kPoolParts * kPoolStride
+};
+
+static int queue_counts(const QueuePlan& q) { return QC_SEGMENTS + 2 * q.shape.segments(); }
 
 // Buffers of the queue path (before a capture).
 static int queue_reserve(const QueuePlan& q, long long items, bool learned) {
   int rc;
-  if ((rc = g_scratch.queue.grow(sizeof(int4) * q.entries()))) return rc;
-  if ((rc = g_scratch.qrec.grow(sizeof(QueueRecord) * q.entries()))) return rc;
-  if ((rc = g_scratch.qcounts.grow(sizeof(unsigned) * kQueueCounts))) return rc;
-  if ((rc = g_scratch.rcount.grow(sizeof(int) * 2 * q.regions))) return rc;
-  if ((rc = g_scratch.rparts.grow(sizeof(int) * 8 * q.regions))) return rc;
+  if ((rc = g_scratch.queue.grow(sizeof(int4) * q.shape.entries()))) return rc;
+  if ((rc = g_scratch.qrec.grow(sizeof(QueueRecord) * q.shape.entries()))) return rc;
+  if ((rc = g_scratch.qcounts.grow(sizeof(unsigned) * queue_counts(q)))) return rc;
+  if ((rc = g_scratch.rparts.grow(sizeof(int) * 8 * q.shape.segments()))) return rc;
   if ((rc = g_scratch.deferred.grow(sizeof(int) * (items + 1)))) return rc;
   if ((rc = g_scratch.wlist.grow(sizeof(WaveItem) * (items + 1)))) return rc;
   if ((rc = g_scratch.found.grow(sizeof(unsigned long long)))) return rc;
-  if (learned) {
-    if ((rc = g_scratch.qflags.grow(sizeof(int) * q.entries()))) return rc;
-    if ((rc = g_scratch.qpq.grow(sizeof(double) * 6 * q.entries()))) return rc;
-    return queue_learned_reserve(q.entries());
-  }
-  return DH_OK;
+  return learned ? queue_learned_reserve(q.shape.entries()) : DH_OK;
 }
 
 static void queue_bind(DetectArgs& a, const QueuePlan& q) {
   unsigned* c = g_scratch.qcounts.as<unsigned>();
   a.queue = g_scratch.queue.as<int4>();
-  a.rcap = q.rcap;
-  a.regions = q.regions;
-  a.rcount = g_scratch.rcount.as<int>();
+  a.shape = q.shape;
+  a.most = q.most;
+  a.pool = c + QC_POOL;
+  a.rcount = reinterpret_cast<int*>(c + QC_SEGMENTS);
   a.rparts = g_scratch.rparts.as<int>();
   a.heavy = q.heavy;
-  a.rwant = reinterpret_cast<int*>(c + QC_RWANT);
   a.rec = g_scratch.qrec.as<QueueRecord>();
   a.deferred = g_scratch.deferred.as<int>();
   a.ndeferred = c + QC_DEFERRED;
@@ -1969,20 +2068,20 @@ static int queue_detect(const DetectArgs& a, const QueuePlan& q, unsigned items,
   DetectArgs f = a;
   f.item_list = a.deferred;
   f.nitems_dev = a.ndeferred;
+  f.item_next = g_scratch.qcounts.as<unsigned>() + QC_NEXT;
   // usually none to do: a grid for the capacity would cost a dispatch per item
   hipLaunchKernelGGL(k_detect<DH_BF>, items < 4 * cus ? items : 4 * cus, 256, 0, st, f,
                      static_cast<int>(items));
-  const unsigned grid = grid_for(q.regions, 4);
   const auto solve = learned ? (a.fp32_screen ? k_queue_solve<true, true> : k_queue_solve<false, true>)
                              : (a.fp32_screen ? k_queue_solve<true, false> : k_queue_solve<false, false>);
-  hipLaunchKernelGGL(solve, grid, 256, 0, st, a);
+  hipLaunchKernelGGL(solve, grid_for(q.shape.regions, 4), 256, 0, st, a);
   if (learned) {
     int rc;
-    if ((rc = queue_learned(a.queue, a.pairs, a.tiles, a.regions, a.rcap, a.rcount, a.x, a.y, a.z,
-                            a.eps, g_scratch.qflags.as<int>(), g_scratch.qpq.as<double>(), st)))
+    static_assert(sizeof(QueueRecord) == 64, "a record's strides below");
+    if ((rc = queue_learned(a.queue, a.pairs, a.tiles, a.shape, a.rcount, a.x, a.y, a.z, a.eps,
+                            &a.rec->rank, 16, a.rec->pq, 8, st)))
       return rc;
-    hipLaunchKernelGGL(k_queue_record, grid, 256, 0, st, a, g_scratch.qflags.as<int>(),
-                       g_scratch.qpq.as<double>());
+    hipLaunchKernelGGL(k_queue_record, grid_for(q.shape.segments(), 4), 256, 0, st, a);
   }
   DH_HIP_CHECK(hipGetLastError());
   return DH_OK;
@@ -2093,15 +2192,19 @@ static int detect_pairs_tiled(int method, const dh_geometry* geom, const int* pa
                                     geom) >= tuning().detect_queue_min_items);
   QueuePlan plan = {};
   if (queued) {
-    plan = queue_plan(nitems, g_scratch.rwant);
-    if (learned) plan.heavy = 0x7fffffff;
-    if ((rc = queue_reserve(plan, nitems, learned))) return rc;
+    // a shorter queue where the memory does not allow this one
+    for (long long total = queue_total(nitems, cap);; total /= 2) {
+      plan = queue_plan(nitems, total, learned);
+      if (!(rc = queue_reserve(plan, nitems, learned))) break;
+      if (total <= 65536) return rc;
+      (void)hipGetLastError();
+    }
     queue_bind(a, plan);
   }
   zero_async(ZeroRegions{{g_scratch.counter.as<unsigned>(), g_scratch.stats.as<unsigned>(),
                           g_scratch.error.as<unsigned>(),
                           queued ? g_scratch.qcounts.as<unsigned>() : nullptr},
-                         {2, 2 * ST_COUNT, 1, kQueueCounts}},
+                         {2, 2 * ST_COUNT, 1, queued ? queue_counts(plan) : 0}},
              st);
   const size_t shm_rows = 2 * kMaxRowTriangles * sizeof(int) + 8 + kMaxRowTriangles * 8;
   const unsigned items = static_cast<unsigned>(nitems);
@@ -2139,9 +2242,8 @@ static int detect_pairs_tiled(int method, const dh_geometry* geom, const int* pa
   report_add(report, g_scratch.error.ptr, 1);
   report_add(report, g_scratch.stats.ptr, 2 * ST_COUNT);
   if (queued) {
-    report_add(report, g_scratch.qcounts.ptr, kQueueCounts);
-    hipLaunchKernelGGL(k_queue_write, static_cast<unsigned>(plan.regions), 256, 0, st, a, offs, out, cap,
-                       a.counter, nullptr, report);
+    hipLaunchKernelGGL(k_queue_write, static_cast<unsigned>(plan.shape.segments()), 256, 0, st, a, offs,
+                       out, cap, a.counter, nullptr, report);
   } else {
     const long long wg = (cap + 255) / 256;
     hipLaunchKernelGGL(k_scatter, static_cast<unsigned>(wg < 1 ? 1 : (wg < 2048 ? wg : 2048)), 256,
@@ -2154,12 +2256,6 @@ static int detect_pairs_tiled(int method, const dh_geometry* geom, const int* pa
   std::memcpy(&total, report.mail, sizeof(total));
   std::memcpy(&err, report.mail + 2, sizeof(err));
   std::memcpy(st_host, report.mail + 3, sizeof(st_host));
-  if (queued) {
-    // the next call's regions hold this call's need
-    const long long want = report.mail[3 + 2 * ST_COUNT + QC_RWANT];
-    if (want > plan.rcap)
-      g_scratch.rwant = static_cast<int>(want + want / 4 < (1 << 29) ? want + want / 4 : 1 << 29);
-  }
   if (err == DE_REF_UB)
     return set_error(DH_ERR_REF_UB,
                      "hybridWithPerTriangleFallBack reads row iA < nTriB of A: nTriB > nTriA is "
@@ -2215,25 +2311,22 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
   const bool learned = method == DH_BF_LEARNED;
   const bool queued = graph_queued(method, geom, pair_cap);
   if (learned) method = DH_BF;
+  const int tiles = graph_tiles(pair_cap);
+  const unsigned items = static_cast<unsigned>(static_cast<long long>(pair_cap) * tiles);
+  const QueuePlan plan =
+      queued ? queue_plan(items, queue_total(items, contact_cap), learned) : QueuePlan{};
   zero_async(ZeroRegions{{g_scratch.counter.as<unsigned>(), g_scratch.stats.as<unsigned>(),
                           g_scratch.error.as<unsigned>(),
                           queued ? g_scratch.qcounts.as<unsigned>() : nullptr},
-                         {2, 2 * ST_COUNT, 1, kQueueCounts}},
+                         {2, 2 * ST_COUNT, 1, queued ? queue_counts(plan) : 0}},
              st);
-  const int tiles = graph_tiles(pair_cap);
   const bool bf = method == DH_BF;
   DetectArgs a = detect_args(geom, pairs, pair_cap, np_dev, contact_cap, tiles,
                              tiles > 1 ? g_scratch.tiles.as<int>() : counts, bf, pbox, bbox, psph);
-  const unsigned items = static_cast<unsigned>(static_cast<long long>(pair_cap) * tiles);
   // the chunk pre-pass on the geometries detect_prepare found walls in
   if (bf && !queued && pbox && bbox && particle_max_tris(geom, st, false) > kRowBlock)
     a.item_skip = g_scratch.iskip.as<unsigned char>();
-  QueuePlan plan = {};
-  if (queued) {
-    plan = queue_plan(items, 0);
-    if (learned) plan.heavy = 0x7fffffff;
-    queue_bind(a, plan);
-  }
+  if (queued) queue_bind(a, plan);
   switch (method) {
     case DH_BF:
       if (!queued) launch_detect<DH_BF>(items, 0, st, a);
@@ -2246,8 +2339,8 @@ int detect_pairs_graph(int method, const dh_geometry* geom, const int* pairs, in
   }
   if ((rc = pair_offsets(a, counts, offs, st))) return rc;
   if (queued) {
-    hipLaunchKernelGGL(k_queue_write, static_cast<unsigned>(plan.regions), 256, 0, st, a, offs, out,
-                       contact_cap, a.counter, g_scratch.found.as<unsigned long long>(), Report{});
+    hipLaunchKernelGGL(k_queue_write, static_cast<unsigned>(plan.shape.segments()), 256, 0, st, a, offs,
+                       out, contact_cap, a.counter, g_scratch.found.as<unsigned long long>(), Report{});
   } else {
     const long long wg = (contact_cap + 255) / 256;
     hipLaunchKernelGGL(k_scatter, static_cast<unsigned>(wg < 2048 ? wg : 2048), 256, 0, st, a.temp,
@@ -2263,7 +2356,9 @@ int detect_reserve(const dh_geometry* geom, int pair_cap, long long contact_cap,
   int rc;
   if (graph_queued(method, geom, pair_cap)) {
     const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
-    if ((rc = queue_reserve(queue_plan(items, 0), items, method == DH_BF_LEARNED))) return rc;
+    const bool learned = method == DH_BF_LEARNED;
+    const QueuePlan plan = queue_plan(items, queue_total(items, contact_cap), learned);
+    if ((rc = queue_reserve(plan, items, learned))) return rc;
   }
   if ((rc = g_scratch.temp.grow(sizeof(dh_contact) * (contact_cap > 0 ? contact_cap : 1)))) return rc;
   if ((rc = g_scratch.counter.grow(sizeof(unsigned long long)))) return rc;

@@ -390,3 +390,17 @@ extern "C" int hc_pair_ranges(int rows, int cols, int tiles) {
   }
   return at == static_cast<long long>(rows) * cols ? 0 : tiles + 1;
 }
+
+#include "queue_shape.hpp"
+
+// The places of a queue's segments (one of several blocks by its first).
+extern "C" long long hc_queue_places(int rcap, int regions, int block, int blocks,
+                                     long long* place) {
+  const dh::QueueShape q{rcap, regions, block, blocks};
+  for (int r = 0; r < q.segments(); ++r) place[r] = q.place(r);
+  return q.entries();
+}
+
+extern "C" int hc_pool_segment(int rcap, int regions, int block, int blocks, int part, int b) {
+  return dh::QueueShape{rcap, regions, block, blocks}.pool_segment(part, b);
+}

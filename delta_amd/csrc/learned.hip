@@ -15,6 +15,7 @@
 #include "exact_math.hpp"
 #include "mlp.hpp"
 #include "pair_features.hpp"
+#include "queue_shape.hpp"
 #include "runtime.hpp"
 
 #include <vector>
@@ -819,17 +820,17 @@ k_learned(LearnedArgs a) {
 // ------------------------------------------------ the step's survivor queue
 // The triangle pairs that the DEM step's box mid-phase leaves (the survivor
 // queue of detect.hip, entries {item, triangle of A, triangle of B, ..} in
-// regions) through the learned decision: a wave per region at a time, 64
+// segments) through the learned decision: a wave per segment at a time, 64
 // entries in a round.  A finished entry
-// sets flags[e] (its pair emits a contact: d <= epsA + epsB, bf.cpp:125) and,
-// when it emits, its P, Q at pq[6e..6e+6); the rest are listed for the
+// sets flags[flag_stride e] (its pair emits a contact: d <= epsA + epsB,
+// bf.cpp:125) and, when it emits, its P, Q from pq[pq_stride e] on; the rest are listed for the
 // brute force (k_queue_fallback).  Both write exactly what the brute-force
 // queue solve would.
 struct QueueLearnArgs {
   const int4* queue;
   const int* pairs;
   int tiles;  // items per particle pair
-  int regions, rcap;     // region r: rcount[r] entries from r * rcap
+  QueueShape shape;  // segment r: rcount[r] entries from shape.place(r)
   const int* rcount;
   const double* x;
   const double* y;
@@ -837,6 +838,7 @@ struct QueueLearnArgs {
   const double* eps;
   int* flags;
   double* pq;
+  int flag_stride, pq_stride;
   const float* W;
   int* fb_list;
   unsigned* fb_count;
@@ -857,8 +859,8 @@ k_queue_learned(QueueLearnArgs a) {
   stage_network<kModeFeatures>(L, a.W);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   unsigned evals = 0;
-  for (int r = blockIdx.x * kInferWaves + wave; r < a.regions; r += gridDim.x * kInferWaves) {
-    const long long at = static_cast<long long>(r) * a.rcap;
+  for (int r = blockIdx.x * kInferWaves + wave; r < a.shape.segments(); r += gridDim.x * kInferWaves) {
+    const long long at = a.shape.place(r);
     const int live = a.rcount[r];
     for (int base = 0; base < live; base += 64) {
       const long long e = at + base + lane;
@@ -877,9 +879,9 @@ k_queue_learned(QueueLearnArgs a) {
       learned_pair<kModeFeatures>(L, A, B, valid, P, Q, done, evals);
       if (base + lane < live && !(valid && !done)) {
         const bool emit = valid && pq_dist(P, Q) <= margin;
-        a.flags[e] = emit ? 1 : 0;
+        a.flags[a.flag_stride * e] = emit ? 1 : 0;
         if (emit) {
-          double* o = a.pq + 6 * e;
+          double* o = a.pq + a.pq_stride * e;
           o[0] = P.x; o[1] = P.y; o[2] = P.z;
           o[3] = Q.x; o[4] = Q.y; o[5] = Q.z;
         }
@@ -908,9 +910,9 @@ __device__ __forceinline__ void queue_fallback_entry(const QueueLearnArgs& a, lo
   V3<double> P, Q;
   bf_solver(A, B, P, Q);
   const bool emit = pq_dist(P, Q) <= a.eps[pa] + a.eps[pb];
-  a.flags[e] = emit ? 1 : 0;
+  a.flags[a.flag_stride * e] = emit ? 1 : 0;
   if (emit) {
-    double* o = a.pq + 6 * e;
+    double* o = a.pq + a.pq_stride * e;
     o[0] = P.x; o[1] = P.y; o[2] = P.z;
     o[3] = Q.x; o[4] = Q.y; o[5] = Q.z;
   }
@@ -946,20 +948,21 @@ int queue_learned_reserve(long long n) {
 
 // The survivor queue's entries through the learned decision, then the brute
 // force for the rest; a fill instead of a memset (captured steps).
-int queue_learned(const int4* queue, const int* pairs, int tiles, int regions, int rcap,
+int queue_learned(const int4* queue, const int* pairs, int tiles, const QueueShape& shape,
                   const int* rcount, const double* x, const double* y, const double* z,
-                  const double* eps, int* flags, double* pq, hipStream_t st) {
-  const long long n = static_cast<long long>(regions) * rcap;
+                  const double* eps, int* flags, int flag_stride, double* pq, int pq_stride,
+                  hipStream_t st) {
+  const long long n = shape.entries();
   if (!g_learned.model)
     return set_error(DH_ERR_ARG, "DH_BF_LEARNED: no network set (dh_learned_set_model)");
   int rc;
   if ((rc = queue_learned_reserve(n))) return rc;
-  QueueLearnArgs a{queue, pairs, tiles, regions, rcap, rcount, x, y, z, eps,
-                   flags, pq, g_learned.model, g_qlearn.fb_list.as<int>(),
+  QueueLearnArgs a{queue, pairs, tiles, shape, rcount, x, y, z, eps,
+                   flags, pq, flag_stride, pq_stride, g_learned.model, g_qlearn.fb_list.as<int>(),
                    g_qlearn.fb_count.as<unsigned>()};
   fill_async(g_qlearn.fb_count.as<unsigned>(), 0u, 1, st);
   const long long cus = device_cus();
-  long long grid = (regions + kInferWaves - 1) / kInferWaves;
+  long long grid = (shape.segments() + kInferWaves - 1) / kInferWaves;
   if (grid > 4 * cus) grid = 4 * cus;
   hipLaunchKernelGGL(k_queue_learned, static_cast<unsigned>(grid), 64 * kInferWaves, 0, st, a);
   long long fgrid = grid_for(n, 256);

@@ -124,18 +124,17 @@ def test_batched_bf_through_the_survivor_queue(max_tiles, screen):
 @pytest.mark.parametrize("max_tiles", [1, 7])
 @pytest.mark.parametrize("eps", [1e-3, 5e-3, 2e-2, 1e-1])
 def test_survivor_queue_at_its_limits(eps, max_tiles):
-    """Regions below and above the 256 entries that one wave takes and the
-    1,024 they hold, items of more than 160 kept boxes, uneven ones, empty ones
-    and one triangle: with and without deferral the contacts, their order and
-    the counters are the oracle's."""
+    """Segments below and above the 256 entries that one wave takes, items that
+    go on in the pool's blocks, of more than the 2,048 entries that may queue
+    and of more than 160 kept boxes, uneven ones, empty ones and one triangle:
+    the contacts, their order and the counters are the oracle's."""
     from delta_amd import tuning
     parts = [soup(80, 1), soup(80, 2, 0.1), soup(320, 3, 0.5), soup(100, 4, 0.7), soup(8, 5, 0.2),
              soup(1, 6), soup(700, 7, 5.0), soup(64, 8, 4.2)]
     pairs = [(0, 1), (0, 2), (0, 4), (1, 2), (1, 3), (2, 3), (2, 4), (4, 2), (5, 0), (0, 6), (6, 7)]
     tuning.set(detect_queue_min_items=0, detect_max_tiles=max_tiles)
     try:
-        for _ in range(2):  # an eager call sizes the next one's regions
-            _batched_pairs("bf", parts, pairs, eps)
+        _batched_pairs("bf", parts, pairs, eps)
     finally:
         tuning.set(**tuning.default())
 

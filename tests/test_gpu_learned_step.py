@@ -110,3 +110,47 @@ def test_learned_step_graph_equals_eager(network, name):
                                       dg.download(f).view(np.uint64)), (s, f)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("method", [_lib.DH_BF, _lib.DH_BF_LEARNED])
+@pytest.mark.parametrize("captured", [False, True])
+def test_step_with_more_survivors_than_the_queue(network, method, captured):
+    """125 icospheres pushed into one another with hardly a margin: several
+    survivors per contact, more than the queue's segments and pool hold and,
+    for some pairs, than an item may queue.  The states are those of the brute
+    force without the queue, bit for bit."""
+    from delta_amd import shapes, tuning
+    rs, rr = shapes.Rng(21), shapes.Rng(22)
+    at = np.stack(np.meshgrid(*[np.arange(5)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    meshes = [shapes.jittered_icosphere(1, 0.5e-3, 0.1, rs) @ shapes.random_rotation(rr).T
+              + 0.35e-3 * c for c in at]
+    hs = engine.HostScene(meshes, 1e-9, 0, np.arange(len(meshes)), 2500.0, 0)
+    prm = lambda m: engine.step_params(method=m, dt=1e-8, spring=1.0, damper=0.1, friction=0.0,
+                                       cell=hs.cell_size())
+    want, got = engine.DeviceScene(hs), engine.DeviceScene(hs)
+    try:
+        tuning.set(detect_queue_min_items=1 << 30)
+        infos = [engine.step(want, prm(_lib.DH_BF)) for _ in range(3)]
+        tuning.set(detect_queue_min_items=0, detect_max_tiles=1)
+        info = infos[0]
+        held = max(16 * 2 * info.candidate_pairs + 65536, 5 * (info.contacts + 1024) // 2)
+        assert info.triangle_checks - info.pairs_culled > held
+        if captured:
+            g = engine.StepGraph(got, prm(method), pair_cap=info.candidate_pairs + 64,
+                                 contact_cap=info.contacts + 1024)
+            try:
+                for i in infos:
+                    g.launch()
+                    s, overflow = g.status()
+                    assert overflow == 0
+                    assert (s.candidate_pairs, s.contacts) == (i.candidate_pairs, i.contacts)
+            finally:
+                g.close()
+        else:
+            for i in infos:
+                s = engine.step(got, prm(method))
+                assert (s.candidate_pairs, s.contacts) == (i.candidate_pairs, i.contacts)
+    finally:
+        tuning.set(**tuning.default())
+    for f in STATE:
+        assert np.array_equal(want.download(f).view(np.uint64), got.download(f).view(np.uint64)), f

@@ -510,3 +510,20 @@ def test_pair_ranges_of_the_tiles(hc, rows, cols, tiles):
     """The flat tiles take every triangle pair once and in order, on both
     sides of the products that pass 31 and 32 bits."""
     assert hc.hc_pair_ranges(C.c_int(rows), C.c_int(cols), C.c_int(tiles)) == 0
+
+
+@pytest.mark.parametrize("shape", [(1024, 2, 1024, 1), (64, 5, 256, 8), (2048, 4096, 1088, 480)])
+def test_queue_places(hc, shape):
+    """The segments of the survivor queue lie side by side and fill it, and the
+    blocks of a part follow one another."""
+    rcap, regions, block, blocks = shape
+    place = np.zeros(regions + 16 * blocks, np.int64)
+    hc.hc_queue_places.restype = C.c_longlong
+    entries = hc.hc_queue_places(*shape, place.ctypes.data_as(C.c_void_p))
+    size = np.where(np.arange(len(place)) < regions, rcap, block)
+    order = np.argsort(place)
+    assert np.array_equal(place[order], np.concatenate([[0], np.cumsum(size[order])[:-1]]))
+    assert entries == size.sum()
+    for part in range(16):
+        at = [place[hc.hc_pool_segment(*shape, part, b)] for b in range(blocks)]
+        assert np.array_equal(np.diff(at), np.full(blocks - 1, block))
