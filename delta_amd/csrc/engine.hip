@@ -2,6 +2,8 @@
 // order of Engine::iterate (Engine.cpp:155-163): broad phase, narrow phase on
 // the current geometry, contact forces, velocity/angular update, gravity,
 // position, rotation and vertex replicas.
+#include <mutex>
+
 #include "runtime.hpp"
 
 namespace dh {
@@ -157,7 +159,9 @@ __global__ void k_step_status(const long long* __restrict__ np,
 // after earlier work on the null stream, whose entry points (dh_step,
 // dh_detect_pairs, ...) share the library's scratch with the graphs.
 static hipStream_t replay_stream() {
+  static std::mutex mu;
   static hipStream_t s = nullptr;
+  std::lock_guard<std::mutex> lock(mu);
   if (!s && hipStreamCreate(&s) != hipSuccess) s = nullptr;
   return s;
 }
@@ -269,14 +273,21 @@ int dh_step_graph_create(const dh_scene* scene, const dh_step_params* params, in
   if (e == hipSuccess) e = hipMemsetAsync(g->status.ptr, 0, sizeof(long long) * 6, g->stream);
   // what detection learns of the geometry with a read-back, before the capture
   if (e == hipSuccess) detect_prepare(&scene->geom, g->stream);
-  if (e == hipSuccess) e = hipStreamBeginCapture(g->stream, hipStreamCaptureModeRelaxed);
+  if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
+  // The capture has a stream of its own, on which nothing runs: replays that
+  // another thread launches meanwhile would be captured on the library's.
+  hipStream_t capture = nullptr;
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&capture, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipStreamBeginCapture(capture, hipStreamCaptureModeRelaxed);
   if (e != hipSuccess) {
+    if (capture) (void)hipStreamDestroy(capture);
     destroy_graph(g);
     return set_error(DH_ERR_HIP, "step graph capture: %s", hipGetErrorString(e));
   }
-  rc = record_step(g, g->stream);
+  rc = record_step(g, capture);
   hipGraph_t graph = nullptr;
-  e = hipStreamEndCapture(g->stream, &graph);
+  e = hipStreamEndCapture(capture, &graph);
+  (void)hipStreamDestroy(capture);
   g->graph = graph;
   if (rc != DH_OK) {
     destroy_graph(g);

@@ -1,6 +1,7 @@
 """Whole time steps on the GPU (broad phase, narrow phase, forces, fused
 update) against the oracle's step, every state array bit for bit."""
 import copy
+import ctypes as C
 
 import numpy as np
 import pytest
@@ -142,6 +143,87 @@ def _graph_vs_eager(method):
                 assert np.array_equal(a, b), f"step {s}: {f}"
     finally:
         g.close()
+
+
+def _two_graphs():
+    """Graphs of two lattices of different time steps, and their scenes."""
+    hs = engine.c1_scene()
+    scenes = [engine.DeviceScene(hs), engine.DeviceScene(hs)]
+    graphs = [engine.StepGraph(d, engine.step_params(method=_lib.DH_BF, dt=dt, spring=1.0,
+                                                     cell=hs.cell_size()),
+                               pair_cap=1024, contact_cap=1 << 15)
+              for d, dt in zip(scenes, (1e-7, 3e-7))]
+    return scenes, graphs
+
+
+def _states(scenes):
+    return [d.download(f).reshape(-1).view(np.uint64) for d in scenes for f in STATE]
+
+
+def test_replays_on_several_streams_follow_each_other():
+    """Two graphs, which share the library's scratch, launched in turn on the
+    library's stream and on two (blocking) streams of the caller's, with no
+    wait between the launches: the states are those of the same launches on
+    the library's stream alone."""
+    hip = C.CDLL("libamdhip64.so")
+    streams = [C.c_void_p(), C.c_void_p()]
+    for s in streams:
+        assert hip.hipStreamCreate(C.byref(s)) == 0
+    lib, one, two = None, *streams
+    order = [lib, one, two, lib, lib, two, one, one, lib]
+    runs = []
+    for pick in (lambda s: s, lambda s: None):
+        scenes, graphs = _two_graphs()
+        try:
+            for k in range(6 * len(order)):
+                graphs[k % 2].launch(pick(order[k % len(order)]))
+            _lib.check(_lib.lib().dh_synchronize(), "sync")
+            assert all(g.status()[1] == 0 for g in graphs)
+            runs.append(_states(scenes))
+        finally:
+            for g in graphs:
+                g.close()
+    for s in streams:
+        assert hip.hipStreamDestroy(s) == 0
+    assert all(np.array_equal(a, b) for a, b in zip(*runs))
+
+
+def test_graph_created_while_another_replays():
+    """A thread replays a graph while this one creates others: each is captured
+    by itself, and the replays are those of a run on their own."""
+    import threading
+    runs = []
+    for busy in (False, True):
+        scenes, graphs = _two_graphs()
+        failed = []
+
+        def replay():
+            try:
+                for _ in range(300):
+                    graphs[0].launch()
+            except Exception as e:  # shown by the assertion below
+                failed.append(e)
+
+        t = threading.Thread(target=replay)
+        t.start()
+        try:
+            if busy:
+                while t.is_alive():
+                    for g in _two_graphs()[1]:
+                        g.close()
+        finally:
+            t.join()
+        assert not failed
+        try:
+            for _ in range(3):
+                graphs[1].launch()
+            _lib.check(_lib.lib().dh_synchronize(), "sync")
+            assert all(g.status()[1] == 0 for g in graphs)
+            runs.append(_states(scenes))
+        finally:
+            for g in graphs:
+                g.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*runs))
 
 
 def test_step_graph_reports_overflow():

@@ -2,8 +2,9 @@
 contacts, bit for bit against the oracle's per-pair sums added in ascending
 partner order.  The lists cross the sizes where the device code changes its
 split: pairs with none, one, a wave's worth and several waves of contacts,
-short and long pair lists, few and many particles, offsets past the contact
-capacity."""
+short and long pair lists, few and many particles.  (What a captured step adds
+up after it ran out of contact capacity is not defined, only that it stays
+within its buffers: tests of the step graph.)"""
 import ctypes as C
 import types
 
