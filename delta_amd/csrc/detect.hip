@@ -2388,9 +2388,9 @@ const unsigned long long* detect_counter_dev(int method, const dh_geometry* geom
 const int* detect_error_dev() { return g_scratch.error.as<int>(); }
 const unsigned long long* detect_stats_dev() { return g_scratch.stats.as<unsigned long long>(); }
 
-// Contacts of a host call that come back through pinned memory (65,536 of them
-// take 9.4 MB); more are copied.
-constexpr size_t kPinnedContactBytes = 16u << 20;
+// Particles and contacts of a host call that go through pinned memory, which is
+// kept (65,536 contacts take 9.4 MB, 233,000 triangles 16); more are copied.
+constexpr size_t kPinnedBytes = 16u << 20;
 
 __global__ __launch_bounds__(256) void k_fetch(const double* __restrict__ src,
                                                double* __restrict__ dst, long long n) {
@@ -2469,10 +2469,10 @@ int dh_detect_pair(int method, const double* xA, const double* yA, const double*
                      "hybridWithPerTriangleFallBack reads row iA < nTriB of A: nTriB > nTriA is "
                      "out of bounds in the reference (hybrid.cpp:130)");
   if (nTriA == 0 || nTriB == 0) return DH_OK;
-  // The two particles go to the device in one block, staged in pinned memory
-  // and fetched from there by a kernel, and the contacts come back into pinned
-  // memory, written by the kernel that orders them: one wait per call (seven
-  // copies in and one out cost 170 of the 205 us of a 20 x 20 call).
+  // The two particles go to the device in one block, up to kPinnedBytes staged
+  // in pinned memory and fetched from there by a kernel, and the contacts come
+  // back into pinned memory, written by the kernel that orders them: one wait per
+  // call (seven copies in and one out cost 170 of the 205 us of a 20 x 20 call).
   struct Meta {
     double eps[2];
     int off[3];
@@ -2487,20 +2487,32 @@ int dh_detect_pair(int method, const double* xA, const double* yA, const double*
   const size_t na = 3 * static_cast<size_t>(nTriA), nb = 3 * static_cast<size_t>(nTriB);
   const size_t nv = na + nb, block = sizeof(Meta) + 3 * nv * sizeof(double);
   if ((rc = geo.grow(block))) return rc;
-  if ((rc = stage.grow(block))) return rc;
   const Meta m = {{epsA, epsB},   {0, nTriA, nTriA + nTriB}, {frictionA ? 1 : 0, frictionB ? 1 : 0},
                   {idA, idB},     {0, 1},                    {0, 0, 0}};
-  std::memcpy(stage.ptr, &m, sizeof(m));
-  double* v = reinterpret_cast<double*>(static_cast<char*>(stage.ptr) + sizeof(Meta));
   const double* axes[3][2] = {{xA, xB}, {yA, yB}, {zA, zB}};
+  const bool staged = block <= kPinnedBytes;
+  if (staged && (rc = stage.grow(block))) return rc;
+  char* to = staged ? static_cast<char*>(stage.ptr) : geo.as<char>();
+  // to the pinned block, or to the device (which waits for earlier calls' work)
+  auto put = [&](size_t at, const void* from, size_t bytes) -> int {
+    if (staged)
+      std::memcpy(to + at, from, bytes);
+    else
+      DH_HIP_CHECK(hipMemcpy(to + at, from, bytes, hipMemcpyHostToDevice));
+    return DH_OK;
+  };
+  if ((rc = put(0, &m, sizeof(m)))) return rc;
   for (int q = 0; q < 3; ++q) {
-    std::memcpy(v + q * nv, axes[q][0], na * sizeof(double));
-    std::memcpy(v + q * nv + na, axes[q][1], nb * sizeof(double));
+    const size_t at = sizeof(Meta) + q * nv * sizeof(double);
+    if ((rc = put(at, axes[q][0], na * sizeof(double)))) return rc;
+    if ((rc = put(at + na * sizeof(double), axes[q][1], nb * sizeof(double)))) return rc;
   }
-  const long long words = static_cast<long long>(block / 8);
-  hipLaunchKernelGGL(k_fetch, grid_for(words, 256) < 256 ? grid_for(words, 256) : 256, 256, 0,
-                     nullptr, static_cast<const double*>(stage.ptr), geo.as<double>(), words);
-  DH_HIP_CHECK(hipGetLastError());
+  if (staged) {
+    const long long words = static_cast<long long>(block / 8);
+    hipLaunchKernelGGL(k_fetch, grid_for(words, 256) < 256 ? grid_for(words, 256) : 256, 256, 0,
+                       nullptr, static_cast<const double*>(stage.ptr), geo.as<double>(), words);
+    DH_HIP_CHECK(hipGetLastError());
+  }
   const Meta* dm = geo.as<Meta>();
   dh_geometry g;
   g.x = reinterpret_cast<double*>(geo.as<char>() + sizeof(Meta));
@@ -2514,7 +2526,7 @@ int dh_detect_pair(int method, const double* xA, const double* yA, const double*
   g.ntri_total = nTriA + nTriB;
   const long long dcap = cap > 0 ? cap : 1;
   const size_t out_bytes = sizeof(dh_contact) * dcap;
-  const bool direct = out_bytes <= kPinnedContactBytes;
+  const bool direct = out_bytes <= kPinnedBytes;
   if ((rc = direct ? pinned_out.grow(out_bytes) : outbuf.grow(out_bytes))) return rc;
   dh_contact* dev_out = direct ? static_cast<dh_contact*>(pinned_out.ptr) : outbuf.as<dh_contact>();
   // Tiles of 256 triangle pairs, one per thread, where each is solved, and of

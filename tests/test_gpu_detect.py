@@ -67,17 +67,17 @@ def soup(n, seed, shift=0.0):
     return t
 
 
-@pytest.mark.parametrize("method", ["bf", "penalty", "hybrid_batch", "hybrid_triangle",
-                                    "hybrid_batch_stat"])
-@pytest.mark.parametrize("na,nb,eps", [(1, 1, 0.2), (16, 16, 0.1), (17, 15, 0.1),
-                                       (321, 79, 1e-3), (321, 79, 1e-5),
-                                       (1100, 1000, 1e-3), (1100, 1000, 1e-5)])
+TILE_SIZES = [(1, 1, 0.2), (16, 16, 0.1), (17, 15, 0.1), (321, 79, 1e-3), (321, 79, 1e-5)]
+NOTED_SIZES = [(1100, 1000, 1e-3), (1100, 1000, 1e-5)]  # the notes are the hybrids'
+
+
+@pytest.mark.parametrize("method,na,nb,eps", [
+    (m, *size) for m in ("bf", "penalty", "hybrid_batch", "hybrid_triangle", "hybrid_batch_stat")
+    for size in TILE_SIZES + (NOTED_SIZES if m in ("hybrid_batch", "hybrid_triangle") else [])])
 def test_tiles_of_one_pair_match_oracle(method, na, nb, eps):
     """Partial tiles, rows over several workgroups, and (1,100 x 1,000) tiles
     of more pairs than a hybrid tile notes; at 1e-5 most rows fall back, at
     the larger margins none."""
-    if na * nb > 1 << 20 and method not in ("hybrid_batch", "hybrid_triangle"):
-        pytest.skip("the notes are the hybrids'")
     A, B = soup(na, 3), soup(nb, 4, 0.4)
     fn, code = METHODS[method]
     contact.reset_all_statistics()
@@ -253,3 +253,17 @@ def test_penalty_over_more_pairs_than_32_bits_number(n):
         want.append(w)
     same_contacts(got, np.concatenate(want))
     assert set(range(0, n, 4001)) <= set(got["triB"].tolist())
+
+
+@pytest.mark.parametrize("n", [233015, 233016])
+def test_largest_particles_through_pinned_memory(n):
+    """The last pair of particles that is staged in pinned memory (16 MiB with
+    its header) and the first that is copied: the oracle's contacts, and a
+    small call after them."""
+    A, _ = _facing_lines(n)
+    B = A[n // 2:n // 2 + 1] + np.array([0.0, 5e-5, 0.0])
+    for a in (A, A[n // 2 - 3:n // 2 + 3]):
+        got = contact.bf(*shapes.to_soa(a), len(a), EPS, True, 7, *shapes.to_soa(B), 1, EPS, True, 9)
+        rc, want, _ = ol.or_detect(_lib.DH_BF, a, B, EPS, EPS, 1, 1, 7, 9)
+        assert rc == 0 and len(want) > 0
+        same_contacts(got, want)
