@@ -2141,18 +2141,6 @@ static int pair_offsets(const DetectArgs& a, int* counts, long long* offs, hipSt
                           g_scratch.sums.as<long long>(), st);
 }
 
-// Items as detect_queue_min_items counts them: one for every 16 triangles of
-// the mean particle.  The queue's launches and their chain of dependent loads
-// cost some 40 us; without it each item is a workgroup's, which the larger
-// particles make the costlier (captured steps with and without the queue: 36
-// pairs of 80 triangles 92 and 83 us, 484 pairs 113 and 124, 2,500 pairs 134
-// and 169, 33,000 pairs 235 and 612).
-static long long queue_items(long long items, const dh_geometry* geom) {
-  const long long per = geom->nparticles > 0
-                            ? static_cast<long long>(geom->ntri_total) / geom->nparticles / 16 : 0;
-  return per > 1 ? items * per : items;
-}
-
 // At least min_tiles tiles per pair.
 static int detect_pairs_tiled(int method, const dh_geometry* geom, const int* pairs, int npairs,
                               int min_tiles, dh_contact* out, long long cap, long long* n_total,
@@ -2189,7 +2177,8 @@ static int detect_pairs_tiled(int method, const dh_geometry* geom, const int* pa
   // the queue costs launches: for many items only
   const bool queued =
       bf && (learned || queue_items(static_cast<long long>(npairs) * tiles_for(npairs, method),
-                                    geom) >= tuning().detect_queue_min_items);
+                                    geom->ntri_total, geom->nparticles) >=
+                            tuning().detect_queue_min_items);
   QueuePlan plan = {};
   if (queued) {
     // a shorter queue where the memory does not allow this one
@@ -2295,7 +2284,8 @@ static int graph_tiles(int pair_cap) { return tiles_for(pair_cap / 2 > 0 ? pair_
 static bool graph_queued(int method, const dh_geometry* geom, int pair_cap) {
   const long long items = static_cast<long long>(pair_cap) * graph_tiles(pair_cap);
   return method == DH_BF_LEARNED ||
-         (method == DH_BF && queue_items(items, geom) >= tuning().detect_queue_min_items);
+         (method == DH_BF && queue_items(items, geom->ntri_total, geom->nparticles) >=
+                                 tuning().detect_queue_min_items);
 }
 
 // Detection for a captured step: launches for `pair_cap` pairs of which

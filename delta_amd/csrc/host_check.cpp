@@ -404,3 +404,7 @@ extern "C" long long hc_queue_places(int rcap, int regions, int block, int block
 extern "C" int hc_pool_segment(int rcap, int regions, int block, int blocks, int part, int b) {
   return dh::QueueShape{rcap, regions, block, blocks}.pool_segment(part, b);
 }
+
+extern "C" long long hc_queue_items(long long items, int ntri, int nparticles) {
+  return dh::queue_items(items, ntri, nparticles);
+}

@@ -1,9 +1,21 @@
-// queue_shape.hpp — the places of the survivor queue's entries (detect.hip,
-// learned.hip; the host build lets CPU tests check them).
+// queue_shape.hpp — when the survivor queue is taken, and the places of its
+// entries (detect.hip, learned.hip; the host build lets CPU tests check them).
 #pragma once
 #include "exact_math.hpp"
 
 namespace dh {
+
+// Items as detect_queue_min_items counts them: one for every 16 triangles of
+// the mean particle.  The queue's launches and their chain of dependent loads
+// cost some 40 us; without it each item is a workgroup's, which the larger
+// particles make the costlier (captured steps with and without the queue: 36
+// pairs of 80 triangles 92 and 83 us, 484 pairs 113 and 124, 2,500 pairs 134
+// and 169, 33,000 pairs 235 and 612).  Never 2^30, the setting for no queue.
+DH_HD long long queue_items(long long items, int ntri, int nparticles) {
+  const long long per = nparticles > 0 ? static_cast<long long>(ntri) / nparticles / 16 : 0;
+  const long long n = per > 1 ? items * per : items;
+  return n < 1ll << 30 ? n : (1ll << 30) - 1;
+}
 
 // Parts of the pool, each with a counter of its own: a wave starts with the part
 // of its workgroup's number and goes on to the next when that is used up.

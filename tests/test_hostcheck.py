@@ -527,3 +527,13 @@ def test_queue_places(hc, shape):
     for part in range(16):
         at = [place[hc.hc_pool_segment(*shape, part, b)] for b in range(blocks)]
         assert np.array_equal(np.diff(at), np.full(blocks - 1, block))
+
+
+@pytest.mark.parametrize("items,ntri,n,want", [
+    (100, 80 * 65, 65, 500), (100, 31 * 65, 65, 100), (0, 0, 0, 0), (7, 5, 0, 7),
+    (10 ** 6, 2 * 10 ** 9, 100000, (1 << 30) - 1), (1 << 31, 80, 1, (1 << 30) - 1)])
+def test_queue_items(hc, items, ntri, n, want):
+    """Weighted by 16 triangles of the mean particle, and below the 2^30 that
+    turns the queue off whatever the particles' sizes."""
+    hc.hc_queue_items.restype = C.c_longlong
+    assert hc.hc_queue_items(C.c_longlong(items), C.c_int(ntri), C.c_int(n)) == want
