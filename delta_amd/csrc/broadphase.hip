@@ -360,11 +360,6 @@ constexpr int kBpWaves = 4;    // particles per workgroup
 constexpr int kBpList = 512;   // partners sorted in LDS per particle (else a serial sort)
 constexpr int kBpKeep = 64;    // partners kept by the count pass per particle (one per lane)
 
-__device__ __forceinline__ int bp_lane_prefix(unsigned long long mask) {
-  return __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
-                                   __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0));
-}
-
 // The partners j > i of a particle i that is not large, by L = 32 or 64 lanes
 // of a wave (`active`: they have one): calls put(position, j) on the finding
 // lane for every partner, positions 0.. in discovery order; returns their
@@ -469,7 +464,7 @@ __device__ __forceinline__ int large_chunk(const GridArgs& g, int i, int c, int*
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const unsigned long long mask = __ballot(e[q]);
-      if (e[q]) put(at + bp_lane_prefix(mask), j0 + 256 * w + 64 * q + lane);
+      if (e[q]) put(at + lane_prefix(mask), j0 + 256 * w + 64 * q + lane);
       at += __popcll(mask);
     }
     __syncthreads();  // the next round overwrites the counts
@@ -684,7 +679,7 @@ __global__ __launch_bounds__(1024) void k_small_pairs(const Aabb* __restrict__ b
       const int j = j0 + lane;
       const bool e = j < n && !(oi && s_obst[j]) && overlap(bi, s_box[j]);
       const unsigned long long mask = __ballot(e);
-      const long long q = s0 + found + bp_lane_prefix(mask);
+      const long long q = s0 + found + lane_prefix(mask);
       if (e && q < cap) {
         pairs[2 * q] = i;
         pairs[2 * q + 1] = j;
@@ -716,7 +711,7 @@ __global__ __launch_bounds__(256) void k_all_pairs(const Aabb* __restrict__ box,
     const int j = j0 + lane;
     const bool e = j < n && !(oi && obstacle[j]) && overlap(bi, box[j]);
     const unsigned long long mask = __ballot(e);
-    const long long q = s0 + found + bp_lane_prefix(mask);
+    const long long q = s0 + found + lane_prefix(mask);
     if (kFill && e && q < cap) {
       pairs[2 * q] = i;
       pairs[2 * q + 1] = j;
@@ -738,7 +733,8 @@ struct BpScratch {
 };
 static BpScratch g_bp;
 
-// Candidates per large-particle chunk: 1024 (one round of a workgroup), more for very large n so that a particle has at most 256 chunks.
+// Candidates per large-particle chunk: 1024 (one round of a workgroup), more
+// for very large n so that a particle has at most 256 chunks.
 static int large_chunk_len(int n) {
   int c = 1024;
   while (static_cast<long long>(c) * 256 < n) c *= 2;

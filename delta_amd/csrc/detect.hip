@@ -192,12 +192,6 @@ __device__ __forceinline__ bool boxes_apart(const Tri<double>& A, const Tri<doub
   return boxes_apart(a, a + 3, b, b + 3, margin);
 }
 
-// Lanes below this one whose predicate is set (wave64).
-__device__ __forceinline__ int lane_prefix(unsigned long long mask) {
-  return __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
-                                   __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0));
-}
-
 struct Pair {
   int pa, pb, oA, oB, nA, nB;
   double epsA, epsB, margin, max_err;
@@ -935,13 +929,6 @@ __global__ __launch_bounds__(1024) void k_lane_cull(DetectArgs g, int items) {
   }
   __syncthreads();
   if (listed) g.wlist[base + wave_cnt[wave] + lane_prefix(m)] = it;
-}
-
-// Orders a wave's LDS writes before its later reads of other lanes' values.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // The largest gap between two boxes along an axis.

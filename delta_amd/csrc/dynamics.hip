@@ -37,13 +37,6 @@ __device__ __forceinline__ void load3(const double* p, int i, double v[3]) {
   v[2] = p[3 * i + 2];
 }
 
-// Orders the wave's LDS writes before its later reads of other lanes' rows.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // np_dev (may be null): the live pair count when npairs is a capacity.
 __device__ __forceinline__ bool past_pairs(int p, int npairs, const long long* np_dev) {
   return p >= npairs || (np_dev && p >= *np_dev);
@@ -89,11 +82,16 @@ constexpr int kForcesFewPairs = 131072;
 // contacts in one lane, one after the other, left a funnel of 3,900 pairs and
 // 17,000 contacts at 300 us and a lattice of 484 pairs and 14,000 contacts at
 // 120 us: a serial chain of scattered loads, square roots and divisions.
-// G = 4 spreads a short list over the GPU (lattice 13.5 us, G = 16 31 us; the
-// funnel's 15,700 pairs 22 against 51 us); with more than kForcesFewPairs pairs
-// there are waves enough, and G = 16 fills more of a wave's lanes where most pairs
-// carry no contact (hopper of 1.9e5 pairs 52 us, G = 4 75 us; G = 64 71 us:
-// its waves meet up to ten rounds of 64 contacts one after the other).
+// G = 4 spreads a short list over the GPU, and a list whose pairs carry many
+// contacts or uneven numbers of them; G = 16 fills more of a wave's lanes
+// where most pairs carry few.  us with G = 4 and 16, by the list's length: lattice, 484
+// pairs, 13.5 and 31; packings (23 contacts a pair), 5,100, 30,800 and 94,000,
+// 17 and 38, 32 and 51, 90 and 129; funnel, 31,500, 21 and 51; drums, 43,000 and
+// 129,000, 10 and 19, 13 and 18; hoppers (3 contacts a pair), 65,000, 118,000,
+// 194,000 and 260,000, 14 and 12, 22 and 16, 32 and 20, 43 and 27.  The number of contacts is not known here, so the line
+// lies where the hoppers' loss passes the others' gain (a captured step's
+// length is its capacity).  G = 64 in the largest hopper: 71 us, G = 16 52, its
+// waves meet up to ten rounds of 64 contacts one after the other.
 template <int G>
 __global__ __launch_bounds__(256) void k_pair_forces(BodiesDev b, const int* __restrict__ pairs,
                                                      int npairs,
@@ -422,8 +420,8 @@ __global__ __launch_bounds__(256) void k_particle_sum_wide(const int* __restrict
   }
 }
 
-// Particles, pairs and contact capacity for which k_forces_small does the
-// force stage in one workgroup.
+// Up to this many particles k_forces_small sums the pairs' forces, in one
+// workgroup (any number of pairs and contacts).
 constexpr int kForcesSmallN = 1024;
 
 // The force stage of a small scene (at most kForcesSmallN particles) after

@@ -293,13 +293,17 @@ DH_HD void bf_features(const Tri<T>& A, const Tri<T>& B, BfBest<T>& best) {
 // whose determinant is in (0, 1e-60), and no feature's distance in (0, 2^-350).
 // Coordinates that are NaN are regular: as in the general form, the distance
 // of each feature that they are part of is NaN, which is never the least.
-// MI355X, 2^24 pairs: 2,807 to about 2,170 vector instructions per wave of 64
-// pairs, 1.467 to 1.198 ms.  A wave leaves as soon as one of its lanes has too
+// MI355X, 2^24 pairs: 2,807 to 2,185 vector instructions per wave of 64 pairs,
+// 1.39 to 1.17 ms.  A wave leaves as soon as one of its lanes has too
 // short or too long an edge: with two such pairs in 100, 2^20 pairs took 148
 // us where the others went on, 102 by the general form alone.
 
 // a / b, correctly rounded, for 2^-400 < |a|, |b| < 2^400 (other operands: any
-// value): the reciprocal by two Newton steps, the quotient by one residual.
+// value): the reciprocal by two Newton steps, then Markstein's final step (the
+// quotient's residual, exact in a fused multiply-add, times the reciprocal),
+// which rounds correctly where the reciprocal is good to half a unit or so
+// (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990).  The GPU tests compare it with the host's division.
 DH_HD double div_regular(double a, double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double y = __builtin_amdgcn_rcp(b);
@@ -348,9 +352,10 @@ DH_HD int least_exponent(int e, double a) {
 constexpr double kSqrtLeast = 0x1p-349;
 
 // sqrt(x), correctly rounded, for x >= 2^-700 and x = 0, by Goldschmidt's
-// iteration and two residual corrections.  Between them the value is positive
-// and below kSqrtLeast: the estimate y of 1 / sqrt(2^-700) gives g = x * y in
-// (0, 2^-350), and every correction adds a factor of 1 to 1.5.
+// iteration and two residual corrections (Markstein, as above).  Between 0 and
+// 2^-700 the value is positive and below kSqrtLeast: the estimate y of
+// 1 / sqrt(2^-700) gives g = x * y in (0, 2^-350), and every correction adds a
+// factor of 1 to 1.5.
 DH_HD double sqrt_regular(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const double y = __builtin_amdgcn_rsq(fmax(x, 0x1p-700));
@@ -728,11 +733,6 @@ DH_HD bool plane_apart(const Tri<double>& A, const Tri<double>& B, double margin
   return plane_side_apart(A, B, thr) || plane_side_apart(B, A, thr);
 }
 
-// plane_apart, then the edge-pair axes (for the pairs the planes leave).
-DH_HD bool axes_apart(const Tri<double>& A, const Tri<double>& B, double margin) {
-  return plane_apart(A, B, margin) || edge_axes_apart(A, B, axis_reach(A, B, margin));
-}
-
 // Screen before bfSolver in binary64: true when A and B are provably farther
 // apart than the contact margin (no contact, bf.cpp:125).  bfSolver in
 // binary32 (coordinates relative to A's first vertex) gives a direction n =
@@ -871,9 +871,9 @@ struct Penalty {
 
   // step() on a regular pair: the same sums, with the penalty terms selected
   // instead of multiplied by 0, 1 or -1, and one reciprocal per pivot for its
-  // quotients (238 vector instructions a step for 333, the divisions' half of
-  // them; the penalty over 363 pairs of 80 x 80 triangles 153 -> 130 us, with
-  // its vector units busy 9 cycles in 10).  The quotients are correctly rounded, as
+  // quotients (238 vector instructions a step for 333 in the assembly; a pair's
+  // four steps and the rest are 1,201 per wave of 64; the penalty over 363 pairs
+  // of 80 x 80 triangles 153 -> 130 us).  The quotients are correctly rounded, as
   // division is, where no pivot is below 2^-10 of the trace, every non-zero
   // numerator is at least 2^-600 (`low` is the least binary exponent seen) and
   // the new x stays within 2^20, which with regular() keeps everything finite;

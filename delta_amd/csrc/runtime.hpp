@@ -58,6 +58,19 @@ inline unsigned grid_for(int64_t n, int block) {
   return static_cast<unsigned>((n + block - 1) / block);
 }
 
+// Lanes below this one whose bit of `mask` is set (wave64).
+__device__ __forceinline__ int lane_prefix(unsigned long long mask) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0));
+}
+
+// Orders a wave's LDS writes before its later reads of other lanes' values.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // p[0..n) = v.  Used instead of hipMemsetAsync in work that may be captured
 // into a HIP graph.
 template <typename T>
