@@ -962,6 +962,8 @@ __device__ __forceinline__ double box_gap(const double* loA, const double* hiA, 
 __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectArgs g) {
   __shared__ double boxes[kWavesPerGroup][kWaveBoxes * 6];
   __shared__ unsigned short act[kWavesPerGroup][kWaveBoxes];
+  // of at most kWaveBoxes / 2 rows by as many columns
+  __shared__ unsigned long long rounds[kWavesPerGroup][kWaveBoxes * kWaveBoxes / 256 + 1];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   double* bx = boxes[w];
@@ -1099,10 +1101,9 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
     const int nc = kept - na, tested = na * nc;
     wave_lds_fence();
     // Survivors in row-major order over the kept rows and columns, 64 pairs a
-    // round (at most 100): put() writes a round's.  Lane l keeps the survivors
-    // of rounds l and 64 + l for an item that turns out not to fit and is
-    // written again, to blocks of the pool that hold it.
-    unsigned long long rounds[2] = {0, 0};
+    // round: put() writes a round's.  The rounds' survivors are kept for an item
+    // that turns out not to fit and is written again, to blocks of the pool that
+    // hold it.
     const int step_r = nc > 0 ? 64 / nc : 0, step_c = 64 - step_r * nc;
     int ra = nc > 0 ? lane / nc : 0, cb = lane - ra * nc;
     auto put = [&](unsigned long long m, int at) {
@@ -1130,7 +1131,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
           keep = !(box_gap(a, a + 3, b, b + 3) > reach);
         }
         const unsigned long long m = __ballot(keep);
-        if (lane == (k & 63)) rounds[k >> 6] = m;
+        if (lane == 0) rounds[w][k] = m;
         put(m, used + S);
         S += __popcll(m);
       }
@@ -1160,9 +1161,9 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, 4) void k_detect_wave(DetectAr
         used = 0;
         ra = lane / nc;
         cb = lane - ra * nc;
+        wave_lds_fence();
         for (int k = 0, at = 0; 64 * k < tested; ++k) {
-          const unsigned long long mine = k < 64 ? rounds[0] : rounds[1];
-          const unsigned long long m = __shfl(mine, k & 63);
+          const unsigned long long m = rounds[w][k];
           put(m, at);
           at += __popcll(m);
         }
@@ -1678,17 +1679,20 @@ __global__ __launch_bounds__(256, 3) void k_queue_solve(DetectArgs g) {
   };
   for (int i0 = 0; i0 < most; i0 += 64) {  // 64 of them at a time
     unsigned long long light, heavy;       // the wave's; the same in all waves
+    int known = 0;  // entries of the first, 0 afterwards (read again)
     {
       const int entries = count(i0 + lane);
       light = __ballot(entries > 0 && entries <= g.heavy && (lane & 3) == w);
       heavy = __ballot(entries > g.heavy);
+      if (light) known = __builtin_amdgcn_readlane(entries, __builtin_ctzll(light));
     }
     while (light | heavy) {
       const bool shared = light == 0;
       const int l = __builtin_ctzll(shared ? heavy : light);
       if (shared) heavy &= heavy - 1;
       else light &= light - 1;
-      const int r = number(i0 + l), total = g.rcount[r];
+      const int r = number(i0 + l), total = known ? known : g.rcount[r];
+      known = 0;
       int begin = 0, n = total;
       if (shared) {
         const int part = segment_part(total);
@@ -1972,14 +1976,15 @@ static long long queue_total(long long items, long long cap) {
   return n < 1ll << 28 ? n : 1ll << 28;
 }
 
-// The queue's shape: half of the entries, and at least 1,024 each, are the
-// waves' own segments (as many waves as the CUs hold at once; 335 MB), the
-// other half the pool.  (Own segments of 512 or 256 entries with the pool for
-// the rest: funnel fill's step 2 and 3 % slower, as a wave whose items go on in
-// the pool waits for it.)  With fewer than 16 items per wave, segments with more
-// than 256 entries are shared by four waves in k_queue_solve; with more, the
-// segments are alike.  An item may queue up to 2,048 entries, 1,024 where one
-// wave alone takes a segment through the learned decision.
+// The queue's shape: half of the entries are the waves' own segments (as many
+// waves as the CUs hold at once), of at least 1,024 each (335 MB), the other
+// half the pool; with 16 items per wave and more, which makes the segments
+// alike, three quarters and one.  (Own segments of 512 or 256 entries: funnel
+// fill's step 2 and 3 % slower, as a wave whose items go on in the pool waits
+// for it.)  Of segments that are not alike, those with more than 256 entries are
+// shared by four waves in k_queue_solve.  An item may queue up to 2,048 entries,
+// 1,024 where one wave alone takes a segment through the learned decision
+// (1,024 always: captured packing of 512 at half its pitch 977 us, 931 so).
 struct QueuePlan {
   unsigned groups;
   QueueShape shape;
@@ -1992,13 +1997,15 @@ static QueuePlan queue_plan(long long items, long long total, bool learned) {
   const long long waves = static_cast<long long>(device_cus()) * 8;
   q.groups = static_cast<unsigned>(wg < 1 ? 1 : (wg < waves ? wg : waves));
   q.shape.regions = static_cast<int>(q.groups) * kWavesPerGroup;
-  const long long half = total / 2, own = half / q.shape.regions / 64 * 64;
+  const bool alike = items >= 16ll * q.shape.regions;
+  const long long pool = alike ? total / 4 : total / 2;
+  const long long own = (total - pool) / q.shape.regions / 64 * 64;
   q.shape.rcap = static_cast<int>(own < 1024 ? 1024 : own);
-  const long long block = (half / 8192 + 63) / 64 * 64;
+  const long long block = (pool / 8192 + 63) / 64 * 64;
   q.shape.block = static_cast<int>(block < 1024 ? 1024 : block);
-  const long long blocks = half / q.shape.block / kPoolParts;
+  const long long blocks = pool / q.shape.block / kPoolParts;
   q.shape.blocks = static_cast<int>(blocks < 1 ? 1 : blocks);
-  q.heavy = !learned && items < 16ll * q.shape.regions ? 256 : 0x7fffffff;
+  q.heavy = learned || alike ? 0x7fffffff : 256;
   q.most = learned ? 1024 : 2048;
   return q;
 }
